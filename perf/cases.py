@@ -281,17 +281,19 @@ class _Arena:
                 group_size=r["query"].shape[0] // r["to_graph"].numel(), aggregation=runtime.config.aggregation,
                 query_heads=r["query"].shape[0], kv_heads=r["key"].shape[1]))
         self.tail = torch.cat(tails)
-        whole = [self.sizes]
-        for layer in self.layers:
-            m = layer.converted.mutable
-            whole += [m.community_counts, layer.converted.current_position, *m.deltas.tensors()]
-        self.groups = [([self.centroids], [self.centroids.clone()]), (whole, [t.clone() for t in whole]),
-                       ([self.weight, self.total], [self.weight.clone(), self.total.clone()])]
+        small = []
+        for layer in self.layers:  # (a community's chunks are unreachable once its head and tail are unset)
+            m, d = layer.converted.mutable, layer.converted.mutable.deltas
+            small += [m.community_counts, layer.converted.current_position, d.community_head, d.community_tail,
+                      d.community_sizes, d.next_free_chunk, d.next_free_position]
+        self.small = small, [t.clone() for t in small]
+        self.large = [(t, t.clone()) for t in (self.centroids, self.sizes, self.weight, self.total)]
 
     def restore(self):
         self.tokens.index_fill_(0, self.tail, -1)
-        for live, kept in self.groups:
-            torch._foreach_copy_(live, kept)
+        torch._foreach_copy_(*self.small)
+        for live, kept in self.large:
+            live.copy_(kept)
 
     def outputs(self):
         return dict(centroids=self.centroids.view(torch.float8_e4m3fn), sizes=self.sizes, weight=self.weight,

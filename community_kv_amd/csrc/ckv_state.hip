@@ -14,16 +14,18 @@
 // not fixed.
 //
 // Launch sequence of ckv_build_layer_state (one stream):
-//   chunk_hist_kernel     per (graph, position chunk): community histogram
-//   csr_scan_kernel       per graph: CSR offsets, each chunk's first slot per
-//                         community, and the table of 64-member blocks
+//   state_prep_kernel     per (graph, position chunk): community histogram; in further
+//                         workgroups labels -> token_communities (-1 past the prompt)
+//                         and the modularity weights cleared
+//   chunk_scan_kernel     per (graph, community): its members in newer chunks, its total
+//   csr_scan_kernel       per graph: CSR offsets and the table of 64-member blocks
 //   csr_scatter_kernel    per (graph, chunk): member positions, newest first
-//   block_sum_kernel      per (retrieval head, block): in-order key sum of 64 members
-//   centroid_kernel       per (retrieval head, community): block sums in order,
-//                         mean -> clamp -> E4M3 / f32
-//   token_table_kernel    labels -> token_communities (-1 past the prompt)
-//   weight_zero_kernel + edge_weight_kernel   modularity weights from an edge list, or
-//   weight_zero_kernel + topk_weight_kernel   the same weights from the prefill top-k edges
+//   block_sum_kernel      per (retrieval head, block): in-order key sum of 64 members; the
+//                         centroid of a community of one block
+//   centroid_kernel       per (retrieval head, community of several blocks or none): block
+//                         sums in order, mean -> clamp -> E4M3 / f32
+//   edge_weight_kernel    modularity weights from an edge list, or
+//   topk_weight_kernel    the same weights from the prefill top-k edges
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -94,16 +96,24 @@ inline size_t state_ws_words(int graphs, int heads, int seq_len, int num_sink, i
 }
 
 // community_counts[g] = 1 + the largest label of a non-sink position, 0 when
-// there is none, -1 when a non-sink label is negative.
+// there is none, -1 when a non-sink label is negative.  One workgroup per
+// graph, bound by load latency: eight loads of a thread are in flight together
+// (32,768 positions: 10.8 us with one, 4.4 us with eight).
 __global__ __launch_bounds__(COUNT_THREADS) void label_count_kernel(const int32_t* __restrict__ labels, int seq_len,
                                                                     int num_sink, int32_t* __restrict__ counts) {
+  constexpr int U = 8;
   const int g = blockIdx.x;
   const int32_t* row = labels + (int64_t)g * seq_len;
   int mx = -1, mn = 0;
-  for (int p = num_sink + threadIdx.x; p < seq_len; p += COUNT_THREADS) {
-    const int v = row[p];
-    mx = max(mx, v);
-    mn = min(mn, v);
+  for (int p0 = num_sink + threadIdx.x; p0 < seq_len; p0 += U * COUNT_THREADS) {
+    int v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = gload_i32(row + min(p0 + u * COUNT_THREADS, seq_len - 1));  // (the last label again)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      mx = max(mx, v[u]);
+      mn = min(mn, v[u]);
+    }
   }
   __shared__ int s_max[COUNT_THREADS / 64], s_min[COUNT_THREADS / 64];
   mx = wave_max_i32(mx);
@@ -122,13 +132,31 @@ __global__ __launch_bounds__(COUNT_THREADS) void label_count_kernel(const int32_
   }
 }
 
-// hist[g][chunk][c]: members of community c among the chunk's positions.
-// Communities below lds_n are counted in LDS, the others in the output row.
-__global__ __launch_bounds__(HIST_THREADS) void chunk_hist_kernel(const int32_t* __restrict__ labels, int seq_len,
-                                                                  int num_sink, int maxc, int lds_n, int chunk_len,
-                                                                  int chunks, int32_t* __restrict__ hist) {
+// Everything that needs the labels alone, in one launch.  Workgroups below
+// graphs * chunks: hist[g][chunk][c] = members of community c among the
+// chunk's positions (communities below lds_n are counted in LDS, the others in
+// the output row).  The others fill the token table and clear the weights.
+__global__ __launch_bounds__(HIST_THREADS) void state_prep_kernel(
+    const int32_t* __restrict__ labels, int seq_len, int num_sink, int maxc, int lds_n, int chunk_len, int chunks,
+    int graphs, int32_t* __restrict__ hist, int token_capacity, int32_t* __restrict__ tokens,
+    float* __restrict__ weight, int64_t weights, float* __restrict__ total) {
   extern __shared__ int h_s[];
-  const int chunk = blockIdx.x, g = blockIdx.y;
+  if ((int)blockIdx.x >= graphs * chunks) {
+    const int64_t i0 = (int64_t)(blockIdx.x - graphs * chunks) * HIST_THREADS + threadIdx.x;
+    const int64_t step = (int64_t)(gridDim.x - graphs * chunks) * HIST_THREADS;
+    const int64_t all = (int64_t)graphs * token_capacity;
+    for (int64_t i = i0; i < all; i += step) {
+      const int g = (int)(i / token_capacity);
+      const int t = (int)(i - (int64_t)g * token_capacity);
+      tokens[i] = t < seq_len ? labels[(int64_t)g * seq_len + t] : -1;
+    }
+    if (weight != nullptr) {
+      for (int64_t i = i0; i < weights; i += step) weight[i] = 0.0f;
+      for (int64_t i = i0; i < graphs; i += step) total[i] = 0.0f;
+    }
+    return;
+  }
+  const int chunk = blockIdx.x % chunks, g = blockIdx.x / chunks;
   int32_t* out = hist + ((int64_t)g * chunks + chunk) * maxc;
   for (int c = threadIdx.x; c < lds_n; c += HIST_THREADS) h_s[c] = 0;
   for (int c = lds_n + threadIdx.x; c < maxc; c += HIST_THREADS) out[c] = 0;
@@ -146,133 +174,217 @@ __global__ __launch_bounds__(HIST_THREADS) void chunk_hist_kernel(const int32_t*
   for (int c = threadIdx.x; c < lds_n; c += HIST_THREADS) out[c] = h_s[c];
 }
 
-// Per graph: offsets[c] = members of communities below c; then every chunk's
-// histogram entry becomes the CSR slot of that chunk's newest member of c
-// (later chunks first: the CSR is recency descending).
-__global__ __launch_bounds__(SCAN_THREADS) void csr_scan_kernel(int maxc, int chunks, int64_t max_blocks,
-                                                                int32_t* __restrict__ hist,
+// Per (graph, community): hist[chunk][c] becomes the members of c in later
+// chunks (the CSR is recency descending), offsets[c] the community's total.
+// Spread over all compute units: with one workgroup per graph walking every
+// community's chunks, 13,000 communities took 146 us.
+__global__ __launch_bounds__(HIST_THREADS) void chunk_scan_kernel(int maxc, int chunks, int32_t* __restrict__ hist,
+                                                                  int32_t* __restrict__ offsets) {
+  const int g = blockIdx.y;
+  const int c = blockIdx.x * HIST_THREADS + threadIdx.x;
+  if (c >= maxc) return;
+  int32_t* h = hist + (int64_t)g * chunks * maxc + c;
+  int run = 0;
+  for (int i0 = chunks - 1; i0 >= 0; i0 -= 16) {  // sixteen loads in flight, then their stores
+    int n[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) n[u] = gload_i32(h + (int64_t)max(i0 - u, 0) * maxc);
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      if (i0 - u >= 0) {
+        h[(int64_t)(i0 - u) * maxc] = run;
+        run += n[u];
+      }
+    }
+  }
+  offsets[(int64_t)g * (maxc + 1) + c] = run;
+}
+
+// Per graph: the communities' totals (in offsets) become CSR offsets and block
+// starts, in place; each thread scans a run of consecutive communities, so the
+// workgroup scans once.
+__global__ __launch_bounds__(SCAN_THREADS) void csr_scan_kernel(int maxc, int64_t max_blocks,
                                                                 int32_t* __restrict__ offsets,
                                                                 int32_t* __restrict__ blk_first,
                                                                 int32_t* __restrict__ blk_comm) {
-  // communities c = k * SCAN_THREADS + tid, one block-wide scan per round k
   const int g = blockIdx.x;
   const int tid = threadIdx.x;
-  int32_t* h = hist + (int64_t)g * chunks * maxc;
   int32_t* off = offsets + (int64_t)g * (maxc + 1);
   int32_t* bf = blk_first + (int64_t)g * (maxc + 1);
   int32_t* bc = blk_comm + (int64_t)g * max_blocks;
   __shared__ int s_wave[SCAN_THREADS / 64], s_wblk[SCAN_THREADS / 64];
-  int carry = 0, bcarry = 0;
-  for (int c0 = 0; c0 < maxc; c0 += SCAN_THREADS) {
-    const int c = c0 + tid;
-    int t = 0;
-    if (c < maxc) {
-#pragma unroll 8
-      for (int i = 0; i < chunks; ++i) t += h[(int64_t)i * maxc + c];
-    }
-    const int nb = (t + SUM_BLOCK - 1) / SUM_BLOCK;
-    const int inc = wave_inclusive_scan(t);
-    const int incb = wave_inclusive_scan(nb);
-    if ((tid & 63) == 63) {
-      s_wave[tid >> 6] = inc;
-      s_wblk[tid >> 6] = incb;
-    }
-    __syncthreads();
-    int base = carry + inc - t, bbase = bcarry + incb - nb;
-    int round = 0, bround = 0;
-    for (int wv = 0; wv < SCAN_THREADS / 64; ++wv) {
-      if (wv < (tid >> 6)) {
-        base += s_wave[wv];
-        bbase += s_wblk[wv];
-      }
-      round += s_wave[wv];
-      bround += s_wblk[wv];
-    }
-    __syncthreads();  // s_wave reused next round
-    if (c < maxc) {
-      off[c] = base;
-      bf[c] = bbase;
-      for (int j = 0; j < nb; ++j) bc[bbase + j] = c;
-      int run = base;
-      for (int i0 = chunks - 1; i0 >= 0; i0 -= 8) {  // eight loads in flight, then their stores
-        int n[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) n[u] = i0 - u >= 0 ? h[(int64_t)(i0 - u) * maxc + c] : 0;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          if (i0 - u >= 0) {
-            h[(int64_t)(i0 - u) * maxc + c] = run;
-            run += n[u];
-          }
-        }
-      }
-    }
-    carry += round;
-    bcarry += bround;
+  const int per = (maxc + SCAN_THREADS - 1) / SCAN_THREADS;
+  const int c0 = min(tid * per, maxc), c1 = min(c0 + per, maxc);
+  int t = 0, nb = 0;
+#pragma unroll 4
+  for (int c = c0; c < c1; ++c) {
+    const int n = off[c];
+    t += n;
+    nb += (n + SUM_BLOCK - 1) / SUM_BLOCK;
   }
-  if (tid == 0) {
-    off[maxc] = carry;
-    bf[maxc] = bcarry;
+  const int inc = wave_inclusive_scan(t);
+  const int incb = wave_inclusive_scan(nb);
+  if ((tid & 63) == 63) {
+    s_wave[tid >> 6] = inc;
+    s_wblk[tid >> 6] = incb;
+  }
+  __syncthreads();
+  int base = inc - t, bbase = incb - nb;
+  for (int wv = 0; wv < (tid >> 6); ++wv) {
+    base += s_wave[wv];
+    bbase += s_wblk[wv];
+  }
+#pragma unroll 4
+  for (int c = c0; c < c1; ++c) {
+    const int n = off[c];
+    const int b = (n + SUM_BLOCK - 1) / SUM_BLOCK;
+    off[c] = base;
+    bf[c] = bbase;
+    for (int j = 0; j < b; ++j) bc[bbase + j] = c;
+    base += n;
+    bbase += b;
+  }
+  if (tid == SCAN_THREADS - 1) {
+    off[maxc] = base;
+    bf[maxc] = bbase;
   }
 }
 
 // One wave per (graph, chunk): walks the chunk's positions from the newest
-// down, 64 at a time (lane l takes the l-th newest); lanes with equal labels
-// are ranked by lane (newer first) one distinct label per round, and an LDS
-// cursor per community advances by each round's members.
-// Cursors of communities below lds_n live in LDS, the others in the chunk's
-// histogram row (which nothing reads afterwards).
+// down, 64 at a time (lane l takes the l-th newest).  Lanes with equal labels
+// find each other bit by bit (one ballot per label bit: at most 17 rounds
+// against one per distinct label, 122 us at 512 communities and 8 x 32,768
+// positions before, 8.2 us now), the lanes before a lane in its set
+// rank it, and the set's first lane advances the community's cursor.
+// Cursors of communities below lds_n live in LDS (members of the chunk placed
+// so far; the community's first slot is prefetched for SCATTER_GROUPS groups at
+// a time), the others in the chunk's histogram row (which nothing reads
+// afterwards).
+constexpr int SCATTER_GROUPS = 8;
+
 __global__ __launch_bounds__(64) void csr_scatter_kernel(const int32_t* __restrict__ labels, int seq_len, int num_sink,
-                                                         int maxc, int lds_n, int chunk_len, int chunks,
-                                                         int32_t* __restrict__ hist,
+                                                         int maxc, int label_bits, int lds_n, int chunk_len, int chunks,
+                                                         const int32_t* __restrict__ offsets, int32_t* hist,
                                                          int32_t* __restrict__ member_positions) {
   extern __shared__ int cur_s[];
   const int chunk = blockIdx.x, g = blockIdx.y;
   const int lane = threadIdx.x;
   int32_t* h = hist + ((int64_t)g * chunks + chunk) * maxc;
-  for (int c = lane; c < lds_n; c += 64) cur_s[c] = h[c];
+  const int32_t* off = offsets + (int64_t)g * (maxc + 1);
+  for (int c = lane; c < lds_n; c += 64) cur_s[c] = 0;
   wave_sync();
   const int32_t* row = labels + (int64_t)g * seq_len;
   int32_t* out = member_positions + (int64_t)g * (seq_len - num_sink);
   const int p0 = num_sink + chunk * chunk_len;
   const int p1 = min(p0 + chunk_len, seq_len);
   const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  for (int top = p1 - 1; top >= p0; top -= 64) {
-    const int p = top - lane;
-    const bool ok = p >= p0;
-    const int c = ok ? row[p] : -1;
-    const bool valid = ok && c >= 0 && c < maxc;
-    uint64_t todo = __ballot(valid);
-    while (todo) {
-      const int leader = __builtin_ctzll(todo);
-      const int lc = __builtin_amdgcn_readlane(c, leader);
-      const uint64_t m = __ballot(valid && c == lc);
-      const int base = lc < lds_n ? cur_s[lc] : h[lc];
-      if (valid && c == lc) out[base + __popcll(m & below)] = p;
-      wave_sync();
-      if (lane == leader) {
-        if (lc < lds_n) cur_s[lc] = base + __popcll(m);
-        else h[lc] = base + __popcll(m);
+  for (int top0 = p1 - 1; top0 >= p0; top0 -= 64 * SCATTER_GROUPS) {
+    int lab[SCATTER_GROUPS], first[SCATTER_GROUPS], later[SCATTER_GROUPS];
+#pragma unroll
+    for (int u = 0; u < SCATTER_GROUPS; ++u) lab[u] = gload_i32(row + max(top0 - 64 * u - lane, p0));
+#pragma unroll
+    for (int u = 0; u < SCATTER_GROUPS; ++u) {
+      const int c = min(max(lab[u], 0), maxc - 1);
+      first[u] = gload_i32(off + c);
+      later[u] = gload_i32(h + c);
+    }
+#pragma unroll
+    for (int u = 0; u < SCATTER_GROUPS; ++u) {
+      const int p = top0 - 64 * u - lane;
+      const int c = lab[u];
+      const bool valid = p >= p0 && c >= 0 && c < maxc;
+      uint64_t peers = __ballot(valid);
+      if (peers == 0) continue;
+      for (int b = 0; b < label_bits; ++b) {
+        const bool bit = (c >> b) & 1;
+        const uint64_t m = __ballot(bit);
+        peers &= bit ? m : ~m;
       }
-      if (lc >= lds_n) wait_vm();  // (wave-uniform) the cursor store lands before a later round reads it
+      const int rank = __popcll(peers & below), size = __popcll(peers);
+      const bool in_lds = valid && c < lds_n;
+      const bool in_row = valid && c >= lds_n;
+      int at = 0;
+      if (in_lds) at = first[u] + later[u] + cur_s[c];
+      if (in_row) at = first[u] + __hip_atomic_load(h + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       wave_sync();
-      todo &= ~m;
+      if (rank == 0 && in_lds) cur_s[c] += size;
+      if (__ballot(in_row)) {
+        if (rank == 0 && in_row) __hip_atomic_fetch_add(h + c, size, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        wait_vm();  // the cursors are advanced before a later group reads them
+      }
+      wave_sync();
+      if (valid) out[at + rank] = p;
+    }
+  }
+}
+
+// Sum and finish of a centroid row (lane = dims 2l and 2l+1): mean, clamp to
+// +-448, then E4M3 or f32.
+template <int CT>
+__device__ __forceinline__ void store_mean(float s0, float s1, int size, bool divide, int64_t row, int lane,
+                                           void* __restrict__ centroids, int32_t* __restrict__ sizes) {
+  if (divide) {
+    const float den = (float)max(size, 1);
+    s0 = s0 / den;
+    s1 = s1 / den;
+  }
+  s0 = fminf(fmaxf(s0, -448.0f), 448.0f);
+  s1 = fminf(fmaxf(s1, -448.0f), 448.0f);
+  if constexpr (CT == CKV_E4M3) {
+    const uint16_t pair = (uint16_t)(ckv_f32_to_e4m3(s0) | ((uint16_t)ckv_f32_to_e4m3(s1) << 8));
+    reinterpret_cast<uint16_t*>(centroids)[row * (D / 2) + lane] = pair;
+  } else {
+    float* dst = reinterpret_cast<float*>(centroids) + row * D + 2 * lane;
+    dst[0] = s0;
+    dst[1] = s1;
+  }
+  if (lane == 0) sizes[row] = size;
+}
+
+// Loads N rows (lanes past n of `mine` repeat the last member) in one round and
+// adds the first n of them in order.
+template <int KT, int N>
+__device__ __forceinline__ void sum_rows(const void* __restrict__ keys, int64_t kb, int64_t token_stride, int mine,
+                                         int n, float& s0, float& s1) {
+  constexpr int W = KT == CKV_BF16 ? 1 : 2;
+  uint32_t x[N][W];
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const int p = __builtin_amdgcn_readlane(mine, u);
+    if constexpr (KT == CKV_BF16) {
+      x[u][0] = (uint32_t)gload_i32(reinterpret_cast<const int32_t*>(reinterpret_cast<const uint16_t*>(keys) + kb +
+                                                                     (int64_t)p * token_stride));
+    } else {
+      const float* kp = reinterpret_cast<const float*>(keys) + kb + (int64_t)p * token_stride;
+      x[u][0] = ckv_f2u(gload_f32(kp));
+      x[u][W - 1] = ckv_f2u(gload_f32(kp + 1));
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    if (u < n) {
+      s0 = s0 + (KT == CKV_BF16 ? ckv_u2f(x[u][0] << 16) : ckv_u2f(x[u][0]));
+      s1 = s1 + (KT == CKV_BF16 ? ckv_u2f(x[u][0] & 0xffff0000u) : ckv_u2f(x[u][W - 1]));
     }
   }
 }
 
 // One wave per (retrieval head, 64-member block): members 64k .. 64k+63 of
 // community c in ascending position order (the CSR lists them newest first),
-// summed in order in f32, lane = dims 2l and 2l+1.  All 64 rows are loaded
-// before the sum, so a block costs one gather round.
-template <int KT>
+// summed in order in f32, lane = dims 2l and 2l+1.  All rows are loaded
+// before the sum, so a block costs one gather round; a block of few members
+// loads 4 or 16 rows instead of 64 (communities of a Leiden partition have two
+// or three members on average: 120 us with 64 rows each, 8 x 13,000 of them, 54 us
+// so).  A community of one block is finished here.
+template <int KT, int CT>
 __global__ __launch_bounds__(64 * CENTROID_WAVES) void block_sum_kernel(
     const void* __restrict__ keys, int64_t head_stride, int64_t token_stride, const int32_t* __restrict__ to_graph,
     const int32_t* __restrict__ to_kv, const int32_t* __restrict__ offsets, const int32_t* __restrict__ positions,
     const int32_t* __restrict__ blk_first, const int32_t* __restrict__ blk_comm, int64_t max_blocks, int seq_len,
-    int num_sink, int maxc, float* __restrict__ partial) {
+    int num_sink, int maxc, int capacity, float* __restrict__ partial, void* __restrict__ centroids,
+    int32_t* __restrict__ sizes) {
   const int r = blockIdx.y;
-  const int64_t b = (int64_t)blockIdx.x * CENTROID_WAVES + (threadIdx.x >> 6);
+  const int64_t b = (int64_t)blockIdx.x * CENTROID_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int g = to_graph[r];
   const int kvh = to_kv[r];
@@ -286,37 +398,22 @@ __global__ __launch_bounds__(64 * CENTROID_WAVES) void block_sum_kernel(
   const int32_t* mem = positions + (int64_t)g * (seq_len - num_sink);
   const int mine = mem[hi - 1 - (i0 + min(lane, n - 1))];
   const int64_t kb = (int64_t)kvh * head_stride + 2 * lane;
-  float x0[SUM_BLOCK], x1[SUM_BLOCK];
-#pragma unroll
-  for (int u = 0; u < SUM_BLOCK; ++u) {
-    const int p = __builtin_amdgcn_readlane(mine, u);  // lanes past n repeat the last member
-    if constexpr (KT == CKV_BF16) {
-      const uint32_t w = (uint32_t)gload_i32(reinterpret_cast<const int32_t*>(
-          reinterpret_cast<const uint16_t*>(keys) + kb + (int64_t)p * token_stride));
-      x0[u] = ckv_u2f(w << 16);
-      x1[u] = ckv_u2f(w & 0xffff0000u);
-    } else {
-      const float* kp = reinterpret_cast<const float*>(keys) + kb + (int64_t)p * token_stride;
-      x0[u] = gload_f32(kp);
-      x1[u] = gload_f32(kp + 1);
-    }
-  }
   float s0 = 0.0f, s1 = 0.0f;  // (+0 start: an all-negative-zero block sums to +0, as scatter_add_ does)
-#pragma unroll
-  for (int u = 0; u < SUM_BLOCK; ++u) {
-    if (u < n) {
-      s0 = s0 + x0[u];
-      s1 = s1 + x1[u];
-    }
+  if (n <= 4) sum_rows<KT, 4>(keys, kb, token_stride, mine, n, s0, s1);
+  else if (n <= 16) sum_rows<KT, 16>(keys, kb, token_stride, mine, n, s0, s1);
+  else sum_rows<KT, SUM_BLOCK>(keys, kb, token_stride, mine, n, s0, s1);
+  if (hi - lo <= SUM_BLOCK) {
+    store_mean<CT>(s0, s1, hi - lo, true, (int64_t)r * capacity + c, lane, centroids, sizes);
+    return;
   }
   float* dst = partial + ((int64_t)r * max_blocks + b) * D + 2 * lane;
   dst[0] = s0;
   dst[1] = s1;
 }
 
-// One wave per (retrieval head, community row): the community's block sums
-// added in order, divided by its size, clamped to +-448, then E4M3 or f32.
-// Rows at or past maxc hold zeros.
+// One wave per (retrieval head, community row) of several blocks or none: the
+// block sums added in order, divided by its size.  Rows at or past maxc hold
+// zeros.
 template <int CT>
 __global__ __launch_bounds__(64 * CENTROID_WAVES) void centroid_kernel(
     const int32_t* __restrict__ to_graph, const int32_t* __restrict__ offsets, const int32_t* __restrict__ blk_first,
@@ -332,6 +429,7 @@ __global__ __launch_bounds__(64 * CENTROID_WAVES) void centroid_kernel(
     size = offsets[(int64_t)g * (maxc + 1) + c + 1] - offsets[(int64_t)g * (maxc + 1) + c];
     b0 = blk_first[(int64_t)g * (maxc + 1) + c];
     nb = blk_first[(int64_t)g * (maxc + 1) + c + 1] - b0;
+    if (nb == 1) return;  // finished by block_sum_kernel
   }
   const float* src = partial + ((int64_t)r * max_blocks + b0) * D + 2 * lane;
   float s0 = 0.0f, s1 = 0.0f;
@@ -351,39 +449,7 @@ __global__ __launch_bounds__(64 * CENTROID_WAVES) void centroid_kernel(
       }
     }
   }
-  if (c < maxc) {
-    const float den = (float)max(size, 1);
-    s0 = s0 / den;
-    s1 = s1 / den;
-  }
-  s0 = fminf(fmaxf(s0, -448.0f), 448.0f);
-  s1 = fminf(fmaxf(s1, -448.0f), 448.0f);
-  const int64_t row = (int64_t)r * capacity + c;
-  if constexpr (CT == CKV_E4M3) {
-    const uint16_t pair = (uint16_t)(ckv_f32_to_e4m3(s0) | ((uint16_t)ckv_f32_to_e4m3(s1) << 8));
-    reinterpret_cast<uint16_t*>(centroids)[row * (D / 2) + lane] = pair;
-  } else {
-    float* dst = reinterpret_cast<float*>(centroids) + row * D + 2 * lane;
-    dst[0] = s0;
-    dst[1] = s1;
-  }
-  if (lane == 0) sizes[row] = size;
-}
-
-__global__ void token_table_kernel(const int32_t* __restrict__ labels, int seq_len, int token_capacity, int graphs,
-                                   int32_t* __restrict__ tokens) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t total = (int64_t)graphs * token_capacity;
-  if (i >= total) return;
-  const int g = (int)(i / token_capacity);
-  const int t = (int)(i % token_capacity);
-  tokens[i] = t < seq_len ? labels[(int64_t)g * seq_len + t] : -1;
-}
-
-__global__ void weight_zero_kernel(float* __restrict__ weight, int64_t n, float* __restrict__ total, int graphs) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) weight[i] = 0.0f;
-  if (i < graphs) total[i] = 0.0f;
+  store_mean<CT>(s0, s1, size, c < maxc, (int64_t)r * capacity + c, lane, centroids, sizes);
 }
 
 // Community degree weights and 2m: each edge (graph * seq_len + position
@@ -449,68 +515,87 @@ __global__ __launch_bounds__(EDGE_THREADS) void edge_weight_kernel(
 // ends), the row position's community gains lam/2 S, and the graph's total
 // 2 x (edge weights) = lam S + (1 - lam) (S^2 + sum p_k^2).  A workgroup's
 // rows share one head, hence one graph: weights gather in LDS first.
-constexpr int TOPK_ROWS_PER_WG = 256;
+//
+// A workgroup walks TOPK_THREADS rows at a time over a share of its head's
+// rows chosen so that about TOPK_WORKGROUPS run: what it gathered leaves with
+// one global atomic per touched community, and with 256 rows per workgroup
+// those (2.1 M at 32 heads x 32,751 rows, 512 communities) were most of the
+// launch.  Rows of 8 or 16 edges at 16-byte aligned addresses are read with
+// 16-byte loads.  82 us before at that size, 58 us now (67 MB of edges).
+constexpr int TOPK_THREADS = 256;
+constexpr int TOPK_WORKGROUPS = 1024;
 
-__global__ __launch_bounds__(TOPK_ROWS_PER_WG) void topk_weight_kernel(
+template <int VEC>  // 16-byte pieces of a row's edges; 0: any kappa, scalar loads
+__global__ __launch_bounds__(TOPK_THREADS) void topk_weight_kernel(
     const int32_t* __restrict__ labels, int seq_len, int capacity, int lds_n, const int32_t* __restrict__ idx,
-    const float* __restrict__ sc, int rows, int kappa, int group, int row0, float lam, float* __restrict__ weight,
-    float* __restrict__ total) {
+    const float* __restrict__ sc, int rows, int rows_per_wg, int kappa, int group, int row0, float lam,
+    float* __restrict__ weight, float* __restrict__ total) {
+  constexpr int K = VEC ? 4 * VEC : 16;
   extern __shared__ float w_s[];  // communities [0, lds_n)
   const int h = blockIdx.y;
   const int g = h / group;
-  for (int c = threadIdx.x; c < lds_n; c += TOPK_ROWS_PER_WG) w_s[c] = 0.0f;
+  for (int c = threadIdx.x; c < lds_n; c += TOPK_THREADS) w_s[c] = 0.0f;
   __syncthreads();
-  const int r = blockIdx.x * TOPK_ROWS_PER_WG + threadIdx.x;
   const int32_t* lab = labels + (int64_t)g * seq_len;
-  float mine = 0.0f;
-  if (r < rows) {
-    const int32_t* ir = idx + ((int64_t)h * rows + r) * kappa;
-    const float* sr = sc + ((int64_t)h * rows + r) * kappa;
-    int col[16];
-    float p[16];
+  auto add = [&](int c, float v) {
+    if (c >= 0 && c < lds_n) unsafeAtomicAdd(w_s + c, v);
+    else if (c >= lds_n && c < capacity) unsafeAtomicAdd(weight + (int64_t)g * capacity + c, v);
+  };
+  const float half = 0.5f * lam, co = 1.0f - lam;
+  double mine = 0.0;
+  const int r1 = min(rows, (int)(blockIdx.x + 1) * rows_per_wg);
+  for (int r = blockIdx.x * rows_per_wg + threadIdx.x; r < r1; r += TOPK_THREADS) {
+    const int64_t at = ((int64_t)h * rows + r) * kappa;
+    int col[K];
+    float p[K];
+    if constexpr (VEC > 0) {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        const uint4 i4 = gload16(idx + at + 4 * v), p4 = gload16(sc + at + 4 * v);
+        col[4 * v] = (int)i4.x; col[4 * v + 1] = (int)i4.y; col[4 * v + 2] = (int)i4.z; col[4 * v + 3] = (int)i4.w;
+        p[4 * v] = ckv_u2f(p4.x); p[4 * v + 1] = ckv_u2f(p4.y);
+        p[4 * v + 2] = ckv_u2f(p4.z); p[4 * v + 3] = ckv_u2f(p4.w);
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        col[k] = k < kappa ? idx[at + k] : -1;
+        p[k] = k < kappa ? sc[at + k] : 0.0f;
+      }
+    }
+    int com[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) com[k] = gload_i32(lab + min(max(col[k], 0), seq_len - 1));
+    const int pos = row0 + r;
+    const bool pos_ok = pos >= 0 && pos < seq_len;
+    const int pos_com = pos_ok ? lab[pos] : -1;
     float s = 0.0f, s2 = 0.0f;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      col[k] = k < kappa ? ir[k] : -1;
-      p[k] = k < kappa ? sr[k] : 0.0f;
-    }
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
+    for (int k = 0; k < K; ++k) {
       if (col[k] >= 0 && col[k] < seq_len) {
         s = s + p[k];
         s2 = s2 + p[k] * p[k];
       }
     }
-    const float half = 0.5f * lam, co = 1.0f - lam;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      if (col[k] >= 0 && col[k] < seq_len) {
-        const int c = lab[col[k]];
-        const float v = half * p[k] + co * (p[k] * (s + p[k]));
-        if (c >= 0 && c < lds_n) atomicAdd(w_s + c, v);
-        else if (c >= lds_n && c < capacity) atomicAdd(weight + (int64_t)g * capacity + c, v);
-      }
+    for (int k = 0; k < K; ++k) {
+      if (col[k] >= 0 && col[k] < seq_len) add(com[k], half * p[k] + co * (p[k] * (s + p[k])));
     }
-    const int pos = row0 + r;
-    if (pos >= 0 && pos < seq_len) {
-      const int c = lab[pos];
-      if (c >= 0 && c < lds_n) atomicAdd(w_s + c, half * s);
-      else if (c >= lds_n && c < capacity) atomicAdd(weight + (int64_t)g * capacity + c, half * s);
-    }
-    mine = lam * s + co * (s * s + s2);
+    if (pos_ok) add(pos_com, half * s);
+    mine += (double)(lam * s + co * (s * s + s2));
   }
-  __shared__ float s_part[TOPK_ROWS_PER_WG / 64];
-  mine = wave_sum_tree(mine);
+  __shared__ double s_part[TOPK_THREADS / 64];
+  for (int o = 32; o >= 1; o >>= 1) mine += __shfl_xor(mine, o);
   if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = mine;
   __syncthreads();
-  for (int c = threadIdx.x; c < lds_n; c += TOPK_ROWS_PER_WG) {
+  for (int c = threadIdx.x; c < lds_n; c += TOPK_THREADS) {
     const float v = w_s[c];
-    if (v != 0.0f) atomicAdd(weight + (int64_t)g * capacity + c, v);
+    if (v != 0.0f) unsafeAtomicAdd(weight + (int64_t)g * capacity + c, v);
   }
   if (threadIdx.x == 0) {
-    float t = 0.0f;
-    for (int i = 0; i < TOPK_ROWS_PER_WG / 64; ++i) t = t + s_part[i];
-    atomicAdd(total + g, t);
+    double t = 0.0;
+    for (int i = 0; i < TOPK_THREADS / 64; ++i) t += s_part[i];
+    unsafeAtomicAdd(total + g, (float)t);
   }
 }
 
@@ -582,20 +667,37 @@ extern "C" int ckv_build_layer_state(const ckv_state_build_args* a, void* stream
   // communities past lds_n are counted in global memory (64 KB of LDS per kernel)
   const int lds_n = std::min(maxc, STATE_LDS_COMMUNITIES);
   const size_t lds = (size_t)lds_n * sizeof(int);
-  hipLaunchKernelGGL(chunk_hist_kernel, dim3(chunks, a->graphs), dim3(HIST_THREADS), lds, s, a->labels, a->seq_len,
-                     a->num_sink, maxc, lds_n, chunk_len, chunks, w.hist);
-  hipLaunchKernelGGL(csr_scan_kernel, dim3(a->graphs), dim3(SCAN_THREADS), 0, s, maxc, chunks, mb, w.hist,
-                     a->member_offsets, w.blk_first, w.blk_comm);
+  const bool weights = a->community_weight && a->total_weight;
+  const int64_t nw = (int64_t)a->graphs * a->community_capacity;
+  const int64_t fill = std::max((int64_t)a->graphs * a->token_capacity, weights ? nw : 0);
+  const unsigned prep = (unsigned)(chunks * a->graphs + std::min<int64_t>((fill + 4 * HIST_THREADS - 1) / (4 * HIST_THREADS), 1024));
+  hipLaunchKernelGGL(state_prep_kernel, dim3(prep), dim3(HIST_THREADS), lds, s, a->labels, a->seq_len, a->num_sink,
+                     maxc, lds_n, chunk_len, chunks, a->graphs, w.hist, a->token_capacity, a->token_communities,
+                     weights ? a->community_weight : nullptr, nw, a->total_weight);
+  hipLaunchKernelGGL(chunk_scan_kernel, dim3((maxc + HIST_THREADS - 1) / HIST_THREADS, a->graphs), dim3(HIST_THREADS),
+                     0, s, maxc, chunks, w.hist, a->member_offsets);
+  hipLaunchKernelGGL(csr_scan_kernel, dim3(a->graphs), dim3(SCAN_THREADS), 0, s, maxc, mb, a->member_offsets,
+                     w.blk_first, w.blk_comm);
+  int label_bits = 1;
+  while (label_bits < 31 && ((maxc - 1) >> label_bits) != 0) ++label_bits;
   hipLaunchKernelGGL(csr_scatter_kernel, dim3(chunks, a->graphs), dim3(64), lds, s, a->labels, a->seq_len,
-                     a->num_sink, maxc, lds_n, chunk_len, chunks, w.hist, a->member_positions);
+                     a->num_sink, maxc, label_bits, lds_n, chunk_len, chunks, (const int32_t*)a->member_offsets, w.hist,
+                     a->member_positions);
   const dim3 bgrid((unsigned)((mb + CENTROID_WAVES - 1) / CENTROID_WAVES), a->retrieval_heads);
   auto sums = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, bgrid, dim3(64 * CENTROID_WAVES), 0, s, a->keys, a->head_stride, a->token_stride,
                        a->retrieval_to_graph, a->retrieval_to_kv, (const int32_t*)a->member_offsets,
                        (const int32_t*)a->member_positions, (const int32_t*)w.blk_first,
-                       (const int32_t*)w.blk_comm, mb, a->seq_len, a->num_sink, maxc, w.partial);
+                       (const int32_t*)w.blk_comm, mb, a->seq_len, a->num_sink, maxc, a->community_capacity,
+                       w.partial, a->centroids, a->community_sizes);
   };
-  if (a->key_dtype == CKV_BF16) sums(block_sum_kernel<CKV_BF16>); else sums(block_sum_kernel<CKV_F32>);
+  if (a->key_dtype == CKV_BF16) {
+    if (a->centroid_dtype == CKV_E4M3) sums(block_sum_kernel<CKV_BF16, CKV_E4M3>);
+    else sums(block_sum_kernel<CKV_BF16, CKV_F32>);
+  } else {
+    if (a->centroid_dtype == CKV_E4M3) sums(block_sum_kernel<CKV_F32, CKV_E4M3>);
+    else sums(block_sum_kernel<CKV_F32, CKV_F32>);
+  }
   const dim3 cgrid((a->community_capacity + CENTROID_WAVES - 1) / CENTROID_WAVES, a->retrieval_heads);
   auto cent = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, cgrid, dim3(64 * CENTROID_WAVES), 0, s, a->retrieval_to_graph,
@@ -603,20 +705,20 @@ extern "C" int ckv_build_layer_state(const ckv_state_build_args* a, void* stream
                        maxc, a->community_capacity, a->centroids, a->community_sizes);
   };
   if (a->centroid_dtype == CKV_E4M3) cent(centroid_kernel<CKV_E4M3>); else cent(centroid_kernel<CKV_F32>);
-  const int64_t ntok = (int64_t)a->graphs * a->token_capacity;
-  hipLaunchKernelGGL(token_table_kernel, dim3((unsigned)((ntok + 255) / 256)), dim3(256), 0, s, a->labels,
-                     a->seq_len, a->token_capacity, a->graphs, a->token_communities);
-  if (a->community_weight && a->total_weight) {
-    const int64_t nw = (int64_t)a->graphs * a->community_capacity;
-    const int64_t nz = nw > a->graphs ? nw : a->graphs;
-    hipLaunchKernelGGL(weight_zero_kernel, dim3((unsigned)((nz + 255) / 256)), dim3(256), 0, s, a->community_weight,
-                       nw, a->total_weight, a->graphs);
+  if (weights) {
     if (a->topk_indices && a->topk_rows > 0) {
-      hipLaunchKernelGGL(topk_weight_kernel,
-                         dim3((a->topk_rows + TOPK_ROWS_PER_WG - 1) / TOPK_ROWS_PER_WG, a->topk_heads),
-                         dim3(TOPK_ROWS_PER_WG), (size_t)lds_n * sizeof(float), s, a->labels,
-                         a->seq_len, a->community_capacity, lds_n, a->topk_indices, a->topk_scores, a->topk_rows,
-                         a->topk_kappa, a->topk_group, a->topk_row0, a->lam, a->community_weight, a->total_weight);
+      const int per_head = std::max(1, TOPK_WORKGROUPS / a->topk_heads);
+      const int rows_per_wg = ((a->topk_rows + per_head - 1) / per_head + TOPK_THREADS - 1) / TOPK_THREADS * TOPK_THREADS;
+      const dim3 tgrid((a->topk_rows + rows_per_wg - 1) / rows_per_wg, a->topk_heads);
+      auto topk = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, tgrid, dim3(TOPK_THREADS), (size_t)lds_n * sizeof(float), s, a->labels, a->seq_len,
+                           a->community_capacity, lds_n, a->topk_indices, a->topk_scores, a->topk_rows, rows_per_wg,
+                           a->topk_kappa, a->topk_group, a->topk_row0, a->lam, a->community_weight, a->total_weight);
+      };
+      const bool aligned = (((uintptr_t)a->topk_indices | (uintptr_t)a->topk_scores) & 15) == 0;
+      if (aligned && a->topk_kappa == 8) topk(topk_weight_kernel<2>);
+      else if (aligned && a->topk_kappa == 16) topk(topk_weight_kernel<4>);
+      else topk(topk_weight_kernel<0>);
     }
     if (a->edges > 0) {
       hipLaunchKernelGGL(edge_weight_kernel, dim3((unsigned)((a->edges + EDGES_PER_WG - 1) / EDGES_PER_WG)),

@@ -147,3 +147,78 @@ def test_state_build_topk_edges_match_coalesced_graph(device, lam, kappa):
     tw64 = np.array([2.0 * w[src // seq_len == g].astype(np.float64).sum() for g in range(graphs)])
     np.testing.assert_allclose(st.total_weight.cpu().numpy(), tw64, rtol=1e-5)
     np.testing.assert_allclose(tw, tw64, rtol=1e-3)
+
+
+@pytest.mark.parametrize("kdt,fp8", [(torch.bfloat16, True), (torch.bfloat16, False), (torch.float32, True)])
+def test_state_build_block_edges(device, kdt, fp8):
+    """Communities whose sizes sit at the edges of the block sums (4, 16 and
+    64 rows loaded; one block finished at once, several added later), newest
+    members in partial 64-position groups, and label counts around a power of
+    two: CSR, sizes and centroids bit for bit."""
+    sizes = [1, 4, 5, 16, 17, 63, 64, 65, 128, 129, 200, 3]
+    for extra in (4, 5, 6):  # 16, 17 and 18 labels: 4, 5 and 5 label bits
+        rng = np.random.default_rng(extra)
+        lab = np.repeat(np.arange(len(sizes) + extra), sizes + [2] * extra).astype(np.int32)
+        rng.shuffle(lab)
+        ids = np.concatenate([np.zeros(3, np.int32), lab])[None]
+        seq_len = ids.shape[1]
+        keys = (torch.randn(1, seq_len, 128, generator=torch.Generator().manual_seed(extra)) * 3.0).to(kdt)
+        print(f"state build block edges {kdt} fp8={fp8} S={seq_len} labels={len(sizes) + extra}", flush=True)
+        one = torch.zeros(1, dtype=torch.int32, device=device)
+        st = build_layer_state(torch.from_numpy(ids).to(device), keys.to(device), retrieval_to_graph=one,
+                               retrieval_to_kv=one, num_sink=3, max_decode_tokens=2, fp8=fp8)
+        counts = np.array([len(sizes) + extra], np.int32)
+        off, pos = co.build_member_csr(ids, counts, num_sink=3)
+        np.testing.assert_array_equal(st.member_offsets.cpu().numpy(), off)
+        np.testing.assert_array_equal(st.member_positions.cpu().numpy(), pos)
+        cent, csizes = co.compute_centroids(ids, counts, keys.float().numpy(), to_graph=np.zeros(1, np.int32),
+                                            to_kv=np.zeros(1, np.int32), num_sink=3, max_decode_tokens=2, fp8=fp8)
+        np.testing.assert_array_equal(st.community_sizes.cpu().numpy(), csizes)
+        got = st.centroids.cpu()
+        if fp8:
+            np.testing.assert_array_equal(got.view(torch.uint8).numpy(), cent)
+        else:
+            np.testing.assert_array_equal(got.numpy().view(np.uint32), cent.view(np.uint32))
+
+
+@pytest.mark.parametrize("kappa,offset", [(8, 0), (8, 1), (16, 0), (16, 3), (5, 0)])
+def test_state_build_topk_load_widths(device, kappa, offset):
+    """Top-k edges read with 16-byte loads (8 or 16 edges a row, aligned) and
+    one by one (any other width, or a view that starts off a 16-byte address)
+    give the weights of the float64 closed form: at most about 3,400 x 9 float
+    terms per community, so 1e-4 relative."""
+    from community_kv_amd.graph.kernels.state_build import TopkEdges
+
+    rng = np.random.default_rng(kappa + offset)
+    graphs, group, seq_len, num_sink, maxc, lam = 2, 2, 1700, 4, 37, 0.5
+    ids = _labels(rng, graphs, seq_len, maxc, num_sink)
+    row0 = num_sink + kappa - 1
+    rows, heads = seq_len - row0, graphs * group
+    idx = rng.integers(0, seq_len, size=(heads, rows, kappa)).astype(np.int32)
+    idx[rng.random(idx.shape) < 0.1] = -1
+    sc = rng.random((heads, rows, kappa)).astype(np.float32)
+
+    def shifted(a):
+        flat = torch.zeros(a.size + offset, dtype=torch.from_numpy(a).dtype, device=device)
+        flat[offset:] = torch.from_numpy(a).to(device).flatten()
+        return flat[offset:].view(a.shape)
+
+    print(f"state build top-k widths kappa={kappa} offset={offset}", flush=True)
+    tg = torch.arange(graphs, dtype=torch.int32, device=device)
+    keys = torch.zeros(graphs, seq_len, 128, dtype=torch.bfloat16, device=device)
+    st = build_layer_state(torch.from_numpy(ids).to(device), keys, retrieval_to_graph=tg, retrieval_to_kv=tg,
+                           num_sink=num_sink, max_decode_tokens=8,
+                           topk_edges=TopkEdges(indices=shifted(idx), scores=shifted(sc), row0=row0, group=group,
+                                                lam=lam))
+    weight = np.zeros((graphs, st.community_weight.shape[1]))
+    total = np.zeros(graphs)
+    for h in range(heads):
+        g = h // group
+        p = np.where(idx[h] >= 0, sc[h], 0.0).astype(np.float64)
+        s, s2 = p.sum(1), (p * p).sum(1)
+        w = lam / 2 * p + (1 - lam) * p * (s[:, None] + p)
+        np.add.at(weight[g], ids[g][np.maximum(idx[h], 0)], w)
+        np.add.at(weight[g], ids[g][row0:], lam / 2 * s)
+        total[g] += (lam * s + (1 - lam) * (s * s + s2)).sum()
+    np.testing.assert_allclose(st.community_weight.cpu().numpy(), weight, rtol=1e-4, atol=1e-4)
+    np.testing.assert_allclose(st.total_weight.cpu().numpy(), total, rtol=1e-5)

@@ -19,7 +19,8 @@ REPO_DIR = os.path.dirname(PACKAGE_DIR)
 LIB_PATH = os.path.join(PACKAGE_DIR, "libckv_amd.so")
 SOURCES = [os.path.join(PACKAGE_DIR, "csrc", name)
            for name in ("ckv_decode.hip", "ckv_select.hip", "ckv_attend.hip", "ckv_prefill.hip", "ckv_diag.hip",
-                                "ckv_state.hip", "ckv_leiden.hip", "ckv_noalloc.hip", "ckv_select_large.hip")]
+                                "ckv_state.hip", "ckv_adjacency.hip", "ckv_leiden.hip", "ckv_noalloc.hip",
+                                "ckv_select_large.hip")]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = [
     "--offload-arch=gfx950",

@@ -1,0 +1,787 @@
+// The coalesced token graph of the prefill's top-k edges (reference:
+// graph/partition.py:168-249): per row of graph g at position p with columns
+// c_i of score s_i, the direct edges (p, c_i) of weight s_i * lam / 2 and, when
+// lam < 1, the co-occurrence edges (c_i, c_j), i <= j, of weight
+// s_i * s_j * (1 - lam); equal (min, max) pairs summed, pairs in order.
+//
+// A row of 8 columns stands for 44 entries, 46.9 M for a 32k layer of 32 query
+// heads, so the entries are never written: a vertex's edges to higher ids are
+// gathered from the rows that name it.
+//
+//   posting_kernel    one (vertex, entry) pair per column, and one per row
+//                     whose position lies below one of its columns
+//   radix sort        pairs by vertex, stable: a vertex's postings are a run in row order
+//   list_kernel       the runs, in two lists by length
+//   gather_kernel     one wave per short run: each posting's row is read, the neighbours
+//                     above the vertex gather in an LDS hash table (f64 sums) and leave
+//                     ordered by id
+//   gather_big_kernel the same by one workgroup per long run
+//   gather_dense_kernel  vertices with more neighbours than that table holds:
+//                     windows of consecutive ids summed in a dense LDS array
+//   scan + emit_kernel   edges to their places in the output
+//
+// The sums are f64 sums of the f32 entry weights, rounded once.
+//
+// Measured at that size (9.8 M edges out): 2.9 ms for the expansion, the
+// 64-bit radix sort of its 46.9 M entries and their reduction before,
+// 1.2 ms so.  What bounds it now: the random reads of the rows (32 bytes
+// of columns and of scores per posting, from L2 and the Infinity Cache) and
+// the LDS inserts.
+#include <hip/hip_runtime.h>
+
+#include <stdint.h>
+
+#include <type_traits>
+
+#include "ckv_amd.h"
+#include "ckv_error.h"
+#include "ckv_sort.h"
+
+namespace ckv {
+namespace {
+
+constexpr int THREADS = 256;
+constexpr int WAVE_SLOTS = 512;        // LDS table of one wave: 6 KB
+constexpr int WAVE_CANDIDATES = 448;   // candidates of a short run at most (table load 7/8)
+constexpr int WAVES = 4;               // waves per workgroup: a run's length decides how long its wave holds the
+                                       // workgroup's LDS, so workgroups are small (24 KB, six fill a compute unit)
+constexpr int WAVE_BLOCKS = 1536;
+constexpr int FLIGHT = 4;              // candidates a thread has in flight: postings, then their rows, then the inserts
+constexpr int BIG_THREADS = 256;
+constexpr int BIG_SLOTS = 2048;        // 24 KB
+constexpr int BIG_MOST = 960;          // neighbours after which a vertex leaves for the dense list
+static_assert(BIG_MOST + FLIGHT * BIG_THREADS < BIG_SLOTS, "every insert between two checks finds a place");
+constexpr int BIG_BLOCKS = 1280;       // five workgroups a compute unit (24 KB + the id bitmap of 32k vertices)
+constexpr int MAP_WORDS = 4096;        // id bitmap of a graph: up to 131,072 vertices
+constexpr int DENSE_THREADS = 1024;
+constexpr int DENSE_WINDOW = 16384;    // ids per window: 128 KB of f64 sums
+constexpr int DENSE_BLOCKS = 256;
+constexpr uint32_t EMPTY = 0xffffffffu;
+
+struct TopkGraph {
+  const int32_t* idx;    // [G * R][K]
+  const float* sc;       // [G * R][K]
+  const int64_t* pos;    // [G * R]
+  int32_t G, R, K, S;
+  int shift;             // bits of a posting below its row
+  float half_lam, co_lam;
+  int co;                // co-occurrence edges (lam < 1)
+};
+
+__device__ inline int lane() { return (int)__lane_id(); }
+// Orders the wave's LDS accesses (all lanes' writes before, reads after).
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ inline double wave_sum_f64(double x) {
+  for (int o = 32; o >= 1; o >>= 1) x += __shfl_xor(x, o);
+  return x;
+}
+__device__ inline uint32_t hash_id(uint32_t x) { return (x * 0x9E3779B1u) >> 8; }
+
+// Postings [first, last) of one vertex.
+struct Run {
+  uint32_t first, last;
+};
+
+enum { LIST_SHORT = 0, LIST_LONG = 1, LIST_DENSE = 2, LIST_TICKET = 3, LIST_WORDS = 4 };
+
+// A posting names (row << shift) | i: column i of the row, or (i == K) its
+// position.  A position is a posting only if one of the row's columns lies
+// above it: then that direct edge starts at the position (a causal prefill has
+// none).  The pair of (i, row) stands at i * rows + row, so the stores of
+// consecutive rows are consecutive.
+template <int KT>
+__global__ __launch_bounds__(THREADS) void posting_kernel(TopkGraph t, uint32_t* __restrict__ keys,
+                                                          uint32_t* __restrict__ vals, int32_t* __restrict__ lists) {
+  const int K = KT ? KT : t.K;
+  const int64_t rows = (int64_t)t.G * t.R;
+  const int64_t row = (int64_t)blockIdx.x * THREADS + threadIdx.x;
+  if (row < LIST_WORDS) lists[row] = 0;  // no run listed yet
+  if (row >= rows) return;
+  const int32_t base = (int32_t)(row / t.R) * t.S;
+  const uint32_t none = (uint32_t)(t.G * t.S);  // sorts last
+  const int64_t p = t.pos[row];
+  bool above = false;
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    const int32_t c = t.idx[row * K + i];
+    const bool ok = c >= 0 && c < t.S;
+    above = above || (ok && c > p);
+    keys[i * rows + row] = ok ? (uint32_t)(base + c) : none;
+    vals[i * rows + row] = ((uint32_t)row << t.shift) | (uint32_t)i;
+  }
+  keys[K * rows + row] = (above && p >= 0 && p < t.S) ? (uint32_t)(base + (int32_t)p) : none;
+  vals[K * rows + row] = ((uint32_t)row << t.shift) | (uint32_t)K;
+}
+
+// A candidate edge of vertex v: column j of a posting's row.
+struct Candidate {
+  uint32_t u;    // the neighbour (> v) when ok
+  bool ok;
+  float w;
+  double self;   // weight it adds to the pair (v, v)
+  bool has_self;
+};
+
+// What a candidate needs from memory.
+struct Loaded {
+  int32_t c;
+  float s, si;   // scores of column j and of the posting's own column
+  int64_t p;     // the row's position (lane j == i only)
+};
+
+template <int KT>
+__device__ __forceinline__ Loaded load_candidate(const TopkGraph& t, uint32_t posting, int j) {
+  const int K = KT ? KT : t.K;
+  const uint32_t row = posting >> t.shift;
+  const int i = (int)(posting & ((1u << t.shift) - 1u));
+  const int64_t at = (int64_t)row * K;
+  Loaded l;
+  l.c = t.idx[at + j];
+  l.s = t.sc[at + j];
+  l.si = t.sc[at + (i < K ? i : j)];
+  l.p = (j == i) ? t.pos[row] : -1;
+  return l;
+}
+
+// The lane of the posting's own column carries the column's pair with itself
+// and the row's direct edge.
+template <int KT>
+__device__ __forceinline__ Candidate candidate(const TopkGraph& t, uint32_t posting, int j, const Loaded& l,
+                                               int32_t v, int32_t base) {
+  const int K = KT ? KT : t.K;
+  const int i = (int)(posting & ((1u << t.shift) - 1u));
+  Candidate r{0u, false, 0.0f, 0.0, false};
+  if (i == K) {  // the vertex is the row's position: direct edges to the columns above it
+    r.u = (uint32_t)(base + l.c);
+    r.ok = l.c < t.S && base + l.c > v;
+    r.w = l.s * t.half_lam;
+  } else if (j == i) {
+    const bool direct = l.p >= 0 && l.p < t.S && base + l.p >= v;
+    const float w = l.s * t.half_lam;
+    r.u = (uint32_t)(base + (int32_t)l.p);
+    r.ok = direct && base + l.p > v;
+    r.w = w;
+    r.has_self = t.co || (direct && !r.ok);
+    if (t.co) r.self += (double)((l.s * l.s) * t.co_lam);
+    if (direct && !r.ok) r.self += (double)w;
+  } else if (t.co && l.c >= 0 && l.c < t.S && base + l.c >= v) {
+    const float w = (l.si * l.s) * t.co_lam;
+    r.u = (uint32_t)(base + l.c);
+    r.ok = base + l.c > v;
+    r.w = w;
+    r.has_self = !r.ok && j > i;  // the column again: one entry of the pair (i, j), i < j
+    if (r.has_self) r.self = (double)w;
+  }
+  return r;
+}
+
+// Walks the candidates q = first, first + step, ... of the run that starts at
+// posting a, FLIGHT at a time; add(candidate) for each, pause() after each FLIGHT
+// (a true return ends the walk).
+template <int KT, class Add, class Pause>
+__device__ __forceinline__ void walk(const TopkGraph& t, const uint32_t* __restrict__ postings, uint32_t a, uint64_t n,
+                                     uint32_t first, uint32_t step, int32_t v, int32_t base, Add add, Pause pause) {
+  const uint32_t K = KT ? KT : (uint32_t)t.K;
+  for (uint64_t q0 = 0; q0 < n; q0 += (uint64_t)FLIGHT * step) {
+    uint32_t post[FLIGHT], j[FLIGHT];
+    Loaded l[FLIGHT];
+#pragma unroll
+    for (int f = 0; f < FLIGHT; ++f) {
+      const uint64_t q = q0 + (uint64_t)f * step + first;
+      const uint64_t qc = q < n ? q : n - 1;  // (past the end: the last one again, not added)
+      const uint64_t p = KT ? qc / KT : qc / K;
+      j[f] = (uint32_t)(qc - p * K);
+      post[f] = postings[a + p];
+    }
+#pragma unroll
+    for (int f = 0; f < FLIGHT; ++f) l[f] = load_candidate<KT>(t, post[f], (int)j[f]);
+#pragma unroll
+    for (int f = 0; f < FLIGHT; ++f) {
+      if (q0 + (uint64_t)f * step + first < n) add(candidate<KT>(t, post[f], (int)j[f], l[f], v, base));
+    }
+    if (pause()) break;
+  }
+}
+
+// Inserts (u, w) into an open-addressing table of size slots (a power of two);
+// returns the number of probes that found no place, 0 when placed.
+__device__ inline bool insert(uint32_t* tk, double* ts, uint32_t size, uint32_t u, float w, int* added) {
+  uint32_t h = hash_id(u) & (size - 1);
+  for (uint32_t probe = 0; probe < size; ++probe) {
+    const uint32_t cur = __hip_atomic_load(tk + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    bool mine = cur == u;
+    if (cur == EMPTY) {
+      const uint32_t prev = atomicCAS(tk + h, EMPTY, u);
+      mine = prev == EMPTY || prev == u;
+      if (prev == EMPTY && added) atomicAdd(added, 1);
+    }
+    if (mine) {
+      unsafeAtomicAdd(ts + h, (double)w);
+      return true;
+    }
+    h = (h + 1) & (size - 1);
+  }
+  return false;
+}
+
+__device__ inline uint32_t table_size(uint64_t most, uint32_t cap) {
+  uint32_t size = 64;
+  while (size < 2 * most && size < cap) size <<= 1;
+  return size;
+}
+
+// The edges of one run [a, b) of vertex v by one wave.
+template <int KT>
+__device__ __forceinline__ void gather_run(const TopkGraph& t, const uint32_t* __restrict__ postings, uint32_t a,
+                                           uint32_t b, int32_t v, uint32_t* tk, double* ts,
+                                           int32_t* __restrict__ count, uint32_t* __restrict__ tmp_id,
+                                           float* __restrict__ tmp_w) {
+  const int ln = lane();
+  const int32_t base = v / t.S * t.S;
+  const uint32_t n = (b - a) * (uint32_t)t.K;
+  const uint32_t size = table_size(min(n, (uint32_t)(base + t.S - v)), WAVE_SLOTS);
+  for (uint32_t j = ln; j < size; j += 64) {
+    tk[j] = EMPTY;
+    ts[j] = 0.0;
+  }
+  wave_sync();
+  double self = 0.0;
+  bool any_self = false;
+  walk<KT>(t, postings, a, n, (uint32_t)ln, 64u, v, base,
+           [&](const Candidate& c) {
+             any_self = any_self || c.has_self;
+             self += c.self;
+             if (c.ok) insert(tk, ts, size, c.u, c.w, nullptr);  // (never more ids than the table holds)
+           },
+           [] { return false; });
+  wave_sync();
+  self = wave_sum_f64(self);
+  const int lead = __ballot(any_self) != 0 ? 1 : 0;
+  // Compact the occupied slots to the front (every lane has read its slots
+  // before any is overwritten), then order them by counting smaller ids.
+  constexpr int PER = WAVE_SLOTS / 64;
+  uint32_t k[PER];
+  float w[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const uint32_t j = ln + 64 * i;
+    k[i] = j < size ? tk[j] : EMPTY;
+    w[i] = k[i] != EMPTY ? (float)ts[j] : 0.0f;
+  }
+  wave_sync();
+  float* tw = reinterpret_cast<float*>(ts);
+  int m = 0;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const uint64_t used = __ballot(k[i] != EMPTY);
+    if (k[i] != EMPTY) {
+      const int at = m + __popcll(used & ((((uint64_t)1) << ln) - 1));
+      tk[at] = k[i];
+      tw[at] = w[i];
+    }
+    m += __popcll(used);
+  }
+  if (ln < 4 && m + ln < WAVE_SLOTS) tk[m + ln] = EMPTY;  // fills the last group of four
+  wave_sync();
+  const int64_t out = (int64_t)a * (t.K + 1);
+  if (lead && ln == 0) {
+    tmp_id[out] = (uint32_t)v;
+    tmp_w[out] = (float)self;
+  }
+  for (int i = ln; i < m; i += 64) {
+    const uint32_t mine = tk[i];
+    int rank = 0;
+    for (int j = 0; j < m; j += 4) {
+      const uint4 o = *reinterpret_cast<const uint4*>(tk + j);
+      rank += (o.x < mine) + (o.y < mine) + (o.z < mine) + (o.w < mine);
+    }
+    tmp_id[out + lead + rank] = mine;
+    tmp_w[out + lead + rank] = tw[i];
+  }
+  if (ln == 0) count[a] = lead + m;
+  wave_sync();  // the wave's next run clears the table
+}
+
+// End of the run of v that starts before `end` and goes on there: the first
+// posting of another vertex in [end, n], found by probing 64 places at a time
+// (the interval narrows 63-fold per round).
+__device__ inline uint32_t run_end(const uint32_t* __restrict__ keys, uint32_t end, uint32_t n, uint32_t v) {
+  uint32_t lo = end, hi = n, step = 1;
+  while (lo < hi) {
+    const uint32_t at = lo + (uint32_t)lane() * step;
+    const uint64_t other = __ballot(at >= hi || keys[at < hi ? at : hi - 1] != v);
+    const uint32_t f = other ? (uint32_t)__builtin_ctzll(other) : 64u;  // probes below f are of v, probe f is not
+    if (f < 64) hi = min(lo + f * step, hi);
+    if (f > 0) lo = min(lo + (f - 1) * step + 1, hi);
+    step = max(1u, (hi - lo + 62) / 63);
+  }
+  return lo;
+}
+
+// Lists the runs by their length.  A workgroup takes LIST_GROUPS x 1,024
+// postings and reserves its places in a list at once: with one reservation per
+// wave, 294,000 atomics on two words took 870 us.
+constexpr int LIST_THREADS = 1024;
+constexpr int LIST_GROUPS = 4;
+
+__global__ __launch_bounds__(LIST_THREADS) void list_kernel(const uint32_t* __restrict__ keys, uint32_t n, uint32_t V,
+                                                            uint32_t short_most, int32_t* __restrict__ count,
+                                                            Run* __restrict__ short_runs, Run* __restrict__ long_runs,
+                                                            int32_t* __restrict__ lists) {
+  __shared__ int s_n[2], s_at[2];
+  const int ln = lane();
+  const uint64_t below = (((uint64_t)1) << ln) - 1;
+  if (threadIdx.x < 2) s_n[threadIdx.x] = 0;
+  __syncthreads();
+  uint32_t stop[LIST_GROUPS];
+  int place[LIST_GROUPS];  // in the workgroup's part of list `kind`; kind 2: no run starts here
+  int kind[LIST_GROUPS];
+#pragma unroll
+  for (int g = 0; g < LIST_GROUPS; ++g) {
+    const uint32_t here = (blockIdx.x * LIST_GROUPS + g) * LIST_THREADS + threadIdx.x;
+    const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)here);
+    const bool in = here < n;
+    const uint32_t key = in ? keys[here] : EMPTY;
+    const bool start = in && (here == 0 || keys[here - 1] != key);
+    const uint64_t starts = __ballot(start);
+    if (in) count[here] = 0;  // runs that have edges store their number later
+    const bool mine = start && key < V;
+    const uint64_t real = __ballot(mine);
+    uint32_t end = first + 64 < n ? first + 64 : n;
+    if (real != 0 && end < n) {
+      const int last = 63 - __builtin_clzll(starts);
+      if ((real >> last) & 1) end = run_end(keys, end, n, (uint32_t)__builtin_amdgcn_readlane((int)key, last));
+    }
+    const uint64_t later = ln == 63 ? 0ull : starts >> (ln + 1);
+    stop[g] = later ? here + 1 + (uint32_t)__builtin_ctzll(later) : end;
+    kind[g] = !mine ? 2 : stop[g] - here <= short_most ? LIST_SHORT : LIST_LONG;
+    const uint64_t ms = __ballot(kind[g] == LIST_SHORT), ml = __ballot(kind[g] == LIST_LONG);
+    int bs = 0, bl = 0;
+    if (ln == 0) {
+      if (ms) bs = atomicAdd(s_n, __popcll(ms));
+      if (ml) bl = atomicAdd(s_n + 1, __popcll(ml));
+    }
+    bs = __builtin_amdgcn_readfirstlane(bs);
+    bl = __builtin_amdgcn_readfirstlane(bl);
+    place[g] = kind[g] == LIST_SHORT ? bs + __popcll(ms & below) : bl + __popcll(ml & below);
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) s_at[threadIdx.x] = s_n[threadIdx.x] ? atomicAdd(lists + threadIdx.x, s_n[threadIdx.x]) : 0;
+  __syncthreads();
+#pragma unroll
+  for (int g = 0; g < LIST_GROUPS; ++g) {
+    const uint32_t here = (blockIdx.x * LIST_GROUPS + g) * LIST_THREADS + threadIdx.x;
+    if (kind[g] == LIST_SHORT) short_runs[s_at[0] + place[g]] = Run{here, stop[g]};
+    if (kind[g] == LIST_LONG) long_runs[s_at[1] + place[g]] = Run{here, stop[g]};
+  }
+}
+
+// The edges of the run that starts at posting a wait in tmp at a * (K + 1): a
+// posting brings at most K neighbours, the run one pair with itself; count[a]
+// holds their number (0 at postings that start no run).
+template <int KT>
+__global__ __launch_bounds__(64 * WAVES) void gather_kernel(TopkGraph t, const uint32_t* __restrict__ keys,
+                                                            const uint32_t* __restrict__ postings,
+                                                            const Run* __restrict__ runs,
+                                                            const int32_t* __restrict__ lists,
+                                                            int32_t* __restrict__ count, uint32_t* __restrict__ tmp_id,
+                                                            float* __restrict__ tmp_w) {
+  __shared__ __align__(16) uint32_t tab_k[WAVES][WAVE_SLOTS];
+  __shared__ double tab_s[WAVES][WAVE_SLOTS];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int32_t listed = lists[LIST_SHORT];
+  for (int32_t it = blockIdx.x * WAVES + wave; it < listed; it += gridDim.x * WAVES) {
+    const Run r = runs[it];
+    gather_run<KT>(t, postings, r.first, r.last, (int32_t)keys[r.first], tab_k[wave], tab_s[wave], count, tmp_id,
+                   tmp_w);
+  }
+}
+
+// One workgroup per long run (taken in turn by a ticket: their lengths differ
+// by a hundredfold).  Up to BIG_MOST neighbours in the LDS table; a vertex that has more goes to the dense list.  The neighbours are
+// ordered by a bitmap of the graph's vertices (words of it dynamic LDS, with a
+// running count per word): the set bits below an id are its rank.  Counting
+// smaller ids instead, as the waves do for their few, grows with the square
+// (and orders graphs of more vertices than the bitmap has).
+template <int KT>
+__global__ __launch_bounds__(BIG_THREADS) void gather_big_kernel(
+    TopkGraph t, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ postings,
+    const Run* __restrict__ runs, Run* __restrict__ dense, int32_t* lists, int32_t* __restrict__ count,
+    uint32_t* __restrict__ tmp_id, float* __restrict__ tmp_w) {
+  __shared__ __align__(16) uint32_t tk[BIG_SLOTS];
+  __shared__ double ts[BIG_SLOTS];
+  extern __shared__ uint32_t map_s[];  // [words] bits, [words] set bits before the word
+  __shared__ double red[BIG_THREADS / 64];
+  __shared__ int wave_n[BIG_THREADS / 64];
+  __shared__ int s_added, s_self, s_ticket;
+  const int tid = threadIdx.x, wv = tid >> 6, ln = lane();
+  const int32_t listed = lists[LIST_LONG];
+  const int words = t.S <= 32 * MAP_WORDS ? (t.S + 31) >> 5 : 0;
+  uint32_t* before_s = map_s + words;
+  while (true) {
+    if (tid == 0) s_ticket = atomicAdd(lists + LIST_TICKET, 1);
+    __syncthreads();
+    const int32_t it = s_ticket;
+    if (it >= listed) return;
+    const uint32_t a = runs[it].first, b = runs[it].last;
+    const int32_t v = (int32_t)keys[a];
+    const int32_t base = v / t.S * t.S;
+    const uint64_t n = (uint64_t)(b - a) * (uint32_t)t.K;
+    const uint64_t room = (uint64_t)(base + t.S - v);
+    const uint32_t size = table_size(n < room ? n : room, BIG_SLOTS);
+    for (uint32_t j = tid; j < size; j += BIG_THREADS) {
+      tk[j] = EMPTY;
+      ts[j] = 0.0;
+    }
+    for (int j = tid; j < words; j += BIG_THREADS) map_s[j] = 0u;
+    if (tid == 0) s_added = s_self = 0;
+    __syncthreads();
+    double self = 0.0;
+    bool any_self = false;
+    walk<KT>(t, postings, a, n, (uint32_t)tid, BIG_THREADS, v, base,
+             [&](const Candidate& c) {
+               any_self = any_self || c.has_self;
+               self += c.self;
+               if (c.ok) insert(tk, ts, size, c.u, c.w, &s_added);
+             },
+             [&] {
+               if (size < BIG_SLOTS) return false;  // room for every candidate
+               __syncthreads();
+               const bool full = s_added > BIG_MOST;
+               __syncthreads();
+               return full;
+             });
+    self = wave_sum_f64(self);
+    if (ln == 0) red[wv] = self;
+    if (any_self) s_self = 1;
+    __syncthreads();
+    if (s_added > BIG_MOST) {
+      if (tid == 0) dense[atomicAdd(lists + LIST_DENSE, 1)] = Run{a, b};
+      __syncthreads();
+      continue;
+    }
+    const int lead = s_self;
+    double total = 0.0;
+    for (int i = 0; i < BIG_THREADS / 64; ++i) total += red[i];
+    const int64_t out = (int64_t)a * (t.K + 1);
+    if (lead && tid == 0) {
+      tmp_id[out] = (uint32_t)v;
+      tmp_w[out] = (float)total;
+    }
+    // Thread t holds the slots t, t + 256, ...
+    constexpr int PER = BIG_SLOTS / BIG_THREADS;
+    uint32_t k[PER];
+    float w[PER];
+    int own = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const uint32_t j = tid + BIG_THREADS * i;
+      k[i] = j < size ? tk[j] : EMPTY;
+      w[i] = k[i] != EMPTY ? (float)ts[j] : 0.0f;
+      own += k[i] != EMPTY ? 1 : 0;
+      if (words > 0 && k[i] != EMPTY) {
+        const uint32_t d = k[i] - (uint32_t)base;
+        atomicOr(map_s + (d >> 5), 1u << (d & 31));
+      }
+    }
+    __syncthreads();
+    const int per = (words + BIG_THREADS - 1) / BIG_THREADS;  // consecutive map words of a thread
+    int mine = own;
+    if (words > 0) {
+      mine = 0;
+      for (int i = 0; i < per; ++i) {
+        const int j = tid * per + i;
+        if (j < words) mine += __popc(map_s[j]);
+      }
+    }
+    int incl = mine;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o);
+      if (ln >= o) incl += y;
+    }
+    if (ln == 63) wave_n[wv] = incl;
+    __syncthreads();
+    int at = incl - mine, m = 0;
+    for (int i = 0; i < BIG_THREADS / 64; ++i) {
+      if (i < wv) at += wave_n[i];
+      m += wave_n[i];
+    }
+    if (words > 0) {
+      for (int i = 0; i < per; ++i) {
+        const int j = tid * per + i;
+        if (j < words) {
+          before_s[j] = (uint32_t)at;
+          at += __popc(map_s[j]);
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        if (k[i] != EMPTY) {
+          const uint32_t d = k[i] - (uint32_t)base;
+          const int rank = (int)before_s[d >> 5] + __popc(map_s[d >> 5] & ((1u << (d & 31)) - 1u));
+          tmp_id[out + lead + rank] = k[i];
+          tmp_w[out + lead + rank] = w[i];
+        }
+      }
+    } else {
+      float* tw = reinterpret_cast<float*>(ts);
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        if (k[i] != EMPTY) {
+          tk[at] = k[i];
+          tw[at] = w[i];
+          ++at;
+        }
+      }
+      if (tid < 4) tk[m + tid] = EMPTY;  // (m <= BIG_MOST: never a compacted place)
+      __syncthreads();
+      for (int i = tid; i < m; i += BIG_THREADS) {
+        int rank = 0;
+        for (int j = 0; j < m; j += 4) {
+          const uint4 o = *reinterpret_cast<const uint4*>(tk + j);
+          rank += (o.x < tk[i]) + (o.y < tk[i]) + (o.z < tk[i]) + (o.w < tk[i]);
+        }
+        tmp_id[out + lead + rank] = tk[i];
+        tmp_w[out + lead + rank] = tw[i];
+      }
+    }
+    if (tid == 0) count[a] = lead + m;
+    __syncthreads();
+  }
+}
+
+// Vertices with more than BIG_MOST neighbours: their rows are read once per
+// window of DENSE_WINDOW consecutive ids, whose sums and marks lie in LDS in
+// id order.
+constexpr size_t dense_lds_bytes() { return DENSE_WINDOW * 8 + DENSE_WINDOW / 8; }
+
+template <int KT>
+__global__ __launch_bounds__(DENSE_THREADS) void gather_dense_kernel(
+    TopkGraph t, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ postings,
+    const Run* __restrict__ dense, const int32_t* __restrict__ lists, int32_t* __restrict__ count,
+    uint32_t* __restrict__ tmp_id, float* __restrict__ tmp_w) {
+  extern __shared__ double dense_s[];
+  uint32_t* mark = reinterpret_cast<uint32_t*>(dense_s + DENSE_WINDOW);
+  __shared__ int wave_n[DENSE_THREADS / 64];
+  constexpr int PER = DENSE_WINDOW / DENSE_THREADS;  // consecutive ids of a thread (half a mark word)
+  static_assert(PER == 16, "a thread owns half a mark word");
+  const int tid = threadIdx.x, wv = tid >> 6, ln = lane();
+  const int32_t listed = lists[LIST_DENSE];
+  for (int32_t it = blockIdx.x; it < listed; it += gridDim.x) {
+    const uint32_t a = dense[it].first, b = dense[it].last;
+    const int32_t v = (int32_t)keys[a];
+    const int32_t base = v / t.S * t.S;
+    const uint64_t n = (uint64_t)(b - a) * (uint32_t)t.K;
+    const int64_t out = (int64_t)a * (t.K + 1);
+    int done = 0;
+    for (int32_t lo = v; lo < base + t.S; lo += DENSE_WINDOW) {
+      for (int j = tid; j < DENSE_WINDOW; j += DENSE_THREADS) dense_s[j] = 0.0;
+      for (int j = tid; j < DENSE_WINDOW / 32; j += DENSE_THREADS) mark[j] = 0u;
+      __syncthreads();
+      walk<KT>(t, postings, a, n, (uint32_t)tid, DENSE_THREADS, v, base,
+               [&](const Candidate& c) {
+                 if (c.has_self && lo == v) {
+                   unsafeAtomicAdd(dense_s, c.self);
+                   atomicOr(mark, 1u);
+                 }
+                 const int32_t d = (int32_t)c.u - lo;
+                 if (c.ok && d >= 0 && d < DENSE_WINDOW) {
+                   unsafeAtomicAdd(dense_s + d, (double)c.w);
+                   atomicOr(mark + (d >> 5), 1u << (d & 31));
+                 }
+               },
+               [] { return false; });
+      __syncthreads();
+      const uint32_t bits = (mark[tid >> 1] >> (16 * (tid & 1))) & 0xffffu;
+      const int own = __popc(bits);
+      int incl = own;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(incl, o);
+        if (ln >= o) incl += y;
+      }
+      if (ln == 63) wave_n[wv] = incl;
+      __syncthreads();
+      int at = done + incl - own, m = 0;
+      for (int i = 0; i < DENSE_THREADS / 64; ++i) {
+        if (i < wv) at += wave_n[i];
+        m += wave_n[i];
+      }
+      for (int i = 0; i < PER; ++i) {
+        if ((bits >> i) & 1u) {
+          const int d = tid * PER + i;
+          tmp_id[out + at] = (uint32_t)(lo + d);
+          tmp_w[out + at] = (float)dense_s[d];
+          ++at;
+        }
+      }
+      done += m;
+      __syncthreads();
+    }
+    if (tid == 0) count[a] = done;
+  }
+}
+
+// Copies the runs' edges to their places; the last posting's place ends the output.
+__global__ __launch_bounds__(64 * WAVES) void emit_kernel(const uint32_t* __restrict__ keys,
+                                                          const int32_t* __restrict__ count,
+                                                          const int32_t* __restrict__ place,
+                                                          const Run* __restrict__ short_runs,
+                                                          const Run* __restrict__ long_runs,
+                                                          const int32_t* __restrict__ lists, uint32_t n, int32_t K,
+                                                          const uint32_t* __restrict__ tmp_id,
+                                                          const float* __restrict__ tmp_w, int32_t* __restrict__ out_src,
+                                                          int32_t* __restrict__ out_dst, float* __restrict__ out_w,
+                                                          int64_t* __restrict__ out_count) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int32_t shorts = lists[LIST_SHORT], listed = shorts + lists[LIST_LONG];
+  for (int32_t it = blockIdx.x * WAVES + wave; it < listed; it += gridDim.x * WAVES) {
+    const uint32_t a = (it < shorts ? short_runs[it] : long_runs[it - shorts]).first;
+    const int m = count[a], at = place[a], v = (int)keys[a];
+    const int64_t from = (int64_t)a * (K + 1);
+    for (int i = lane(); i < m; i += 64) {
+      out_src[at + i] = v;
+      out_dst[at + i] = (int32_t)tmp_id[from + i];
+      out_w[at + i] = tmp_w[from + i];
+    }
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) *out_count = (int64_t)place[n - 1] + count[n - 1];
+}
+
+struct AdjLayout {
+  size_t keys_in, vals_in, keys, vals, temp, temp_bytes, count, place, short_runs, long_runs, dense, lists, tmp_id,
+      tmp_w, total;
+};
+
+// n: postings (rows x (kappa + 1)).  A long run has more than WAVE_CANDIDATES / kappa of them.
+AdjLayout adj_layout(int64_t n, int32_t kappa) {
+  AdjLayout L{};
+  size_t off = 0;
+  auto take = [&](size_t bytes) {
+    const size_t at = off;
+    off += align256(bytes);
+    return at;
+  };
+  const size_t sort = sort_pairs_bytes((size_t)n), scan = scan_bytes((size_t)n);
+  const size_t runs = (size_t)n / (size_t)(WAVE_CANDIDATES / kappa + 1) + 1;
+  L.keys_in = take((size_t)n * 4);
+  L.vals_in = take((size_t)n * 4);
+  L.keys = take((size_t)n * 4);
+  L.vals = take((size_t)n * 4);
+  L.count = take((size_t)n * 4);
+  L.place = take((size_t)n * 4);
+  L.short_runs = take((size_t)n * sizeof(Run));
+  L.long_runs = take(runs * sizeof(Run));
+  L.dense = take(runs * sizeof(Run));
+  L.lists = take(LIST_WORDS * 4);
+  L.temp_bytes = sort > scan ? sort : scan;
+  L.temp = take(L.temp_bytes);
+  L.tmp_id = take((size_t)n * (size_t)(kappa + 1) * 4);
+  L.tmp_w = take((size_t)n * (size_t)(kappa + 1) * 4);
+  L.total = off;
+  return L;
+}
+
+inline unsigned blocks_for(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
+
+inline int64_t adjacency_entries(int32_t graphs, int32_t rows, int32_t kappa, float lam) {
+  const int per_row = kappa + (lam < 1.0f ? kappa * (kappa + 1) / 2 : 0);
+  return (int64_t)graphs * rows * per_row;
+}
+inline int64_t adjacency_postings(int32_t graphs, int32_t rows, int32_t kappa) {
+  return (int64_t)graphs * rows * (kappa + 1);
+}
+
+int launch_check() {
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : ckv_internal::set_error(CKV_E_LAUNCH, hipGetErrorString(e));
+}
+
+}  // namespace
+}  // namespace ckv
+
+using namespace ckv;
+
+extern "C" size_t ckv_adjacency_workspace_bytes(int32_t graphs, int32_t rows, int32_t kappa, float lam) {
+  if (graphs <= 0 || rows <= 0 || kappa <= 0) return 0;
+  (void)lam;
+  return adj_layout(adjacency_postings(graphs, rows, kappa), kappa).total;
+}
+
+extern "C" int64_t ckv_adjacency_capacity(int32_t graphs, int32_t rows, int32_t kappa, float lam) {
+  if (graphs <= 0 || rows < 0 || kappa <= 0) return 0;
+  return adjacency_entries(graphs, rows, kappa, lam);
+}
+
+extern "C" int ckv_build_adjacency(const int32_t* topk_indices, const float* topk_scores,
+                                   const int64_t* query_positions, int32_t graphs, int32_t rows, int32_t kappa,
+                                   int32_t seq_len, float lam, int32_t* out_src, int32_t* out_dst, float* out_weight,
+                                   int64_t* out_count, void* workspace, void* stream) {
+  if (graphs <= 0 || rows < 0 || kappa <= 0 || kappa > 64 || seq_len <= 0 || !out_count || !(lam >= 0.0f && lam <= 1.0f))
+    return ckv_internal::set_error(CKV_E_INVALID, "bad adjacency sizes (kappa <= 64, lam in [0, 1])");
+  hipStream_t st = (hipStream_t)stream;
+  if (rows == 0) {
+    if (hipMemsetAsync(out_count, 0, 8, st) != hipSuccess) return launch_check();
+    return 0;
+  }
+  if (!topk_indices || !topk_scores || !query_positions || !out_src || !out_dst || !out_weight || !workspace)
+    return ckv_internal::set_error(CKV_E_INVALID, "null adjacency pointer");
+  const int64_t V = (int64_t)graphs * seq_len;
+  const int64_t n = adjacency_postings(graphs, rows, kappa);
+  if (adjacency_entries(graphs, rows, kappa, lam) >= ((int64_t)1 << 31) - 1 || V >= (int64_t)1 << 30)
+    return ckv_internal::set_error(CKV_E_LIMIT, "adjacency too large");
+  const AdjLayout L = adj_layout(n, kappa);
+  char* ws = (char*)workspace;
+  uint32_t* keys_in = (uint32_t*)(ws + L.keys_in);
+  uint32_t* vals_in = (uint32_t*)(ws + L.vals_in);
+  uint32_t* keys = (uint32_t*)(ws + L.keys);
+  uint32_t* vals = (uint32_t*)(ws + L.vals);
+  int32_t* count = (int32_t*)(ws + L.count);
+  int32_t* place = (int32_t*)(ws + L.place);
+  Run* short_runs = (Run*)(ws + L.short_runs);
+  Run* long_runs = (Run*)(ws + L.long_runs);
+  Run* dense = (Run*)(ws + L.dense);
+  int32_t* lists = (int32_t*)(ws + L.lists);
+  uint32_t* tmp_id = (uint32_t*)(ws + L.tmp_id);
+  float* tmp_w = (float*)(ws + L.tmp_w);
+  const TopkGraph t{topk_indices, topk_scores, query_positions, graphs, rows, kappa, seq_len,
+                    bits_for((uint64_t)kappa), lam / 2.0f, 1.0f - lam, lam < 1.0f ? 1 : 0};
+  auto gather = [&](auto width) -> int {
+    constexpr int KT = decltype(width)::value;
+    posting_kernel<KT><<<blocks_for((int64_t)graphs * rows, THREADS), THREADS, 0, st>>>(t, keys_in, vals_in, lists);
+    if (sort_pairs(ws + L.temp, L.temp_bytes, keys_in, keys, vals_in, vals, (size_t)n, bits_for((uint64_t)V), st) !=
+        hipSuccess)
+      return ckv_internal::set_error(CKV_E_LAUNCH, "posting sort failed");
+    list_kernel<<<blocks_for(n, LIST_GROUPS * LIST_THREADS), LIST_THREADS, 0, st>>>(
+        keys, (uint32_t)n, (uint32_t)V, (uint32_t)(WAVE_CANDIDATES / kappa), count, short_runs, long_runs, lists);
+    gather_kernel<KT><<<WAVE_BLOCKS, 64 * WAVES, 0, st>>>(t, keys, vals, short_runs, lists, count, tmp_id, tmp_w);
+    const size_t map_bytes = seq_len <= 32 * MAP_WORDS ? (size_t)((seq_len + 31) / 32) * 8 : 0;
+    gather_big_kernel<KT><<<BIG_BLOCKS, BIG_THREADS, map_bytes, st>>>(t, keys, vals, long_runs, dense, lists, count,
+                                                                      tmp_id, tmp_w);
+    if (seq_len > BIG_MOST) {  // (a vertex has fewer neighbours than its graph has vertices)
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gather_dense_kernel<KT>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)dense_lds_bytes());
+      if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return ckv_internal::set_error(CKV_E_LAUNCH, hipGetErrorString(e));
+      }
+      gather_dense_kernel<KT><<<DENSE_BLOCKS, DENSE_THREADS, dense_lds_bytes(), st>>>(
+          t, keys, vals, dense, lists, count, tmp_id, tmp_w);
+    }
+    return 0;
+  };
+  // the reference's edge width has its own code (divisions become shifts)
+  const int rc = kappa == 8 ? gather(std::integral_constant<int, 8>{})
+                            : kappa == 16 ? gather(std::integral_constant<int, 16>{})
+                                          : gather(std::integral_constant<int, 0>{});
+  if (rc != 0) return rc;
+  if (exclusive_scan_i32(ws + L.temp, L.temp_bytes, count, place, (size_t)n, st) != hipSuccess)
+    return ckv_internal::set_error(CKV_E_LAUNCH, "edge scan failed");
+  emit_kernel<<<2048, 64 * WAVES, 0, st>>>(keys, count, place, short_runs, long_runs, lists, (uint32_t)n, kappa, tmp_id,
+                                           tmp_w, out_src, out_dst, out_weight, out_count);
+  return launch_check();
+}

@@ -84,8 +84,8 @@ def build_adjacency(topk_indices: torch.Tensor, topk_scores: torch.Tensor, query
                     *, seq_len: int, lam: float) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Coalesced disjoint batched token graph from top-k edges (partition.py:168-249):
     direct edges weighted lam/2 * p, co-occurrence edges (1 - lam) * p_i * p_j.
-    Device tensors run ``ckv_build_adjacency`` (one radix sort of the edge
-    keys, equal pairs summed); the torch ops below serve host tensors."""
+    Device tensors run ``ckv_build_adjacency`` (each vertex's edges gathered
+    from the rows that name it); the torch ops below serve host tensors."""
     if topk_indices.device.type == "cuda":
         return _native_adjacency(topk_indices, topk_scores, query_positions, seq_len=seq_len, lam=lam)
     graphs, _, kappa = topk_indices.shape

@@ -239,3 +239,44 @@ def test_overflow_raised_during_local_moving_reaches_the_caller(device):
     torch.cuda.synchronize()
     _vertex, _part, q = algorithm.run_leiden(s, d, x, G=2, seq_len=300)
     assert np.isfinite(q)
+
+
+ADJACENCY_TIERS = [
+    # graphs, rows, kappa, seq_len, hub columns and the share of rows that name them
+    (2, 1500, 8, 900, 0, 0.0),       # short and long runs, fewer vertices than the workgroup table
+    (1, 400, 16, 3000, 2, 0.2),      # the width with its own code; runs of 80 rows: the id bitmap orders them
+    (1, 300, 5, 2000, 1, 1.0),       # any other width
+    (2, 6000, 8, 5000, 2, 1.0),      # more neighbours than the table: one dense window
+    (1, 4000, 8, 40000, 1, 1.0),     # three dense windows
+    (1, 700, 8, 140000, 1, 0.15),    # more vertices than the bitmap holds: ordered by counting
+    (1, 57, 8, 300, 1, 1.0),         # a run one posting past the short ones
+    (1, 1, 1, 1, 0, 0.0),            # the smallest graph: one vertex, one self loop
+]
+
+
+@pytest.mark.parametrize("G,R,kappa,S,hubs,share", ADJACENCY_TIERS)
+def test_build_adjacency_run_lengths(device, G, R, kappa, S, hubs, share):
+    """Every way a vertex's edges are gathered (one wave, one workgroup, dense
+    windows) and ordered, with columns on both sides of the row's position,
+    repeated within a row and outside the sequence; dyadic scores make the sums
+    exact, so the edge list must equal the oracle's bit for bit."""
+    from community_kv_amd.graph.partition import build_adjacency
+    from oracle import ckv_oracle as co
+
+    rng = np.random.default_rng(R + S)
+    idx = rng.integers(0, S, (G, R, kappa)).astype(np.int32)
+    if kappa > 1:
+        for h in range(hubs):
+            named = rng.random((G, R)) < share
+            idx[..., h][named] = (7 + 11 * h) % S
+        idx[:, ::5, -1] = idx[:, ::5, -2]
+        idx[rng.random(idx.shape) < 0.03] = -1
+        idx[rng.random(idx.shape) < 0.02] = S
+    sc = (rng.integers(1, 9, idx.shape) / 16.0).astype(np.float32)
+    pos = rng.integers(0, S, (G, R)).astype(np.int64)
+    print(f"build_adjacency tiers G={G} R={R} kappa={kappa} S={S} hubs={hubs} share={share}", flush=True)
+    for lam in (0.5, 1.0):
+        got = build_adjacency(*_dev(device, idx, sc, pos), seq_len=S, lam=lam)
+        ref = co.build_adjacency(idx, sc, pos, seq_len=S, lam=lam)
+        for a, b in zip(got, ref):
+            np.testing.assert_array_equal(a.cpu().numpy(), b)

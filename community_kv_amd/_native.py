@@ -77,8 +77,13 @@ EXPORTED_SYMBOLS = (
     "ckv_state_workspace_bytes",
     "ckv_label_counts",
     "ckv_build_layer_state",
+    "ckv_degree_weights",
     "ckv_leiden_workspace_bytes",
     "ckv_batched_leiden",
+    "ckv_leiden_run_workspace_bytes",
+    "ckv_leiden_run",
+    "ckv_dense_communities_workspace_bytes",
+    "ckv_dense_communities",
     "ckv_leiden_test_raise_overflow",
     "ckv_aggregate_coo_workspace_bytes",
     "ckv_aggregate_coo",
@@ -267,6 +272,17 @@ def lib() -> ctypes.CDLL:
     handle.ckv_batched_leiden.argtypes = [_p, _p, _p, _i64, _i32, _i32, _f32, _f32, _i32, _i32, _i32, _p, _p, _p,
                                           _p]
     handle.ckv_batched_leiden.restype = ctypes.c_int
+    handle.ckv_degree_weights.argtypes = [_p, _p, _p, _p, _i64, _i32, _i32, _i32, _p, _p, _p]
+    handle.ckv_degree_weights.restype = ctypes.c_int
+    handle.ckv_leiden_run_workspace_bytes.argtypes = [_i64, _i32, _i32]
+    handle.ckv_leiden_run_workspace_bytes.restype = ctypes.c_size_t
+    handle.ckv_leiden_run.argtypes = [_p, _p, _p, _i64, _i32, _i32, _i32, _f32, _f32, _i32, _i32, _i32, _p, _p,
+                                      ctypes.POINTER(_i32), ctypes.POINTER(ctypes.c_double), _p, _p]
+    handle.ckv_leiden_run.restype = ctypes.c_int
+    handle.ckv_dense_communities_workspace_bytes.argtypes = [_i32, _i32, _i32]
+    handle.ckv_dense_communities_workspace_bytes.restype = ctypes.c_size_t
+    handle.ckv_dense_communities.argtypes = [_p, _i32, _i32, _i32, _p, _p, _p, _p]
+    handle.ckv_dense_communities.restype = ctypes.c_int
     handle.ckv_leiden_test_raise_overflow.argtypes = [_i32]
     handle.ckv_leiden_test_raise_overflow.restype = None
     handle.ckv_aggregate_coo_workspace_bytes.argtypes = [_i64]

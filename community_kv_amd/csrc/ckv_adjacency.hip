@@ -36,6 +36,7 @@
 #include "ckv_amd.h"
 #include "ckv_error.h"
 #include "ckv_sort.h"
+#include "ckv_table.h"
 
 namespace ckv {
 namespace {
@@ -56,7 +57,6 @@ constexpr int MAP_WORDS = 4096;        // id bitmap of a graph: up to 131,072 ve
 constexpr int DENSE_THREADS = 1024;
 constexpr int DENSE_WINDOW = 16384;    // ids per window: 128 KB of f64 sums
 constexpr int DENSE_BLOCKS = 256;
-constexpr uint32_t EMPTY = 0xffffffffu;
 
 struct TopkGraph {
   const int32_t* idx;    // [G * R][K]
@@ -67,19 +67,6 @@ struct TopkGraph {
   float half_lam, co_lam;
   int co;                // co-occurrence edges (lam < 1)
 };
-
-__device__ inline int lane() { return (int)__lane_id(); }
-// Orders the wave's LDS accesses (all lanes' writes before, reads after).
-__device__ inline void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-__device__ inline double wave_sum_f64(double x) {
-  for (int o = 32; o >= 1; o >>= 1) x += __shfl_xor(x, o);
-  return x;
-}
-__device__ inline uint32_t hash_id(uint32_t x) { return (x * 0x9E3779B1u) >> 8; }
 
 // Postings [first, last) of one vertex.
 struct Run {
@@ -207,33 +194,6 @@ __device__ __forceinline__ void walk(const TopkGraph& t, const uint32_t* __restr
   }
 }
 
-// Inserts (u, w) into an open-addressing table of size slots (a power of two);
-// returns the number of probes that found no place, 0 when placed.
-__device__ inline bool insert(uint32_t* tk, double* ts, uint32_t size, uint32_t u, float w, int* added) {
-  uint32_t h = hash_id(u) & (size - 1);
-  for (uint32_t probe = 0; probe < size; ++probe) {
-    const uint32_t cur = __hip_atomic_load(tk + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    bool mine = cur == u;
-    if (cur == EMPTY) {
-      const uint32_t prev = atomicCAS(tk + h, EMPTY, u);
-      mine = prev == EMPTY || prev == u;
-      if (prev == EMPTY && added) atomicAdd(added, 1);
-    }
-    if (mine) {
-      unsafeAtomicAdd(ts + h, (double)w);
-      return true;
-    }
-    h = (h + 1) & (size - 1);
-  }
-  return false;
-}
-
-__device__ inline uint32_t table_size(uint64_t most, uint32_t cap) {
-  uint32_t size = 64;
-  while (size < 2 * most && size < cap) size <<= 1;
-  return size;
-}
-
 // The edges of one run [a, b) of vertex v by one wave.
 template <int KT>
 __device__ __forceinline__ void gather_run(const TopkGraph& t, const uint32_t* __restrict__ postings, uint32_t a,
@@ -248,7 +208,7 @@ __device__ __forceinline__ void gather_run(const TopkGraph& t, const uint32_t* _
     tk[j] = EMPTY;
     ts[j] = 0.0;
   }
-  wave_sync();
+  wave_lds_sync();
   double self = 0.0;
   bool any_self = false;
   walk<KT>(t, postings, a, n, (uint32_t)ln, 64u, v, base,
@@ -258,7 +218,7 @@ __device__ __forceinline__ void gather_run(const TopkGraph& t, const uint32_t* _
              if (c.ok) insert(tk, ts, size, c.u, c.w, nullptr);  // (never more ids than the table holds)
            },
            [] { return false; });
-  wave_sync();
+  wave_lds_sync();
   self = wave_sum_f64(self);
   const int lead = __ballot(any_self) != 0 ? 1 : 0;
   // Compact the occupied slots to the front (every lane has read its slots
@@ -272,7 +232,7 @@ __device__ __forceinline__ void gather_run(const TopkGraph& t, const uint32_t* _
     k[i] = j < size ? tk[j] : EMPTY;
     w[i] = k[i] != EMPTY ? (float)ts[j] : 0.0f;
   }
-  wave_sync();
+  wave_lds_sync();
   float* tw = reinterpret_cast<float*>(ts);
   int m = 0;
 #pragma unroll
@@ -286,7 +246,7 @@ __device__ __forceinline__ void gather_run(const TopkGraph& t, const uint32_t* _
     m += __popcll(used);
   }
   if (ln < 4 && m + ln < WAVE_SLOTS) tk[m + ln] = EMPTY;  // fills the last group of four
-  wave_sync();
+  wave_lds_sync();
   const int64_t out = (int64_t)a * (t.K + 1);
   if (lead && ln == 0) {
     tmp_id[out] = (uint32_t)v;
@@ -303,7 +263,7 @@ __device__ __forceinline__ void gather_run(const TopkGraph& t, const uint32_t* _
     tmp_w[out + lead + rank] = tw[i];
   }
   if (ln == 0) count[a] = lead + m;
-  wave_sync();  // the wave's next run clears the table
+  wave_lds_sync();  // the wave's next run clears the table
 }
 
 // End of the run of v that starts before `end` and goes on there: the first

@@ -507,6 +507,120 @@ __global__ __launch_bounds__(EDGE_THREADS) void edge_weight_kernel(
   }
 }
 
+// The same weights where the vertices' degrees are known (row sums of the
+// graph, a self loop counted twice): an edge's two ends add its weight to
+// their communities, so a community weighs the sum of its members' degrees.
+// 262,144 degrees in place of 9.8 M edges with two label reads and LDS adds
+// each: 488 us (8 graphs of 32,768, 13,000 communities) and 1,434 us (32 of
+// 8,192) in edge_weight_kernel, 150 us with the totals here.
+constexpr int DEGREE_THREADS = 256;
+
+__global__ __launch_bounds__(DEGREE_THREADS) void degree_weight_kernel(
+    const int32_t* __restrict__ labels, const double* __restrict__ degree, int seq_len, int graphs, int capacity,
+    float* __restrict__ weight) {
+  const int64_t v = (int64_t)blockIdx.x * DEGREE_THREADS + threadIdx.x;
+  if (v >= (int64_t)graphs * seq_len) return;
+  const int g = (int)(v / seq_len);
+  const int c = labels[v];
+  const float w = (float)degree[v];
+  if (c >= 0 && c < capacity && w != 0.0f) unsafeAtomicAdd(weight + (int64_t)g * capacity + c, w);
+}
+
+// The graphs' totals.  In edge_weight_kernel a block of EDGES_PER_WG edges
+// sends one sum to the graph of its first edge, and the edges of the graphs
+// that begin inside the block are added to their totals one by one, 8,000
+// atomics on one word (430 us); the block sums arrive after about 1,500 of them
+// with 8 graphs, after 4,000 with 32 (whose atomics queue with theirs).  Float
+// totals of 10^5 depend on that order by up to 3e-5 (a single edge is smaller
+// than half their last bit), so it is kept, with the single edges added in a
+// register: one wave per graph, before and after the blocks (within 7e-6 of
+// the atomics on 4,000 to 32,768 positions, 2 to 32 graphs; 140 us in all at
+// 9.8 M edges).
+constexpr int REST_EARLY_PER_GRAPH = 192, REST_EARLY_MOST = 4096;
+
+__global__ __launch_bounds__(EDGE_THREADS) void edge_total_kernel(const int32_t* __restrict__ src,
+                                                                  const float* __restrict__ w, int64_t edges,
+                                                                  int seq_len, float* __restrict__ total) {
+  constexpr int U = 8;
+  const int64_t e0 = (int64_t)blockIdx.x * EDGES_PER_WG;
+  const int64_t e1 = min(edges, e0 + EDGES_PER_WG);
+  const int g0 = src[e0] / seq_len;
+  const bool whole = src[e1 - 1] / seq_len == g0;  // (the list is grouped by graph)
+  float mine = 0.0f;
+  for (int64_t b = e0 + threadIdx.x; b < e1; b += U * EDGE_THREADS) {
+    float x[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t e = min(b + u * EDGE_THREADS, e1 - 1);
+      x[u] = gload_f32(w + e);
+      if (!whole && src[e] / seq_len != g0) x[u] = 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (b + u * EDGE_THREADS < e1) mine = mine + 2.0f * x[u];
+    }
+  }
+  __shared__ float s_part[EDGE_THREADS / 64];
+  mine = wave_sum_tree(mine);
+  if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = mine;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float t = 0.0f;
+    for (int i = 0; i < EDGE_THREADS / 64; ++i) t = t + s_part[i];
+    unsafeAtomicAdd(total + g0, t);
+  }
+}
+
+// t plus the edges [e0, last) of graph g in order, up to the graph's end.
+__device__ inline float add_edges(const int32_t* __restrict__ src, const float* __restrict__ w, int64_t e0,
+                                  int64_t last, int g, int seq_len, float t) {
+  const int lane = lane_id();
+  for (; e0 < last; e0 += 64) {
+    const int64_t e = min(e0 + lane, last - 1);
+    const float x = 2.0f * w[e];
+    const int n = __popcll(__ballot(e0 + lane < last && src[e] / seq_len == g));
+    if (n == 64) {
+#pragma unroll
+      for (int i = 0; i < 64; ++i) t = t + ckv_u2f((uint32_t)__builtin_amdgcn_readlane((int)ckv_f2u(x), i));
+    } else {
+      for (int i = 0; i < n; ++i) t = t + ckv_u2f((uint32_t)__builtin_amdgcn_readlane((int)ckv_f2u(x), i));
+      break;
+    }
+  }
+  return t;
+}
+
+// One wave per graph: its edges that lie in an earlier graph's block, the
+// first `early` of them into a cleared total (late == 0) or the others.
+__global__ __launch_bounds__(64) void edge_rest_kernel(const int32_t* __restrict__ src, const float* __restrict__ w,
+                                                       int64_t edges, int seq_len, int early, int late,
+                                                       float* __restrict__ total) {
+  const int g = blockIdx.x;
+  const int lane = threadIdx.x;
+  const int64_t v0 = (int64_t)g * seq_len;
+  // the first edge of this graph or a later one, 64 probes a round
+  int64_t lo = 0, hi = edges;
+  while (lo < hi) {
+    const int64_t step = (hi - lo + 63) / 64;
+    const int64_t at = lo + (int64_t)lane * step;
+    const uint64_t here = __ballot(at >= hi || src[min(at, hi - 1)] >= v0);
+    const int f = here ? __builtin_ctzll(here) : 64;  // probe f is the first at or past the graph
+    const int64_t top = lo + (int64_t)f * step;
+    if (f > 0) lo = lo + (int64_t)(f - 1) * step + 1;
+    hi = min(hi, top);
+  }
+  const int64_t last = min(edges, (lo + EDGES_PER_WG - 1) / EDGES_PER_WG * EDGES_PER_WG);
+  const int64_t mid = min(last, lo + early);
+  const float t = late ? add_edges(src, w, mid, last, g, seq_len, total[g]) : add_edges(src, w, lo, mid, g, seq_len, 0.0f);
+  if (lane == 0) total[g] = t;
+}
+
+__global__ void weight_zero_kernel(float* __restrict__ weight, int64_t n, float* __restrict__ total, int graphs) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) weight[i] = 0.0f;
+  if (i < graphs) total[i] = 0.0f;
+}
+
 // Modularity weights straight from the prefill top-k edges: one thread per
 // (query head, row).  With the row's valid columns k (score p_k), S = sum p_k:
 // the direct edges (position, column k) weigh lam/2 p_k, the co-occurrence
@@ -725,6 +839,33 @@ extern "C" int ckv_build_layer_state(const ckv_state_build_args* a, void* stream
                          dim3(EDGE_THREADS), (size_t)lds_n * sizeof(float), s, a->labels, a->seq_len, a->graphs,
                          a->community_capacity, lds_n, a->edge_src, a->edge_dst, a->edge_weight, a->edges, a->community_weight, a->total_weight);
     }
+  }
+  return launch_check();
+}
+
+extern "C" int ckv_degree_weights(const int32_t* labels, const double* degree, const int32_t* edge_src,
+                                  const float* edge_weight, int64_t edges, int32_t graphs, int32_t seq_len,
+                                  int32_t community_capacity, float* community_weight, float* total_weight,
+                                  void* stream) {
+  if (!labels || !degree || !community_weight || !total_weight || (edges > 0 && (!edge_src || !edge_weight)))
+    return ckv_internal::set_error(CKV_E_INVALID, "null degree-weight argument");
+  if (graphs <= 0 || seq_len <= 0 || community_capacity <= 0 || edges < 0)
+    return ckv_internal::set_error(CKV_E_INVALID, "graphs, seq_len and community_capacity must be positive");
+  const hipStream_t s = (hipStream_t)stream;
+  const int64_t n = (int64_t)graphs * community_capacity, v = (int64_t)graphs * seq_len;
+  hipLaunchKernelGGL(weight_zero_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, community_weight, n,
+                     total_weight, graphs);
+  hipLaunchKernelGGL(degree_weight_kernel, dim3((unsigned)((v + DEGREE_THREADS - 1) / DEGREE_THREADS)),
+                     dim3(DEGREE_THREADS), 0, s, labels, degree, seq_len, graphs, community_capacity,
+                     community_weight);
+  if (edges > 0) {
+    const int early = std::min(REST_EARLY_MOST, REST_EARLY_PER_GRAPH * graphs);
+    hipLaunchKernelGGL(edge_rest_kernel, dim3(graphs), dim3(64), 0, s, edge_src, edge_weight, edges, seq_len, early, 0,
+                       total_weight);
+    hipLaunchKernelGGL(edge_total_kernel, dim3((unsigned)((edges + EDGES_PER_WG - 1) / EDGES_PER_WG)),
+                       dim3(EDGE_THREADS), 0, s, edge_src, edge_weight, edges, seq_len, total_weight);
+    hipLaunchKernelGGL(edge_rest_kernel, dim3(graphs), dim3(64), 0, s, edge_src, edge_weight, edges, seq_len, early, 1,
+                       total_weight);
   }
   return launch_check();
 }

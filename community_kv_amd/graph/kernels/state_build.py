@@ -67,10 +67,12 @@ class StateBuild:
                  retrieval_to_kv: torch.Tensor, num_sink: int, max_decode_tokens: int, fp8: bool = True,
                  edges: tuple[torch.Tensor, torch.Tensor, torch.Tensor] | None = None,
                  token_capacity: int | None = None, topk_edges: "TopkEdges | None" = None,
-                 count_sink_labels: bool = False):
+                 count_sink_labels: bool = False, vertex_degree: torch.Tensor | None = None):
         device = nat.require_device(community_ids, keys, retrieval_to_graph, retrieval_to_kv)
         if edges is not None and topk_edges is not None:
             raise ValueError("give either an edge list or top-k edges")
+        if vertex_degree is not None and edges is None:
+            raise ValueError("vertex degrees come with the edge list they belong to")
         if keys.ndim != 3 or keys.shape[-1] != nat.HEAD_DIM or keys.stride(-1) != 1:
             raise ValueError("keys must be [KV heads, sequence, 128] with unit dim stride")
         graphs, seq_len = community_ids.shape
@@ -80,6 +82,11 @@ class StateBuild:
             raise ValueError("num_sink must be below the sequence length")
         if retrieval_to_graph.dtype != torch.int32 or retrieval_to_kv.dtype != torch.int32:
             raise TypeError("aggregation mappings must be int32")
+        if vertex_degree is not None and (vertex_degree.dtype != torch.float64 or not vertex_degree.is_contiguous()
+                                          or vertex_degree.numel() != graphs * seq_len
+                                          or vertex_degree.device != device):
+            raise TypeError("vertex degrees must be contiguous float64, one per graph and position, on the labels' device")
+        self.degree = vertex_degree
         self.device = device
         self.ids = community_ids.to(torch.int32).contiguous()
         counts = label_counts(self.ids, num_sink=0 if count_sink_labels else num_sink)
@@ -138,17 +145,26 @@ class StateBuild:
             labels=nat.ptr(self.ids), keys=nat.ptr(keys), head_stride=keys.stride(0),
             token_stride=keys.stride(1), retrieval_to_graph=nat.ptr(self.maps[0]),
             retrieval_to_kv=nat.ptr(self.maps[1]), edge_src=nat.ptr(src), edge_dst=nat.ptr(dst),
-            edge_weight=nat.ptr(w), edges=n_edges, graphs=graphs, seq_len=seq_len, num_sink=num_sink,
+            edge_weight=nat.ptr(w), edges=0 if vertex_degree is not None else n_edges, graphs=graphs, seq_len=seq_len, num_sink=num_sink,
             retrieval_heads=heads, kv_heads=keys.shape[0], key_dtype=nat.dtype_code(keys.dtype),
             centroid_dtype=nat.CKV_E4M3 if fp8 else nat.CKV_F32, max_communities=maxc,
             community_capacity=capacity, token_capacity=token_capacity,
             member_offsets=nat.ptr(o.member_offsets), member_positions=nat.ptr(o.member_positions),
             centroids=nat.ptr(o.centroids), community_sizes=nat.ptr(o.community_sizes),
-            community_weight=nat.ptr(o.community_weight), total_weight=nat.ptr(o.total_weight),
+            community_weight=None if vertex_degree is not None else nat.ptr(o.community_weight),
+            total_weight=None if vertex_degree is not None else nat.ptr(o.total_weight),
             token_communities=nat.ptr(o.token_communities), workspace=nat.ptr(self.workspace), **tk)
 
     def run(self) -> LayerStateTensors:
-        nat.check(nat.lib().ckv_build_layer_state(self.args, nat.stream_handle(self.device)))
+        stream = nat.stream_handle(self.device)
+        nat.check(nat.lib().ckv_build_layer_state(self.args, stream))
+        if self.degree is not None:
+            o = self.out
+            src, _, w = self.edges if self.edges is not None else (None, None, None)
+            nat.check(nat.lib().ckv_degree_weights(nat.ptr(self.ids), nat.ptr(self.degree), nat.ptr(src), nat.ptr(w),
+                                                   0 if src is None else src.numel(), self.ids.shape[0],
+                                                   self.ids.shape[1], o.community_weight.shape[1],
+                                                   nat.ptr(o.community_weight), nat.ptr(o.total_weight), stream))
         return self.out
 
 
@@ -156,18 +172,21 @@ def build_layer_state(community_ids: torch.Tensor, keys: torch.Tensor, *, retrie
                       retrieval_to_kv: torch.Tensor, num_sink: int, max_decode_tokens: int, fp8: bool = True,
                       edges: tuple[torch.Tensor, torch.Tensor, torch.Tensor] | None = None,
                       token_capacity: int | None = None, topk_edges: "TopkEdges | None" = None,
-                      count_sink_labels: bool = False) -> LayerStateTensors:
+                      count_sink_labels: bool = False,
+                      vertex_degree: torch.Tensor | None = None) -> LayerStateTensors:
     """Every prefill state tensor of one layer from labels ``[graphs, S]`` and
     keys ``[Hkv, S, 128]`` (bf16 or f32, token stride may exceed 128).  Reads
     the community counts back once to size the outputs, as the reference
     does with ``.item()``.  ``count_sink_labels`` counts communities over all
-    positions (sinks included) instead of the non-sink ones.  (The workspace and edge copies return to the
+    positions (sinks included) instead of the non-sink ones;
+    ``vertex_degree`` (f64, one per graph and position, of the graph of
+    ``edges``) saves the pass over the edges' labels where it is known.  (The workspace and edge copies return to the
     caching allocator on this stream, so later work on it cannot overwrite
     them before the launches run.)"""
     return StateBuild(community_ids, keys, retrieval_to_graph=retrieval_to_graph, retrieval_to_kv=retrieval_to_kv,
                       num_sink=num_sink, max_decode_tokens=max_decode_tokens, fp8=fp8, edges=edges,
                       token_capacity=token_capacity, topk_edges=topk_edges,
-                      count_sink_labels=count_sink_labels).run()
+                      count_sink_labels=count_sink_labels, vertex_degree=vertex_degree).run()
 
 
 __all__ = ["LayerStateTensors", "StateBuild", "TopkEdges", "build_layer_state", "label_counts"]

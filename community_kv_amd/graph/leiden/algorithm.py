@@ -1,16 +1,16 @@
 """Batched multi-level Leiden over the HIP kernels of ``ckv_leiden.hip``
 (reference: community_kv/graph/leiden/algorithm.py:1-202).
 
-Each level runs one ``ckv_batched_leiden`` (local moving + refinement, no host
-round trips inside), densifies the labels per graph (``ckv_densify_count`` /
-``ckv_densify_apply``) and contracts the edge list (``ckv_aggregate_coo``);
-the chain of relabellings is composed back to the original vertices.  The
-level loop reads two small device values per level (the densified width and
-the aggregated edge count), as the reference does.
+Device edges run ``ckv_leiden_run``: every level's local moving, refinement,
+densified labels and contraction on the device, one small read back per level.
+The extension's entry points (``batched_leiden``, ``aggregate_coo``) stay
+available one by one (``_load_module``); over host tensors ``run_leiden`` is
+the reference's own level loop around them.
 """
 
 from __future__ import annotations
 
+import ctypes
 import functools
 import os
 
@@ -106,6 +106,50 @@ def _densify_per_graph(labels: torch.Tensor, G: int, seq_len: int) -> tuple[torc
     return dense, width
 
 
+def native_run(edge_src: torch.Tensor, edge_dst: torch.Tensor, edge_weight: torch.Tensor, *, G: int, seq_len: int,
+               max_level: int, resolution: float, theta: float, max_inner_iter: int, seed: int,
+               use_boltzmann: bool) -> tuple[torch.Tensor, torch.Tensor, int, float]:
+    """``ckv_leiden_run`` over device edges (at least one): labels ``[G * seq_len]`` (graph * width + rank of
+    the community in its graph, -1 for vertices without edges), the vertices' degrees (f64), width, modularity."""
+    device = nat.require_device(edge_src, edge_dst, edge_weight)
+    _check_edges(edge_src, edge_dst, edge_weight)
+    if G <= 0 or seq_len <= 0:
+        raise RuntimeError("G and seq_len must be positive")
+    lib = nat.lib()
+    E = edge_src.numel()
+    labels = torch.empty(G * seq_len, dtype=torch.int32, device=device)
+    degree = torch.empty(G * seq_len, dtype=torch.float64, device=device)
+    ws = torch.empty(max(1, (lib.ckv_leiden_run_workspace_bytes(E, G, seq_len) + 7) // 8), dtype=torch.int64,
+                     device=device)
+    width, modularity = ctypes.c_int32(), ctypes.c_double()
+    rc = lib.ckv_leiden_run(nat.ptr(edge_src), nat.ptr(edge_dst), nat.ptr(edge_weight), E, G, seq_len, int(max_level),
+                            float(resolution), float(theta), int(max_inner_iter), int(seed),
+                            1 if use_boltzmann else 0, nat.ptr(labels), nat.ptr(degree), ctypes.byref(width),
+                            ctypes.byref(modularity), nat.ptr(ws), nat.stream_handle(device))
+    if rc != 0:
+        message = lib.ckv_last_error().decode(errors="replace")
+        if "same graph" in message:
+            raise ValueError("edges must join two vertices of the same graph, ids in [0, G * seq_len)")
+        if "overflowed" in message:
+            raise RuntimeError("Leiden: " + message)
+    nat.check(rc)
+    return labels, degree, int(width.value), float(modularity.value)
+
+
+def leiden_options(theta: float, max_inner_iter: int, use_boltzmann: bool) -> tuple[float, int, bool]:
+    """The options after the reference's environment overrides (algorithm.py:71-84)."""
+    theta_env = os.environ.get("COMMUNITY_KV_LEIDEN_THETA")
+    if theta_env is not None:
+        theta = float(theta_env)
+    iter_env = os.environ.get("COMMUNITY_KV_LEIDEN_MAX_INNER_ITER")
+    if iter_env is not None:
+        max_inner_iter = int(iter_env)
+    boltzmann_env = os.environ.get("COMMUNITY_KV_LEIDEN_BOLTZMANN")
+    if boltzmann_env is not None:
+        use_boltzmann = boltzmann_env not in ("", "0", "false", "False")
+    return theta, max_inner_iter, use_boltzmann
+
+
 def run_leiden(edge_src: torch.Tensor, edge_dst: torch.Tensor, edge_weight: torch.Tensor, *, G: int, seq_len: int,
                max_level: int = 6, resolution: float = 1.0, theta: float = 0.01, max_inner_iter: int = 16,
                seed: int = 0, use_boltzmann: bool = False) -> tuple[torch.Tensor, torch.Tensor, float]:
@@ -122,22 +166,22 @@ def run_leiden(edge_src: torch.Tensor, edge_dst: torch.Tensor, edge_weight: torc
     edge_weight = edge_weight.contiguous()
     V_orig = G * seq_len
     device = edge_src.device
+    theta, max_inner_iter, use_boltzmann = leiden_options(theta, max_inner_iter, use_boltzmann)
+    if device.type == "cuda":
+        if edge_src.numel() == 0:
+            none = torch.empty(0, dtype=torch.int32, device=device)
+            return none.long(), none, 0.0
+        labels, _, _, modularity = native_run(edge_src, edge_dst, edge_weight, G=G, seq_len=seq_len,
+                                              max_level=max_level, resolution=resolution, theta=theta,
+                                              max_inner_iter=max_inner_iter, seed=seed, use_boltzmann=use_boltzmann)
+        vertex = torch.nonzero(labels >= 0, as_tuple=False).squeeze(-1)
+        return vertex, labels[vertex], modularity
     if edge_src.numel():
         # every edge inside one graph: the per-graph relabelling depends on it
         lo = torch.minimum(edge_src, edge_dst)
         bad = (lo < 0) | (torch.maximum(edge_src, edge_dst) >= V_orig) | (edge_src // seq_len != edge_dst // seq_len)
         if bool(bad.any()):
             raise ValueError("edges must join two vertices of the same graph, ids in [0, G * seq_len)")
-
-    theta_env = os.environ.get("COMMUNITY_KV_LEIDEN_THETA")
-    if theta_env is not None:
-        theta = float(theta_env)
-    iter_env = os.environ.get("COMMUNITY_KV_LEIDEN_MAX_INNER_ITER")
-    if iter_env is not None:
-        max_inner_iter = int(iter_env)
-    boltzmann_env = os.environ.get("COMMUNITY_KV_LEIDEN_BOLTZMANN")
-    if boltzmann_env is not None:
-        use_boltzmann = boltzmann_env not in ("", "0", "false", "False")
 
     level_modularity = []
     labels0, mod0 = module.batched_leiden(edge_src, edge_dst, edge_weight, G, seq_len, max_level, float(resolution),
@@ -217,4 +261,4 @@ def _compute_disjoint_modularity(edge_src: torch.Tensor, edge_dst: torch.Tensor,
     return in_total / two_m - resolution * float((sigma * sigma).sum()) / (two_m * two_m)
 
 
-__all__ = ["run_leiden"]
+__all__ = ["leiden_options", "native_run", "run_leiden"]

@@ -38,6 +38,7 @@ class PartitionResult:
     edge_src: torch.Tensor
     edge_dst: torch.Tensor
     edge_weight: torch.Tensor
+    degree: torch.Tensor | None = None  # the vertices' degrees, f64 [graphs * S] (None without edges)
 
 
 @dataclass(slots=True)
@@ -210,13 +211,15 @@ def build_layer_from_labels(*, layer_idx: int, community_ids: torch.Tensor, keys
                             num_sink: int, max_decode_tokens: int, query_heads: int,
                             aggregation: GraphAggregation = GraphAggregation.PER_QUERY_HEAD,
                             edges: tuple[torch.Tensor, torch.Tensor, torch.Tensor] | None = None,
-                            fp8: bool = True, topk_edges: Any = None,
-                            count_sink_labels: bool = False) -> PartitionedLayer:
+                            fp8: bool = True, topk_edges: Any = None, count_sink_labels: bool = False,
+                            vertex_degree: torch.Tensor | None = None) -> PartitionedLayer:
     """Everything ``build_partitioned_layer`` (partition.py:538-618) produces
     after Leiden, from given dense labels ``community_ids [graphs, S]``.  The
     modularity weights come from ``edges`` (a coalesced edge list) or from
     ``topk_edges`` (a ``graph.kernels.state_build.TopkEdges``: the prefill
-    top-k edges, device tensors only), or are zero.  The community count is
+    top-k edges, device tensors only), or are zero; ``vertex_degree`` (the f64
+    degrees of the graph of ``edges``, device tensors only) saves the pass over
+    the edges' labels.  The community count is
     1 + the largest non-sink label, or, with ``count_sink_labels``, 1 + the
     largest label of any position (the reference's count after Leiden, whose
     sink singletons may carry the largest ids)."""
@@ -234,7 +237,7 @@ def build_layer_from_labels(*, layer_idx: int, community_ids: torch.Tensor, keys
 
         st = build_layer_state(ids, keys, retrieval_to_graph=to_graph, retrieval_to_kv=to_kv, num_sink=num_sink,
                                max_decode_tokens=max_decode_tokens, fp8=fp8, edges=edges, topk_edges=topk_edges,
-                               count_sink_labels=count_sink_labels)
+                               count_sink_labels=count_sink_labels, vertex_degree=vertex_degree)
         return PartitionedLayer(layer_idx=layer_idx, prefill_seq_len=seq_len, aggregation=aggregation,
                                 query_heads=query_heads, kv_heads=kv_heads, retrieval_to_graph=to_graph,
                                 retrieval_to_kv=to_kv, member_offsets=st.member_offsets,
@@ -242,8 +245,8 @@ def build_layer_from_labels(*, layer_idx: int, community_ids: torch.Tensor, keys
                                 centroids=st.centroids, community_sizes=st.community_sizes,
                                 community_weight=st.community_weight, total_weight=st.total_weight,
                                 token_communities=st.token_communities)
-    if topk_edges is not None:
-        raise ValueError("top-k edges are taken by the device state build only; pass a coalesced edge list")
+    if topk_edges is not None or vertex_degree is not None:
+        raise ValueError("top-k edges and degrees are taken by the device state build only; pass a coalesced edge list")
     counts = (ids[:, 0 if count_sink_labels else num_sink:].amax(dim=1) + 1).to(torch.int32)
     centroids, sizes = compute_centroids(ids, counts, keys, retrieval_to_graph=to_graph, retrieval_to_kv=to_kv,
                                          num_sink=num_sink, max_decode_tokens=max_decode_tokens, fp8=fp8)
@@ -287,14 +290,6 @@ def _reshape_by_aggregation(topk_indices: torch.Tensor, topk_scores: torch.Tenso
             base.repeat(query_heads).unsqueeze(0))
 
 
-def _scatter_membership(vertex: torch.Tensor, labels: torch.Tensor, *, graph_count: int,
-                        seq_len: int) -> torch.Tensor:
-    """partition.py:252-266: Leiden labels into a [graphs, S] table, -1 elsewhere."""
-    membership = torch.full((graph_count * seq_len,), -1, dtype=torch.int32, device=vertex.device)
-    membership[vertex] = labels
-    return membership.view(graph_count, seq_len)
-
-
 def _fill_isolated_vertices(membership: torch.Tensor) -> torch.Tensor:
     """partition.py:269-273: vertices without edges become singletons numbered
     after the graph's largest label, in position order."""
@@ -321,25 +316,32 @@ def partition_graphs(topk_indices: torch.Tensor, topk_scores: torch.Tensor, *, a
                      leiden_seed: int) -> PartitionResult:
     """Top-k edges -> coalesced graph -> native batched Leiden -> dense
     per-graph community ids (partition.py:289-353).  Device tensors only."""
-    from community_kv_amd.graph.leiden import run_leiden
+    from community_kv_amd import _native as nat
+    from community_kv_amd.graph.leiden.algorithm import leiden_options, native_run
 
     grouped_idx, grouped_scores, positions = _reshape_by_aggregation(
         topk_indices, topk_scores, aggregation=aggregation, num_kv_heads=num_kv_heads, num_sink=num_sink)
+    device = nat.require_device(grouped_idx, grouped_scores)
     graph_count = grouped_idx.shape[0]
     src, dst, weight = build_adjacency(grouped_idx, grouped_scores, positions, seq_len=prefill_seq_len, lam=lam)
+    degree, width, modularity = None, 0, 0.0
     if src.numel():
-        vertex, labels, modularity = run_leiden(src, dst, weight, G=graph_count, seq_len=prefill_seq_len,
-                                                resolution=leiden_resolution,
-                                                max_inner_iter=leiden_max_iterations(prefill_seq_len),
-                                                seed=leiden_seed)
-        membership = _scatter_membership(vertex, labels, graph_count=graph_count, seq_len=prefill_seq_len)
+        theta, sweeps, boltzmann = leiden_options(0.01, leiden_max_iterations(prefill_seq_len), False)
+        labels, degree, width, modularity = native_run(src, dst, weight, G=graph_count, seq_len=prefill_seq_len,
+                                                       max_level=6, resolution=leiden_resolution, theta=theta,
+                                                       max_inner_iter=sweeps, seed=leiden_seed,
+                                                       use_boltzmann=boltzmann)
     else:
-        modularity = 0.0
-        membership = torch.full((graph_count, prefill_seq_len), -1, dtype=torch.int32, device=topk_indices.device)
-    community_ids = _dense_remap(_fill_isolated_vertices(membership))
-    community_counts = (community_ids.amax(dim=1) + 1).to(torch.int32)
+        labels = torch.full((graph_count * prefill_seq_len,), -1, dtype=torch.int32, device=device)
+    community_ids = torch.empty((graph_count, prefill_seq_len), dtype=torch.int32, device=device)
+    community_counts = torch.empty(graph_count, dtype=torch.int32, device=device)
+    lib = nat.lib()
+    ws = torch.empty(lib.ckv_dense_communities_workspace_bytes(graph_count, prefill_seq_len, width), dtype=torch.uint8,
+                     device=device)
+    nat.check(lib.ckv_dense_communities(nat.ptr(labels), graph_count, prefill_seq_len, width, nat.ptr(community_ids),
+                                        nat.ptr(community_counts), nat.ptr(ws), nat.stream_handle(device)))
     return PartitionResult(community_ids=community_ids, community_counts=community_counts, modularity=modularity,
-                           edge_src=src, edge_dst=dst, edge_weight=weight)
+                           edge_src=src, edge_dst=dst, edge_weight=weight, degree=degree)
 
 
 def partition_query_groups(topk_indices: torch.Tensor, topk_scores: torch.Tensor, *, num_kv_heads: int,
@@ -357,7 +359,7 @@ def build_partitioned_layer(*, layer_idx: int, topk_indices: torch.Tensor, topk_
                             aggregation: GraphAggregation = GraphAggregation.PER_QUERY_HEAD) -> PartitionedLayer:
     """Full prefill partition of one layer and its decode state
     (partition.py:538-618): Leiden on the top-k graph, then the state build
-    with the community count over all positions, sinks included, as the
+    (modularity weights from the graph's degrees) with the community count over all positions, sinks included, as the
     reference counts them."""
     if max_decode_tokens <= 0:
         raise ValueError("max_decode_tokens must be positive")
@@ -370,7 +372,7 @@ def build_partitioned_layer(*, layer_idx: int, topk_indices: torch.Tensor, topk_
     return build_layer_from_labels(layer_idx=layer_idx, community_ids=result.community_ids, keys=keys,
                                    num_sink=num_sink, max_decode_tokens=max_decode_tokens,
                                    query_heads=topk_indices.shape[0], aggregation=aggregation, edges=edges,
-                                   count_sink_labels=True)
+                                   count_sink_labels=True, vertex_degree=result.degree)
 
 
 __all__ = [

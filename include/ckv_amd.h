@@ -28,8 +28,8 @@
  *                           prefill_attention_topk()          attention/flash_attention.py:23-51
  *                           (patched FA3 op, third_party/flash_attention/community-kv.patch:31-120)
  *   ckv_label_counts,       the state build of build_partitioned_layer() after Leiden
- *   ckv_build_layer_state   (graph/partition.py:538-618): compute_centroids 382-454,
- *                           build_member_csr 457-492, init_modularity_state 495-535
+ *   ckv_build_layer_state,  (graph/partition.py:538-618): compute_centroids 382-454,
+ *   ckv_degree_weights      build_member_csr 457-492, init_modularity_state 495-535
  *   ckv_build_adjacency     build_adjacency()                 graph/partition.py:168-249
  *   ckv_batched_leiden      batched_leiden() of the Leiden extension (graph/leiden/_csrc/bindings.cpp:40-103,
  *                           launch_batched_leiden in leiden.cu:43-205), called by run_leiden()
@@ -302,6 +302,14 @@ size_t ckv_state_workspace_bytes(int32_t graphs, int32_t retrieval_heads, int32_
 int ckv_label_counts(const int32_t* labels, int32_t graphs, int32_t seq_len, int32_t num_sink,
                      int32_t* community_counts, void* stream);
 int ckv_build_layer_state(const ckv_state_build_args* args, void* stream);
+/* init_modularity_state() where the vertices' degrees are known (f64
+ * [graphs][seq_len], as ckv_leiden_run leaves them): community_weight[g][c] =
+ * degrees of the positions labelled c (labels outside
+ * [0, community_capacity) are dropped), total_weight[g] = twice the weight of
+ * the graph's edges (the coalesced list that the degrees belong to). */
+int ckv_degree_weights(const int32_t* labels, const double* degree, const int32_t* edge_src, const float* edge_weight,
+                       int64_t edges, int32_t graphs, int32_t seq_len, int32_t community_capacity,
+                       float* community_weight, float* total_weight, void* stream);
 
 /* One Leiden level over `graphs` vertex-disjoint graphs of seq_len vertices
  * each (vertex ids g * seq_len + i).  Edges: upper-triangular COO (self loops
@@ -319,11 +327,39 @@ int ckv_batched_leiden(const int32_t* edge_src, const int32_t* edge_dst, const f
                        int32_t seed, int32_t use_boltzmann, int32_t* labels, double* modularity,
                        void* workspace, void* stream);
 
+/* The multi-level run of run_leiden() (graph/leiden/algorithm.py:51-161):
+ * levels of local moving, refinement and contraction until max_level levels
+ * have run or a level merges nothing.  Edges as above, at least one, both ends
+ * in the same graph (else CKV_E_INVALID); an ascending (src, dst) list, as
+ * ckv_build_adjacency leaves it, is taken without the general sort.  Outputs:
+ * labels [graphs * seq_len] (device; graph * *width + rank of the community
+ * among its graph's, -1 for vertices without edges), degree [graphs * seq_len]
+ * (device f64; row sums, a self loop counted twice), and on the host *width
+ * (the largest number of communities of a graph) and *result (modularity of
+ * the disjoint union).  SYNCHRONISES the stream once per level and at the end
+ * (a level's size decides the next one's launches), so it is not for capture;
+ * workspace of ckv_leiden_run_workspace_bytes(edges, graphs, seq_len) bytes. */
+size_t ckv_leiden_run_workspace_bytes(int64_t edges, int32_t graphs, int32_t seq_len);
+int ckv_leiden_run(const int32_t* edge_src, const int32_t* edge_dst, const float* edge_weight, int64_t edges,
+                   int32_t graphs, int32_t seq_len, int32_t max_level, float resolution, float theta,
+                   int32_t max_inner_iter, int32_t seed, int32_t use_boltzmann, int32_t* labels, double* degree,
+                   int32_t* width, double* result, void* workspace, void* stream);
+
+/* Labels of a Leiden run (graph g's in [g * width, (g + 1) * width), -1 for
+ * vertices without edges) to dense community ids per graph: each label becomes
+ * its rank among its graph's labels, the vertices without edges become
+ * singletons after them in position order (graph/partition.py:252-286).
+ * community_counts [graphs]. */
+size_t ckv_dense_communities_workspace_bytes(int32_t graphs, int32_t seq_len, int32_t width);
+int ckv_dense_communities(const int32_t* labels, int32_t graphs, int32_t seq_len, int32_t width,
+                          int32_t* community_ids, int32_t* community_counts, void* workspace, void* stream);
+
 /* Test hook with no counterpart in the reference: while enabled, every
- * ckv_batched_leiden call raises its table-overflow word after the
- * local-moving sweeps, as a broken neighbour-table bound would, so a test can
- * check that the flag survives refinement and turns the level's modularity
- * into NaN (run_leiden then raises).  Process-wide, not thread-safe. */
+ * ckv_batched_leiden call and level of a ckv_leiden_run raises its
+ * table-overflow word after the local-moving sweeps, as a broken
+ * neighbour-table bound would, so a test can check that the flag survives
+ * refinement and turns the call's modularity into NaN, or the run into an
+ * error (run_leiden then raises).  Process-wide, not thread-safe. */
 void ckv_leiden_test_raise_overflow(int32_t enable);
 
 /* Contract an upper-triangular COO by `labels` (super-vertex per vertex, in

@@ -280,3 +280,72 @@ def test_build_adjacency_run_lengths(device, G, R, kappa, S, hubs, share):
         ref = co.build_adjacency(idx, sc, pos, seq_len=S, lam=lam)
         for a, b in zip(got, ref):
             np.testing.assert_array_equal(a.cpu().numpy(), b)
+
+
+CONTRACTIONS = [
+    # seed, graphs, seq_len, hub leaves, isolated, shuffled: rows of one member, many members, a workgroup's and dense
+    (41, 2, 700, 0, 5, False),
+    (42, 1, 2400, 1500, 0, False),
+    (43, 3, 500, 0, 0, True),
+    (44, 1, 20000, 17000, 100, False),
+    (45, 1, 20000, 17000, 0, True),
+]
+
+
+@pytest.mark.parametrize("seed,G,S,leaves,isolated,shuffled", CONTRACTIONS)
+def test_run_leiden_contractions(device, seed, G, S, leaves, isolated, shuffled):
+    """The whole native run on sorted edge lists and on shuffled ones (general
+    sort), with hubs whose contracted rows take one wave, one workgroup and
+    dense windows of ids: labels equal the oracle's level by level (dyadic
+    weights: every sum exact), degrees equal the rows' sums."""
+    src, dst, w = lg.planted(seed, G, S, 12, edges_per_vertex=5.0, self_loops=4, isolated=isolated)
+    if leaves:  # one vertex joined to many, as a token every row attends to
+        rng = np.random.default_rng(seed)
+        far = rng.choice(np.arange(1, S - isolated), leaves, replace=False).astype(np.int32)
+        src = np.concatenate([src, np.zeros(leaves, np.int32)])
+        dst = np.concatenate([dst, far])
+        w = np.concatenate([w, (rng.integers(1, 5, leaves) / 64.0).astype(np.float32)])
+        total = int(G * S)
+        key, inv = np.unique(np.minimum(src, dst).astype(np.int64) * total + np.maximum(src, dst), return_inverse=True)
+        src, dst = (key // total).astype(np.int32), (key % total).astype(np.int32)
+        w = np.bincount(inv, weights=w).astype(np.float32)
+    else:
+        order = np.lexsort((dst, src))
+        src, dst, w = src[order], dst[order], w[order]
+    if shuffled:
+        order = np.random.default_rng(seed).permutation(src.size)
+        src, dst, w = src[order], dst[order], w[order]
+    print(f"leiden run G={G} S={S} edges={src.size} leaves={leaves} shuffled={shuffled}", flush=True)
+    s, d, x = _dev(device, src, dst, w)
+    vertex, part, q = algorithm.run_leiden(s, d, x, G=G, seq_len=S, max_inner_iter=5, seed=seed)
+    rv, rp, rq = L.run_leiden(src, dst, w, graphs=G, seq_len=S, max_inner_iter=5, seed=seed)
+    np.testing.assert_array_equal(vertex.cpu().numpy(), rv)
+    np.testing.assert_array_equal(part.cpu().numpy(), rp)
+    assert q == pytest.approx(rq, abs=1e-9)
+    labels, degree, width, _ = algorithm.native_run(s, d, x, G=G, seq_len=S, max_level=6, resolution=1.0, theta=0.01,
+                                                    max_inner_iter=5, seed=seed, use_boltzmann=False)
+    k = np.bincount(src, weights=w, minlength=G * S) + np.bincount(dst, weights=w, minlength=G * S)
+    np.testing.assert_array_equal(degree.cpu().numpy(), k)
+    assert (labels.cpu().numpy() < 0).sum() == G * S - rv.size and int(labels.max()) < G * width
+
+
+def test_dense_communities_match_oracle(device):
+    """Native fill of isolated vertices and dense renumbering against the oracle's two steps."""
+    from community_kv_amd import _native as nat
+
+    rng = np.random.default_rng(9)
+    for G, S, W in ((3, 257, 40), (1, 64, 1), (2, 5, 0)):
+        lab = np.full((G, S), -1, np.int32)
+        if W:
+            lab = (rng.integers(0, W, (G, S)) + np.arange(G)[:, None] * W).astype(np.int32)
+            lab[rng.random(lab.shape) < 0.2] = -1
+        t = torch.from_numpy(lab).to(device)
+        ids = torch.empty_like(t)
+        counts = torch.empty(G, dtype=torch.int32, device=device)
+        ws = torch.empty(nat.lib().ckv_dense_communities_workspace_bytes(G, S, W), dtype=torch.uint8, device=device)
+        print(f"dense communities G={G} S={S} W={W}", flush=True)
+        nat.check(nat.lib().ckv_dense_communities(t.data_ptr(), G, S, W, ids.data_ptr(), counts.data_ptr(),
+                                                  ws.data_ptr(), nat.stream_handle(t.device)))
+        ref = L.dense_remap(L.fill_isolated(lab))
+        np.testing.assert_array_equal(ids.cpu().numpy(), ref)
+        assert counts.cpu().tolist() == (ref.max(axis=1) + 1).tolist()

@@ -222,3 +222,29 @@ def test_state_build_topk_load_widths(device, kappa, offset):
         total[g] += (lam * s + (1 - lam) * (s * s + s2)).sum()
     np.testing.assert_allclose(st.community_weight.cpu().numpy(), weight, rtol=1e-4, atol=1e-4)
     np.testing.assert_allclose(st.total_weight.cpu().numpy(), total, rtol=1e-5)
+
+
+@pytest.mark.parametrize("graphs,seq_len,n", [(1, 300, 200), (3, 1000, 5000), (2, 4000, 40000), (5, 700, 9000)])
+def test_state_build_weights_from_degrees(device, graphs, seq_len, n):
+    """Weights from the vertices' degrees and totals from the edges equal those
+    of the edge list alone (dyadic weights, sums below 2^11: exact), with graphs
+    that end inside a block of 8,192 edges, span several, or share one."""
+    rng = np.random.default_rng(n)
+    ids = rng.integers(0, 50, (graphs, seq_len)).astype(np.int32)
+    src, dst, _ = _edges(rng, graphs, seq_len, 0, n)
+    w = (rng.integers(1, 64, n) / 4096.0).astype(np.float32)
+    degree = (np.bincount(src, weights=w, minlength=graphs * seq_len)
+              + np.bincount(dst, weights=w, minlength=graphs * seq_len))
+    keys = torch.zeros(graphs, seq_len, 128, dtype=torch.bfloat16, device=device)
+    tg = torch.arange(graphs, dtype=torch.int32, device=device)
+    edges = tuple(torch.from_numpy(e).to(device) for e in (src, dst, w))
+    print(f"state build degrees graphs={graphs} S={seq_len} edges={n}", flush=True)
+    kw = dict(retrieval_to_graph=tg, retrieval_to_kv=tg, num_sink=0, max_decode_tokens=4, edges=edges)
+    a = build_layer_state(torch.from_numpy(ids).to(device), keys, **kw)
+    b = build_layer_state(torch.from_numpy(ids).to(device), keys, vertex_degree=torch.from_numpy(degree).to(device), **kw)
+    assert torch.equal(a.community_weight, b.community_weight) and torch.equal(a.total_weight, b.total_weight)
+    np.testing.assert_array_equal(b.total_weight.cpu().numpy(),
+                                  np.bincount(src // seq_len, weights=2.0 * w, minlength=graphs).astype(np.float32))
+    with pytest.raises(ValueError, match="edge list"):
+        build_layer_state(torch.from_numpy(ids).to(device), keys, retrieval_to_graph=tg, retrieval_to_kv=tg, num_sink=0,
+                          max_decode_tokens=4, vertex_degree=torch.from_numpy(degree).to(device))

@@ -26,14 +26,11 @@
 // communities (the reference's table size), in order of first appearance.
 //
 // Launch sequence of ckv_batched_leiden (one stream, no host sync):
-//   mirror_kernel, radix sort, row_ptr_kernel, col_kernel, zero_kernel, hub_list_kernel, degree_kernel,
-//   graph_sum_kernel (2m), identity_kernel
-//   local moving x max_inner_iter: sigma_zero, sigma_scatter, local_moving_kernel (small rows, then
-//                                  hubs), local_moving_giant_kernel, lm_control_kernel
-//   refine_init_kernel, parent sigma
-//   refinement x max_inner_iter: sigma_zero, sigma_scatter, refine_propose_kernel (small, hubs),
-//                                refine_propose_giant_kernel,
-//                                refine_commit_kernel, refine_control_kernel
+//   mirror_kernel, radix sort, row_ptr_kernel, col_kernel, degree_kernel, graph_sum_kernel (2m)
+//   level_init_kernel, hub_list_kernel
+//   local moving x max_inner_iter: local_moving_kernel, local_moving_giant_kernel
+//   pair_init_kernel
+//   refinement x max_inner_iter: refine_propose_kernel, refine_propose_giant_kernel, refine_commit_kernel
 //   sigma of the result, modularity_kernel, graph_sum_kernel, finish_kernel (labels, -1 for isolated)
 //
 // ckv_leiden_run keeps the graph as a CSR from level to level.  The first
@@ -43,7 +40,7 @@
 // level's result contracts the CSR row by row in LDS hash tables, where the
 // edge list was relabelled, sorted by 64-bit keys, reduced, and sorted again
 // into a CSR (2.0 ms at 9.7 M edges, 0.35 ms now).  Launch sequence per level:
-//   level_init, hub_list, sweeps as above, flag_zero, flag_mark, scan, width
+//   level_init, hub_list, sweeps as above (giants only where rows can be so long), flag_zero, flag_mark, scan, width
 //   [the host reads the width], densify_apply, chain_kernel,
 //   agg_zero, agg_hist, scan, agg_fill (members by super-vertex), agg_list,
 //   agg_short (one wave per row), agg_long (workgroup), agg_dense, graph_sum
@@ -53,6 +50,7 @@
 #include <stdint.h>
 
 #include "ckv_amd.h"
+#include "ckv_device.h"
 #include "ckv_error.h"
 #include "ckv_sort.h"
 #include "ckv_table.h"
@@ -65,10 +63,18 @@ constexpr int LTHREADS = 64 * LWAVES;
 constexpr int TABLE_CAP = 1024;  // distinct neighbour communities per vertex
 constexpr int ETHREADS = 256;
 
-enum { CTL_MOVED = 0,  // nonzero once a vertex moved in the current sweep
-       CTL_UPDOWN = 1, CTL_STALE = 2, CTL_DONE = 3,
-       CTL_OVERFLOW = 4,  // nonzero when a workgroup table overflowed (a broken table bound)
-       CTL_WORDS = 8 };
+// Control words of a level.  A sweep marks its slot of its phase's ring when a
+// vertex moves; the next sweeps read the ring themselves, so no kernel runs
+// between sweeps to advance a state.  Every RING sweeps fold_kernel moves the
+// ring's outcome to the base words.
+constexpr int RING = 64;
+enum { CTL_OVERFLOW = 0,  // nonzero when a workgroup table overflowed (a broken table bound)
+       CTL_STALLS = 1,    // local moving: stalled sweeps before the ring, modulo 2
+       CTL_LAST = 2,      // the last sweep before the ring stalled
+       CTL_DONE = 3,      // the phase ended before the ring
+       CTL_LM = 4,                  // local moving's ring
+       CTL_REFINE = CTL_LM + RING,  // refinement's ring
+       CTL_WORDS = CTL_REFINE + RING };
 
 // ----------------------------------------------------------------- hashing (rng.cuh)
 __device__ __host__ inline uint32_t pcg_hash(uint32_t x) {
@@ -115,122 +121,48 @@ __device__ inline uint32_t ordered(float f) {
 __device__ inline uint64_t pack(float score, uint32_t pref) { return ((uint64_t)ordered(score) << 32) | pref; }
 
 // ----------------------------------------------------------------- wave helpers
-__device__ inline uint64_t wave_max_u64(uint64_t x) {
-  for (int o = 32; o >= 1; o >>= 1) {
-    const uint64_t y = (uint64_t)__shfl_xor((long long)x, o);
-    x = y > x ? y : x;
-  }
-  return x;
-}
 __device__ inline int first_lane(uint64_t m) { return __ffsll((long long)m) - 1; }
 
-// The control kernels only test the moved word for zero: set it once per
-// sweep (read first, so that later movers do not queue writes to one line).
-__device__ inline void mark_moved(int32_t* ctl) {
-  if (__hip_atomic_load(ctl + CTL_MOVED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
-    __hip_atomic_store(ctl + CTL_MOVED, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// Marks a sweep that moved a vertex (read first, so that later movers do not
+// queue writes to one line).
+__device__ inline void mark_moved(int32_t* word) {
+  if (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+    __hip_atomic_store(word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Neighbour-community table of vertex v over its row [a, b): self loops
-// skipped; with `parent`, only neighbours u with parent[u] == pv.  Returns the
-// number of table slots to scan (wave-uniform; empty slots hold -1); *e_sum
-// gets the summed weight of the admitted entries (every lane).
-//
-// Rows of at most CAP entries (all rows the per-wave kernels take): every
-// lane inserts its neighbour's community into an open-addressing table of
-// min(2 x degree, CAP) slots (LDS compare-and-swap) and adds its weight with an
-// LDS f64 atomic.  Longer rows (the workgroup kernels' fallback): a leader
-// loop over the chunk's distinct communities, entries in order of first
-// appearance along the row, later ones dropped once CAP are held.
-template <int CAP>
-__device__ int build_table(int32_t* tc, double* ts, const int32_t* __restrict__ col,
-                           const float* __restrict__ wt, const int32_t* __restrict__ lab,
-                           const int32_t* __restrict__ parent, int32_t pv, int32_t v, int32_t a, int32_t b,
-                           double* e_sum) {
-  const int ln = lane();
-  double e_acc = 0.0;
-  if (b - a <= CAP) {  // at most CAP distinct communities: no capacity rule to apply
-    int size = 64;
-    while (size < 2 * (b - a) && size < CAP) size <<= 1;
-    for (int j = ln; j < size; j += 64) {
-      tc[j] = -1;
-      ts[j] = 0.0;
-    }
-    __builtin_amdgcn_wave_barrier();
-    for (int32_t e0 = a; e0 < b; e0 += 64) {
-      const int32_t e = e0 + ln;
-      bool ok = e < b;
-      const int32_t u = ok ? col[e] : v;
-      ok = ok && u != v;
-      if (parent) ok = ok && parent[u] == pv;
-      if (ok) {
-        const float w = wt[e];
-        const int32_t c = lab[u];
-        e_acc += (double)w;
-        uint32_t h = pcg_hash((uint32_t)c) & (uint32_t)(size - 1);
-        while (true) {
-          const int32_t cur = __hip_atomic_load(tc + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-          if (cur == c) break;
-          if (cur == -1) {
-            const int32_t prev = atomicCAS(tc + h, -1, c);
-            if (prev == -1 || prev == c) break;
-          }
-          h = (h + 1) & (uint32_t)(size - 1);
-        }
-        unsafeAtomicAdd(ts + h, (double)w);
-      }
-    }
-    __builtin_amdgcn_wave_barrier();
-    *e_sum = wave_sum_f64(e_acc);
-    return size;
-  }
-  int n = 0;
-  for (int32_t e0 = a; e0 < b; e0 += 64) {
-    const int32_t e = e0 + ln;
-    bool ok = e < b;
-    const int32_t u = ok ? col[e] : v;
-    ok = ok && u != v;
-    const float w = ok ? wt[e] : 0.0f;
-    if (parent) ok = ok && parent[u] == pv;
-    const int32_t c = ok ? lab[u] : -1;
-    if (ok) e_acc += (double)w;
-    uint64_t active = __ballot(ok);
-    while (active) {
-      const int32_t c0 = __shfl(c, first_lane(active));
-      const uint64_t m = __ballot(ok && c == c0);
-      const double s = wave_sum_f64(((m >> ln) & 1) ? (double)w : 0.0);
-      int idx = -1;
-      for (int j0 = 0; j0 < n; j0 += 64) {
-        const int j = j0 + ln;
-        const uint64_t hit = __ballot(j < n && tc[j] == c0);
-        if (hit) {
-          idx = j0 + first_lane(hit);
-          break;
-        }
-      }
-      if (idx < 0 && n < CAP) {
-        idx = n++;
-        if (ln == 0) {
-          tc[idx] = c0;
-          ts[idx] = 0.0;
-        }
-      }
-      if (idx >= 0 && ln == 0) ts[idx] += s;
-      __builtin_amdgcn_wave_barrier();
-      active &= ~m;
-    }
-  }
-  *e_sum = wave_sum_f64(e_acc);
-  return n;
+// Local moving before sweep `sweep` (wave-uniform): done after two stalled
+// sweeps in a row; up or down moves, flipped by every stalled sweep
+// (leiden.cu:113-135).
+struct MoveState {
+  bool done;
+  int up;
+};
+__device__ inline MoveState move_state(const int32_t* __restrict__ ctl, int sweep) {
+  const int n = sweep & (RING - 1);  // sweeps in the ring
+  const int base = ctl[CTL_DONE], parity = ctl[CTL_STALLS], last = ctl[CTL_LAST];
+  const uint64_t below = n == 0 ? 0ull : ~0ull >> (64 - n);
+  const uint64_t stalled = ~__ballot(ctl[CTL_LM + lane()] != 0) & below;
+  const uint64_t twice = stalled & ((stalled << 1) | (last ? 1ull : 0ull));
+  return MoveState{base != 0 || twice != 0, 1 ^ (((int)__popcll(stalled) + parity) & 1)};
+}
+// Refinement ends with the first sweep that moves nothing (later ones mark nothing).
+__device__ inline bool refine_done(const int32_t* __restrict__ ctl, int sweep) {
+  const int n = sweep & (RING - 1);
+  return ctl[CTL_DONE] != 0 || (n > 0 && ctl[CTL_REFINE + n - 1] == 0);
 }
 
-__device__ float table_lookup(const int32_t* tc, const double* ts, int n, int32_t c) {
-  for (int j0 = 0; j0 < n; j0 += 64) {
-    const int j = j0 + lane();
-    const uint64_t hit = __ballot(j < n && tc[j] == c && c >= 0);
-    if (hit) return (float)ts[j0 + first_lane(hit)];
+// Folds a full ring (RING sweeps of one phase) into the base words; or, with
+// reset, clears the words of the phase that begins.
+__global__ void fold_kernel(int32_t* __restrict__ ctl, int lm, int reset) {
+  const uint64_t stalled = ~__ballot(ctl[(lm ? CTL_LM : CTL_REFINE) + lane()] != 0);
+  if (lane() == 0) {
+    const uint64_t twice = stalled & ((stalled << 1) | (ctl[CTL_LAST] ? 1ull : 0ull));
+    const bool ended = lm ? twice != 0 : stalled != 0;
+    ctl[CTL_DONE] = reset ? 0 : (ctl[CTL_DONE] != 0 || ended ? 1 : 0);
+    ctl[CTL_STALLS] = reset ? 0 : (ctl[CTL_STALLS] + __popcll(stalled)) & 1;
+    ctl[CTL_LAST] = reset ? 0 : (int32_t)(stalled >> 63);
   }
-  return 0.0f;
+  ctl[(lm ? CTL_LM : CTL_REFINE) + lane()] = 0;
 }
 
 // ----------------------------------------------------------------- CSR build
@@ -266,21 +198,6 @@ __global__ void row_ptr_kernel(const uint64_t* __restrict__ keys, int64_t n, int
 __global__ void col_kernel(const uint64_t* __restrict__ keys, int64_t n, int bits, int32_t* __restrict__ col) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) col[i] = (int32_t)(keys[i] & (((uint64_t)1 << bits) - 1));
-}
-
-__global__ void zero_kernel(double* __restrict__ two_m, int32_t G, double* __restrict__ modularity,
-                            int32_t* __restrict__ ctl, int32_t* __restrict__ hub_count,
-                            int32_t* __restrict__ giant_count) {
-  const int i = threadIdx.x;
-  for (int g = i; g < G; g += blockDim.x) {
-    two_m[g] = 0.0;
-    modularity[g] = 0.0;
-  }
-  if (i < CTL_WORDS) ctl[i] = i == CTL_UPDOWN ? 1 : 0;  // local moving starts with upward moves
-  if (i == 0) {
-    *hub_count = 0;
-    *giant_count = 0;
-  }
 }
 
 __global__ __launch_bounds__(LTHREADS) void degree_kernel(const int32_t* __restrict__ row_ptr,
@@ -326,21 +243,14 @@ __global__ __launch_bounds__(SUM_THREADS) void graph_sum_kernel(const double* __
   }
 }
 
-__global__ void identity_kernel(int32_t V, int32_t* __restrict__ labels) {
-  const int32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v < V) labels[v] = v;
-}
-
 // ----------------------------------------------------------------- sweeps
-__global__ void sigma_zero_kernel(double* __restrict__ sigma, int32_t V, const int32_t* __restrict__ ctl) {
-  if (ctl && ctl[CTL_DONE]) return;
+__global__ void sigma_zero_kernel(double* __restrict__ sigma, int32_t V) {
   const int32_t v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v < V) sigma[v] = 0.0;
 }
 
 __global__ void sigma_scatter_kernel(const int32_t* __restrict__ labels, const double* __restrict__ k_v, int32_t V,
-                                     double* __restrict__ sigma, const int32_t* __restrict__ ctl) {
-  if (ctl && ctl[CTL_DONE]) return;
+                                     double* __restrict__ sigma) {
   const int32_t v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= V) return;
   const int32_t c = labels[v];
@@ -359,184 +269,44 @@ struct Graph {
   const double* two_m;
   int32_t V;
   int32_t S;
+  bool unique;  // no row names another vertex twice
 };
 
-template <int CAP>
-__device__ void local_moving_vertex(const Graph& gr, const double* __restrict__ sigma, const int32_t* __restrict__ lin,
-                                    int32_t* __restrict__ lout, int32_t* __restrict__ ctl, float resolution,
-                                    uint32_t level, uint32_t sweep, uint32_t seed, int32_t v, int32_t* tc,
-                                    double* ts) {
-  const int32_t old = lin[v];
-  const bool done = ctl[CTL_DONE] != 0;
-  const int32_t a = gr.beg[v], b = gr.end[v];
-  const int32_t g = v / gr.S;
-  const double tm = gr.two_m[g];
-  if (done || a == b || !(tm > 0.0)) {
-    if (lane() == 0) lout[v] = old;
-    return;
-  }
-  const int up_down = ctl[CTL_UPDOWN];
-  double e_sum;
-  const int n = build_table<CAP>(tc, ts, gr.col, gr.wt, lin, nullptr, 0, v, a, b, &e_sum);
-  const float k_old = table_lookup(tc, ts, n, old);
-  const double kv = gr.k_v[v];
-  const double m_g = 0.5 * tm;
-  const double inv_m = 1.0 / m_g;
-  const double inv_2m2 = 1.0 / (2.0 * m_g * m_g);
-  const double sig_old_excl = sigma[old] - kv;
-  const float jitter = (rand_uniform((uint32_t)g, (uint32_t)v, level, sweep, seed) - 0.5f) * 1e-9f;
-  uint64_t mine = 0;
-  int32_t mine_c = old;
-  // every slot's community total is loaded before any is used, so a lane's
-  // gathers are in flight together
-  constexpr int PER = CAP / 64;
-  int32_t cs[PER];
-  double sg[PER];
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int j = lane() + 64 * k;
-    const int32_t c = j < n ? tc[j] : -1;
-    cs[k] = (c < 0 || c == old || (c > old ? 1 : 0) != up_down) ? -1 : c;
-  }
-#pragma unroll
-  for (int k = 0; k < PER; ++k) sg[k] = cs[k] >= 0 ? sigma[cs[k]] : 0.0;
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int32_t c = cs[k];
-    if (c < 0) continue;
-    const float kn = (float)ts[lane() + 64 * k];
-    const double dq = ((double)kn - (double)k_old) * inv_m
-                      + (double)resolution * kv * (sig_old_excl - sg[k]) * inv_2m2;
-    const float dqf = (float)dq + jitter;
-    const uint64_t p = pack(dqf, cand_pref(c));
-    if (p > mine) {
-      mine = p;
-      mine_c = c;
-    }
-  }
-  const uint64_t best = wave_max_u64(mine);
-  int32_t choice = old;
-  if (best > pack(0.0f, STAY_PREF)) choice = __shfl(mine_c, first_lane(__ballot(mine == best)));
-  if (lane() == 0) {
-    lout[v] = choice;
-    if (choice != old) mark_moved(ctl);
-  }
-}
+// Sweeps.  A vertex of at most SMALL_ROW entries (nearly all) is handled by
+// half a wave, a longer one (listed once per level by hub_list_kernel) by a
+// workgroup of HUB_THREADS, both with up to ROW_PER entries per thread held in
+// registers, so that a vertex costs four rounds of loads whatever its row:
+// bounds, degree and label; entries; the neighbours' labels; the community
+// totals.  Rows longer than GIANT_MIN have kernels of their own.
+//
+// What bounds a sweep is the scattered reads of the neighbours' labels and of
+// the community totals.  Over the 24 sweeps a phase takes in the six levels of
+// eight 32k graphs (262,144 vertices, 19.4 M entries at first) a local-moving
+// sweep averages 115 us and a refinement sweep 200 us.  With a wave per vertex
+// that walked its row 64 entries at a time through a 256-slot table, longer
+// rows by one wave each in a launch behind it, and kernels that cleared and
+// refilled sigma and advanced the control words, it was 205 and 305 us (that
+// partition 16.0 -> 11.5 ms; of eight 2k graphs 2.95 -> 2.27 ms).
+//
+// Sigma, the communities' total degrees, needs no pass of its own: a sweep
+// adds every vertex's degree to its new community in the buffer the next sweep
+// reads, and clears the buffer after that (three buffers in turn).  In a
+// phase's first sweep every vertex is its own community: sigma is k_v, and
+// where no row names a neighbour twice every neighbour is a candidate by
+// itself, so no table is built (FIRST).
+constexpr int SMALL_ROW = 128;
+constexpr int ROW_PER = 4;
+constexpr int HUB_THREADS = 256;
+constexpr int HUB_BLOCKS = 512;  // a multiple of 8, so the blocks behind them keep their XCD
+constexpr int SMALL_SLOTS = 192, HUB_SLOTS = 1536;  // table load at most 2/3
+constexpr int GROUPS = HUB_THREADS / 32;            // half waves per workgroup: 8 x 192 slots = 1,536
+static_assert(GROUPS * SMALL_SLOTS == HUB_SLOTS, "both kinds of workgroup use the same LDS (18 KB, eight a compute unit)");
 
-// After a local-moving sweep: a stalled sweep flips the direction, two in a
-// row end local moving (leiden.cu:113-135).
-__global__ void lm_control_kernel(int32_t* __restrict__ ctl) {
-  if (threadIdx.x != 0) return;
-  if (!ctl[CTL_DONE]) {
-    if (ctl[CTL_MOVED] == 0) {
-      ctl[CTL_UPDOWN] ^= 1;
-      if (++ctl[CTL_STALE] >= 2) ctl[CTL_DONE] = 1;
-    } else {
-      ctl[CTL_STALE] = 0;
-    }
-  }
-  ctl[CTL_MOVED] = 0;
-}
-
-__global__ void refine_init_kernel(const int32_t* __restrict__ lm, int32_t V, int32_t* __restrict__ parent,
-                                   int32_t* __restrict__ labels, int32_t* __restrict__ ctl) {
-  const int32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v < V) {
-    parent[v] = lm[v];
-    labels[v] = v;
-  }
-  if (v < CTL_WORDS && v != CTL_OVERFLOW) ctl[v] = 0;  // an overflow of the local-moving sweeps stays raised
-}
-
-// Test hook: raises the overflow word as a broken local-moving table would.
-__global__ void raise_overflow_kernel(int32_t* __restrict__ ctl) {
-  if (threadIdx.x == 0) ctl[CTL_OVERFLOW] = 1;
-}
-
-template <int CAP>
-__device__ void refine_propose_vertex(const Graph& gr, const int32_t* __restrict__ parent,
-                                      const double* __restrict__ sigma, const double* __restrict__ parent_sigma,
-                                      const int32_t* __restrict__ lin, int32_t* __restrict__ prop,
-                                      uint32_t* __restrict__ rank, float resolution, float inv_theta, int boltzmann,
-                                      uint32_t level, uint32_t sweep, uint32_t seed, int32_t v, int32_t* tc,
-                                      double* ts) {
-  const int32_t g = v / gr.S;
-  if (lane() == 0) rank[v] = mix4((uint32_t)g, (uint32_t)v, (level << 16) | sweep, seed);
-  const int32_t old = lin[v];
-  const int32_t a = gr.beg[v], b = gr.end[v];
-  const double tm = gr.two_m[g];
-  if (a == b || !(tm > 0.0)) {
-    if (lane() == 0) prop[v] = old;
-    return;
-  }
-  const int32_t pv = parent[v];
-  double e_sum;
-  const int n = build_table<CAP>(tc, ts, gr.col, gr.wt, lin, parent, pv, v, a, b, &e_sum);
-  const double kv = gr.k_v[v];
-  double vol_minus = parent_sigma[pv] - kv;
-  if (vol_minus < 0.0) vol_minus = 0.0;
-  const double bound = (double)resolution * kv * vol_minus / tm;
-  if ((double)(float)e_sum < bound) {  // {v} is not well connected to its parent community
-    if (lane() == 0) prop[v] = old;
-    return;
-  }
-  const float k_old = table_lookup(tc, ts, n, old);
-  const double m_g = 0.5 * tm;
-  const double inv_m = 1.0 / m_g;
-  const double inv_2m2 = 1.0 / (2.0 * m_g * m_g);
-  const double sig_old_excl = sigma[old] - kv;
-  uint64_t mine = 0;
-  int32_t mine_c = old;
-  constexpr int PER = CAP / 64;  // community totals gathered together, as in local moving
-  int32_t cs[PER];
-  double sg[PER];
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int j = lane() + 64 * k;
-    const int32_t c = j < n ? tc[j] : -1;
-    cs[k] = (c < 0 || c == old) ? -1 : c;
-  }
-#pragma unroll
-  for (int k = 0; k < PER; ++k) sg[k] = cs[k] >= 0 ? sigma[cs[k]] : 0.0;
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int32_t c = cs[k];
-    if (c < 0) continue;
-    const float kn = (float)ts[lane() + 64 * k];
-    const double dq = ((double)kn - (double)k_old) * inv_m
-                      + (double)resolution * kv * (sig_old_excl - sg[k]) * inv_2m2;
-    if (dq < 0.0) continue;
-    const float score = boltzmann
-        ? (float)(dq * (double)inv_theta)
-              + gumbel(rand_uniform_pair((uint32_t)g, (uint32_t)v, (uint32_t)c, level, sweep, seed))
-        : (float)dq;
-    const uint64_t p = pack(score, cand_pref(c));
-    if (p > mine) {
-      mine = p;
-      mine_c = c;
-    }
-  }
-  const uint64_t best = wave_max_u64(mine);
-  const float stay = boltzmann
-      ? gumbel(rand_uniform_pair((uint32_t)g, (uint32_t)v, (uint32_t)old, level, sweep, seed))
-      : 0.0f;
-  int32_t choice = old;
-  if (best > pack(stay, STAY_PREF)) choice = __shfl(mine_c, first_lane(__ballot(mine == best)));
-  if (lane() == 0) prop[v] = choice;
-}
-
-// Vertices with at most SMALL_CAP / 2 row entries (nearly all) run with a
-// small LDS table and 8 waves per workgroup; the rest (hubs, listed once per
-// call by hub_list_kernel) run with the full TABLE_CAP table, grid-striding
-// over the list.
-constexpr int SMALL_CAP = 256;
-constexpr int SWAVES = 8;
-constexpr int HUB_BLOCKS = 768;  // three 48 KB workgroups per CU
-
-constexpr int GIANT_MIN = TABLE_CAP;  // rows longer than this take a whole workgroup
+constexpr int GIANT_MIN = TABLE_CAP;  // rows longer than this take a workgroup of GIANT_THREADS
 constexpr int GIANT_SLOTS = 4096;
 constexpr int GIANT_THREADS = 1024;
 constexpr int GIANT_BLOCKS = 512;  // two 65 KB workgroups per CU
+static_assert(SMALL_ROW == 32 * ROW_PER && GIANT_MIN == HUB_THREADS * ROW_PER, "rows fit their threads' registers");
 
 // (Places in the lists are reserved once per workgroup: one atomic per wave and
 // list queues thousands of them on two words.)
@@ -551,7 +321,7 @@ __global__ __launch_bounds__(LIST_THREADS) void hub_list_kernel(const int32_t* _
   __shared__ int s_n[2], s_at[2];
   const int32_t v = blockIdx.x * LIST_THREADS + threadIdx.x;
   const int32_t d = v < V ? end[v] - beg[v] : 0;
-  const bool giant = d > GIANT_MIN, hub = !giant && d > SMALL_CAP / 2;
+  const bool giant = d > GIANT_MIN, hub = !giant && d > SMALL_ROW;
   if (threadIdx.x < 2) s_n[threadIdx.x] = 0;
   __syncthreads();
   const uint64_t mg = __ballot(giant), mh = __ballot(hub);
@@ -569,6 +339,471 @@ __global__ __launch_bounds__(LIST_THREADS) void hub_list_kernel(const int32_t* _
   __syncthreads();
   if (hub) hubs[s_at[0] + bh + __popcll(mh & below)] = v;
   if (giant) giants[s_at[1] + bg + __popcll(mg & below)] = v;
+}
+
+// The threads of one vertex.
+struct HalfWave {
+  static constexpr int N = 32, SLOTS = SMALL_SLOTS;
+  int32_t* tc;
+  double* ts;
+  __device__ int tid() const { return lane() & 31; }
+  __device__ void sync() const { wave_lds_sync(); }
+  __device__ uint64_t max(uint64_t x) const {
+    x = pick_u64<true>(x, xor_u64<1>(x));
+    x = pick_u64<true>(x, xor_u64<2>(x));
+    x = pick_u64<true>(x, xor_u64<4>(x));
+    x = pick_u64<true>(x, xor_u64<8>(x));
+    return pick_u64<true>(x, xor_u64<16>(x));
+  }
+  __device__ double sum(double x) const {
+    x += __builtin_bit_cast(double, xor_u64<1>(__builtin_bit_cast(uint64_t, x)));
+    x += __builtin_bit_cast(double, xor_u64<2>(__builtin_bit_cast(uint64_t, x)));
+    x += __builtin_bit_cast(double, xor_u64<4>(__builtin_bit_cast(uint64_t, x)));
+    x += __builtin_bit_cast(double, xor_u64<8>(__builtin_bit_cast(uint64_t, x)));
+    return x + __builtin_bit_cast(double, xor_u64<16>(__builtin_bit_cast(uint64_t, x)));
+  }
+  // The value of the thread that holds the winning key.
+  __device__ int32_t of(uint64_t best, uint64_t mine, int32_t value) const {
+    const uint64_t m = __ballot(mine == best) >> (lane() & 32);
+    return __shfl(value, (lane() & 32) + __builtin_ctz((uint32_t)m));
+  }
+  __device__ bool any(bool x) const { return (uint32_t)(__ballot(x) >> (lane() & 32)) != 0; }
+};
+
+struct WorkgroupShared {
+  uint64_t best[HUB_THREADS / 64];
+  int32_t value[HUB_THREADS / 64];
+  double sum[HUB_THREADS / 64];
+};
+struct Workgroup {
+  static constexpr int N = HUB_THREADS, SLOTS = HUB_SLOTS;
+  int32_t* tc;
+  double* ts;
+  WorkgroupShared* sh;
+  __device__ int tid() const { return threadIdx.x; }
+  __device__ void sync() const { __syncthreads(); }
+  __device__ uint64_t max(uint64_t x) const {
+    x = wave_max_u64(x);
+    if (lane() == 0) sh->best[threadIdx.x >> 6] = x;
+    __syncthreads();
+    for (int i = 0; i < HUB_THREADS / 64; ++i) x = pick_u64<true>(x, sh->best[i]);
+    __syncthreads();
+    return x;
+  }
+  __device__ double sum(double x) const {
+    x = wave_sum_f64(x);
+    if (lane() == 0) sh->sum[threadIdx.x >> 6] = x;
+    __syncthreads();
+    double t = 0.0;
+    for (int i = 0; i < HUB_THREADS / 64; ++i) t += sh->sum[i];
+    __syncthreads();
+    return t;
+  }
+  __device__ int32_t of(uint64_t best, uint64_t mine, int32_t value) const {
+    if (mine == best) sh->value[0] = value;  // (keys of different candidates differ; equal keys are one candidate)
+    __syncthreads();
+    const int32_t r = sh->value[0];
+    __syncthreads();
+    return r;
+  }
+  __device__ bool any(bool x) const { return __syncthreads_or(x) != 0; }
+};
+
+// One vertex's row in its threads' registers: neighbour, weight and whether
+// the entry counts (self loops do not).
+struct Row {
+  int32_t u[ROW_PER];
+  float w[ROW_PER];
+  bool ok[ROW_PER];
+};
+template <class P>
+__device__ __forceinline__ void load_row(const P& p, const Graph& gr, int32_t v, int32_t a, int32_t b, Row& r) {
+#pragma unroll
+  for (int i = 0; i < ROW_PER; ++i) {
+    const int32_t e = a + i * P::N + p.tid();
+    const int32_t at = min(e, b - 1);  // (past the row: its last entry again, not counted)
+    r.u[i] = gr.col[at];
+    r.w[i] = gr.wt[at];
+    r.ok[i] = e < b && r.u[i] != v;
+  }
+}
+
+// Sums the entries' weights by community c[i] into the group's table; returns
+// its size in slots.
+template <class P>
+__device__ __forceinline__ int fill_table(const P& p, const Row& r, const int32_t* c, int32_t row) {
+  int size = 2 * P::N;
+  while (size < P::SLOTS && 2 * size < 3 * row) size = min(2 * size, P::SLOTS);
+  for (int j = p.tid(); j < size; j += P::N) {
+    p.tc[j] = -1;
+    p.ts[j] = 0.0;
+  }
+  p.sync();
+#pragma unroll
+  for (int i = 0; i < ROW_PER; ++i) {
+    if (r.ok[i]) {
+      int h = (int)__umulhi(pcg_hash((uint32_t)c[i]), (uint32_t)size);
+      while (true) {  // (at most `row` <= 2/3 size communities: a free slot or the community's is found)
+        const int32_t cur = __hip_atomic_load(p.tc + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (cur == c[i]) break;
+        if (cur == -1) {
+          const int32_t prev = atomicCAS(p.tc + h, -1, c[i]);
+          if (prev == -1 || prev == c[i]) break;
+        }
+        h = h + 1 == size ? 0 : h + 1;
+      }
+      unsafeAtomicAdd(p.ts + h, (double)r.w[i]);
+    }
+  }
+  p.sync();
+  return size;
+}
+
+// Weight to community c in the table (every thread probes alike).
+template <class P>
+__device__ __forceinline__ float table_weight(const P& p, int size, int32_t c) {
+  int h = (int)__umulhi(pcg_hash((uint32_t)c), (uint32_t)size);
+  while (true) {
+    const int32_t cur = p.tc[h];
+    if (cur == c) return (float)p.ts[h];
+    if (cur == -1) return 0.0f;
+    h = h + 1 == size ? 0 : h + 1;
+  }
+}
+
+// Calls f(community, weight to it, its total) for every candidate other than
+// `old` that want() admits; all totals are loaded before any is used.
+template <class P, bool FIRST, class Want, class F>
+__device__ __forceinline__ void each_candidate(const P& p, const Row& r, const double* first_total, int size,
+                                               const double* __restrict__ sigma, int32_t old, Want want, F f) {
+  if constexpr (FIRST) {
+#pragma unroll
+    for (int i = 0; i < ROW_PER; ++i) {
+      if (r.ok[i] && want(r.u[i])) f(r.u[i], r.w[i], first_total[i]);
+    }
+  } else {
+    constexpr int PER = P::SLOTS / P::N;
+    int32_t cs[PER];
+    double sg[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int j = p.tid() + P::N * k;
+      const int32_t c = j < size ? p.tc[j] : -1;
+      cs[k] = c >= 0 && c != old && want(c) ? c : -1;
+    }
+#pragma unroll
+    for (int k = 0; k < PER; ++k) sg[k] = cs[k] >= 0 ? sigma[cs[k]] : 0.0;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      if (cs[k] >= 0) f(cs[k], (float)p.ts[p.tid() + P::N * k], sg[k]);
+    }
+  }
+}
+
+// What a sweep reads and writes.
+struct MoveSweep {
+  const double* sigma;
+  double* next;        // totals for the next sweep
+  double* clear;       // cleared for the sweep after it
+  const int32_t* lin;  // labels (not read in a FIRST sweep)
+  int32_t* lout;
+  int32_t* ctl;
+  int32_t sweep;
+  float resolution;
+  uint32_t seed;
+};
+
+__device__ inline void finish_move(const MoveSweep& s, int32_t v, int32_t old, int32_t choice, double kv) {
+  s.lout[v] = choice;
+  s.clear[v] = 0.0;
+  if (kv != 0.0) unsafeAtomicAdd(s.next + choice, kv);
+  if (choice != old) mark_moved(s.ctl + CTL_LM + (s.sweep & (RING - 1)));
+}
+
+template <class P, bool FIRST>
+__device__ __forceinline__ void move_vertex(const P& p, const Graph& gr, const MoveSweep& s, const MoveState& st,
+                                            int32_t v, int32_t a, int32_t b) {
+  const int32_t old = FIRST ? v : s.lin[v];
+  const double kv = gr.k_v[v];
+  const int32_t g = v / gr.S;
+  const double tm = gr.two_m[g];
+  int32_t choice = old;
+  if (!st.done && a != b && tm > 0.0) {
+    Row r;
+    load_row(p, gr, v, a, b, r);
+    const double sig_old_excl = s.sigma[old] - kv;
+    double total[ROW_PER];
+    float k_old = 0.0f;
+    int size = 0;
+    if constexpr (FIRST) {
+#pragma unroll
+      for (int i = 0; i < ROW_PER; ++i) total[i] = s.sigma[r.u[i]];
+    } else {
+      int32_t c[ROW_PER];
+#pragma unroll
+      for (int i = 0; i < ROW_PER; ++i) c[i] = s.lin[r.u[i]];
+      size = fill_table(p, r, c, b - a);
+      k_old = table_weight(p, size, old);
+    }
+    const double m_g = 0.5 * tm;
+    const double inv_m = 1.0 / m_g;
+    const double inv_2m2 = 1.0 / (2.0 * m_g * m_g);
+    const float jitter = (rand_uniform((uint32_t)g, (uint32_t)v, 0u, (uint32_t)s.sweep, s.seed) - 0.5f) * 1e-9f;
+    uint64_t mine = 0;
+    int32_t mine_c = old;
+    each_candidate<P, FIRST>(
+        p, r, total, size, s.sigma, old, [&](int32_t c) { return (c > old ? 1 : 0) == st.up; },
+        [&](int32_t c, float kn, double sg) {
+          const double dq = ((double)kn - (double)k_old) * inv_m
+                            + (double)s.resolution * kv * (sig_old_excl - sg) * inv_2m2;
+          const uint64_t key = pack((float)dq + jitter, cand_pref(c));
+          if (key > mine) {
+            mine = key;
+            mine_c = c;
+          }
+        });
+    const uint64_t best = p.max(mine);
+    if (best > pack(0.0f, STAY_PREF)) choice = p.of(best, mine, mine_c);
+  }
+  if (p.tid() == 0) finish_move(s, v, old, choice, kv);
+}
+
+// Block b of n of a vertex range: each XCD (blocks run on the eight in turn)
+// gets a contiguous run, so that a graph's labels and totals stay in one L2.
+__device__ inline int32_t xcd_block(int32_t b, int32_t n) {
+  const int32_t per = n >> 3;
+  return b < 8 * per ? (b & 7) * per + (b >> 3) : b;
+}
+
+template <bool FIRST>
+__global__ __launch_bounds__(HUB_THREADS, 8) void local_moving_kernel(Graph gr, MoveSweep s,
+                                                                      const int32_t* __restrict__ hubs,
+                                                                      const int32_t* __restrict__ hub_count) {
+  __shared__ int32_t tab_c[FIRST ? 1 : HUB_SLOTS];
+  __shared__ double tab_s[FIRST ? 1 : HUB_SLOTS];
+  __shared__ WorkgroupShared sh;
+  const MoveState st = move_state(s.ctl, s.sweep);
+  if (blockIdx.x < HUB_BLOCKS) {
+    const int32_t n = *hub_count;
+    const Workgroup p{tab_c, tab_s, &sh};
+    for (int32_t i = blockIdx.x; i < n; i += HUB_BLOCKS) {
+      const int32_t v = hubs[i];
+      move_vertex<Workgroup, FIRST>(p, gr, s, st, v, gr.beg[v], gr.end[v]);
+      __syncthreads();  // the next vertex takes the table
+    }
+    return;
+  }
+  const int group = threadIdx.x >> 5;
+  const HalfWave p{tab_c + (FIRST ? 0 : group * SMALL_SLOTS), tab_s + (FIRST ? 0 : group * SMALL_SLOTS)};
+  const int32_t v = xcd_block(blockIdx.x - HUB_BLOCKS, gridDim.x - HUB_BLOCKS) * GROUPS + group;
+  if (v >= gr.V) return;
+  const int32_t a = gr.beg[v], b = gr.end[v];
+  if (b - a > SMALL_ROW) return;
+  move_vertex<HalfWave, FIRST>(p, gr, s, st, v, a, b);
+}
+
+// Refinement: a vertex proposes a community inside its parent community (x of
+// the label pairs; y is its community), then the proposals' independent set
+// commits.  mover[v] holds the parent of a vertex that wants to move, -1 of
+// the others: one gather per neighbour tells the commit all it needs.
+struct RefineSweep {
+  const double* sigma;
+  const double* parent_sigma;
+  double* next;
+  double* clear;
+  const int32_t* parent;  // read in a FIRST sweep in place of the pairs
+  const int2* lin;
+  int2* lout;
+  int32_t* labels;        // the communities alone
+  int32_t* prop;
+  int32_t* mover;
+  int32_t* ctl;
+  int32_t sweep;
+  float resolution;
+  float inv_theta;
+  int boltzmann;
+  uint32_t seed;
+};
+
+template <class P, bool FIRST>
+__device__ __forceinline__ void propose_vertex(const P& p, const Graph& gr, const RefineSweep& s, int32_t v, int32_t a,
+                                               int32_t b) {
+  int2 self;
+  if constexpr (FIRST) self = int2{s.parent[v], v};
+  else self = s.lin[v];
+  const int32_t pv = self.x, old = self.y;
+  const double kv = gr.k_v[v];
+  const int32_t g = v / gr.S;
+  const double tm = gr.two_m[g];
+  int32_t choice = old;
+  if (a != b && tm > 0.0) {
+    Row r;
+    load_row(p, gr, v, a, b, r);
+    double vol_minus = s.parent_sigma[pv] - kv;
+    if (vol_minus < 0.0) vol_minus = 0.0;
+    const double bound = (double)s.resolution * kv * vol_minus / tm;
+    const double sig_old_excl = s.sigma[old] - kv;
+    int32_t c[ROW_PER];
+    double total[ROW_PER];
+    double e_sum = 0.0;
+#pragma unroll
+    for (int i = 0; i < ROW_PER; ++i) {
+      if constexpr (FIRST) {
+        total[i] = s.sigma[r.u[i]];
+        r.ok[i] = r.ok[i] && s.parent[r.u[i]] == pv;
+      } else {
+        const int2 q = s.lin[r.u[i]];
+        r.ok[i] = r.ok[i] && q.x == pv;
+        c[i] = q.y;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < ROW_PER; ++i) e_sum += r.ok[i] ? (double)r.w[i] : 0.0;
+    e_sum = p.sum(e_sum);
+    if (!((double)(float)e_sum < bound)) {  // {v} is well connected to its parent community
+      float k_old = 0.0f;
+      int size = 0;
+      if constexpr (!FIRST) {
+        size = fill_table(p, r, c, b - a);
+        k_old = table_weight(p, size, old);
+      }
+      const double m_g = 0.5 * tm;
+      const double inv_m = 1.0 / m_g;
+      const double inv_2m2 = 1.0 / (2.0 * m_g * m_g);
+      uint64_t mine = 0;
+      int32_t mine_c = old;
+      each_candidate<P, FIRST>(
+          p, r, total, size, s.sigma, old, [](int32_t) { return true; },
+          [&](int32_t cand, float kn, double sg) {
+            const double dq = ((double)kn - (double)k_old) * inv_m
+                              + (double)s.resolution * kv * (sig_old_excl - sg) * inv_2m2;
+            if (dq < 0.0) return;
+            const float score = s.boltzmann
+                ? (float)(dq * (double)s.inv_theta)
+                      + gumbel(rand_uniform_pair((uint32_t)g, (uint32_t)v, (uint32_t)cand, 1u, (uint32_t)s.sweep,
+                                                 s.seed))
+                : (float)dq;
+            const uint64_t key = pack(score, cand_pref(cand));
+            if (key > mine) {
+              mine = key;
+              mine_c = cand;
+            }
+          });
+      const uint64_t best = p.max(mine);
+      const float stay = s.boltzmann
+          ? gumbel(rand_uniform_pair((uint32_t)g, (uint32_t)v, (uint32_t)old, 1u, (uint32_t)s.sweep, s.seed))
+          : 0.0f;
+      if (best > pack(stay, STAY_PREF)) choice = p.of(best, mine, mine_c);
+    }
+  }
+  if (p.tid() == 0) {
+    s.prop[v] = choice;
+    s.mover[v] = choice != old ? pv : -1;
+  }
+}
+
+template <bool FIRST>
+__global__ __launch_bounds__(HUB_THREADS, 8) void refine_propose_kernel(Graph gr, RefineSweep s,
+                                                                        const int32_t* __restrict__ hubs,
+                                                                        const int32_t* __restrict__ hub_count) {
+  __shared__ int32_t tab_c[FIRST ? 1 : HUB_SLOTS];
+  __shared__ double tab_s[FIRST ? 1 : HUB_SLOTS];
+  __shared__ WorkgroupShared sh;
+  if (refine_done(s.ctl, s.sweep)) return;
+  if (blockIdx.x < HUB_BLOCKS) {
+    const int32_t n = *hub_count;
+    const Workgroup p{tab_c, tab_s, &sh};
+    for (int32_t i = blockIdx.x; i < n; i += HUB_BLOCKS) {
+      const int32_t v = hubs[i];
+      propose_vertex<Workgroup, FIRST>(p, gr, s, v, gr.beg[v], gr.end[v]);
+      __syncthreads();
+    }
+    return;
+  }
+  const int group = threadIdx.x >> 5;
+  const HalfWave p{tab_c + (FIRST ? 0 : group * SMALL_SLOTS), tab_s + (FIRST ? 0 : group * SMALL_SLOTS)};
+  const int32_t v = xcd_block(blockIdx.x - HUB_BLOCKS, gridDim.x - HUB_BLOCKS) * GROUPS + group;
+  if (v >= gr.V) return;
+  const int32_t a = gr.beg[v], b = gr.end[v];
+  if (b - a > SMALL_ROW) return;
+  propose_vertex<HalfWave, FIRST>(p, gr, s, v, a, b);
+}
+
+// A mover commits unless a moving neighbour in its parent community outranks
+// it on (rank, id) (refinement.cu:263-300); the rank is the neighbour's hash,
+// computed where it is needed.
+template <class P, bool FIRST>
+__device__ __forceinline__ void commit_vertex(const P& p, const Graph& gr, const RefineSweep& s, bool done, int32_t v,
+                                              int32_t a, int32_t b) {
+  int2 self;
+  if constexpr (FIRST) self = int2{s.parent[v], v};
+  else self = s.lin[v];
+  const double kv = gr.k_v[v];
+  const int32_t wants = done ? -1 : s.mover[v];
+  const int32_t to = done ? self.y : s.prop[v];
+  bool lost = false;
+  if (wants >= 0) {
+    const uint32_t rv = mix4((uint32_t)(v / gr.S), (uint32_t)v, (1u << 16) | (uint32_t)s.sweep, s.seed);
+    for (int32_t e0 = a; e0 < b; e0 += ROW_PER * P::N) {
+      int32_t u[ROW_PER], m[ROW_PER];
+#pragma unroll
+      for (int i = 0; i < ROW_PER; ++i) u[i] = gr.col[min(e0 + i * P::N + p.tid(), b - 1)];
+#pragma unroll
+      for (int i = 0; i < ROW_PER; ++i) m[i] = s.mover[u[i]];
+#pragma unroll
+      for (int i = 0; i < ROW_PER; ++i) {
+        if (u[i] != v && m[i] == self.x) {
+          const uint32_t ru = mix4((uint32_t)(u[i] / gr.S), (uint32_t)u[i], (1u << 16) | (uint32_t)s.sweep, s.seed);
+          lost = lost || ru > rv || (ru == rv && u[i] > v);
+        }
+      }
+    }
+    lost = p.any(lost);
+  }
+  if (p.tid() == 0) {
+    const int32_t label = wants >= 0 && !lost ? to : self.y;
+    s.lout[v] = int2{self.x, label};
+    s.labels[v] = label;
+    s.clear[v] = 0.0;
+    if (kv != 0.0) unsafeAtomicAdd(s.next + label, kv);
+    if (label != self.y) mark_moved(s.ctl + CTL_REFINE + (s.sweep & (RING - 1)));
+  }
+}
+
+template <bool FIRST>
+__global__ __launch_bounds__(HUB_THREADS, 8) void refine_commit_kernel(Graph gr, RefineSweep s,
+                                                                       const int32_t* __restrict__ hubs,
+                                                                       const int32_t* __restrict__ hub_count,
+                                                                       const int32_t* __restrict__ giants,
+                                                                       const int32_t* __restrict__ giant_count) {
+  __shared__ WorkgroupShared sh;
+  const bool done = refine_done(s.ctl, s.sweep);
+  if (blockIdx.x < HUB_BLOCKS) {
+    const int32_t n = *hub_count, all = n + *giant_count;
+    const Workgroup p{nullptr, nullptr, &sh};
+    for (int32_t i = blockIdx.x; i < all; i += HUB_BLOCKS) {
+      const int32_t v = i < n ? hubs[i] : giants[i - n];
+      commit_vertex<Workgroup, FIRST>(p, gr, s, done, v, gr.beg[v], gr.end[v]);
+    }
+    return;
+  }
+  const HalfWave p{nullptr, nullptr};
+  const int32_t v = xcd_block(blockIdx.x - HUB_BLOCKS, gridDim.x - HUB_BLOCKS) * GROUPS + (threadIdx.x >> 5);
+  if (v >= gr.V) return;
+  const int32_t a = gr.beg[v], b = gr.end[v];
+  if (b - a > SMALL_ROW) return;
+  commit_vertex<HalfWave, FIRST>(p, gr, s, done, v, a, b);
+}
+
+// Test hook: raises the overflow word as a broken local-moving table would.
+__global__ void raise_overflow_kernel(int32_t* __restrict__ ctl) {
+  if (threadIdx.x == 0) ctl[CTL_OVERFLOW] = 1;
+}
+
+// Label pairs of singletons, for graphs whose first refinement sweep reads them.
+__global__ void pair_init_kernel(const int32_t* __restrict__ parent, int32_t V, int2* __restrict__ pairs) {
+  const int32_t v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v < V) pairs[v] = int2{parent[v], v};
 }
 
 // Rows longer than GIANT_MIN: one 1024-thread workgroup per vertex.  All
@@ -603,10 +838,10 @@ __device__ inline double block_sum_giant(double x, GiantShared& sh) {
 
 // Returns false when the table overflowed (caller falls back); on success
 // *thr bounds the kept first positions and *e_sum is the admitted weight.
-template <bool REFINE>
-__device__ bool giant_table(const Graph& gr, const int32_t* __restrict__ parent, const int32_t* __restrict__ lin,
-                            int32_t v, int32_t pv, int32_t a, int32_t b, GiantShared& sh, int32_t* thr,
-                            double* e_sum) {
+// community_of(u): the neighbour's community, -1 when the entry does not count.
+template <class Of>
+__device__ bool giant_table(const Graph& gr, Of community_of, int32_t v, int32_t a, int32_t b, GiantShared& sh,
+                            int32_t* thr, double* e_sum) {
   const int tid = threadIdx.x;
   for (int j = tid; j < GIANT_SLOTS; j += GIANT_THREADS) {
     sh.c[j] = -1;
@@ -624,10 +859,9 @@ __device__ bool giant_table(const Graph& gr, const int32_t* __restrict__ parent,
     const int32_t e = e0 + tid;
     if (e < b) {
       const int32_t u = gr.col[e];
-      const bool ok = u != v && (!REFINE || parent[u] == pv);
-      if (ok) {
+      const int32_t c = u != v ? community_of(u) : -1;
+      if (c >= 0) {
         const float w = gr.wt[e];
-        const int32_t c = lin[u];
         e_acc += (double)w;
         uint32_t h = pcg_hash((uint32_t)c) & (GIANT_SLOTS - 1);
         int probes = 0;
@@ -715,97 +949,48 @@ __device__ float giant_k_old(GiantShared& sh, int32_t old, int32_t thr) {
   return slot >= 0 ? (float)sh.s[slot] : 0.0f;
 }
 
-template <bool HUB>
-__global__ __launch_bounds__(HUB ? LTHREADS : 64 * SWAVES) void local_moving_kernel(
-    Graph gr, const double* __restrict__ sigma, const int32_t* __restrict__ lin, int32_t* __restrict__ lout,
-    int32_t* __restrict__ ctl, const int32_t* __restrict__ hubs, const int32_t* __restrict__ hub_count,
-    float resolution, uint32_t level, uint32_t sweep, uint32_t seed) {
-  constexpr int W = HUB ? LWAVES : SWAVES;
-  constexpr int CAP = HUB ? TABLE_CAP : SMALL_CAP;
-  __shared__ int32_t tab_c[W][CAP];
-  __shared__ double tab_s[W][CAP];
-  const int wv = threadIdx.x >> 6;
-  if (HUB) {
-    const int32_t n = *hub_count;
-    for (int32_t i = blockIdx.x * W + wv; i < n; i += gridDim.x * W)
-      local_moving_vertex<CAP>(gr, sigma, lin, lout, ctl, resolution, level, sweep, seed, hubs[i], tab_c[wv],
-                               tab_s[wv]);
-  } else {
-    const int32_t v = blockIdx.x * W + wv;
-    if (v >= gr.V || gr.end[v] - gr.beg[v] > CAP / 2) return;
-    local_moving_vertex<CAP>(gr, sigma, lin, lout, ctl, resolution, level, sweep, seed, v, tab_c[wv], tab_s[wv]);
-  }
-}
-
-template <bool HUB>
-__global__ __launch_bounds__(HUB ? LTHREADS : 64 * SWAVES) void refine_propose_kernel(
-    Graph gr, const int32_t* __restrict__ parent, const double* __restrict__ sigma,
-    const double* __restrict__ parent_sigma, const int32_t* __restrict__ lin, int32_t* __restrict__ prop,
-    uint32_t* __restrict__ rank, const int32_t* __restrict__ ctl, const int32_t* __restrict__ hubs,
-    const int32_t* __restrict__ hub_count, float resolution, float inv_theta, int boltzmann, uint32_t level,
-    uint32_t sweep, uint32_t seed) {
-  constexpr int W = HUB ? LWAVES : SWAVES;
-  constexpr int CAP = HUB ? TABLE_CAP : SMALL_CAP;
-  __shared__ int32_t tab_c[W][CAP];
-  __shared__ double tab_s[W][CAP];
-  if (ctl[CTL_DONE]) return;
-  const int wv = threadIdx.x >> 6;
-  if (HUB) {
-    const int32_t n = *hub_count;
-    for (int32_t i = blockIdx.x * W + wv; i < n; i += gridDim.x * W)
-      refine_propose_vertex<CAP>(gr, parent, sigma, parent_sigma, lin, prop, rank, resolution, inv_theta,
-                                 boltzmann, level, sweep, seed, hubs[i], tab_c[wv], tab_s[wv]);
-  } else {
-    const int32_t v = blockIdx.x * W + wv;
-    if (v >= gr.V || gr.end[v] - gr.beg[v] > CAP / 2) return;
-    refine_propose_vertex<CAP>(gr, parent, sigma, parent_sigma, lin, prop, rank, resolution, inv_theta, boltzmann,
-                               level, sweep, seed, v, tab_c[wv], tab_s[wv]);
-  }
-}
-
-__global__ __launch_bounds__(GIANT_THREADS) void local_moving_giant_kernel(
-    Graph gr, const double* __restrict__ sigma, const int32_t* __restrict__ lin, int32_t* __restrict__ lout,
-    int32_t* __restrict__ ctl, const int32_t* __restrict__ giants, const int32_t* __restrict__ giant_count,
-    float resolution, uint32_t level, uint32_t sweep, uint32_t seed) {
+template <bool FIRST>
+__global__ __launch_bounds__(GIANT_THREADS) void local_moving_giant_kernel(Graph gr, MoveSweep s,
+                                                                           const int32_t* __restrict__ giants,
+                                                                           const int32_t* __restrict__ giant_count) {
   __shared__ GiantShared sh;
   const int32_t count = *giant_count;
-  const bool done = ctl[CTL_DONE] != 0;
-  const int up_down = ctl[CTL_UPDOWN];
+  const MoveState st = move_state(s.ctl, s.sweep);
   for (int32_t i = blockIdx.x; i < count; i += gridDim.x) {
     const int32_t v = giants[i];
-    const int32_t old = lin[v];
+    const int32_t old = FIRST ? v : s.lin[v];
     const int32_t g = v / gr.S;
     const double tm = gr.two_m[g];
-    if (done || !(tm > 0.0)) {
-      if (threadIdx.x == 0) lout[v] = old;
+    const double kv = gr.k_v[v];
+    if (st.done || !(tm > 0.0)) {
+      if (threadIdx.x == 0) finish_move(s, v, old, old, kv);
       continue;
     }
     const int32_t a = gr.beg[v], b = gr.end[v];
     int32_t thr;
     double e_sum;
-    if (!giant_table<false>(gr, nullptr, lin, v, 0, a, b, sh, &thr, &e_sum)) {  // cannot happen: stay, flagged
+    if (!giant_table(gr, [&](int32_t u) { return FIRST ? u : s.lin[u]; }, v, a, b, sh, &thr, &e_sum)) {  // cannot happen
       if (threadIdx.x == 0) {
-        lout[v] = old;
-        ctl[CTL_OVERFLOW] = 1;
+        finish_move(s, v, old, old, kv);  // stay, flagged
+        s.ctl[CTL_OVERFLOW] = 1;
       }
       __syncthreads();
       continue;
     }
     const float k_old = giant_k_old(sh, old, thr);
-    const double kv = gr.k_v[v];
     const double m_g = 0.5 * tm;
     const double inv_m = 1.0 / m_g;
     const double inv_2m2 = 1.0 / (2.0 * m_g * m_g);
-    const double sig_old_excl = sigma[old] - kv;
-    const float jitter = (rand_uniform((uint32_t)g, (uint32_t)v, level, sweep, seed) - 0.5f) * 1e-9f;
+    const double sig_old_excl = s.sigma[old] - kv;
+    const float jitter = (rand_uniform((uint32_t)g, (uint32_t)v, 0u, (uint32_t)s.sweep, s.seed) - 0.5f) * 1e-9f;
     uint64_t mine = 0;
     int32_t mine_c = old;
     for (int j = threadIdx.x; j < GIANT_SLOTS; j += GIANT_THREADS) {
       const int32_t c = sh.c[j];
-      if (c < 0 || sh.first[j] >= thr || c == old || (c > old ? 1 : 0) != up_down) continue;
+      if (c < 0 || sh.first[j] >= thr || c == old || (c > old ? 1 : 0) != st.up) continue;
       const float kn = (float)sh.s[j];
       const double dq = ((double)kn - (double)k_old) * inv_m
-                        + (double)resolution * kv * (sig_old_excl - sigma[c]) * inv_2m2;
+                        + (double)s.resolution * kv * (sig_old_excl - s.sigma[c]) * inv_2m2;
       const float dqf = (float)dq + jitter;
       const uint64_t p = pack(dqf, cand_pref(c));
       if (p > mine) {
@@ -814,50 +999,55 @@ __global__ __launch_bounds__(GIANT_THREADS) void local_moving_giant_kernel(
       }
     }
     const int32_t choice = giant_pick(mine, mine_c, pack(0.0f, STAY_PREF), old, sh);
-    if (threadIdx.x == 0) {
-      lout[v] = choice;
-      if (choice != old) mark_moved(ctl);
-    }
+    if (threadIdx.x == 0) finish_move(s, v, old, choice, kv);
   }
 }
 
-__global__ __launch_bounds__(GIANT_THREADS) void refine_propose_giant_kernel(
-    Graph gr, const int32_t* __restrict__ parent, const double* __restrict__ sigma,
-    const double* __restrict__ parent_sigma, const int32_t* __restrict__ lin, int32_t* __restrict__ prop,
-    uint32_t* __restrict__ rank, int32_t* __restrict__ ctl, const int32_t* __restrict__ giants,
-    const int32_t* __restrict__ giant_count, float resolution, float inv_theta, int boltzmann, uint32_t level,
-    uint32_t sweep, uint32_t seed) {
+template <bool FIRST>
+__global__ __launch_bounds__(GIANT_THREADS) void refine_propose_giant_kernel(Graph gr, RefineSweep s,
+                                                                             const int32_t* __restrict__ giants,
+                                                                             const int32_t* __restrict__ giant_count) {
   __shared__ GiantShared sh;
-  if (ctl[CTL_DONE]) return;
+  if (refine_done(s.ctl, s.sweep)) return;
   const int32_t count = *giant_count;
   for (int32_t i = blockIdx.x; i < count; i += gridDim.x) {
     const int32_t v = giants[i];
     const int32_t g = v / gr.S;
-    if (threadIdx.x == 0) rank[v] = mix4((uint32_t)g, (uint32_t)v, (level << 16) | sweep, seed);
-    const int32_t old = lin[v];
+    int2 self;
+    if constexpr (FIRST) self = int2{s.parent[v], v};
+    else self = s.lin[v];
+    const int32_t pv = self.x, old = self.y;
     const double tm = gr.two_m[g];
+    auto propose = [&](int32_t choice) {
+      if (threadIdx.x == 0) {
+        s.prop[v] = choice;
+        s.mover[v] = choice != old ? pv : -1;
+      }
+    };
     if (!(tm > 0.0)) {
-      if (threadIdx.x == 0) prop[v] = old;
+      propose(old);
       continue;
     }
     const int32_t a = gr.beg[v], b = gr.end[v];
-    const int32_t pv = parent[v];
     int32_t thr;
     double e_sum;
-    if (!giant_table<true>(gr, parent, lin, v, pv, a, b, sh, &thr, &e_sum)) {  // cannot happen: stay, flagged
-      if (threadIdx.x == 0) {
-        prop[v] = old;
-        ctl[CTL_OVERFLOW] = 1;
-      }
+    auto community_of = [&](int32_t u) {
+      if constexpr (FIRST) return s.parent[u] == pv ? u : -1;
+      const int2 q = FIRST ? int2{} : s.lin[u];
+      return q.x == pv ? q.y : -1;
+    };
+    if (!giant_table(gr, community_of, v, a, b, sh, &thr, &e_sum)) {  // cannot happen: stay, flagged
+      propose(old);
+      if (threadIdx.x == 0) s.ctl[CTL_OVERFLOW] = 1;
       __syncthreads();
       continue;
     }
     const double kv = gr.k_v[v];
-    double vol_minus = parent_sigma[pv] - kv;
+    double vol_minus = s.parent_sigma[pv] - kv;
     if (vol_minus < 0.0) vol_minus = 0.0;
-    const double bound = (double)resolution * kv * vol_minus / tm;
+    const double bound = (double)s.resolution * kv * vol_minus / tm;
     if ((double)(float)e_sum < bound) {  // {v} is not well connected to its parent community
-      if (threadIdx.x == 0) prop[v] = old;
+      propose(old);
       __syncthreads();
       continue;
     }
@@ -865,7 +1055,7 @@ __global__ __launch_bounds__(GIANT_THREADS) void refine_propose_giant_kernel(
     const double m_g = 0.5 * tm;
     const double inv_m = 1.0 / m_g;
     const double inv_2m2 = 1.0 / (2.0 * m_g * m_g);
-    const double sig_old_excl = sigma[old] - kv;
+    const double sig_old_excl = s.sigma[old] - kv;
     uint64_t mine = 0;
     int32_t mine_c = old;
     for (int j = threadIdx.x; j < GIANT_SLOTS; j += GIANT_THREADS) {
@@ -873,11 +1063,11 @@ __global__ __launch_bounds__(GIANT_THREADS) void refine_propose_giant_kernel(
       if (c < 0 || sh.first[j] >= thr || c == old) continue;
       const float kn = (float)sh.s[j];
       const double dq = ((double)kn - (double)k_old) * inv_m
-                        + (double)resolution * kv * (sig_old_excl - sigma[c]) * inv_2m2;
+                        + (double)s.resolution * kv * (sig_old_excl - s.sigma[c]) * inv_2m2;
       if (dq < 0.0) continue;
-      const float score = boltzmann
-          ? (float)(dq * (double)inv_theta)
-                + gumbel(rand_uniform_pair((uint32_t)g, (uint32_t)v, (uint32_t)c, level, sweep, seed))
+      const float score = s.boltzmann
+          ? (float)(dq * (double)s.inv_theta)
+                + gumbel(rand_uniform_pair((uint32_t)g, (uint32_t)v, (uint32_t)c, 1u, (uint32_t)s.sweep, s.seed))
           : (float)dq;
       const uint64_t p = pack(score, cand_pref(c));
       if (p > mine) {
@@ -885,55 +1075,14 @@ __global__ __launch_bounds__(GIANT_THREADS) void refine_propose_giant_kernel(
         mine_c = c;
       }
     }
-    const float stay = boltzmann
-        ? gumbel(rand_uniform_pair((uint32_t)g, (uint32_t)v, (uint32_t)old, level, sweep, seed))
+    const float stay = s.boltzmann
+        ? gumbel(rand_uniform_pair((uint32_t)g, (uint32_t)v, (uint32_t)old, 1u, (uint32_t)s.sweep, s.seed))
         : 0.0f;
     const int32_t choice = giant_pick(mine, mine_c, pack(stay, STAY_PREF), old, sh);
-    if (threadIdx.x == 0) prop[v] = choice;
+    propose(choice);
   }
 }
 
-// Commit an independent set of the proposals: a mover commits unless a
-// moving neighbour in its parent community outranks it on (rank, id)
-// (refinement.cu:263-300).
-__global__ __launch_bounds__(LTHREADS) void refine_commit_kernel(
-    Graph gr, const int32_t* __restrict__ parent, const int32_t* __restrict__ lin,
-    const int32_t* __restrict__ prop, const uint32_t* __restrict__ rank, int32_t* __restrict__ lout,
-    int32_t* __restrict__ ctl) {
-  const int32_t v = blockIdx.x * LWAVES + (threadIdx.x >> 6);
-  if (v >= gr.V) return;
-  const int32_t old = lin[v];
-  if (ctl[CTL_DONE]) {
-    if (lane() == 0) lout[v] = old;
-    return;
-  }
-  const int32_t p = prop[v];
-  if (p == old) {
-    if (lane() == 0) lout[v] = old;
-    return;
-  }
-  const int32_t pv = parent[v];
-  const uint32_t rv = rank[v];
-  const int32_t a = gr.beg[v], b = gr.end[v];
-  bool lost = false;
-  for (int32_t e = a + lane(); e < b; e += 64) {
-    const int32_t u = gr.col[e];
-    if (u == v || parent[u] != pv || prop[u] == lin[u]) continue;
-    const uint32_t ru = rank[u];
-    lost = lost || ru > rv || (ru == rv && u > v);
-  }
-  const bool any_lost = __ballot(lost) != 0;
-  if (lane() == 0) {
-    lout[v] = any_lost ? old : p;
-    if (!any_lost) mark_moved(ctl);
-  }
-}
-
-__global__ void refine_control_kernel(int32_t* __restrict__ ctl) {
-  if (threadIdx.x != 0) return;
-  if (!ctl[CTL_DONE] && ctl[CTL_MOVED] == 0) ctl[CTL_DONE] = 1;
-  ctl[CTL_MOVED] = 0;
-}
 
 // q_v = in(v) / 2m - gamma k_v Sigma[c_v] / (4 m^2); Q_g is their sum over
 // the graph (helpers.cu:41-78).
@@ -1576,14 +1725,22 @@ __global__ __launch_bounds__(AGG_DENSE_THREADS) void agg_dense_kernel(Contract c
 }
 
 // ----------------------------------------------------------------- the run's own small kernels
-// Start of a level: identity labels and cleared lists (the overflow word stays raised).
+// Start of a level: identity labels, the first sweep's cleared totals, cleared
+// lists and control words (the overflow word stays raised after the first level).
 __global__ __launch_bounds__(ETHREADS) void level_init_kernel(int32_t V, int32_t* __restrict__ labels,
+                                                              int32_t* __restrict__ moves, double* __restrict__ total,
                                                               int32_t* __restrict__ ctl,
                                                               int32_t* __restrict__ hub_count,
                                                               int32_t* __restrict__ giant_count, int first) {
   const int32_t v = blockIdx.x * ETHREADS + threadIdx.x;
-  if (v < V) labels[v] = v;
-  if (v < CTL_WORDS && (v != CTL_OVERFLOW || first)) ctl[v] = v == CTL_UPDOWN ? 1 : 0;
+  if (v < V) {
+    labels[v] = v;
+    moves[v] = v;
+    total[v] = 0.0;
+  }
+  for (int32_t i = v; i < CTL_WORDS; i += gridDim.x * ETHREADS) {
+    if (i != CTL_OVERFLOW || first) ctl[i] = 0;
+  }
   if (v == 0) {
     *hub_count = 0;
     *giant_count = 0;
@@ -1699,8 +1856,8 @@ int launch_check() {
 }
 
 struct LeidenLayout {
-  size_t keys_a, keys_b, vals_a, vals_b, temp, temp_bytes, row_ptr, col, k_v, two_m, sigma, psigma, lab_a, lab_b,
-      parent, prop, rank, ctl, hubs, hub_count, giants, giant_count, total;
+  size_t keys_a, keys_b, vals_a, vals_b, temp, temp_bytes, row_ptr, col, k_v, two_m, totals[4], lab, moves[2], pairs[2],
+      prop, mover, ctl, hubs, hub_count, giants, giant_count, total;
 };
 
 LeidenLayout leiden_layout(int64_t E, int32_t G, int32_t S) {
@@ -1727,13 +1884,14 @@ LeidenLayout leiden_layout(int64_t E, int32_t G, int32_t S) {
   L.col = take(n * 4);
   L.k_v = take(V * 8);
   L.two_m = take(G * 8);
-  L.sigma = take(V * 8);
-  L.psigma = take(V * 8);
-  L.lab_a = take(V * 4);
-  L.lab_b = take(V * 4);
-  L.parent = take(V * 4);
+  for (size_t& at : L.totals) at = take(V * 8);
+  L.lab = take(V * 4);
+  for (int i = 0; i < 2; ++i) {
+    L.moves[i] = take(V * 4);
+    L.pairs[i] = take(V * 8);
+  }
   L.prop = take(V * 4);
-  L.rank = take(V * 4);
+  L.mover = take(V * 4);
   L.ctl = take(CTL_WORDS * 4);
   L.hubs = take(V * 4);
   L.hub_count = take(4);
@@ -1812,12 +1970,12 @@ namespace {
 
 // The arrays of one level's sweeps.
 struct SweepBuffers {
-  double* sigma;
-  double* psigma;
-  int32_t* lab[2];  // lab[0] is the identity on entry
-  int32_t* parent;
+  double* total[4];    // communities' total degrees, in turn
+  int32_t* labels;     // the result; identity on entry
+  int32_t* moves[2];   // local moving's labels; moves[0] is the identity on entry
+  int2* pairs[2];      // refinement's (parent, label)
   int32_t* prop;
-  uint32_t* rank;
+  int32_t* mover;
   int32_t* ctl;
   int32_t* hubs;
   int32_t* hub_count;
@@ -1825,53 +1983,58 @@ struct SweepBuffers {
   int32_t* giant_count;
 };
 
-// Local moving and refinement of one level; returns the index of the label
-// buffer that holds the result.
-int run_sweeps(const Graph& gr, const SweepBuffers& b, float resolution, float theta, int32_t max_inner_iter,
-               int32_t seed, int32_t use_boltzmann, hipStream_t st) {
+// Queues a level: cleared state, lists of long rows, local moving and
+// refinement.  The communities end in b.labels.
+void run_sweeps(const Graph& gr, const SweepBuffers& b, float resolution, float theta, int32_t max_inner_iter,
+                int32_t seed, int32_t use_boltzmann, bool first_level, hipStream_t st) {
   const int32_t V = gr.V;
-  const unsigned egrid = blocks(V, ETHREADS), vgrid = blocks(V, LWAVES);
-  int cur = 0;
-  for (int sweep = 0; sweep < max_inner_iter; ++sweep) {
-    sigma_zero_kernel<<<egrid, ETHREADS, 0, st>>>(b.sigma, V, b.ctl);
-    sigma_scatter_kernel<<<egrid, ETHREADS, 0, st>>>(b.lab[cur], gr.k_v, V, b.sigma, b.ctl);
-    local_moving_kernel<false><<<blocks(V, SWAVES), 64 * SWAVES, 0, st>>>(
-        gr, b.sigma, b.lab[cur], b.lab[cur ^ 1], b.ctl, b.hubs, b.hub_count, resolution, 0u, (uint32_t)sweep,
-        (uint32_t)seed);
-    local_moving_kernel<true><<<HUB_BLOCKS, LTHREADS, 0, st>>>(gr, b.sigma, b.lab[cur], b.lab[cur ^ 1], b.ctl, b.hubs,
-                                                              b.hub_count, resolution, 0u, (uint32_t)sweep,
-                                                              (uint32_t)seed);
-    local_moving_giant_kernel<<<GIANT_BLOCKS, GIANT_THREADS, 0, st>>>(gr, b.sigma, b.lab[cur], b.lab[cur ^ 1], b.ctl,
-                                                                     b.giants, b.giant_count, resolution, 0u,
-                                                                     (uint32_t)sweep, (uint32_t)seed);
-    lm_control_kernel<<<1, 64, 0, st>>>(b.ctl);
-    cur ^= 1;
+  level_init_kernel<<<blocks(V, ETHREADS), ETHREADS, 0, st>>>(V, b.labels, b.moves[0], b.total[0], b.ctl, b.hub_count,
+                                                              b.giant_count, first_level);
+  hub_list_kernel<<<blocks(V, LIST_THREADS), LIST_THREADS, 0, st>>>(gr.beg, gr.end, V, b.hubs, b.hub_count, b.giants,
+                                                                   b.giant_count);
+  const unsigned grid = HUB_BLOCKS + blocks(V, GROUPS);
+  // (a row of different neighbours, its self loop twice, is at most one longer than its graph)
+  const bool giants = !gr.unique || gr.S >= GIANT_MIN;
+  double* const* t = b.total;
+  for (int32_t i = 0; i < max_inner_iter; ++i) {
+    if (i > 0 && i % RING == 0) fold_kernel<<<1, 64, 0, st>>>(b.ctl, 1, 0);
+    const MoveSweep s{i == 0 ? gr.k_v : t[(i - 1) % 3], t[i % 3], t[(i + 1) % 3], b.moves[i & 1], b.moves[(i & 1) ^ 1],
+                      b.ctl, i, resolution, (uint32_t)seed};
+    if (i == 0 && gr.unique) {
+      local_moving_kernel<true><<<grid, HUB_THREADS, 0, st>>>(gr, s, b.hubs, b.hub_count);
+      if (giants) local_moving_giant_kernel<true><<<GIANT_BLOCKS, GIANT_THREADS, 0, st>>>(gr, s, b.giants, b.giant_count);
+    } else {
+      local_moving_kernel<false><<<grid, HUB_THREADS, 0, st>>>(gr, s, b.hubs, b.hub_count);
+      if (giants)
+        local_moving_giant_kernel<false><<<GIANT_BLOCKS, GIANT_THREADS, 0, st>>>(gr, s, b.giants, b.giant_count);
+    }
   }
   if (g_test_raise_overflow) raise_overflow_kernel<<<1, 64, 0, st>>>(b.ctl);
   // refinement from singletons inside the local-moving communities
-  refine_init_kernel<<<egrid, ETHREADS, 0, st>>>(b.lab[cur], V, b.parent, b.lab[cur ^ 1], b.ctl);
-  cur ^= 1;
-  sigma_zero_kernel<<<egrid, ETHREADS, 0, st>>>(b.psigma, V, nullptr);
-  sigma_scatter_kernel<<<egrid, ETHREADS, 0, st>>>(b.parent, gr.k_v, V, b.psigma, nullptr);
-  const float t = theta > 0.0f ? theta : 1.0e-3f;
-  const float inv_theta = 1.0f / t;
-  for (int sweep = 0; sweep < max_inner_iter; ++sweep) {
-    sigma_zero_kernel<<<egrid, ETHREADS, 0, st>>>(b.sigma, V, b.ctl);
-    sigma_scatter_kernel<<<egrid, ETHREADS, 0, st>>>(b.lab[cur], gr.k_v, V, b.sigma, b.ctl);
-    refine_propose_kernel<false><<<blocks(V, SWAVES), 64 * SWAVES, 0, st>>>(
-        gr, b.parent, b.sigma, b.psigma, b.lab[cur], b.prop, b.rank, b.ctl, b.hubs, b.hub_count, resolution, inv_theta,
-        use_boltzmann ? 1 : 0, 1u, (uint32_t)sweep, (uint32_t)seed);
-    refine_propose_kernel<true><<<HUB_BLOCKS, LTHREADS, 0, st>>>(
-        gr, b.parent, b.sigma, b.psigma, b.lab[cur], b.prop, b.rank, b.ctl, b.hubs, b.hub_count, resolution, inv_theta,
-        use_boltzmann ? 1 : 0, 1u, (uint32_t)sweep, (uint32_t)seed);
-    refine_propose_giant_kernel<<<GIANT_BLOCKS, GIANT_THREADS, 0, st>>>(
-        gr, b.parent, b.sigma, b.psigma, b.lab[cur], b.prop, b.rank, b.ctl, b.giants, b.giant_count, resolution,
-        inv_theta, use_boltzmann ? 1 : 0, 1u, (uint32_t)sweep, (uint32_t)seed);
-    refine_commit_kernel<<<vgrid, LTHREADS, 0, st>>>(gr, b.parent, b.lab[cur], b.prop, b.rank, b.lab[cur ^ 1], b.ctl);
-    refine_control_kernel<<<1, 64, 0, st>>>(b.ctl);
-    cur ^= 1;
+  const int32_t* parent = b.moves[max_inner_iter & 1];
+  const double* parent_total = max_inner_iter == 0 ? gr.k_v : t[(max_inner_iter - 1) % 3];
+  double* r[3] = {t[max_inner_iter % 3], t[(max_inner_iter + 1) % 3], t[3]};  // r[0] was cleared by the last sweep
+  const float temperature = theta > 0.0f ? theta : 1.0e-3f;
+  const float inv_theta = 1.0f / temperature;
+  if (max_inner_iter > RING) fold_kernel<<<1, 64, 0, st>>>(b.ctl, 1, 1);
+  if (!gr.unique) pair_init_kernel<<<blocks(V, ETHREADS), ETHREADS, 0, st>>>(parent, V, b.pairs[0]);
+  for (int32_t i = 0; i < max_inner_iter; ++i) {
+    if (i > 0 && i % RING == 0) fold_kernel<<<1, 64, 0, st>>>(b.ctl, 0, 0);
+    const RefineSweep s{i == 0 ? gr.k_v : r[(i - 1) % 3], parent_total, r[i % 3], r[(i + 1) % 3], parent,
+                        b.pairs[i & 1], b.pairs[(i & 1) ^ 1], b.labels, b.prop, b.mover, b.ctl, i, resolution,
+                        inv_theta, use_boltzmann ? 1 : 0, (uint32_t)seed};
+    if (i == 0 && gr.unique) {
+      refine_propose_kernel<true><<<grid, HUB_THREADS, 0, st>>>(gr, s, b.hubs, b.hub_count);
+      if (giants)
+        refine_propose_giant_kernel<true><<<GIANT_BLOCKS, GIANT_THREADS, 0, st>>>(gr, s, b.giants, b.giant_count);
+      refine_commit_kernel<true><<<grid, HUB_THREADS, 0, st>>>(gr, s, b.hubs, b.hub_count, b.giants, b.giant_count);
+    } else {
+      refine_propose_kernel<false><<<grid, HUB_THREADS, 0, st>>>(gr, s, b.hubs, b.hub_count);
+      if (giants)
+        refine_propose_giant_kernel<false><<<GIANT_BLOCKS, GIANT_THREADS, 0, st>>>(gr, s, b.giants, b.giant_count);
+      refine_commit_kernel<false><<<grid, HUB_THREADS, 0, st>>>(gr, s, b.hubs, b.hub_count, b.giants, b.giant_count);
+    }
   }
-  return cur;
 }
 
 }  // namespace
@@ -1915,17 +2078,9 @@ extern "C" int ckv_batched_leiden(const int32_t* edge_src, const int32_t* edge_d
   int32_t* col = (int32_t*)(ws + L.col);
   double* k_v = (double*)(ws + L.k_v);
   double* two_m = (double*)(ws + L.two_m);
-  double* sigma = (double*)(ws + L.sigma);
-  double* psigma = (double*)(ws + L.psigma);
-  int32_t* lab[2] = {(int32_t*)(ws + L.lab_a), (int32_t*)(ws + L.lab_b)};
-  int32_t* parent = (int32_t*)(ws + L.parent);
-  int32_t* prop = (int32_t*)(ws + L.prop);
-  uint32_t* rank = (uint32_t*)(ws + L.rank);
+  double* sigma = (double*)(ws + L.totals[0]);
+  int32_t* lab = (int32_t*)(ws + L.lab);
   int32_t* ctl = (int32_t*)(ws + L.ctl);
-  int32_t* hubs = (int32_t*)(ws + L.hubs);
-  int32_t* hub_count = (int32_t*)(ws + L.hub_count);
-  int32_t* giants = (int32_t*)(ws + L.giants);
-  int32_t* giant_count = (int32_t*)(ws + L.giant_count);
 
   const int bits = bits_for((uint64_t)V - 1);
   const int end_bit = bits + bits_for((uint64_t)V);
@@ -1938,23 +2093,25 @@ extern "C" int ckv_batched_leiden(const int32_t* edge_src, const int32_t* edge_d
     return ckv_internal::set_error(CKV_E_LAUNCH, "Leiden CSR sort failed");
   row_ptr_kernel<<<blocks(V + 1, ETHREADS), ETHREADS, 0, st>>>(keys_b, n, V, bits, row_ptr);
   col_kernel<<<blocks(n, ETHREADS), ETHREADS, 0, st>>>(keys_b, n, bits, col);
-  zero_kernel<<<1, 256, 0, st>>>(two_m, graphs, modularity, ctl, hub_count, giant_count);
-  hub_list_kernel<<<blocks(V, LIST_THREADS), LIST_THREADS, 0, st>>>(row_ptr, row_ptr + 1, V, hubs, hub_count, giants,
-                                                                   giant_count);
-  const unsigned vgrid = blocks(V, LWAVES);
+  const unsigned vgrid = blocks(V, LWAVES), egrid = blocks(V, ETHREADS);
   degree_kernel<<<vgrid, LTHREADS, 0, st>>>(row_ptr, vals_b, V, k_v);
   graph_sum_kernel<<<graphs, SUM_THREADS, 0, st>>>(k_v, seq_len, two_m);
-  identity_kernel<<<blocks(V, ETHREADS), ETHREADS, 0, st>>>(V, lab[0]);
-  const Graph gr{row_ptr, row_ptr + 1, col, vals_b, k_v, two_m, V, seq_len};
-  const SweepBuffers buf{sigma, psigma, {lab[0], lab[1]}, parent, prop, rank, ctl, hubs, hub_count, giants, giant_count};
-  const unsigned egrid = blocks(V, ETHREADS);
-  const int cur = run_sweeps(gr, buf, resolution, theta, max_inner_iter, seed, use_boltzmann, st);
-  sigma_zero_kernel<<<egrid, ETHREADS, 0, st>>>(sigma, V, nullptr);
-  sigma_scatter_kernel<<<egrid, ETHREADS, 0, st>>>(lab[cur], k_v, V, sigma, nullptr);
-  modularity_kernel<<<vgrid, LTHREADS, 0, st>>>(gr, lab[cur], sigma, resolution, psigma);
-  graph_sum_kernel<<<graphs, SUM_THREADS, 0, st>>>(psigma, seq_len, modularity);
+  const Graph gr{row_ptr, row_ptr + 1, col, vals_b, k_v, two_m, V, seq_len, false};
+  const SweepBuffers buf{{(double*)(ws + L.totals[0]), (double*)(ws + L.totals[1]), (double*)(ws + L.totals[2]),
+                          (double*)(ws + L.totals[3])},
+                         lab,
+                         {(int32_t*)(ws + L.moves[0]), (int32_t*)(ws + L.moves[1])},
+                         {(int2*)(ws + L.pairs[0]), (int2*)(ws + L.pairs[1])},
+                         (int32_t*)(ws + L.prop), (int32_t*)(ws + L.mover), ctl, (int32_t*)(ws + L.hubs),
+                         (int32_t*)(ws + L.hub_count), (int32_t*)(ws + L.giants), (int32_t*)(ws + L.giant_count)};
+  run_sweeps(gr, buf, resolution, theta, max_inner_iter, seed, use_boltzmann, true, st);
+  sigma_zero_kernel<<<egrid, ETHREADS, 0, st>>>(sigma, V);
+  sigma_scatter_kernel<<<egrid, ETHREADS, 0, st>>>(lab, k_v, V, sigma);
+  double* share = (double*)(ws + L.totals[1]);
+  modularity_kernel<<<vgrid, LTHREADS, 0, st>>>(gr, lab, sigma, resolution, share);
+  graph_sum_kernel<<<graphs, SUM_THREADS, 0, st>>>(share, seq_len, modularity);
   overflow_mark_kernel<<<blocks(graphs, ETHREADS), ETHREADS, 0, st>>>(ctl, graphs, modularity);
-  finish_kernel<<<egrid, ETHREADS, 0, st>>>(row_ptr, lab[cur], V, labels);
+  finish_kernel<<<egrid, ETHREADS, 0, st>>>(row_ptr, lab, V, labels);
   return launch_check();
 }
 
@@ -2057,8 +2214,8 @@ namespace ckv {
 namespace {
 
 struct RunLayout {
-  size_t row_ptr, col0, wt0, col[2], wt[2], beg[2], end[2], k[2], two_m, two_m0, sigma, psigma, square, lab[2], parent,
-      prop, rank, ctl, hubs, giants, counts, flags, scan, dense, hist, first, members, dense_list, lists, words, temp,
+  size_t row_ptr, col0, wt0, col[2], wt[2], beg[2], end[2], k[2], two_m, two_m0, totals[4], lab, moves[2], pairs[2], prop,
+      mover, ctl, hubs, giants, counts, flags, scan, dense, hist, first, members, dense_list, lists, words, temp,
       temp_bytes, sort, total;
 };
 
@@ -2080,16 +2237,15 @@ RunLayout run_layout(int64_t E, int32_t G, int32_t S) {
     L.beg[i] = take(V * 4);
     L.end[i] = take(V * 4);
     L.k[i] = take(V * 8);
-    L.lab[i] = take(V * 4);
+    L.moves[i] = take(V * 4);
+    L.pairs[i] = take(V * 8);
   }
   L.two_m = take(G * 8);
   L.two_m0 = take(G * 8);
-  L.sigma = take(V * 8);
-  L.psigma = take(V * 8);
-  L.square = take(V * 8);
-  L.parent = take(V * 4);
+  for (size_t& at : L.totals) at = take(V * 8);
+  L.lab = take(V * 4);
   L.prop = take(V * 4);
-  L.rank = take(V * 4);
+  L.mover = take(V * 4);
   L.ctl = take(CTL_WORDS * 4);
   L.hubs = take(V * 4);
   L.giants = take(V * 4);
@@ -2210,18 +2366,18 @@ extern "C" int ckv_leiden_run(const int32_t* edge_src, const int32_t* edge_dst, 
   graph_sum_kernel<<<graphs, SUM_THREADS, 0, st>>>(degree, seq_len, f64(L.two_m0));
 
   // ---- levels
-  const Graph gr0{row_ptr, row_ptr + 1, col0, wt0, degree, f64(L.two_m0), V0, seq_len};
+  const Graph gr0{row_ptr, row_ptr + 1, col0, wt0, degree, f64(L.two_m0), V0, seq_len, host[1] == 0};
   Graph gr = gr0;
   for (int32_t level = 0;; ++level) {
     const unsigned egrid = blocks(gr.V, ETHREADS);
-    level_init_kernel<<<egrid, ETHREADS, 0, st>>>(gr.V, i32(L.lab[0]), ctl, hub_count, giant_count, level == 0);
-    hub_list_kernel<<<blocks(gr.V, LIST_THREADS), LIST_THREADS, 0, st>>>(gr.beg, gr.end, gr.V, i32(L.hubs), hub_count,
-                                                                        i32(L.giants), giant_count);
-    const SweepBuffers buf{f64(L.sigma), f64(L.psigma), {i32(L.lab[0]), i32(L.lab[1])}, i32(L.parent), i32(L.prop),
-                           (uint32_t*)(ws + L.rank), ctl, i32(L.hubs), hub_count, i32(L.giants), giant_count};
-    const int cur = run_sweeps(gr, buf, resolution, theta, max_inner_iter, seed + level, use_boltzmann, st);
+    const SweepBuffers buf{{f64(L.totals[0]), f64(L.totals[1]), f64(L.totals[2]), f64(L.totals[3])},
+                           i32(L.lab),
+                           {i32(L.moves[0]), i32(L.moves[1])},
+                           {(int2*)(ws + L.pairs[0]), (int2*)(ws + L.pairs[1])},
+                           i32(L.prop), i32(L.mover), ctl, i32(L.hubs), hub_count, i32(L.giants), giant_count};
+    run_sweeps(gr, buf, resolution, theta, max_inner_iter, seed + level, use_boltzmann, level == 0, st);
     // ranks of the labels in use, per graph
-    const int32_t* lab = i32(L.lab[cur]);
+    const int32_t* lab = i32(L.lab);
     int32_t* flags = i32(L.flags);
     int32_t* scan = i32(L.scan);
     int32_t* dense = i32(L.dense);
@@ -2257,19 +2413,19 @@ extern "C" int ckv_leiden_run(const int32_t* edge_src, const int32_t* edge_dst, 
       agg_dense_kernel<<<AGG_DENSE_BLOCKS, AGG_DENSE_THREADS, agg_dense_lds(), st>>>(c, i32(L.dense_list), lists);
     }
     gr = Graph{i32(L.beg[to]), i32(L.end[to]), i32(L.col[to]), (float*)(ws + L.wt[to]), f64(L.k[to]), f64(L.two_m), Vs,
-               *width};
+               *width, true};
     graph_sum_kernel<<<graphs, SUM_THREADS, 0, st>>>(gr.k_v, gr.S, f64(L.two_m));
   }
 
   // ---- modularity of the result on the first level's graph
   const unsigned egrid = blocks(V0, ETHREADS);
-  sigma_zero_kernel<<<egrid, ETHREADS, 0, st>>>(f64(L.sigma), V0, nullptr);
-  sigma_scatter_kernel<<<egrid, ETHREADS, 0, st>>>(labels, degree, V0, f64(L.sigma), nullptr);
-  inside_kernel<<<blocks(V0, LWAVES), LTHREADS, 0, st>>>(gr0, labels, f64(L.sigma), f64(L.psigma), f64(L.square));
+  sigma_zero_kernel<<<egrid, ETHREADS, 0, st>>>(f64(L.totals[0]), V0);
+  sigma_scatter_kernel<<<egrid, ETHREADS, 0, st>>>(labels, degree, V0, f64(L.totals[0]));
+  inside_kernel<<<blocks(V0, LWAVES), LTHREADS, 0, st>>>(gr0, labels, f64(L.totals[0]), f64(L.totals[1]), f64(L.totals[2]));
   double* sums = f64(L.k[0]);  // per graph: inside, square; then the result
   double* squares = f64(L.k[1]);
-  graph_sum_kernel<<<graphs, SUM_THREADS, 0, st>>>(f64(L.psigma), seq_len, sums);
-  graph_sum_kernel<<<graphs, SUM_THREADS, 0, st>>>(f64(L.square), seq_len, squares);
+  graph_sum_kernel<<<graphs, SUM_THREADS, 0, st>>>(f64(L.totals[1]), seq_len, sums);
+  graph_sum_kernel<<<graphs, SUM_THREADS, 0, st>>>(f64(L.totals[2]), seq_len, squares);
   union_modularity_kernel<<<1, 64, 0, st>>>(f64(L.two_m0), sums, squares, graphs, resolution, ctl, f64(L.hist));
   isolated_kernel<<<egrid, ETHREADS, 0, st>>>(row_ptr, V0, labels);
   if (int rc = launch_check()) return rc;

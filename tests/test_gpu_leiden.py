@@ -349,3 +349,56 @@ def test_dense_communities_match_oracle(device):
         ref = L.dense_remap(L.fill_isolated(lab))
         np.testing.assert_array_equal(ids.cpu().numpy(), ref)
         assert counts.cpu().tolist() == (ref.max(axis=1) + 1).tolist()
+
+
+SWEEP_ROWS = [
+    # seed, row lengths, vertices, self loops, sweeps: each side of the row classes' edges; more sweeps than one ring of
+    # marks; the longest row of a graph that needs no workgroup of 1,024 threads, and of one that does
+    (51, (1, 2, 31, 32, 33, 63, 64, 65), 400, 3, 5),
+    (52, (127, 128, 129, 130), 700, 0, 4),
+    (53, (255, 256, 257, 511, 512, 513), 1500, 0, 4),
+    (54, (1022, 1021), 1023, 1, 3),
+    (55, (1023, 1022), 1024, 1, 3),
+    (56, (1023, 1024, 1025), 2200, 1, 3),
+    (57, (40, 90), 300, 0, 130),
+]
+
+
+@pytest.mark.parametrize("ordered", [True, False])
+@pytest.mark.parametrize("seed,rows,S,loops,sweeps", SWEEP_ROWS)
+def test_sweep_row_classes(device, seed, rows, S, loops, sweeps, ordered):
+    """Rows at the edges of the sweeps' classes (half a wave, a workgroup of
+    256, one of 1,024), on an ascending list (each row names a neighbour once:
+    the first sweeps build no table) and on a shuffled one: labels equal the
+    oracle's (dyadic weights: every sum exact)."""
+    rng = np.random.default_rng(seed)
+    src, dst, w = lg.planted(seed, 2, S, 10, edges_per_vertex=4.0, self_loops=loops)
+    key = {}
+    for a, b, x in zip(src.tolist(), dst.tolist(), w.tolist()):
+        key[min(a, b), max(a, b)] = x
+    for i, n in enumerate(rows):  # vertex i of the second graph gets a row of exactly n other vertices
+        v = S + i
+        have = {b if a == v else a for a, b in key if (a == v) != (b == v)}
+        far = [u for u in rng.permutation(np.arange(S + len(rows), 2 * S)).tolist() if u not in have]
+        for u in far[:max(0, n - len(have))]:
+            key[v, u] = int(rng.integers(1, 9)) / 64.0
+    if loops:
+        key[S, S] = 0.25
+    order = sorted(key)
+    if not ordered:
+        order = [order[i] for i in rng.permutation(len(order))]
+    src, dst = (np.array([p[i] for p in order], np.int32) for i in (0, 1))
+    w = np.array([key[p] for p in order], np.float32)
+    print(f"leiden rows {rows} S={S} edges={src.size} ordered={ordered} sweeps={sweeps}", flush=True)
+    s, d, x = _dev(device, src, dst, w)
+    kw = dict(seq_len=S, max_level=1, max_inner_iter=sweeps, seed=seed)
+    vertex, part, _ = algorithm.run_leiden(s, d, x, G=2, **kw)
+    rv, rp, _ = L.run_leiden(src, dst, w, graphs=2, **kw)
+    np.testing.assert_array_equal(vertex.cpu().numpy(), rv)
+    np.testing.assert_array_equal(part.cpu().numpy(), rp)
+    # with noise in the scores, the same sweeps through the general path (logf is the device's on both sides)
+    vertex, part, _ = algorithm.run_leiden(s, d, x, G=2, use_boltzmann=True, **kw)
+    general, _ = _native_level(device, src, dst, w, 2, S, use_boltzmann=True, max_inner_iter=sweeps, seed=seed)
+    general = general[vertex.cpu().numpy()]
+    pairs = np.unique(np.stack([general, part.cpu().numpy()]), axis=1).shape[1]
+    assert pairs == np.unique(general).size == np.unique(part.cpu().numpy()).size

@@ -88,14 +88,16 @@ __device__ inline uint32_t mix4(uint32_t a, uint32_t b, uint32_t c, uint32_t d) 
   h = pcg_hash(h ^ c);
   return pcg_hash(h ^ d);
 }
+// mix4 of a salt = pcg_hash(pcg_hash(graph) ^ vertex) kept per vertex.
+__device__ inline uint32_t salt_of(uint32_t g, uint32_t v) { return pcg_hash(pcg_hash(g) ^ v); }
+__device__ inline uint32_t mix_salt(uint32_t salt, uint32_t c, uint32_t d) { return pcg_hash(pcg_hash(salt ^ c) ^ d); }
 __device__ inline float unit_float(uint32_t h) { return (float)(h >> 8) * (1.0f / 16777216.0f); }
-__device__ inline float rand_uniform(uint32_t g, uint32_t v, uint32_t level, uint32_t sweep, uint32_t seed) {
-  return unit_float(mix4(g, v, (level << 16) | sweep, seed));
+__device__ inline float rand_uniform(uint32_t salt, uint32_t level, uint32_t sweep, uint32_t seed) {
+  return unit_float(mix_salt(salt, (level << 16) | sweep, seed));
 }
-__device__ inline float rand_uniform_pair(uint32_t g, uint32_t v, uint32_t c, uint32_t level, uint32_t sweep,
-                                          uint32_t seed) {
+__device__ inline float rand_uniform_pair(uint32_t salt, uint32_t c, uint32_t level, uint32_t sweep, uint32_t seed) {
   const uint32_t s = pcg_hash((sweep << 16) ^ c);
-  return unit_float(mix4(g, v, (level << 16) | (s & 0xFFFFu), seed));
+  return unit_float(mix_salt(salt, (level << 16) | (s & 0xFFFFu), seed));
 }
 __device__ inline float gumbel(float u) {
   u = fmaxf(u, 1.0e-7f);
@@ -272,6 +274,31 @@ struct Graph {
   bool unique;  // no row names another vertex twice
 };
 
+// v / S for 0 <= v < 2^31 by a multiplication (a 32-bit division is some 40 issue slots).
+struct Divisor {
+  uint32_t mul;
+  int32_t shift;
+  explicit Divisor(int32_t S) : mul(0), shift(0) {
+    if (S < 2) return;  // one vertex a graph: v itself
+    int bits = 1;
+    while (((int64_t)1 << bits) < S) ++bits;
+    // mul S - 2^(31 + bits) < S <= 2^bits, so the quotient of every v below 2^31 is exact
+    mul = (uint32_t)((((uint64_t)1 << (31 + bits)) + (uint64_t)S - 1) / (uint64_t)S);
+    shift = bits - 1;
+  }
+  __device__ int32_t of(int32_t v) const { return mul == 0 ? v : (int32_t)(__umulhi((uint32_t)v, mul) >> shift); }
+};
+
+// A load that stays where it is written (the compiler would move one whose
+// value is used late behind the loads it should travel with).
+template <class T>
+__device__ __forceinline__ T load_now(const T* p) {
+  if constexpr (sizeof(T) == 4)
+    return __builtin_bit_cast(T, __hip_atomic_load((const uint32_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT));
+  else
+    return __builtin_bit_cast(T, __hip_atomic_load((const uint64_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT));
+}
+
 // Sweeps.  A vertex of at most SMALL_ROW entries (nearly all) is handled by
 // half a wave, a longer one (listed once per level by hub_list_kernel) by a
 // workgroup of HUB_THREADS, both with up to ROW_PER entries per thread held in
@@ -298,9 +325,10 @@ constexpr int SMALL_ROW = 128;
 constexpr int ROW_PER = 4;
 constexpr int HUB_THREADS = 256;
 constexpr int HUB_BLOCKS = 512;  // a multiple of 8, so the blocks behind them keep their XCD
-constexpr int SMALL_SLOTS = 192, HUB_SLOTS = 1536;  // table load at most 2/3
-constexpr int GROUPS = HUB_THREADS / 32;            // half waves per workgroup: 8 x 192 slots = 1,536
-static_assert(GROUPS * SMALL_SLOTS == HUB_SLOTS, "both kinds of workgroup use the same LDS (18 KB, eight a compute unit)");
+constexpr int SMALL_SLOTS = 184, HUB_SLOTS = 1472;  // table load at most 70%
+constexpr int GROUPS = HUB_THREADS / 32;            // half waves per workgroup
+// Both kinds of workgroup use the same LDS (20 KB, eight a compute unit).
+static_assert(GROUPS * SMALL_SLOTS == HUB_SLOTS && GROUPS * SMALL_ROW == HUB_THREADS * ROW_PER, "tables and lists");
 
 constexpr int GIANT_MIN = TABLE_CAP;  // rows longer than this take a workgroup of GIANT_THREADS
 constexpr int GIANT_SLOTS = 4096;
@@ -341,11 +369,23 @@ __global__ __launch_bounds__(LIST_THREADS) void hub_list_kernel(const int32_t* _
   if (giant) giants[s_at[1] + bg + __popcll(mg & below)] = v;
 }
 
-// The threads of one vertex.
+// The threads of one vertex, with their part of the workgroup's LDS.
+struct SweepShared {
+  int32_t tc[HUB_SLOTS];                    // communities, -1 free
+  double ts[HUB_SLOTS];                     // weight to them
+  uint16_t list[HUB_THREADS * ROW_PER];     // slots in use
+  uint64_t best[HUB_THREADS / 64];
+  double sum[HUB_THREADS / 64];
+  int32_t value, count;
+};
 struct HalfWave {
   static constexpr int N = 32, SLOTS = SMALL_SLOTS;
   int32_t* tc;
   double* ts;
+  uint16_t* list;
+  __device__ explicit HalfWave(SweepShared& sh)
+      : tc(sh.tc + (threadIdx.x >> 5) * SMALL_SLOTS), ts(sh.ts + (threadIdx.x >> 5) * SMALL_SLOTS),
+        list(sh.list + (threadIdx.x >> 5) * SMALL_ROW) {}
   __device__ int tid() const { return lane() & 31; }
   __device__ void sync() const { wave_lds_sync(); }
   __device__ uint64_t max(uint64_t x) const {
@@ -362,24 +402,29 @@ struct HalfWave {
     x += __builtin_bit_cast(double, xor_u64<8>(__builtin_bit_cast(uint64_t, x)));
     return x + __builtin_bit_cast(double, xor_u64<16>(__builtin_bit_cast(uint64_t, x)));
   }
+  __device__ uint32_t ballot(bool x) const { return (uint32_t)(__ballot(x) >> (lane() & 32)); }
   // The value of the thread that holds the winning key.
   __device__ int32_t of(uint64_t best, uint64_t mine, int32_t value) const {
-    const uint64_t m = __ballot(mine == best) >> (lane() & 32);
-    return __shfl(value, (lane() & 32) + __builtin_ctz((uint32_t)m));
+    return __shfl(value, (lane() & 32) + __builtin_ctz(ballot(mine == best)));
   }
-  __device__ bool any(bool x) const { return (uint32_t)(__ballot(x) >> (lane() & 32)) != 0; }
+  __device__ bool any(bool x) const { return ballot(x) != 0; }
+  // Lists slot h of the threads that took a free one, behind the n listed before.
+  __device__ void start_list() const {}
+  __device__ int append(bool taken, int h, int n) const {
+    const uint32_t m = ballot(taken);
+    if (taken) list[n + __popc(m & ((1u << tid()) - 1))] = (uint16_t)h;
+    return n + __popc(m);
+  }
+  __device__ int listed(int n) const { return n; }
 };
 
-struct WorkgroupShared {
-  uint64_t best[HUB_THREADS / 64];
-  int32_t value[HUB_THREADS / 64];
-  double sum[HUB_THREADS / 64];
-};
 struct Workgroup {
   static constexpr int N = HUB_THREADS, SLOTS = HUB_SLOTS;
+  SweepShared* sh;
   int32_t* tc;
   double* ts;
-  WorkgroupShared* sh;
+  uint16_t* list;
+  __device__ explicit Workgroup(SweepShared& s) : sh(&s), tc(s.tc), ts(s.ts), list(s.list) {}
   __device__ int tid() const { return threadIdx.x; }
   __device__ void sync() const { __syncthreads(); }
   __device__ uint64_t max(uint64_t x) const {
@@ -400,13 +445,26 @@ struct Workgroup {
     return t;
   }
   __device__ int32_t of(uint64_t best, uint64_t mine, int32_t value) const {
-    if (mine == best) sh->value[0] = value;  // (keys of different candidates differ; equal keys are one candidate)
+    if (mine == best) sh->value = value;  // (equal keys are one candidate)
     __syncthreads();
-    const int32_t r = sh->value[0];
+    const int32_t r = sh->value;
     __syncthreads();
     return r;
   }
   __device__ bool any(bool x) const { return __syncthreads_or(x) != 0; }
+  __device__ void start_list() const {
+    if (threadIdx.x == 0) sh->count = 0;
+  }
+  __device__ int append(bool taken, int h, int) const {
+    const uint64_t m = __ballot(taken);
+    if (m == 0) return 0;
+    int at = 0;
+    if (lane() == 0) at = atomicAdd(&sh->count, __popcll(m));
+    at = __shfl(at, 0);
+    if (taken) list[at + __popcll(m & ((((uint64_t)1) << lane()) - 1))] = (uint16_t)h;
+    return 0;
+  }
+  __device__ int listed(int) const { return sh->count; }
 };
 
 // One vertex's row in its threads' registers: neighbour, weight and whether
@@ -418,18 +476,24 @@ struct Row {
 };
 template <class P>
 __device__ __forceinline__ void load_row(const P& p, const Graph& gr, int32_t v, int32_t a, int32_t b, Row& r) {
+  const int32_t* col = gr.col + a + p.tid();
+  const float* wt = gr.wt + a + p.tid();
+  const int32_t left = b - a - p.tid();
 #pragma unroll
   for (int i = 0; i < ROW_PER; ++i) {
-    const int32_t e = a + i * P::N + p.tid();
-    const int32_t at = min(e, b - 1);  // (past the row: its last entry again, not counted)
-    r.u[i] = gr.col[at];
-    r.w[i] = gr.wt[at];
-    r.ok[i] = e < b && r.u[i] != v;
+    r.u[i] = v;
+    r.w[i] = 0.0f;
+    if (i * P::N < left) {
+      r.u[i] = col[i * P::N];
+      r.w[i] = wt[i * P::N];
+    }
   }
+#pragma unroll
+  for (int i = 0; i < ROW_PER; ++i) r.ok[i] = r.u[i] != v;
 }
 
-// Sums the entries' weights by community c[i] into the group's table; returns
-// its size in slots.
+// Sums the weights of the entries that count by community c[i] into the
+// group's table and lists the slots in use; returns their number.
 template <class P>
 __device__ __forceinline__ int fill_table(const P& p, const Row& r, const int32_t* c, int32_t row) {
   int size = 2 * P::N;
@@ -438,67 +502,72 @@ __device__ __forceinline__ int fill_table(const P& p, const Row& r, const int32_
     p.tc[j] = -1;
     p.ts[j] = 0.0;
   }
+  p.start_list();
   p.sync();
+  int n = 0;
 #pragma unroll
   for (int i = 0; i < ROW_PER; ++i) {
+    bool taken = false;
+    int h = 0;
     if (r.ok[i]) {
-      int h = (int)__umulhi(pcg_hash((uint32_t)c[i]), (uint32_t)size);
-      while (true) {  // (at most `row` <= 2/3 size communities: a free slot or the community's is found)
+      h = (int)(__umul24(((uint32_t)c[i] * 0x9E3779B1u) >> 16, (uint32_t)size) >> 16);
+      while (true) {  // (at most `row` <= 70% of size communities: a free slot or the community's is found)
         const int32_t cur = __hip_atomic_load(p.tc + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         if (cur == c[i]) break;
         if (cur == -1) {
           const int32_t prev = atomicCAS(p.tc + h, -1, c[i]);
-          if (prev == -1 || prev == c[i]) break;
+          taken = prev == -1;
+          if (taken || prev == c[i]) break;
         }
         h = h + 1 == size ? 0 : h + 1;
       }
       unsafeAtomicAdd(p.ts + h, (double)r.w[i]);
     }
+    n = p.append(taken, h, n);
   }
   p.sync();
-  return size;
+  return p.listed(n);
 }
 
-// Weight to community c in the table (every thread probes alike).
-template <class P>
-__device__ __forceinline__ float table_weight(const P& p, int size, int32_t c) {
-  int h = (int)__umulhi(pcg_hash((uint32_t)c), (uint32_t)size);
-  while (true) {
-    const int32_t cur = p.tc[h];
-    if (cur == c) return (float)p.ts[h];
-    if (cur == -1) return 0.0f;
-    h = h + 1 == size ? 0 : h + 1;
+// Calls f(community, weight to it, its total) for the candidates: the entries
+// that count where no community has two (FIRST), else the n listed slots.  All
+// totals are loaded before any is used.
+template <class P, bool FIRST, class F>
+__device__ __forceinline__ void each_candidate(const P& p, const Row& r, int n, const double* __restrict__ sigma,
+                                               F f) {
+  int32_t c[ROW_PER];
+  float w[ROW_PER];
+  double total[ROW_PER];
+  bool ok[ROW_PER];
+#pragma unroll
+  for (int i = 0; i < ROW_PER; ++i) {
+    if constexpr (FIRST) {
+      ok[i] = r.ok[i];
+      c[i] = r.u[i];
+      w[i] = r.w[i];
+    } else {
+      const int j = p.tid() + P::N * i;
+      ok[i] = j < n;
+      if (ok[i]) {
+        const int h = p.list[j];
+        c[i] = p.tc[h];
+        w[i] = (float)p.ts[h];
+      }
+    }
+    if (ok[i]) total[i] = sigma[c[i]];
+  }
+#pragma unroll
+  for (int i = 0; i < ROW_PER; ++i) {
+    if (ok[i]) f(c[i], w[i], total[i]);
   }
 }
 
-// Calls f(community, weight to it, its total) for every candidate other than
-// `old` that want() admits; all totals are loaded before any is used.
-template <class P, bool FIRST, class Want, class F>
-__device__ __forceinline__ void each_candidate(const P& p, const Row& r, const double* first_total, int size,
-                                               const double* __restrict__ sigma, int32_t old, Want want, F f) {
-  if constexpr (FIRST) {
-#pragma unroll
-    for (int i = 0; i < ROW_PER; ++i) {
-      if (r.ok[i] && want(r.u[i])) f(r.u[i], r.w[i], first_total[i]);
-    }
-  } else {
-    constexpr int PER = P::SLOTS / P::N;
-    int32_t cs[PER];
-    double sg[PER];
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-      const int j = p.tid() + P::N * k;
-      const int32_t c = j < size ? p.tc[j] : -1;
-      cs[k] = c >= 0 && c != old && want(c) ? c : -1;
-    }
-#pragma unroll
-    for (int k = 0; k < PER; ++k) sg[k] = cs[k] >= 0 ? sigma[cs[k]] : 0.0;
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-      if (cs[k] >= 0) f(cs[k], (float)p.ts[p.tid() + P::N * k], sg[k]);
-    }
-  }
-}
+// What a level's sweeps read of a vertex's graph: 1 / m and 1 / (2 m^2).
+struct LevelConst {
+  const double2* scale;
+  const uint32_t* salt;
+  Divisor graph_of;
+};
 
 // What a sweep reads and writes.
 struct MoveSweep {
@@ -511,6 +580,7 @@ struct MoveSweep {
   int32_t sweep;
   float resolution;
   uint32_t seed;
+  LevelConst lc;
 };
 
 __device__ inline void finish_move(const MoveSweep& s, int32_t v, int32_t old, int32_t choice, double kv) {
@@ -520,52 +590,73 @@ __device__ inline void finish_move(const MoveSweep& s, int32_t v, int32_t old, i
   if (choice != old) mark_moved(s.ctl + CTL_LM + (s.sweep & (RING - 1)));
 }
 
+// What a sweep reads of vertex v before its row: loads that depend on v alone,
+// issued together.
+struct Vertex {
+  int32_t v, a, b, g;
+  double kv, tm;
+  double2 scale;
+  uint32_t salt;
+};
+__device__ __forceinline__ Vertex load_vertex(const Graph& gr, const LevelConst& lc, int32_t v) {
+  Vertex x;
+  x.v = v;
+  x.g = lc.graph_of.of(v);
+  x.a = load_now(gr.beg + v);
+  x.b = load_now(gr.end + v);
+  x.kv = load_now(gr.k_v + v);
+  x.tm = load_now(gr.two_m + x.g);
+  x.scale.x = load_now(&lc.scale[x.g].x);
+  x.scale.y = load_now(&lc.scale[x.g].y);
+  x.salt = load_now(lc.salt + v);
+  return x;
+}
+
 template <class P, bool FIRST>
 __device__ __forceinline__ void move_vertex(const P& p, const Graph& gr, const MoveSweep& s, const MoveState& st,
-                                            int32_t v, int32_t a, int32_t b) {
-  const int32_t old = FIRST ? v : s.lin[v];
-  const double kv = gr.k_v[v];
-  const int32_t g = v / gr.S;
-  const double tm = gr.two_m[g];
+                                            const Vertex& x, int32_t old) {
   int32_t choice = old;
-  if (!st.done && a != b && tm > 0.0) {
+  if (!st.done && x.a != x.b && x.tm > 0.0) {
     Row r;
-    load_row(p, gr, v, a, b, r);
-    const double sig_old_excl = s.sigma[old] - kv;
-    double total[ROW_PER];
+    load_row(p, gr, x.v, x.a, x.b, r);
+    const double sig_old_excl = load_now(s.sigma + old) - x.kv;
     float k_old = 0.0f;
-    int size = 0;
+    int n = 0;
     if constexpr (FIRST) {
 #pragma unroll
-      for (int i = 0; i < ROW_PER; ++i) total[i] = s.sigma[r.u[i]];
+      for (int i = 0; i < ROW_PER; ++i) r.ok[i] = r.ok[i] && (r.u[i] > old ? 1 : 0) == st.up;
     } else {
       int32_t c[ROW_PER];
 #pragma unroll
-      for (int i = 0; i < ROW_PER; ++i) c[i] = s.lin[r.u[i]];
-      size = fill_table(p, r, c, b - a);
-      k_old = table_weight(p, size, old);
+      for (int i = 0; i < ROW_PER; ++i) {
+        c[i] = old;
+        if (r.ok[i]) c[i] = s.lin[r.u[i]];
+      }
+      double own = 0.0;
+#pragma unroll
+      for (int i = 0; i < ROW_PER; ++i) {
+        own += r.ok[i] && c[i] == old ? (double)r.w[i] : 0.0;
+        r.ok[i] = c[i] != old && (c[i] > old ? 1 : 0) == st.up;  // the others are no candidates
+      }
+      k_old = (float)p.sum(own);
+      n = fill_table(p, r, c, x.b - x.a);
     }
-    const double m_g = 0.5 * tm;
-    const double inv_m = 1.0 / m_g;
-    const double inv_2m2 = 1.0 / (2.0 * m_g * m_g);
-    const float jitter = (rand_uniform((uint32_t)g, (uint32_t)v, 0u, (uint32_t)s.sweep, s.seed) - 0.5f) * 1e-9f;
+    const double gain = (double)s.resolution * x.kv;
+    const float jitter = (rand_uniform(x.salt, 0u, (uint32_t)s.sweep, s.seed) - 0.5f) * 1e-9f;
     uint64_t mine = 0;
     int32_t mine_c = old;
-    each_candidate<P, FIRST>(
-        p, r, total, size, s.sigma, old, [&](int32_t c) { return (c > old ? 1 : 0) == st.up; },
-        [&](int32_t c, float kn, double sg) {
-          const double dq = ((double)kn - (double)k_old) * inv_m
-                            + (double)s.resolution * kv * (sig_old_excl - sg) * inv_2m2;
-          const uint64_t key = pack((float)dq + jitter, cand_pref(c));
-          if (key > mine) {
-            mine = key;
-            mine_c = c;
-          }
-        });
+    each_candidate<P, FIRST>(p, r, n, s.sigma, [&](int32_t c, float kn, double sg) {
+      const double dq = ((double)kn - (double)k_old) * x.scale.x + gain * (sig_old_excl - sg) * x.scale.y;
+      const uint64_t key = pack((float)dq + jitter, cand_pref(c));
+      if (key > mine) {
+        mine = key;
+        mine_c = c;
+      }
+    });
     const uint64_t best = p.max(mine);
     if (best > pack(0.0f, STAY_PREF)) choice = p.of(best, mine, mine_c);
   }
-  if (p.tid() == 0) finish_move(s, v, old, choice, kv);
+  if (p.tid() == 0) finish_move(s, x.v, old, choice, x.kv);
 }
 
 // Block b of n of a vertex range: each XCD (blocks run on the eight in turn)
@@ -579,27 +670,25 @@ template <bool FIRST>
 __global__ __launch_bounds__(HUB_THREADS, 8) void local_moving_kernel(Graph gr, MoveSweep s,
                                                                       const int32_t* __restrict__ hubs,
                                                                       const int32_t* __restrict__ hub_count) {
-  __shared__ int32_t tab_c[FIRST ? 1 : HUB_SLOTS];
-  __shared__ double tab_s[FIRST ? 1 : HUB_SLOTS];
-  __shared__ WorkgroupShared sh;
+  __shared__ SweepShared sh;  // (FIRST leaves the table out of use; its occupancy is full all the same)
   const MoveState st = move_state(s.ctl, s.sweep);
   if (blockIdx.x < HUB_BLOCKS) {
     const int32_t n = *hub_count;
-    const Workgroup p{tab_c, tab_s, &sh};
+    const Workgroup p(sh);
     for (int32_t i = blockIdx.x; i < n; i += HUB_BLOCKS) {
-      const int32_t v = hubs[i];
-      move_vertex<Workgroup, FIRST>(p, gr, s, st, v, gr.beg[v], gr.end[v]);
+      const Vertex x = load_vertex(gr, s.lc, hubs[i]);
+      move_vertex<Workgroup, FIRST>(p, gr, s, st, x, FIRST ? x.v : s.lin[x.v]);
       __syncthreads();  // the next vertex takes the table
     }
     return;
   }
-  const int group = threadIdx.x >> 5;
-  const HalfWave p{tab_c + (FIRST ? 0 : group * SMALL_SLOTS), tab_s + (FIRST ? 0 : group * SMALL_SLOTS)};
-  const int32_t v = xcd_block(blockIdx.x - HUB_BLOCKS, gridDim.x - HUB_BLOCKS) * GROUPS + group;
+  const HalfWave p(sh);
+  const int32_t v = xcd_block(blockIdx.x - HUB_BLOCKS, gridDim.x - HUB_BLOCKS) * GROUPS + (threadIdx.x >> 5);
   if (v >= gr.V) return;
-  const int32_t a = gr.beg[v], b = gr.end[v];
-  if (b - a > SMALL_ROW) return;
-  move_vertex<HalfWave, FIRST>(p, gr, s, st, v, a, b);
+  const Vertex x = load_vertex(gr, s.lc, v);
+  const int32_t old = FIRST ? v : load_now(s.lin + v);
+  if (x.b - x.a > SMALL_ROW) return;
+  move_vertex<HalfWave, FIRST>(p, gr, s, st, x, old);
 }
 
 // Refinement: a vertex proposes a community inside its parent community (x of
@@ -623,82 +712,88 @@ struct RefineSweep {
   float inv_theta;
   int boltzmann;
   uint32_t seed;
+  LevelConst lc;
 };
 
+template <bool FIRST>
+__device__ __forceinline__ int2 refine_self(const RefineSweep& s, int32_t v) {
+  if constexpr (FIRST) return int2{load_now(s.parent + v), v};
+  return load_now(s.lin + v);
+}
+
+// e < x / tm, without the division (some 35 issue slots) unless they are close.
+__device__ __forceinline__ bool below_quotient(double e, double x, double tm) {
+  const double lhs = e * tm, slack = fabs(x) * 1e-12;
+  if (lhs > x + slack) return false;
+  if (lhs < x - slack) return true;
+  return e < x / tm;
+}
+
 template <class P, bool FIRST>
-__device__ __forceinline__ void propose_vertex(const P& p, const Graph& gr, const RefineSweep& s, int32_t v, int32_t a,
-                                               int32_t b) {
-  int2 self;
-  if constexpr (FIRST) self = int2{s.parent[v], v};
-  else self = s.lin[v];
+__device__ __forceinline__ void propose_vertex(const P& p, const Graph& gr, const RefineSweep& s, const Vertex& x,
+                                               int2 self) {
   const int32_t pv = self.x, old = self.y;
-  const double kv = gr.k_v[v];
-  const int32_t g = v / gr.S;
-  const double tm = gr.two_m[g];
   int32_t choice = old;
-  if (a != b && tm > 0.0) {
+  if (x.a != x.b && x.tm > 0.0) {
     Row r;
-    load_row(p, gr, v, a, b, r);
-    double vol_minus = s.parent_sigma[pv] - kv;
+    load_row(p, gr, x.v, x.a, x.b, r);
+    double vol_minus = load_now(s.parent_sigma + pv) - x.kv;
     if (vol_minus < 0.0) vol_minus = 0.0;
-    const double bound = (double)s.resolution * kv * vol_minus / tm;
-    const double sig_old_excl = s.sigma[old] - kv;
+    const double sig_old_excl = load_now(s.sigma + old) - x.kv;
     int32_t c[ROW_PER];
-    double total[ROW_PER];
-    double e_sum = 0.0;
+    double own = 0.0, e_sum = 0.0;
 #pragma unroll
     for (int i = 0; i < ROW_PER; ++i) {
-      if constexpr (FIRST) {
-        total[i] = s.sigma[r.u[i]];
-        r.ok[i] = r.ok[i] && s.parent[r.u[i]] == pv;
-      } else {
-        const int2 q = s.lin[r.u[i]];
-        r.ok[i] = r.ok[i] && q.x == pv;
-        c[i] = q.y;
+      int2 q{-1, old};
+      if (r.ok[i]) {
+        if constexpr (FIRST) q = int2{s.parent[r.u[i]], r.u[i]};
+        else q = s.lin[r.u[i]];
       }
+      r.ok[i] = q.x == pv;  // (parents are vertices, never -1)
+      c[i] = q.y;
     }
 #pragma unroll
     for (int i = 0; i < ROW_PER; ++i) e_sum += r.ok[i] ? (double)r.w[i] : 0.0;
     e_sum = p.sum(e_sum);
-    if (!((double)(float)e_sum < bound)) {  // {v} is well connected to its parent community
+    if (!below_quotient((double)(float)e_sum, (double)s.resolution * x.kv * vol_minus, x.tm)) {
+      // {v} is well connected to its parent community
       float k_old = 0.0f;
-      int size = 0;
+      int n = 0;
       if constexpr (!FIRST) {
-        size = fill_table(p, r, c, b - a);
-        k_old = table_weight(p, size, old);
+#pragma unroll
+        for (int i = 0; i < ROW_PER; ++i) {
+          own += r.ok[i] && c[i] == old ? (double)r.w[i] : 0.0;
+          r.ok[i] = r.ok[i] && c[i] != old;
+        }
+        k_old = (float)p.sum(own);
+        n = fill_table(p, r, c, x.b - x.a);
       }
-      const double m_g = 0.5 * tm;
-      const double inv_m = 1.0 / m_g;
-      const double inv_2m2 = 1.0 / (2.0 * m_g * m_g);
+      const double gain = (double)s.resolution * x.kv;
       uint64_t mine = 0;
       int32_t mine_c = old;
-      each_candidate<P, FIRST>(
-          p, r, total, size, s.sigma, old, [](int32_t) { return true; },
-          [&](int32_t cand, float kn, double sg) {
-            const double dq = ((double)kn - (double)k_old) * inv_m
-                              + (double)s.resolution * kv * (sig_old_excl - sg) * inv_2m2;
-            if (dq < 0.0) return;
-            const float score = s.boltzmann
-                ? (float)(dq * (double)s.inv_theta)
-                      + gumbel(rand_uniform_pair((uint32_t)g, (uint32_t)v, (uint32_t)cand, 1u, (uint32_t)s.sweep,
-                                                 s.seed))
-                : (float)dq;
-            const uint64_t key = pack(score, cand_pref(cand));
-            if (key > mine) {
-              mine = key;
-              mine_c = cand;
-            }
-          });
+      each_candidate<P, FIRST>(p, r, n, s.sigma, [&](int32_t cand, float kn, double sg) {
+        const double dq = ((double)kn - (double)k_old) * x.scale.x + gain * (sig_old_excl - sg) * x.scale.y;
+        if (dq < 0.0) return;
+        const float score = s.boltzmann
+            ? (float)(dq * (double)s.inv_theta)
+                  + gumbel(rand_uniform_pair(x.salt, (uint32_t)cand, 1u, (uint32_t)s.sweep, s.seed))
+            : (float)dq;
+        const uint64_t key = pack(score, cand_pref(cand));
+        if (key > mine) {
+          mine = key;
+          mine_c = cand;
+        }
+      });
       const uint64_t best = p.max(mine);
       const float stay = s.boltzmann
-          ? gumbel(rand_uniform_pair((uint32_t)g, (uint32_t)v, (uint32_t)old, 1u, (uint32_t)s.sweep, s.seed))
+          ? gumbel(rand_uniform_pair(x.salt, (uint32_t)old, 1u, (uint32_t)s.sweep, s.seed))
           : 0.0f;
       if (best > pack(stay, STAY_PREF)) choice = p.of(best, mine, mine_c);
     }
   }
   if (p.tid() == 0) {
-    s.prop[v] = choice;
-    s.mover[v] = choice != old ? pv : -1;
+    s.prop[x.v] = choice;
+    s.mover[x.v] = choice != old ? pv : -1;
   }
 }
 
@@ -706,67 +801,88 @@ template <bool FIRST>
 __global__ __launch_bounds__(HUB_THREADS, 8) void refine_propose_kernel(Graph gr, RefineSweep s,
                                                                         const int32_t* __restrict__ hubs,
                                                                         const int32_t* __restrict__ hub_count) {
-  __shared__ int32_t tab_c[FIRST ? 1 : HUB_SLOTS];
-  __shared__ double tab_s[FIRST ? 1 : HUB_SLOTS];
-  __shared__ WorkgroupShared sh;
+  __shared__ SweepShared sh;
   if (refine_done(s.ctl, s.sweep)) return;
   if (blockIdx.x < HUB_BLOCKS) {
     const int32_t n = *hub_count;
-    const Workgroup p{tab_c, tab_s, &sh};
+    const Workgroup p(sh);
     for (int32_t i = blockIdx.x; i < n; i += HUB_BLOCKS) {
-      const int32_t v = hubs[i];
-      propose_vertex<Workgroup, FIRST>(p, gr, s, v, gr.beg[v], gr.end[v]);
+      const Vertex x = load_vertex(gr, s.lc, hubs[i]);
+      propose_vertex<Workgroup, FIRST>(p, gr, s, x, refine_self<FIRST>(s, x.v));
       __syncthreads();
     }
     return;
   }
-  const int group = threadIdx.x >> 5;
-  const HalfWave p{tab_c + (FIRST ? 0 : group * SMALL_SLOTS), tab_s + (FIRST ? 0 : group * SMALL_SLOTS)};
-  const int32_t v = xcd_block(blockIdx.x - HUB_BLOCKS, gridDim.x - HUB_BLOCKS) * GROUPS + group;
+  const HalfWave p(sh);
+  const int32_t v = xcd_block(blockIdx.x - HUB_BLOCKS, gridDim.x - HUB_BLOCKS) * GROUPS + (threadIdx.x >> 5);
   if (v >= gr.V) return;
-  const int32_t a = gr.beg[v], b = gr.end[v];
-  if (b - a > SMALL_ROW) return;
-  propose_vertex<HalfWave, FIRST>(p, gr, s, v, a, b);
+  const Vertex x = load_vertex(gr, s.lc, v);
+  const int2 self = refine_self<FIRST>(s, v);
+  if (x.b - x.a > SMALL_ROW) return;
+  propose_vertex<HalfWave, FIRST>(p, gr, s, x, self);
 }
 
 // A mover commits unless a moving neighbour in its parent community outranks
 // it on (rank, id) (refinement.cu:263-300); the rank is the neighbour's hash,
 // computed where it is needed.
-template <class P, bool FIRST>
-__device__ __forceinline__ void commit_vertex(const P& p, const Graph& gr, const RefineSweep& s, bool done, int32_t v,
-                                              int32_t a, int32_t b) {
+struct Commit {
+  int32_t v, a, b, to, wants;
   int2 self;
-  if constexpr (FIRST) self = int2{s.parent[v], v};
-  else self = s.lin[v];
-  const double kv = gr.k_v[v];
-  const int32_t wants = done ? -1 : s.mover[v];
-  const int32_t to = done ? self.y : s.prop[v];
+  double kv;
+};
+template <bool FIRST>
+__device__ __forceinline__ Commit load_commit(const Graph& gr, const RefineSweep& s, int32_t v) {
+  Commit x;
+  x.v = v;
+  x.a = load_now(gr.beg + v);
+  x.b = load_now(gr.end + v);
+  x.wants = load_now(s.mover + v);
+  x.to = load_now(s.prop + v);
+  x.self = refine_self<FIRST>(s, v);
+  x.kv = load_now(gr.k_v + v);
+  return x;
+}
+
+template <class P>
+__device__ __forceinline__ void commit_vertex(const P& p, const Graph& gr, const RefineSweep& s, bool done,
+                                              const Commit& x) {
+  const bool wants = !done && x.wants >= 0;  // (after the end the proposals are an earlier sweep's)
   bool lost = false;
-  if (wants >= 0) {
-    const uint32_t rv = mix4((uint32_t)(v / gr.S), (uint32_t)v, (1u << 16) | (uint32_t)s.sweep, s.seed);
-    for (int32_t e0 = a; e0 < b; e0 += ROW_PER * P::N) {
+  if (wants) {
+    const int32_t g = s.lc.graph_of.of(x.v);
+    const uint32_t key = (1u << 16) | (uint32_t)s.sweep, gh = pcg_hash((uint32_t)g);
+    const uint32_t rv = mix_salt(pcg_hash(gh ^ (uint32_t)x.v), key, s.seed);
+    for (int32_t e0 = x.a; e0 < x.b; e0 += ROW_PER * P::N) {
       int32_t u[ROW_PER], m[ROW_PER];
 #pragma unroll
-      for (int i = 0; i < ROW_PER; ++i) u[i] = gr.col[min(e0 + i * P::N + p.tid(), b - 1)];
-#pragma unroll
-      for (int i = 0; i < ROW_PER; ++i) m[i] = s.mover[u[i]];
+      for (int i = 0; i < ROW_PER; ++i) {
+        const int32_t e = e0 + i * P::N + p.tid();
+        u[i] = x.v;
+        if (e < x.b) u[i] = gr.col[e];
+      }
 #pragma unroll
       for (int i = 0; i < ROW_PER; ++i) {
-        if (u[i] != v && m[i] == self.x) {
-          const uint32_t ru = mix4((uint32_t)(u[i] / gr.S), (uint32_t)u[i], (1u << 16) | (uint32_t)s.sweep, s.seed);
-          lost = lost || ru > rv || (ru == rv && u[i] > v);
+        m[i] = -1;
+        if (u[i] != x.v) m[i] = s.mover[u[i]];
+      }
+#pragma unroll
+      for (int i = 0; i < ROW_PER; ++i) {
+        if (m[i] == x.self.x) {
+          const int32_t gu = s.lc.graph_of.of(u[i]);
+          const uint32_t ru = mix_salt(pcg_hash((gu == g ? gh : pcg_hash((uint32_t)gu)) ^ (uint32_t)u[i]), key, s.seed);
+          lost = lost || ru > rv || (ru == rv && u[i] > x.v);
         }
       }
     }
     lost = p.any(lost);
   }
   if (p.tid() == 0) {
-    const int32_t label = wants >= 0 && !lost ? to : self.y;
-    s.lout[v] = int2{self.x, label};
-    s.labels[v] = label;
-    s.clear[v] = 0.0;
-    if (kv != 0.0) unsafeAtomicAdd(s.next + label, kv);
-    if (label != self.y) mark_moved(s.ctl + CTL_REFINE + (s.sweep & (RING - 1)));
+    const int32_t label = wants && !lost ? x.to : x.self.y;
+    s.lout[x.v] = int2{x.self.x, label};
+    s.labels[x.v] = label;
+    s.clear[x.v] = 0.0;
+    if (x.kv != 0.0) unsafeAtomicAdd(s.next + label, x.kv);
+    if (label != x.self.y) mark_moved(s.ctl + CTL_REFINE + (s.sweep & (RING - 1)));
   }
 }
 
@@ -776,23 +892,21 @@ __global__ __launch_bounds__(HUB_THREADS, 8) void refine_commit_kernel(Graph gr,
                                                                        const int32_t* __restrict__ hub_count,
                                                                        const int32_t* __restrict__ giants,
                                                                        const int32_t* __restrict__ giant_count) {
-  __shared__ WorkgroupShared sh;
+  __shared__ SweepShared sh;  // (the table stays out of use)
   const bool done = refine_done(s.ctl, s.sweep);
   if (blockIdx.x < HUB_BLOCKS) {
     const int32_t n = *hub_count, all = n + *giant_count;
-    const Workgroup p{nullptr, nullptr, &sh};
-    for (int32_t i = blockIdx.x; i < all; i += HUB_BLOCKS) {
-      const int32_t v = i < n ? hubs[i] : giants[i - n];
-      commit_vertex<Workgroup, FIRST>(p, gr, s, done, v, gr.beg[v], gr.end[v]);
-    }
+    const Workgroup p(sh);
+    for (int32_t i = blockIdx.x; i < all; i += HUB_BLOCKS)
+      commit_vertex(p, gr, s, done, load_commit<FIRST>(gr, s, i < n ? hubs[i] : giants[i - n]));
     return;
   }
-  const HalfWave p{nullptr, nullptr};
+  const HalfWave p(sh);
   const int32_t v = xcd_block(blockIdx.x - HUB_BLOCKS, gridDim.x - HUB_BLOCKS) * GROUPS + (threadIdx.x >> 5);
   if (v >= gr.V) return;
-  const int32_t a = gr.beg[v], b = gr.end[v];
-  if (b - a > SMALL_ROW) return;
-  commit_vertex<HalfWave, FIRST>(p, gr, s, done, v, a, b);
+  const Commit x = load_commit<FIRST>(gr, s, v);
+  if (x.b - x.a > SMALL_ROW) return;
+  commit_vertex(p, gr, s, done, x);
 }
 
 // Test hook: raises the overflow word as a broken local-moving table would.
@@ -982,7 +1096,7 @@ __global__ __launch_bounds__(GIANT_THREADS) void local_moving_giant_kernel(Graph
     const double inv_m = 1.0 / m_g;
     const double inv_2m2 = 1.0 / (2.0 * m_g * m_g);
     const double sig_old_excl = s.sigma[old] - kv;
-    const float jitter = (rand_uniform((uint32_t)g, (uint32_t)v, 0u, (uint32_t)s.sweep, s.seed) - 0.5f) * 1e-9f;
+    const float jitter = (rand_uniform(s.lc.salt[v], 0u, (uint32_t)s.sweep, s.seed) - 0.5f) * 1e-9f;
     uint64_t mine = 0;
     int32_t mine_c = old;
     for (int j = threadIdx.x; j < GIANT_SLOTS; j += GIANT_THREADS) {
@@ -1067,7 +1181,7 @@ __global__ __launch_bounds__(GIANT_THREADS) void refine_propose_giant_kernel(Gra
       if (dq < 0.0) continue;
       const float score = s.boltzmann
           ? (float)(dq * (double)s.inv_theta)
-                + gumbel(rand_uniform_pair((uint32_t)g, (uint32_t)v, (uint32_t)c, 1u, (uint32_t)s.sweep, s.seed))
+                + gumbel(rand_uniform_pair(s.lc.salt[v], (uint32_t)c, 1u, (uint32_t)s.sweep, s.seed))
           : (float)dq;
       const uint64_t p = pack(score, cand_pref(c));
       if (p > mine) {
@@ -1076,7 +1190,7 @@ __global__ __launch_bounds__(GIANT_THREADS) void refine_propose_giant_kernel(Gra
       }
     }
     const float stay = s.boltzmann
-        ? gumbel(rand_uniform_pair((uint32_t)g, (uint32_t)v, (uint32_t)old, 1u, (uint32_t)s.sweep, s.seed))
+        ? gumbel(rand_uniform_pair(s.lc.salt[v], (uint32_t)old, 1u, (uint32_t)s.sweep, s.seed))
         : 0.0f;
     const int32_t choice = giant_pick(mine, mine_c, pack(stay, STAY_PREF), old, sh);
     propose(choice);
@@ -1726,14 +1840,24 @@ __global__ __launch_bounds__(AGG_DENSE_THREADS) void agg_dense_kernel(Contract c
 
 // ----------------------------------------------------------------- the run's own small kernels
 // Start of a level: identity labels, the first sweep's cleared totals, cleared
-// lists and control words (the overflow word stays raised after the first level).
+// lists and control words (the overflow word stays raised after the first
+// level), and what the sweeps would compute of every vertex or graph again and again.
 __global__ __launch_bounds__(ETHREADS) void level_init_kernel(int32_t V, int32_t* __restrict__ labels,
                                                               int32_t* __restrict__ moves, double* __restrict__ total,
                                                               int32_t* __restrict__ ctl,
                                                               int32_t* __restrict__ hub_count,
-                                                              int32_t* __restrict__ giant_count, int first) {
+                                                              int32_t* __restrict__ giant_count,
+                                                              const double* __restrict__ two_m,
+                                                              double2* __restrict__ scale,
+                                                              uint32_t* __restrict__ salt, Divisor graph_of,
+                                                              int32_t G, int first) {
   const int32_t v = blockIdx.x * ETHREADS + threadIdx.x;
+  if (v < G) {
+    const double m = 0.5 * two_m[v];  // (a graph without weight is not asked for these)
+    scale[v] = double2{1.0 / m, 1.0 / (2.0 * m * m)};
+  }
   if (v < V) {
+    salt[v] = salt_of((uint32_t)graph_of.of(v), (uint32_t)v);
     labels[v] = v;
     moves[v] = v;
     total[v] = 0.0;
@@ -1857,7 +1981,7 @@ int launch_check() {
 
 struct LeidenLayout {
   size_t keys_a, keys_b, vals_a, vals_b, temp, temp_bytes, row_ptr, col, k_v, two_m, totals[4], lab, moves[2], pairs[2],
-      prop, mover, ctl, hubs, hub_count, giants, giant_count, total;
+      prop, mover, ctl, hubs, hub_count, giants, giant_count, scale, salt, total;
 };
 
 LeidenLayout leiden_layout(int64_t E, int32_t G, int32_t S) {
@@ -1892,6 +2016,8 @@ LeidenLayout leiden_layout(int64_t E, int32_t G, int32_t S) {
   }
   L.prop = take(V * 4);
   L.mover = take(V * 4);
+  L.salt = take(V * 4);
+  L.scale = take(G * 16);
   L.ctl = take(CTL_WORDS * 4);
   L.hubs = take(V * 4);
   L.hub_count = take(4);
@@ -1981,6 +2107,8 @@ struct SweepBuffers {
   int32_t* hub_count;
   int32_t* giants;
   int32_t* giant_count;
+  double2* scale;
+  uint32_t* salt;
 };
 
 // Queues a level: cleared state, lists of long rows, local moving and
@@ -1988,8 +2116,11 @@ struct SweepBuffers {
 void run_sweeps(const Graph& gr, const SweepBuffers& b, float resolution, float theta, int32_t max_inner_iter,
                 int32_t seed, int32_t use_boltzmann, bool first_level, hipStream_t st) {
   const int32_t V = gr.V;
+  const Divisor graph_of(gr.S);
+  const LevelConst lc{b.scale, b.salt, graph_of};
   level_init_kernel<<<blocks(V, ETHREADS), ETHREADS, 0, st>>>(V, b.labels, b.moves[0], b.total[0], b.ctl, b.hub_count,
-                                                              b.giant_count, first_level);
+                                                              b.giant_count, gr.two_m, b.scale, b.salt, graph_of,
+                                                              V / gr.S, first_level);
   hub_list_kernel<<<blocks(V, LIST_THREADS), LIST_THREADS, 0, st>>>(gr.beg, gr.end, V, b.hubs, b.hub_count, b.giants,
                                                                    b.giant_count);
   const unsigned grid = HUB_BLOCKS + blocks(V, GROUPS);
@@ -1999,7 +2130,7 @@ void run_sweeps(const Graph& gr, const SweepBuffers& b, float resolution, float 
   for (int32_t i = 0; i < max_inner_iter; ++i) {
     if (i > 0 && i % RING == 0) fold_kernel<<<1, 64, 0, st>>>(b.ctl, 1, 0);
     const MoveSweep s{i == 0 ? gr.k_v : t[(i - 1) % 3], t[i % 3], t[(i + 1) % 3], b.moves[i & 1], b.moves[(i & 1) ^ 1],
-                      b.ctl, i, resolution, (uint32_t)seed};
+                      b.ctl, i, resolution, (uint32_t)seed, lc};
     if (i == 0 && gr.unique) {
       local_moving_kernel<true><<<grid, HUB_THREADS, 0, st>>>(gr, s, b.hubs, b.hub_count);
       if (giants) local_moving_giant_kernel<true><<<GIANT_BLOCKS, GIANT_THREADS, 0, st>>>(gr, s, b.giants, b.giant_count);
@@ -2022,7 +2153,7 @@ void run_sweeps(const Graph& gr, const SweepBuffers& b, float resolution, float 
     if (i > 0 && i % RING == 0) fold_kernel<<<1, 64, 0, st>>>(b.ctl, 0, 0);
     const RefineSweep s{i == 0 ? gr.k_v : r[(i - 1) % 3], parent_total, r[i % 3], r[(i + 1) % 3], parent,
                         b.pairs[i & 1], b.pairs[(i & 1) ^ 1], b.labels, b.prop, b.mover, b.ctl, i, resolution,
-                        inv_theta, use_boltzmann ? 1 : 0, (uint32_t)seed};
+                        inv_theta, use_boltzmann ? 1 : 0, (uint32_t)seed, lc};
     if (i == 0 && gr.unique) {
       refine_propose_kernel<true><<<grid, HUB_THREADS, 0, st>>>(gr, s, b.hubs, b.hub_count);
       if (giants)
@@ -2103,7 +2234,8 @@ extern "C" int ckv_batched_leiden(const int32_t* edge_src, const int32_t* edge_d
                          {(int32_t*)(ws + L.moves[0]), (int32_t*)(ws + L.moves[1])},
                          {(int2*)(ws + L.pairs[0]), (int2*)(ws + L.pairs[1])},
                          (int32_t*)(ws + L.prop), (int32_t*)(ws + L.mover), ctl, (int32_t*)(ws + L.hubs),
-                         (int32_t*)(ws + L.hub_count), (int32_t*)(ws + L.giants), (int32_t*)(ws + L.giant_count)};
+                         (int32_t*)(ws + L.hub_count), (int32_t*)(ws + L.giants), (int32_t*)(ws + L.giant_count),
+                         (double2*)(ws + L.scale), (uint32_t*)(ws + L.salt)};
   run_sweeps(gr, buf, resolution, theta, max_inner_iter, seed, use_boltzmann, true, st);
   sigma_zero_kernel<<<egrid, ETHREADS, 0, st>>>(sigma, V);
   sigma_scatter_kernel<<<egrid, ETHREADS, 0, st>>>(lab, k_v, V, sigma);
@@ -2215,7 +2347,7 @@ namespace {
 
 struct RunLayout {
   size_t row_ptr, col0, wt0, col[2], wt[2], beg[2], end[2], k[2], two_m, two_m0, totals[4], lab, moves[2], pairs[2], prop,
-      mover, ctl, hubs, giants, counts, flags, scan, dense, hist, first, members, dense_list, lists, words, temp,
+      mover, salt, scale, ctl, hubs, giants, counts, flags, scan, dense, hist, first, members, dense_list, lists, words, temp,
       temp_bytes, sort, total;
 };
 
@@ -2246,6 +2378,8 @@ RunLayout run_layout(int64_t E, int32_t G, int32_t S) {
   L.lab = take(V * 4);
   L.prop = take(V * 4);
   L.mover = take(V * 4);
+  L.salt = take(V * 4);
+  L.scale = take(G * 16);
   L.ctl = take(CTL_WORDS * 4);
   L.hubs = take(V * 4);
   L.giants = take(V * 4);
@@ -2374,7 +2508,8 @@ extern "C" int ckv_leiden_run(const int32_t* edge_src, const int32_t* edge_dst, 
                            i32(L.lab),
                            {i32(L.moves[0]), i32(L.moves[1])},
                            {(int2*)(ws + L.pairs[0]), (int2*)(ws + L.pairs[1])},
-                           i32(L.prop), i32(L.mover), ctl, i32(L.hubs), hub_count, i32(L.giants), giant_count};
+                           i32(L.prop), i32(L.mover), ctl, i32(L.hubs), hub_count, i32(L.giants), giant_count,
+                           (double2*)(ws + L.scale), (uint32_t*)(ws + L.salt)};
     run_sweeps(gr, buf, resolution, theta, max_inner_iter, seed + level, use_boltzmann, level == 0, st);
     // ranks of the labels in use, per graph
     const int32_t* lab = i32(L.lab);

@@ -27,7 +27,7 @@
 //
 // Launch sequence of ckv_batched_leiden (one stream, no host sync):
 //   mirror_kernel, radix sort, row_ptr_kernel, col_kernel, degree_kernel, graph_sum_kernel (2m)
-//   level_init_kernel, hub_list_kernel
+//   level_init_kernel, row_list_kernel
 //   local moving x max_inner_iter: local_moving_kernel, local_moving_giant_kernel
 //   pair_init_kernel
 //   refinement x max_inner_iter: refine_propose_kernel, refine_propose_giant_kernel, refine_commit_kernel
@@ -40,7 +40,7 @@
 // level's result contracts the CSR row by row in LDS hash tables, where the
 // edge list was relabelled, sorted by 64-bit keys, reduced, and sorted again
 // into a CSR (2.0 ms at 9.7 M edges, 0.35 ms now).  Launch sequence per level:
-//   level_init, hub_list, sweeps as above (giants only where rows can be so long), flag_zero, flag_mark, scan, width
+//   level_init, row_list, sweeps as above (giants only where rows can be so long), flag_zero, flag_mark, scan, width
 //   [the host reads the width], densify_apply, chain_kernel,
 //   agg_zero, agg_hist, scan, agg_fill (members by super-vertex), agg_list,
 //   agg_short (one wave per row), agg_long (workgroup), agg_dense, graph_sum
@@ -63,18 +63,22 @@ constexpr int LTHREADS = 64 * LWAVES;
 constexpr int TABLE_CAP = 1024;  // distinct neighbour communities per vertex
 constexpr int ETHREADS = 256;
 
-// Control words of a level.  A sweep marks its slot of its phase's ring when a
-// vertex moves; the next sweeps read the ring themselves, so no kernel runs
-// between sweeps to advance a state.  Every RING sweeps fold_kernel moves the
-// ring's outcome to the base words.
-constexpr int RING = 64;
+// Control words of a level.  A sweep in which a vertex moves marks its slot of
+// its phase's ring; the next sweeps read the ring themselves, so no kernel runs
+// between sweeps to advance a state.  A slot is a word per XCD, each in a line
+// of its own: with a mark per moved vertex on one word a first sweep of 57,000
+// vertices took 64 us, 31 now.  Every RING sweeps fold_kernel moves the ring's
+// outcome to the base words.
+constexpr int RING = 16;
+constexpr int MARK_STRIDE = 32;              // words from one XCD's mark to the next
+constexpr int SLOT_WORDS = 8 * MARK_STRIDE;  // a sweep's slot
 enum { CTL_OVERFLOW = 0,  // nonzero when a workgroup table overflowed (a broken table bound)
        CTL_STALLS = 1,    // local moving: stalled sweeps before the ring, modulo 2
        CTL_LAST = 2,      // the last sweep before the ring stalled
        CTL_DONE = 3,      // the phase ended before the ring
-       CTL_LM = 4,                  // local moving's ring
-       CTL_REFINE = CTL_LM + RING,  // refinement's ring
-       CTL_WORDS = CTL_REFINE + RING };
+       CTL_LM = MARK_STRIDE,                     // local moving's ring
+       CTL_REFINE = CTL_LM + RING * SLOT_WORDS,  // refinement's ring
+       CTL_WORDS = CTL_REFINE + RING * SLOT_WORDS };
 
 // ----------------------------------------------------------------- hashing (rng.cuh)
 __device__ __host__ inline uint32_t pcg_hash(uint32_t x) {
@@ -125,11 +129,12 @@ __device__ inline uint64_t pack(float score, uint32_t pref) { return ((uint64_t)
 // ----------------------------------------------------------------- wave helpers
 __device__ inline int first_lane(uint64_t m) { return __ffsll((long long)m) - 1; }
 
-// Marks a sweep that moved a vertex (read first, so that later movers do not
-// queue writes to one line).
-__device__ inline void mark_moved(int32_t* word) {
-  if (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
-    __hip_atomic_store(word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// Marks a sweep (its slot of the ring) in which a thread of the wave moved a
+// vertex: once per wave at its end, and only while the XCD's word reads zero.
+__device__ inline void mark_moved(int32_t* slot, bool moved) {
+  int32_t* word = slot + (blockIdx.x & 7) * MARK_STRIDE;
+  if (__ballot(moved) != 0 && lane() == 0 && *word == 0)
+    __hip_atomic_store(word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // Local moving before sweep `sweep` (wave-uniform): done after two stalled
@@ -139,32 +144,51 @@ struct MoveState {
   bool done;
   int up;
 };
-__device__ inline MoveState move_state(const int32_t* __restrict__ ctl, int sweep) {
-  const int n = sweep & (RING - 1);  // sweeps in the ring
-  const int base = ctl[CTL_DONE], parity = ctl[CTL_STALLS], last = ctl[CTL_LAST];
-  const uint64_t below = n == 0 ? 0ull : ~0ull >> (64 - n);
-  const uint64_t stalled = ~__ballot(ctl[CTL_LM + lane()] != 0) & below;
-  const uint64_t twice = stalled & ((stalled << 1) | (last ? 1ull : 0ull));
-  return MoveState{base != 0 || twice != 0, 1 ^ (((int)__popcll(stalled) + parity) & 1)};
+struct RingState {
+  bool done, last;
+  int stalls;
+};
+// The state after the first n <= RING sweeps of a ring; a single stalled sweep
+// ends refinement, two in a row local moving.
+__device__ inline RingState ring_state(const int32_t* __restrict__ ctl, bool lm, int n) {
+  RingState r{ctl[CTL_DONE] != 0, ctl[CTL_LAST] != 0, ctl[CTL_STALLS]};
+  const int32_t* ring = ctl + (lm ? CTL_LM : CTL_REFINE);
+  for (int s0 = 0; s0 < n; s0 += 8) {
+    const int at = s0 * 8 + lane();
+    const uint64_t marks = __ballot(at < 8 * n && ring[at * MARK_STRIDE] != 0);
+    for (int k = s0; k < n && k < s0 + 8; ++k) {
+      const bool stalled = ((marks >> (8 * (k - s0))) & 0xff) == 0;
+      r.done = r.done || (stalled && (!lm || r.last));
+      r.stalls ^= stalled ? 1 : 0;
+      r.last = stalled;
+    }
+  }
+  return r;
 }
-// Refinement ends with the first sweep that moves nothing (later ones mark nothing).
+__device__ inline MoveState move_state(const int32_t* __restrict__ ctl, int sweep) {
+  const RingState r = ring_state(ctl, true, sweep & (RING - 1));
+  return MoveState{r.done, 1 ^ (r.stalls & 1)};
+}
 __device__ inline bool refine_done(const int32_t* __restrict__ ctl, int sweep) {
-  const int n = sweep & (RING - 1);
-  return ctl[CTL_DONE] != 0 || (n > 0 && ctl[CTL_REFINE + n - 1] == 0);
+  return ring_state(ctl, false, sweep & (RING - 1)).done;
+}
+__device__ inline int32_t* mark_slot(int32_t* ctl, bool lm, int sweep) {
+  return ctl + (lm ? CTL_LM : CTL_REFINE) + (sweep & (RING - 1)) * SLOT_WORDS;
 }
 
-// Folds a full ring (RING sweeps of one phase) into the base words; or, with
-// reset, clears the words of the phase that begins.
+// Folds a full ring (RING sweeps of one phase) into the base words; with reset,
+// clears the words of the phase that begins (its ring is clear).
 __global__ void fold_kernel(int32_t* __restrict__ ctl, int lm, int reset) {
-  const uint64_t stalled = ~__ballot(ctl[(lm ? CTL_LM : CTL_REFINE) + lane()] != 0);
+  RingState r{false, false, 0};
+  if (!reset) r = ring_state(ctl, lm != 0, RING);
+  __syncthreads();
   if (lane() == 0) {
-    const uint64_t twice = stalled & ((stalled << 1) | (ctl[CTL_LAST] ? 1ull : 0ull));
-    const bool ended = lm ? twice != 0 : stalled != 0;
-    ctl[CTL_DONE] = reset ? 0 : (ctl[CTL_DONE] != 0 || ended ? 1 : 0);
-    ctl[CTL_STALLS] = reset ? 0 : (ctl[CTL_STALLS] + __popcll(stalled)) & 1;
-    ctl[CTL_LAST] = reset ? 0 : (int32_t)(stalled >> 63);
+    ctl[CTL_DONE] = r.done ? 1 : 0;
+    ctl[CTL_STALLS] = r.stalls & 1;
+    ctl[CTL_LAST] = r.last ? 1 : 0;
   }
-  ctl[(lm ? CTL_LM : CTL_REFINE) + lane()] = 0;
+  if (reset) return;
+  for (int at = lane(); at < 8 * RING; at += 64) ctl[(lm ? CTL_LM : CTL_REFINE) + at * MARK_STRIDE] = 0;
 }
 
 // ----------------------------------------------------------------- CSR build
@@ -300,20 +324,21 @@ __device__ __forceinline__ T load_now(const T* p) {
 }
 
 // Sweeps.  A vertex of at most SMALL_ROW entries (nearly all) is handled by
-// half a wave, a longer one (listed once per level by hub_list_kernel) by a
-// workgroup of HUB_THREADS, both with up to ROW_PER entries per thread held in
-// registers, so that a vertex costs four rounds of loads whatever its row:
-// bounds, degree and label; entries; the neighbours' labels; the community
-// totals.  Rows longer than GIANT_MIN have kernels of their own.
+// half a wave; the longer ones, listed once per level, of up to MID_ROW entries
+// by a wave and up to GIANT_MIN by a workgroup.  All hold up to ROW_PER entries
+// per thread in registers, so that a vertex costs four rounds of loads whatever
+// its row: bounds, degree and label; entries; the neighbours' labels; the
+// community totals.  Rows longer than GIANT_MIN have kernels of their own.
 //
-// What bounds a sweep is the scattered reads of the neighbours' labels and of
-// the community totals.  Over the 24 sweeps a phase takes in the six levels of
-// eight 32k graphs (262,144 vertices, 19.4 M entries at first) a local-moving
-// sweep averages 115 us and a refinement sweep 200 us.  With a wave per vertex
-// that walked its row 64 entries at a time through a 256-slot table, longer
-// rows by one wave each in a launch behind it, and kernels that cleared and
-// refilled sigma and advanced the control words, it was 205 and 305 us (that
-// partition 16.0 -> 11.5 ms; of eight 2k graphs 2.95 -> 2.27 ms).
+// What bounds a sweep is the instructions issued per entry and the latency of
+// those rounds.  Over the 24 sweeps a phase takes in the six levels of eight
+// 32k graphs (262,144 vertices, 19.4 M entries, 29,400 rows of more than 128 at
+// first) a local-moving sweep averages 70 us and a refinement sweep 88 + 46 us
+// (first level: 120 us, 150 + 75 us).  With a wave per vertex that walked its
+// row 64 entries at a time through a 256-slot table, longer rows by one wave
+// each in a launch behind it, and kernels that cleared and refilled sigma and
+// advanced the control words, it was 205 and 305 us.  Rows of 129-256 entries
+// on a workgroup each waited at its barriers: 100 and 118 + 57 us.
 //
 // Sigma, the communities' total degrees, needs no pass of its own: a sweep
 // adds every vertex's degree to its new community in the buffer the next sweep
@@ -322,9 +347,11 @@ __device__ __forceinline__ T load_now(const T* p) {
 // where no row names a neighbour twice every neighbour is a candidate by
 // itself, so no table is built (FIRST).
 constexpr int SMALL_ROW = 128;
+constexpr int MID_ROW = 256;
 constexpr int ROW_PER = 4;
 constexpr int HUB_THREADS = 256;
-constexpr int HUB_BLOCKS = 512;  // a multiple of 8, so the blocks behind them keep their XCD
+constexpr int SWEEP_BLOCKS = 2048;  // eight a compute unit
+constexpr int LONG_BLOCKS = 512;    // a multiple of eight
 constexpr int SMALL_SLOTS = 184, HUB_SLOTS = 1472;  // table load at most 70%
 constexpr int GROUPS = HUB_THREADS / 32;            // half waves per workgroup
 // Both kinds of workgroup use the same LDS (20 KB, eight a compute unit).
@@ -334,39 +361,48 @@ constexpr int GIANT_MIN = TABLE_CAP;  // rows longer than this take a workgroup 
 constexpr int GIANT_SLOTS = 4096;
 constexpr int GIANT_THREADS = 1024;
 constexpr int GIANT_BLOCKS = 512;  // two 65 KB workgroups per CU
-static_assert(SMALL_ROW == 32 * ROW_PER && GIANT_MIN == HUB_THREADS * ROW_PER, "rows fit their threads' registers");
+static_assert(SMALL_ROW == 32 * ROW_PER && MID_ROW == 64 * ROW_PER && GIANT_MIN == HUB_THREADS * ROW_PER, "rows fit their threads' registers");
+
+// The rows longer than SMALL_ROW: mids (a wave each) from the front of `rows`,
+// hubs (a workgroup each) from its back, giants in a list of their own.
+struct RowLists {
+  int32_t* rows;
+  int32_t* giants;
+  int32_t* counts;      // mids, hubs, giants
+  int32_t long_blocks;  // workgroups of a sweep that take mids and hubs
+  int32_t first;        // workgroups before those that take the other rows
+  __device__ int32_t start(int32_t block) const { return block < long_blocks ? block : 0x7fffffff; }
+};
 
 // (Places in the lists are reserved once per workgroup: one atomic per wave and
-// list queues thousands of them on two words.)
+// list queues thousands of them on a few words.)
 constexpr int LIST_THREADS = 1024;
 
-__global__ __launch_bounds__(LIST_THREADS) void hub_list_kernel(const int32_t* __restrict__ beg,
+__global__ __launch_bounds__(LIST_THREADS) void row_list_kernel(const int32_t* __restrict__ beg,
                                                                 const int32_t* __restrict__ end, int32_t V,
-                                                                int32_t* __restrict__ hubs,
-                                                                int32_t* __restrict__ hub_count,
-                                                                int32_t* __restrict__ giants,
-                                                                int32_t* __restrict__ giant_count) {
-  __shared__ int s_n[2], s_at[2];
+                                                                RowLists l) {
+  __shared__ int s_n[3], s_at[3];
   const int32_t v = blockIdx.x * LIST_THREADS + threadIdx.x;
   const int32_t d = v < V ? end[v] - beg[v] : 0;
-  const bool giant = d > GIANT_MIN, hub = !giant && d > SMALL_ROW;
-  if (threadIdx.x < 2) s_n[threadIdx.x] = 0;
+  const int kind = d > GIANT_MIN ? 2 : (d > MID_ROW ? 1 : (d > SMALL_ROW ? 0 : -1));
+  if (threadIdx.x < 3) s_n[threadIdx.x] = 0;
   __syncthreads();
-  const uint64_t mg = __ballot(giant), mh = __ballot(hub);
-  const uint64_t below = (((uint64_t)1) << lane()) - 1;
-  int bh = 0, bg = 0;
-  if (lane() == 0) {
-    if (mh) bh = atomicAdd(s_n, __popcll(mh));
-    if (mg) bg = atomicAdd(s_n + 1, __popcll(mg));
+  int at = 0;
+  for (int k = 0; k < 3; ++k) {
+    const uint64_t m = __ballot(kind == k);
+    if (m == 0) continue;
+    int base = 0;
+    if (lane() == 0) base = atomicAdd(s_n + k, __popcll(m));
+    base = __shfl(base, 0);
+    if (kind == k) at = base + __popcll(m & ((((uint64_t)1) << lane()) - 1));
   }
-  bh = __shfl(bh, 0);
-  bg = __shfl(bg, 0);
   __syncthreads();
-  if (threadIdx.x == 0) s_at[0] = s_n[0] ? atomicAdd(hub_count, s_n[0]) : 0;
-  if (threadIdx.x == 1) s_at[1] = s_n[1] ? atomicAdd(giant_count, s_n[1]) : 0;
+  if (threadIdx.x < 3) s_at[threadIdx.x] = s_n[threadIdx.x] ? atomicAdd(l.counts + threadIdx.x, s_n[threadIdx.x]) : 0;
   __syncthreads();
-  if (hub) hubs[s_at[0] + bh + __popcll(mh & below)] = v;
-  if (giant) giants[s_at[1] + bg + __popcll(mg & below)] = v;
+  if (kind < 0) return;
+  at += s_at[kind];
+  if (kind == 2) l.giants[at] = v;
+  else l.rows[kind == 0 ? at : V - 1 - at] = v;
 }
 
 // The threads of one vertex, with their part of the workgroup's LDS.
@@ -378,6 +414,28 @@ struct SweepShared {
   double sum[HUB_THREADS / 64];
   int32_t value, count;
 };
+// (pairs of mirrored lanes in place of xor 4 and 8: the lanes of a pair's side hold equal values by then)
+__device__ __forceinline__ uint64_t half_wave_max(uint64_t x) {
+  x = pick_u64<true>(x, dpp_u64<0xB1>(x));
+  x = pick_u64<true>(x, dpp_u64<0x4E>(x));
+  x = pick_u64<true>(x, dpp_u64<0x141>(x));
+  x = pick_u64<true>(x, dpp_u64<0x140>(x));
+  return pick_u64<true>(x, xor_u64<16>(x));
+}
+__device__ __forceinline__ double f64_of(uint64_t x) { return __builtin_bit_cast(double, x); }
+__device__ __forceinline__ uint64_t u64_of(double x) { return __builtin_bit_cast(uint64_t, x); }
+__device__ __forceinline__ double half_wave_sum(double x) {
+  x += f64_of(dpp_u64<0xB1>(u64_of(x)));
+  x += f64_of(dpp_u64<0x4E>(u64_of(x)));
+  x += f64_of(dpp_u64<0x141>(u64_of(x)));
+  x += f64_of(dpp_u64<0x140>(u64_of(x)));
+  return x + f64_of(xor_u64<16>(u64_of(x)));
+}
+__device__ __forceinline__ double full_wave_sum(double x) {
+  x = half_wave_sum(x);
+  return x + f64_of(xor_u64<32>(u64_of(x)));
+}
+
 struct HalfWave {
   static constexpr int N = 32, SLOTS = SMALL_SLOTS;
   int32_t* tc;
@@ -388,20 +446,8 @@ struct HalfWave {
         list(sh.list + (threadIdx.x >> 5) * SMALL_ROW) {}
   __device__ int tid() const { return lane() & 31; }
   __device__ void sync() const { wave_lds_sync(); }
-  __device__ uint64_t max(uint64_t x) const {
-    x = pick_u64<true>(x, xor_u64<1>(x));
-    x = pick_u64<true>(x, xor_u64<2>(x));
-    x = pick_u64<true>(x, xor_u64<4>(x));
-    x = pick_u64<true>(x, xor_u64<8>(x));
-    return pick_u64<true>(x, xor_u64<16>(x));
-  }
-  __device__ double sum(double x) const {
-    x += __builtin_bit_cast(double, xor_u64<1>(__builtin_bit_cast(uint64_t, x)));
-    x += __builtin_bit_cast(double, xor_u64<2>(__builtin_bit_cast(uint64_t, x)));
-    x += __builtin_bit_cast(double, xor_u64<4>(__builtin_bit_cast(uint64_t, x)));
-    x += __builtin_bit_cast(double, xor_u64<8>(__builtin_bit_cast(uint64_t, x)));
-    return x + __builtin_bit_cast(double, xor_u64<16>(__builtin_bit_cast(uint64_t, x)));
-  }
+  __device__ uint64_t max(uint64_t x) const { return half_wave_max(x); }
+  __device__ double sum(double x) const { return half_wave_sum(x); }
   __device__ uint32_t ballot(bool x) const { return (uint32_t)(__ballot(x) >> (lane() & 32)); }
   // The value of the thread that holds the winning key.
   __device__ int32_t of(uint64_t best, uint64_t mine, int32_t value) const {
@@ -414,6 +460,31 @@ struct HalfWave {
     const uint32_t m = ballot(taken);
     if (taken) list[n + __popc(m & ((1u << tid()) - 1))] = (uint16_t)h;
     return n + __popc(m);
+  }
+  __device__ int listed(int n) const { return n; }
+};
+
+struct Wave {
+  static constexpr int N = 64, SLOTS = 2 * SMALL_SLOTS;
+  int32_t* tc;
+  double* ts;
+  uint16_t* list;
+  __device__ explicit Wave(SweepShared& sh)
+      : tc(sh.tc + (threadIdx.x >> 6) * SLOTS), ts(sh.ts + (threadIdx.x >> 6) * SLOTS),
+        list(sh.list + (threadIdx.x >> 6) * MID_ROW) {}
+  __device__ int tid() const { return lane(); }
+  __device__ void sync() const { wave_lds_sync(); }
+  __device__ uint64_t max(uint64_t x) const { return wave_max_u64(x); }
+  __device__ double sum(double x) const { return full_wave_sum(x); }
+  __device__ int32_t of(uint64_t best, uint64_t mine, int32_t value) const {
+    return __shfl(value, first_lane(__ballot(mine == best)));
+  }
+  __device__ bool any(bool x) const { return __ballot(x) != 0; }
+  __device__ void start_list() const {}
+  __device__ int append(bool taken, int h, int n) const {
+    const uint64_t m = __ballot(taken);
+    if (taken) list[n + __popcll(m & ((((uint64_t)1) << lane()) - 1))] = (uint16_t)h;
+    return n + __popcll(m);
   }
   __device__ int listed(int n) const { return n; }
 };
@@ -436,7 +507,7 @@ struct Workgroup {
     return x;
   }
   __device__ double sum(double x) const {
-    x = wave_sum_f64(x);
+    x = full_wave_sum(x);
     if (lane() == 0) sh->sum[threadIdx.x >> 6] = x;
     __syncthreads();
     double t = 0.0;
@@ -492,26 +563,30 @@ __device__ __forceinline__ void load_row(const P& p, const Graph& gr, int32_t v,
   for (int i = 0; i < ROW_PER; ++i) r.ok[i] = r.u[i] != v;
 }
 
+// Frees the slots of all tables of a workgroup; afterwards each vertex frees
+// the ones it used.
+__device__ __forceinline__ void clear_tables(SweepShared& sh) {
+  for (int j = threadIdx.x; j < HUB_SLOTS; j += HUB_THREADS) {
+    sh.tc[j] = -1;
+    sh.ts[j] = 0.0;
+  }
+  __syncthreads();
+}
+
 // Sums the weights of the entries that count by community c[i] into the
 // group's table and lists the slots in use; returns their number.
 template <class P>
-__device__ __forceinline__ int fill_table(const P& p, const Row& r, const int32_t* c, int32_t row) {
-  int size = 2 * P::N;
-  while (size < P::SLOTS && 2 * size < 3 * row) size = min(2 * size, P::SLOTS);
-  for (int j = p.tid(); j < size; j += P::N) {
-    p.tc[j] = -1;
-    p.ts[j] = 0.0;
-  }
+__device__ __forceinline__ int fill_table(const P& p, const Row& r, const int32_t* c) {
   p.start_list();
-  p.sync();
+  p.sync();  // (the vertex before has freed its slots)
   int n = 0;
 #pragma unroll
   for (int i = 0; i < ROW_PER; ++i) {
     bool taken = false;
     int h = 0;
     if (r.ok[i]) {
-      h = (int)(__umul24(((uint32_t)c[i] * 0x9E3779B1u) >> 16, (uint32_t)size) >> 16);
-      while (true) {  // (at most `row` <= 70% of size communities: a free slot or the community's is found)
+      h = (int)(__umul24(((uint32_t)c[i] * 0x9E3779B1u) >> 16, (uint32_t)P::SLOTS) >> 16);
+      while (true) {  // (at most 70% of the slots are taken: a free one or the community's is found)
         const int32_t cur = __hip_atomic_load(p.tc + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         if (cur == c[i]) break;
         if (cur == -1) {
@@ -519,7 +594,7 @@ __device__ __forceinline__ int fill_table(const P& p, const Row& r, const int32_
           taken = prev == -1;
           if (taken || prev == c[i]) break;
         }
-        h = h + 1 == size ? 0 : h + 1;
+        h = h + 1 == P::SLOTS ? 0 : h + 1;
       }
       unsafeAtomicAdd(p.ts + h, (double)r.w[i]);
     }
@@ -552,6 +627,8 @@ __device__ __forceinline__ void each_candidate(const P& p, const Row& r, int n, 
         const int h = p.list[j];
         c[i] = p.tc[h];
         w[i] = (float)p.ts[h];
+        p.tc[h] = -1;
+        p.ts[h] = 0.0;
       }
     }
     if (ok[i]) total[i] = sigma[c[i]];
@@ -583,11 +660,10 @@ struct MoveSweep {
   LevelConst lc;
 };
 
-__device__ inline void finish_move(const MoveSweep& s, int32_t v, int32_t old, int32_t choice, double kv) {
+__device__ inline void finish_move(const MoveSweep& s, int32_t v, int32_t choice, double kv) {
   s.lout[v] = choice;
   s.clear[v] = 0.0;
   if (kv != 0.0) unsafeAtomicAdd(s.next + choice, kv);
-  if (choice != old) mark_moved(s.ctl + CTL_LM + (s.sweep & (RING - 1)));
 }
 
 // What a sweep reads of vertex v before its row: loads that depend on v alone,
@@ -612,8 +688,9 @@ __device__ __forceinline__ Vertex load_vertex(const Graph& gr, const LevelConst&
   return x;
 }
 
+// Returns whether the vertex moves.
 template <class P, bool FIRST>
-__device__ __forceinline__ void move_vertex(const P& p, const Graph& gr, const MoveSweep& s, const MoveState& st,
+__device__ __forceinline__ bool move_vertex(const P& p, const Graph& gr, const MoveSweep& s, const MoveState& st,
                                             const Vertex& x, int32_t old) {
   int32_t choice = old;
   if (!st.done && x.a != x.b && x.tm > 0.0) {
@@ -639,7 +716,7 @@ __device__ __forceinline__ void move_vertex(const P& p, const Graph& gr, const M
         r.ok[i] = c[i] != old && (c[i] > old ? 1 : 0) == st.up;  // the others are no candidates
       }
       k_old = (float)p.sum(own);
-      n = fill_table(p, r, c, x.b - x.a);
+      n = fill_table(p, r, c);
     }
     const double gain = (double)s.resolution * x.kv;
     const float jitter = (rand_uniform(x.salt, 0u, (uint32_t)s.sweep, s.seed) - 0.5f) * 1e-9f;
@@ -656,39 +733,77 @@ __device__ __forceinline__ void move_vertex(const P& p, const Graph& gr, const M
     const uint64_t best = p.max(mine);
     if (best > pack(0.0f, STAY_PREF)) choice = p.of(best, mine, mine_c);
   }
-  if (p.tid() == 0) finish_move(s, x.v, old, choice, x.kv);
+  if (p.tid() == 0) finish_move(s, x.v, choice, x.kv);
+  return choice != old;
 }
 
-// Block b of n of a vertex range: each XCD (blocks run on the eight in turn)
-// gets a contiguous run, so that a graph's labels and totals stay in one L2.
-__device__ inline int32_t xcd_block(int32_t b, int32_t n) {
-  const int32_t per = n >> 3;
-  return b < 8 * per ? (b & 7) * per + (b >> 3) : b;
+// A workgroup's vertices: chunks of GROUPS, strided over the workgroups of its
+// XCD, each XCD (workgroups run on the eight in turn; the grid is a multiple of
+// eight) a contiguous run, so that a graph's labels and totals stay in one L2.
+// The half waves go through their chunks without waiting for each other: with
+// a workgroup per chunk, the LDS of the waves that were done stayed taken until
+// the slowest was (20 of 32 waves a compute unit at work).
+//
+// Below two chunks a workgroup the long rows take LONG_BLOCKS workgroups of
+// their own in the same launch (all sweeps of eight 2k graphs, 2,000 chunks:
+// 577 us against 669 with every workgroup taking both); above, all workgroups
+// share both (57,000 vertices, 7,100 chunks: 1,885 us against 1,964).
+struct Share {
+  int32_t at, end, step;
+};
+struct Split {
+  unsigned grid;
+  int32_t long_blocks;  // workgroups that take long rows: the first ones
+  int32_t first;        // workgroups before the first that takes chunks
+};
+inline Split split_of(int32_t V) {
+  const int32_t chunks = (V + GROUPS - 1) / GROUPS;
+  if (chunks >= 2 * SWEEP_BLOCKS) return Split{SWEEP_BLOCKS, SWEEP_BLOCKS, 0};
+  return Split{(unsigned)(LONG_BLOCKS + (chunks + 7) / 8 * 8), LONG_BLOCKS, LONG_BLOCKS};
+}
+// A wave's mids: a run of the list (about ascending) for each XCD, as the chunks.
+__device__ __forceinline__ Share mid_share(const RowLists& l) {
+  if ((int32_t)blockIdx.x >= l.long_blocks) return Share{0, 0, 1};
+  const int64_t mids = l.counts[0];
+  const int32_t x = blockIdx.x & 7, waves = HUB_THREADS / 64;
+  return Share{(int32_t)(mids * x / 8) + (int32_t)(blockIdx.x >> 3) * waves + (int32_t)(threadIdx.x >> 6),
+               (int32_t)(mids * (x + 1) / 8), (l.long_blocks >> 3) * waves};
+}
+__device__ __forceinline__ Share share_of(int32_t V, int32_t first) {
+  if ((int32_t)blockIdx.x < first) return Share{0, 0, 1};
+  const int64_t chunks = (V + GROUPS - 1) / GROUPS;
+  const int32_t b = (int32_t)blockIdx.x - first, x = b & 7;
+  return Share{(int32_t)(chunks * x / 8) + (b >> 3), (int32_t)(chunks * (x + 1) / 8), ((int32_t)gridDim.x - first) >> 3};
 }
 
 template <bool FIRST>
 __global__ __launch_bounds__(HUB_THREADS, 8) void local_moving_kernel(Graph gr, MoveSweep s,
-                                                                      const int32_t* __restrict__ hubs,
-                                                                      const int32_t* __restrict__ hub_count) {
+                                                                      RowLists l) {
   __shared__ SweepShared sh;  // (FIRST leaves the table out of use; its occupancy is full all the same)
+  bool moved = false;
   const MoveState st = move_state(s.ctl, s.sweep);
-  if (blockIdx.x < HUB_BLOCKS) {
-    const int32_t n = *hub_count;
-    const Workgroup p(sh);
-    for (int32_t i = blockIdx.x; i < n; i += HUB_BLOCKS) {
-      const Vertex x = load_vertex(gr, s.lc, hubs[i]);
-      move_vertex<Workgroup, FIRST>(p, gr, s, st, x, FIRST ? x.v : s.lin[x.v]);
-      __syncthreads();  // the next vertex takes the table
-    }
-    return;
+  if constexpr (!FIRST) clear_tables(sh);
+  const int32_t hubs = l.counts[1];
+  const Share share = mid_share(l);
+  for (int32_t i = l.start(blockIdx.x); i < hubs; i += l.long_blocks) {
+    const Vertex x = load_vertex(gr, s.lc, l.rows[gr.V - 1 - i]);
+    moved |= move_vertex<Workgroup, FIRST>(Workgroup(sh), gr, s, st, x, FIRST ? x.v : s.lin[x.v]);
+    __syncthreads();  // the next vertex takes the table
   }
+  for (int32_t i = share.at; i < share.end; i += share.step) {
+    const Vertex x = load_vertex(gr, s.lc, l.rows[i]);
+    moved |= move_vertex<Wave, FIRST>(Wave(sh), gr, s, st, x, FIRST ? x.v : load_now(s.lin + x.v));
+  }
+  const Share mine = share_of(gr.V, l.first);
   const HalfWave p(sh);
-  const int32_t v = xcd_block(blockIdx.x - HUB_BLOCKS, gridDim.x - HUB_BLOCKS) * GROUPS + (threadIdx.x >> 5);
-  if (v >= gr.V) return;
-  const Vertex x = load_vertex(gr, s.lc, v);
-  const int32_t old = FIRST ? v : load_now(s.lin + v);
-  if (x.b - x.a > SMALL_ROW) return;
-  move_vertex<HalfWave, FIRST>(p, gr, s, st, x, old);
+  for (int32_t c = mine.at; c < mine.end; c += mine.step) {
+    const int32_t v = c * GROUPS + (int32_t)(threadIdx.x >> 5);
+    if (v >= gr.V) break;
+    const Vertex x = load_vertex(gr, s.lc, v);
+    const int32_t old = FIRST ? v : load_now(s.lin + v);
+    if (x.b - x.a <= SMALL_ROW) moved |= move_vertex<HalfWave, FIRST>(p, gr, s, st, x, old);
+  }
+  mark_moved(mark_slot(s.ctl, true, s.sweep), moved);
 }
 
 // Refinement: a vertex proposes a community inside its parent community (x of
@@ -766,7 +881,7 @@ __device__ __forceinline__ void propose_vertex(const P& p, const Graph& gr, cons
           r.ok[i] = r.ok[i] && c[i] != old;
         }
         k_old = (float)p.sum(own);
-        n = fill_table(p, r, c, x.b - x.a);
+        n = fill_table(p, r, c);
       }
       const double gain = (double)s.resolution * x.kv;
       uint64_t mine = 0;
@@ -799,27 +914,30 @@ __device__ __forceinline__ void propose_vertex(const P& p, const Graph& gr, cons
 
 template <bool FIRST>
 __global__ __launch_bounds__(HUB_THREADS, 8) void refine_propose_kernel(Graph gr, RefineSweep s,
-                                                                        const int32_t* __restrict__ hubs,
-                                                                        const int32_t* __restrict__ hub_count) {
+                                                                        RowLists l) {
   __shared__ SweepShared sh;
   if (refine_done(s.ctl, s.sweep)) return;
-  if (blockIdx.x < HUB_BLOCKS) {
-    const int32_t n = *hub_count;
-    const Workgroup p(sh);
-    for (int32_t i = blockIdx.x; i < n; i += HUB_BLOCKS) {
-      const Vertex x = load_vertex(gr, s.lc, hubs[i]);
-      propose_vertex<Workgroup, FIRST>(p, gr, s, x, refine_self<FIRST>(s, x.v));
-      __syncthreads();
-    }
-    return;
+  if constexpr (!FIRST) clear_tables(sh);
+  const int32_t hubs = l.counts[1];
+  const Share share = mid_share(l);
+  for (int32_t i = l.start(blockIdx.x); i < hubs; i += l.long_blocks) {
+    const Vertex x = load_vertex(gr, s.lc, l.rows[gr.V - 1 - i]);
+    propose_vertex<Workgroup, FIRST>(Workgroup(sh), gr, s, x, refine_self<FIRST>(s, x.v));
+    __syncthreads();
   }
+  for (int32_t i = share.at; i < share.end; i += share.step) {
+    const Vertex x = load_vertex(gr, s.lc, l.rows[i]);
+    propose_vertex<Wave, FIRST>(Wave(sh), gr, s, x, refine_self<FIRST>(s, x.v));
+  }
+  const Share mine = share_of(gr.V, l.first);
   const HalfWave p(sh);
-  const int32_t v = xcd_block(blockIdx.x - HUB_BLOCKS, gridDim.x - HUB_BLOCKS) * GROUPS + (threadIdx.x >> 5);
-  if (v >= gr.V) return;
-  const Vertex x = load_vertex(gr, s.lc, v);
-  const int2 self = refine_self<FIRST>(s, v);
-  if (x.b - x.a > SMALL_ROW) return;
-  propose_vertex<HalfWave, FIRST>(p, gr, s, x, self);
+  for (int32_t c = mine.at; c < mine.end; c += mine.step) {
+    const int32_t v = c * GROUPS + (int32_t)(threadIdx.x >> 5);
+    if (v >= gr.V) break;
+    const Vertex x = load_vertex(gr, s.lc, v);
+    const int2 self = refine_self<FIRST>(s, v);
+    if (x.b - x.a <= SMALL_ROW) propose_vertex<HalfWave, FIRST>(p, gr, s, x, self);
+  }
 }
 
 // A mover commits unless a moving neighbour in its parent community outranks
@@ -843,8 +961,9 @@ __device__ __forceinline__ Commit load_commit(const Graph& gr, const RefineSweep
   return x;
 }
 
+// Returns whether the vertex moves.
 template <class P>
-__device__ __forceinline__ void commit_vertex(const P& p, const Graph& gr, const RefineSweep& s, bool done,
+__device__ __forceinline__ bool commit_vertex(const P& p, const Graph& gr, const RefineSweep& s, bool done,
                                               const Commit& x) {
   const bool wants = !done && x.wants >= 0;  // (after the end the proposals are an earlier sweep's)
   bool lost = false;
@@ -876,37 +995,38 @@ __device__ __forceinline__ void commit_vertex(const P& p, const Graph& gr, const
     }
     lost = p.any(lost);
   }
+  const int32_t label = wants && !lost ? x.to : x.self.y;
   if (p.tid() == 0) {
-    const int32_t label = wants && !lost ? x.to : x.self.y;
     s.lout[x.v] = int2{x.self.x, label};
     s.labels[x.v] = label;
     s.clear[x.v] = 0.0;
     if (x.kv != 0.0) unsafeAtomicAdd(s.next + label, x.kv);
-    if (label != x.self.y) mark_moved(s.ctl + CTL_REFINE + (s.sweep & (RING - 1)));
   }
+  return label != x.self.y;
 }
 
 template <bool FIRST>
 __global__ __launch_bounds__(HUB_THREADS, 8) void refine_commit_kernel(Graph gr, RefineSweep s,
-                                                                       const int32_t* __restrict__ hubs,
-                                                                       const int32_t* __restrict__ hub_count,
-                                                                       const int32_t* __restrict__ giants,
-                                                                       const int32_t* __restrict__ giant_count) {
+                                                                       RowLists l) {
   __shared__ SweepShared sh;  // (the table stays out of use)
   const bool done = refine_done(s.ctl, s.sweep);
-  if (blockIdx.x < HUB_BLOCKS) {
-    const int32_t n = *hub_count, all = n + *giant_count;
-    const Workgroup p(sh);
-    for (int32_t i = blockIdx.x; i < all; i += HUB_BLOCKS)
-      commit_vertex(p, gr, s, done, load_commit<FIRST>(gr, s, i < n ? hubs[i] : giants[i - n]));
-    return;
-  }
+  bool moved = false;
+  const int32_t hubs = l.counts[1], long_rows = hubs + l.counts[2];
+  const Share share = mid_share(l);
+  for (int32_t i = l.start(blockIdx.x); i < long_rows; i += l.long_blocks)
+    moved |= commit_vertex(Workgroup(sh), gr, s, done,
+                  load_commit<FIRST>(gr, s, i < hubs ? l.rows[gr.V - 1 - i] : l.giants[i - hubs]));
+  for (int32_t i = share.at; i < share.end; i += share.step)
+    moved |= commit_vertex(Wave(sh), gr, s, done, load_commit<FIRST>(gr, s, l.rows[i]));
+  const Share mine = share_of(gr.V, l.first);
   const HalfWave p(sh);
-  const int32_t v = xcd_block(blockIdx.x - HUB_BLOCKS, gridDim.x - HUB_BLOCKS) * GROUPS + (threadIdx.x >> 5);
-  if (v >= gr.V) return;
-  const Commit x = load_commit<FIRST>(gr, s, v);
-  if (x.b - x.a > SMALL_ROW) return;
-  commit_vertex(p, gr, s, done, x);
+  for (int32_t c = mine.at; c < mine.end; c += mine.step) {
+    const int32_t v = c * GROUPS + (int32_t)(threadIdx.x >> 5);
+    if (v >= gr.V) break;
+    const Commit x = load_commit<FIRST>(gr, s, v);
+    if (x.b - x.a <= SMALL_ROW) moved |= commit_vertex(p, gr, s, done, x);
+  }
+  mark_moved(mark_slot(s.ctl, false, s.sweep), moved);
 }
 
 // Test hook: raises the overflow word as a broken local-moving table would.
@@ -1065,19 +1185,18 @@ __device__ float giant_k_old(GiantShared& sh, int32_t old, int32_t thr) {
 
 template <bool FIRST>
 __global__ __launch_bounds__(GIANT_THREADS) void local_moving_giant_kernel(Graph gr, MoveSweep s,
-                                                                           const int32_t* __restrict__ giants,
-                                                                           const int32_t* __restrict__ giant_count) {
+                                                                           RowLists l) {
   __shared__ GiantShared sh;
-  const int32_t count = *giant_count;
+  const int32_t count = l.counts[2];
   const MoveState st = move_state(s.ctl, s.sweep);
   for (int32_t i = blockIdx.x; i < count; i += gridDim.x) {
-    const int32_t v = giants[i];
+    const int32_t v = l.giants[i];
     const int32_t old = FIRST ? v : s.lin[v];
     const int32_t g = v / gr.S;
     const double tm = gr.two_m[g];
     const double kv = gr.k_v[v];
     if (st.done || !(tm > 0.0)) {
-      if (threadIdx.x == 0) finish_move(s, v, old, old, kv);
+      if (threadIdx.x == 0) finish_move(s, v, old, kv);
       continue;
     }
     const int32_t a = gr.beg[v], b = gr.end[v];
@@ -1085,7 +1204,7 @@ __global__ __launch_bounds__(GIANT_THREADS) void local_moving_giant_kernel(Graph
     double e_sum;
     if (!giant_table(gr, [&](int32_t u) { return FIRST ? u : s.lin[u]; }, v, a, b, sh, &thr, &e_sum)) {  // cannot happen
       if (threadIdx.x == 0) {
-        finish_move(s, v, old, old, kv);  // stay, flagged
+        finish_move(s, v, old, kv);  // stay, flagged
         s.ctl[CTL_OVERFLOW] = 1;
       }
       __syncthreads();
@@ -1113,19 +1232,19 @@ __global__ __launch_bounds__(GIANT_THREADS) void local_moving_giant_kernel(Graph
       }
     }
     const int32_t choice = giant_pick(mine, mine_c, pack(0.0f, STAY_PREF), old, sh);
-    if (threadIdx.x == 0) finish_move(s, v, old, choice, kv);
+    if (threadIdx.x == 0) finish_move(s, v, choice, kv);
+    if (threadIdx.x < 64) mark_moved(mark_slot(s.ctl, true, s.sweep), choice != old);
   }
 }
 
 template <bool FIRST>
 __global__ __launch_bounds__(GIANT_THREADS) void refine_propose_giant_kernel(Graph gr, RefineSweep s,
-                                                                             const int32_t* __restrict__ giants,
-                                                                             const int32_t* __restrict__ giant_count) {
+                                                                             RowLists l) {
   __shared__ GiantShared sh;
   if (refine_done(s.ctl, s.sweep)) return;
-  const int32_t count = *giant_count;
+  const int32_t count = l.counts[2];
   for (int32_t i = blockIdx.x; i < count; i += gridDim.x) {
-    const int32_t v = giants[i];
+    const int32_t v = l.giants[i];
     const int32_t g = v / gr.S;
     int2 self;
     if constexpr (FIRST) self = int2{s.parent[v], v};
@@ -1845,8 +1964,7 @@ __global__ __launch_bounds__(AGG_DENSE_THREADS) void agg_dense_kernel(Contract c
 __global__ __launch_bounds__(ETHREADS) void level_init_kernel(int32_t V, int32_t* __restrict__ labels,
                                                               int32_t* __restrict__ moves, double* __restrict__ total,
                                                               int32_t* __restrict__ ctl,
-                                                              int32_t* __restrict__ hub_count,
-                                                              int32_t* __restrict__ giant_count,
+                                                              int32_t* __restrict__ counts,
                                                               const double* __restrict__ two_m,
                                                               double2* __restrict__ scale,
                                                               uint32_t* __restrict__ salt, Divisor graph_of,
@@ -1865,10 +1983,7 @@ __global__ __launch_bounds__(ETHREADS) void level_init_kernel(int32_t V, int32_t
   for (int32_t i = v; i < CTL_WORDS; i += gridDim.x * ETHREADS) {
     if (i != CTL_OVERFLOW || first) ctl[i] = 0;
   }
-  if (v == 0) {
-    *hub_count = 0;
-    *giant_count = 0;
-  }
+  if (v < 3) counts[v] = 0;
 }
 
 // width = the largest number of distinct labels of a graph.
@@ -1981,7 +2096,7 @@ int launch_check() {
 
 struct LeidenLayout {
   size_t keys_a, keys_b, vals_a, vals_b, temp, temp_bytes, row_ptr, col, k_v, two_m, totals[4], lab, moves[2], pairs[2],
-      prop, mover, ctl, hubs, hub_count, giants, giant_count, scale, salt, total;
+      prop, mover, ctl, rows, giants, counts, scale, salt, total;
 };
 
 LeidenLayout leiden_layout(int64_t E, int32_t G, int32_t S) {
@@ -2019,10 +2134,9 @@ LeidenLayout leiden_layout(int64_t E, int32_t G, int32_t S) {
   L.salt = take(V * 4);
   L.scale = take(G * 16);
   L.ctl = take(CTL_WORDS * 4);
-  L.hubs = take(V * 4);
-  L.hub_count = take(4);
+  L.rows = take(V * 4);
   L.giants = take(V * 4);
-  L.giant_count = take(4);
+  L.counts = take(12);
   L.total = off;
   return L;
 }
@@ -2103,10 +2217,7 @@ struct SweepBuffers {
   int32_t* prop;
   int32_t* mover;
   int32_t* ctl;
-  int32_t* hubs;
-  int32_t* hub_count;
-  int32_t* giants;
-  int32_t* giant_count;
+  RowLists lists;
   double2* scale;
   uint32_t* salt;
 };
@@ -2118,12 +2229,15 @@ void run_sweeps(const Graph& gr, const SweepBuffers& b, float resolution, float 
   const int32_t V = gr.V;
   const Divisor graph_of(gr.S);
   const LevelConst lc{b.scale, b.salt, graph_of};
-  level_init_kernel<<<blocks(V, ETHREADS), ETHREADS, 0, st>>>(V, b.labels, b.moves[0], b.total[0], b.ctl, b.hub_count,
-                                                              b.giant_count, gr.two_m, b.scale, b.salt, graph_of,
+  level_init_kernel<<<blocks(V, ETHREADS), ETHREADS, 0, st>>>(V, b.labels, b.moves[0], b.total[0], b.ctl,
+                                                              b.lists.counts, gr.two_m, b.scale, b.salt, graph_of,
                                                               V / gr.S, first_level);
-  hub_list_kernel<<<blocks(V, LIST_THREADS), LIST_THREADS, 0, st>>>(gr.beg, gr.end, V, b.hubs, b.hub_count, b.giants,
-                                                                   b.giant_count);
-  const unsigned grid = HUB_BLOCKS + blocks(V, GROUPS);
+  row_list_kernel<<<blocks(V, LIST_THREADS), LIST_THREADS, 0, st>>>(gr.beg, gr.end, V, b.lists);
+  const Split split = split_of(V);
+  const unsigned grid = split.grid;
+  RowLists lists = b.lists;
+  lists.long_blocks = split.long_blocks;
+  lists.first = split.first;
   // (a row of different neighbours, its self loop twice, is at most one longer than its graph)
   const bool giants = !gr.unique || gr.S >= GIANT_MIN;
   double* const* t = b.total;
@@ -2132,12 +2246,12 @@ void run_sweeps(const Graph& gr, const SweepBuffers& b, float resolution, float 
     const MoveSweep s{i == 0 ? gr.k_v : t[(i - 1) % 3], t[i % 3], t[(i + 1) % 3], b.moves[i & 1], b.moves[(i & 1) ^ 1],
                       b.ctl, i, resolution, (uint32_t)seed, lc};
     if (i == 0 && gr.unique) {
-      local_moving_kernel<true><<<grid, HUB_THREADS, 0, st>>>(gr, s, b.hubs, b.hub_count);
-      if (giants) local_moving_giant_kernel<true><<<GIANT_BLOCKS, GIANT_THREADS, 0, st>>>(gr, s, b.giants, b.giant_count);
+      local_moving_kernel<true><<<grid, HUB_THREADS, 0, st>>>(gr, s, lists);
+      if (giants) local_moving_giant_kernel<true><<<GIANT_BLOCKS, GIANT_THREADS, 0, st>>>(gr, s, lists);
     } else {
-      local_moving_kernel<false><<<grid, HUB_THREADS, 0, st>>>(gr, s, b.hubs, b.hub_count);
+      local_moving_kernel<false><<<grid, HUB_THREADS, 0, st>>>(gr, s, lists);
       if (giants)
-        local_moving_giant_kernel<false><<<GIANT_BLOCKS, GIANT_THREADS, 0, st>>>(gr, s, b.giants, b.giant_count);
+        local_moving_giant_kernel<false><<<GIANT_BLOCKS, GIANT_THREADS, 0, st>>>(gr, s, lists);
     }
   }
   if (g_test_raise_overflow) raise_overflow_kernel<<<1, 64, 0, st>>>(b.ctl);
@@ -2155,15 +2269,15 @@ void run_sweeps(const Graph& gr, const SweepBuffers& b, float resolution, float 
                         b.pairs[i & 1], b.pairs[(i & 1) ^ 1], b.labels, b.prop, b.mover, b.ctl, i, resolution,
                         inv_theta, use_boltzmann ? 1 : 0, (uint32_t)seed, lc};
     if (i == 0 && gr.unique) {
-      refine_propose_kernel<true><<<grid, HUB_THREADS, 0, st>>>(gr, s, b.hubs, b.hub_count);
+      refine_propose_kernel<true><<<grid, HUB_THREADS, 0, st>>>(gr, s, lists);
       if (giants)
-        refine_propose_giant_kernel<true><<<GIANT_BLOCKS, GIANT_THREADS, 0, st>>>(gr, s, b.giants, b.giant_count);
-      refine_commit_kernel<true><<<grid, HUB_THREADS, 0, st>>>(gr, s, b.hubs, b.hub_count, b.giants, b.giant_count);
+        refine_propose_giant_kernel<true><<<GIANT_BLOCKS, GIANT_THREADS, 0, st>>>(gr, s, lists);
+      refine_commit_kernel<true><<<grid, HUB_THREADS, 0, st>>>(gr, s, lists);
     } else {
-      refine_propose_kernel<false><<<grid, HUB_THREADS, 0, st>>>(gr, s, b.hubs, b.hub_count);
+      refine_propose_kernel<false><<<grid, HUB_THREADS, 0, st>>>(gr, s, lists);
       if (giants)
-        refine_propose_giant_kernel<false><<<GIANT_BLOCKS, GIANT_THREADS, 0, st>>>(gr, s, b.giants, b.giant_count);
-      refine_commit_kernel<false><<<grid, HUB_THREADS, 0, st>>>(gr, s, b.hubs, b.hub_count, b.giants, b.giant_count);
+        refine_propose_giant_kernel<false><<<GIANT_BLOCKS, GIANT_THREADS, 0, st>>>(gr, s, lists);
+      refine_commit_kernel<false><<<grid, HUB_THREADS, 0, st>>>(gr, s, lists);
     }
   }
 }
@@ -2233,8 +2347,8 @@ extern "C" int ckv_batched_leiden(const int32_t* edge_src, const int32_t* edge_d
                          lab,
                          {(int32_t*)(ws + L.moves[0]), (int32_t*)(ws + L.moves[1])},
                          {(int2*)(ws + L.pairs[0]), (int2*)(ws + L.pairs[1])},
-                         (int32_t*)(ws + L.prop), (int32_t*)(ws + L.mover), ctl, (int32_t*)(ws + L.hubs),
-                         (int32_t*)(ws + L.hub_count), (int32_t*)(ws + L.giants), (int32_t*)(ws + L.giant_count),
+                         (int32_t*)(ws + L.prop), (int32_t*)(ws + L.mover), ctl,
+                         {(int32_t*)(ws + L.rows), (int32_t*)(ws + L.giants), (int32_t*)(ws + L.counts), 0, 0},
                          (double2*)(ws + L.scale), (uint32_t*)(ws + L.salt)};
   run_sweeps(gr, buf, resolution, theta, max_inner_iter, seed, use_boltzmann, true, st);
   sigma_zero_kernel<<<egrid, ETHREADS, 0, st>>>(sigma, V);
@@ -2453,8 +2567,6 @@ extern "C" int ckv_leiden_run(const int32_t* edge_src, const int32_t* edge_dst, 
   int32_t* col0 = i32(L.col0);
   float* wt0 = (float*)(ws + L.wt0);
   int32_t* ctl = i32(L.ctl);
-  int32_t* hub_count = i32(L.counts);
-  int32_t* giant_count = i32(L.counts) + 1;
   int32_t* words = i32(L.words);  // edge flags, then the level's width
   int32_t* lists = i32(L.lists);
   uint64_t* hist = (uint64_t*)(ws + L.hist);
@@ -2508,7 +2620,7 @@ extern "C" int ckv_leiden_run(const int32_t* edge_src, const int32_t* edge_dst, 
                            i32(L.lab),
                            {i32(L.moves[0]), i32(L.moves[1])},
                            {(int2*)(ws + L.pairs[0]), (int2*)(ws + L.pairs[1])},
-                           i32(L.prop), i32(L.mover), ctl, i32(L.hubs), hub_count, i32(L.giants), giant_count,
+                           i32(L.prop), i32(L.mover), ctl, {i32(L.hubs), i32(L.giants), i32(L.counts), 0, 0},
                            (double2*)(ws + L.scale), (uint32_t*)(ws + L.salt)};
     run_sweeps(gr, buf, resolution, theta, max_inner_iter, seed + level, use_boltzmann, level == 0, st);
     // ranks of the labels in use, per graph

@@ -7,7 +7,7 @@
 // merges four lanes, an approximation), kappa is a parameter (<= 16) and the
 // stored value can be the reference probability or the dequantised raw score.
 //
-// prefill_mfma_kernel: one workgroup = 8 waves = 256 packed rows
+// prefill_mfma_kernel: one workgroup = 8 waves = 256 packed rows (4 waves = 128 in short prompts)
 // (row r <-> position r / G, query head kv_head * G + r % G, PackGQA), so every
 // K/V tile staged in LDS serves all G query heads of the KV head.  Each wave
 // owns 32 packed rows and computes S^T = K Q^T with v_mfma_f32_32x32x16_bf16:
@@ -38,8 +38,17 @@ namespace {
 using namespace ckv;
 
 constexpr int D = CKV_HEAD_DIM;
+// Waves per workgroup, 32 packed (position, head) rows each.  A workgroup has a
+// compute unit to itself (LDS), so a short prompt lasts as long as its last row
+// block's chain of tiles: with PF_SHORT_WAVES the chain's tiles take less and
+// twice as many workgroups share the work.  Up to PF_SHORT_GRID workgroups of
+// PF_WAVES (two a compute unit; 32 query heads over 8 KV heads: 4,096 positions)
+// that is faster, above it the tiles staged for half the rows cost more:
+// 500 / 1,000 / 2,000 / 4,000 positions 53 / 93 / 200 / 339 us with eight waves
+// and 48 / 89 / 169 / 319 with four, 6,000 positions 509 and 616.
 constexpr int PF_WAVES = 8;
-constexpr int PF_ROWS = 32 * PF_WAVES;  // packed (position, head) rows per workgroup
+constexpr int PF_SHORT_WAVES = 4;
+constexpr int PF_SHORT_GRID = 512;
 constexpr int PF_KEYS = 64;             // keys per LDS tile
 constexpr int K_STRIDE = D + 8;         // 272-byte (17-chunk) K rows: 16-lane b128 reads hit distinct banks
 constexpr int V_STRIDE = D + 32;        // 320-byte (20-chunk) V rows: transposed b64 reads hit distinct banks
@@ -55,8 +64,8 @@ constexpr int PF_BUF = 8;
 // Columns per candidate group: a group is inspected only when its maximum
 // reaches the filter (4 measured faster than 2 or 8).
 constexpr int PF_GROUP = 4;
-template <int QN>
-constexpr size_t pf_lds_bytes() { return PF_STAGE_BYTES + (size_t)(QN + PF_BUF) * 4 * 64 * PF_WAVES; }
+template <int QN, int WAVES>
+constexpr size_t pf_lds_bytes() { return PF_STAGE_BYTES + (size_t)(QN + PF_BUF) * 4 * 64 * WAVES; }
 constexpr int MAX_KAPPA = 16;
 constexpr int MAX_SEQ = (1 << 17) - 1;  // column + 1 must fit the 17-bit index field
 constexpr float NEG_INF = -__builtin_huge_valf();
@@ -136,8 +145,10 @@ __device__ inline void sort8_desc(uint32_t (&b)[8]) {
   ce_desc(b[1], b[2]); ce_desc(b[3], b[4]); ce_desc(b[5], b[6]);
 }
 
-template <int QN>
-__global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(ckv_prefill_args a, int group, int blocks) {
+template <int QN, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, WAVES / 4) void prefill_mfma_kernel(ckv_prefill_args a, int group, int blocks) {
+  constexpr int ROWS = 32 * WAVES;                       // packed rows of the workgroup
+  constexpr int DMA_PER = (20 + WAVES - 1) / WAVES;      // staging instructions per wave and tile
   extern __shared__ __align__(16) uint16_t pf_lds[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -150,13 +161,13 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(ckv_pref
   const int blk = blocks - 1 - (int)(blockIdx.x / kv_heads);
   const int kvh = (int)(blockIdx.x % kv_heads);
   const int S = a.seq_len;
-  const int64_t pr0 = (int64_t)blk * PF_ROWS;
+  const int64_t pr0 = (int64_t)blk * ROWS;
   const int64_t pr = pr0 + wave * 32 + row;
   const int pos = (int)(pr / group);
   const int head = kvh * group + (int)(pr % group);
   const bool row_ok = pos < S;
   const int pos_lo = (int)(pr0 / group);
-  const int pos_hi = min(S - 1, (int)((pr0 + PF_ROWS - 1) / group));
+  const int pos_hi = min(S - 1, (int)((pr0 + ROWS - 1) / group));
   const int tiles = pos_hi / PF_KEYS + 1;
   const float sl2 = a.softmax_scale * LOG2E;
 
@@ -180,10 +191,10 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(ckv_pref
   // Pad chunks load the row's first chunk (never read).  Byte offsets of each
   // lane's source within a tile are fixed; the tile base is uniform.
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  int k_src[3], v_src[3];
+  int k_src[DMA_PER], v_src[DMA_PER];
 #pragma unroll
-  for (int j = 0; j < 3; ++j) {
-    const int p = (wave_u + PF_WAVES * j) * 64 + lane;
+  for (int j = 0; j < DMA_PER; ++j) {
+    const int p = (wave_u + WAVES * j) * 64 + lane;
     const int kc = p % 17;
     k_src[j] = (int)((int64_t)(p / 17) * kstride * 2) + 16 * (kc == 16 ? 0 : kc);
     const int vc = p % 20;
@@ -198,8 +209,8 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(ckv_pref
     const char* vb = reinterpret_cast<const char*>(Vg + (int64_t)key0 * kstride);
     const bool tail = key0 + PF_KEYS > S;  // rows past the sequence re-read row S - 1
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const int n = wave_u + PF_WAVES * j;
+    for (int j = 0; j < DMA_PER; ++j) {
+      const int n = wave_u + WAVES * j;
       int ko = k_src[j], vo = v_src[j];
       if (tail) {
         const int p = n * 64 + lane;
@@ -223,11 +234,11 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(ckv_pref
   // entry stays in a register.
   uint4* q_lds = reinterpret_cast<uint4*>(reinterpret_cast<char*>(pf_lds) + PF_STAGE_BYTES) + tid;
 #pragma unroll
-  for (int j = 0; j < QN / 4; ++j) q_lds[j * 64 * PF_WAVES] = uint4{0u, 0u, 0u, 0u};
+  for (int j = 0; j < QN / 4; ++j) q_lds[j * 64 * WAVES] = uint4{0u, 0u, 0u, 0u};
   auto load_queue = [&](uint32_t (&q)[QN]) {
 #pragma unroll
     for (int j = 0; j < QN / 4; ++j) {
-      const uint4 w = q_lds[j * 64 * PF_WAVES];
+      const uint4 w = q_lds[j * 64 * WAVES];
       q[4 * j] = w.x;
       q[4 * j + 1] = w.y;
       q[4 * j + 2] = w.z;
@@ -237,7 +248,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(ckv_pref
   // This lane's pending candidates (nbuf of PF_BUF, unsorted), entry e at
   // buf_lds[e * threads].
   uint32_t* buf_lds = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(pf_lds) + PF_STAGE_BYTES +
-                                                  (size_t)QN * 4 * 64 * PF_WAVES) + tid;
+                                                  (size_t)QN * 4 * 64 * WAVES) + tid;
   int nbuf = 0;
   uint32_t q_min = 0u;
   uint32_t row_thr = 0u;  // a lower bound of the row's QN-th best key (both halves)
@@ -261,7 +272,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(ckv_pref
     load_queue(qk);
     uint32_t b[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) b[i] = buf_lds[i * 64 * PF_WAVES];
+    for (int i = 0; i < 8; ++i) b[i] = buf_lds[i * 64 * WAVES];
 #pragma unroll
     for (int i = 0; i < 8; ++i) b[i] = (i < nbuf && (int)(b[i] & 0x1ffffu) > num_sink) ? b[i] : 0u;
     sort8_desc(b);
@@ -275,7 +286,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(ckv_pref
       }
     }
 #pragma unroll
-    for (int j = 0; j < QN / 4; ++j) q_lds[j * 64 * PF_WAVES] = uint4{qk[4 * j], qk[4 * j + 1], qk[4 * j + 2], qk[4 * j + 3]};
+    for (int j = 0; j < QN / 4; ++j) q_lds[j * 64 * WAVES] = uint4{qk[4 * j], qk[4 * j + 1], qk[4 * j + 2], qk[4 * j + 3]};
     q_min = qk[QN - 1];
     nbuf = 0;
     uint32_t rt = 0xffffffffu;
@@ -374,7 +385,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(ckv_pref
             const float sv = cur[b][v];
             const int col = c0 + 32 * b + 8 * (v >> 2) + 4 * half + (v & 3);
             if (sv >= tf) {
-              buf_lds[nbuf * (64 * PF_WAVES)] =
+              buf_lds[nbuf * (64 * WAVES)] =
                   (quantise_score(sv) << 17) | (uint32_t)(col + 1);
               ++nbuf;
             }
@@ -505,27 +516,35 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void prefill_mfma_kernel(ckv_pref
   }
 }
 
-template <int QN>
-int launch_prefill(const ckv_prefill_args& a, hipStream_t s) {
+template <int QN, int WAVES>
+int launch_rows(const ckv_prefill_args& a, hipStream_t s) {
   const int group = a.query_heads / a.kv_heads;
   const int64_t packed = (int64_t)a.seq_len * group;
-  const int blocks = (int)((packed + PF_ROWS - 1) / PF_ROWS);
-  auto kernel = prefill_mfma_kernel<QN>;
+  const int blocks = (int)((packed + 32 * WAVES - 1) / (32 * WAVES));
+  auto kernel = prefill_mfma_kernel<QN, WAVES>;
+  constexpr size_t lds = pf_lds_bytes<QN, WAVES>();
   static bool attr_set = false;
   if (!attr_set) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)pf_lds_bytes<QN>());
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) {
       (void)hipGetLastError();
       return ckv_internal::set_error(CKV_E_LAUNCH, hipGetErrorString(e));
     }
     attr_set = true;
   }
-  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks * a.kv_heads), dim3(64 * PF_WAVES), pf_lds_bytes<QN>(), s, a, group,
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks * a.kv_heads), dim3(64 * WAVES), lds, s, a, group,
                      blocks);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return ckv_internal::set_error(CKV_E_LAUNCH, hipGetErrorString(e));
   return CKV_OK;
+}
+
+template <int QN>
+int launch_prefill(const ckv_prefill_args& a, hipStream_t s) {
+  const int64_t packed = (int64_t)a.seq_len * (a.query_heads / a.kv_heads);
+  const int64_t workgroups = (packed + 32 * PF_WAVES - 1) / (32 * PF_WAVES) * a.kv_heads;
+  return workgroups <= PF_SHORT_GRID ? launch_rows<QN, PF_SHORT_WAVES>(a, s) : launch_rows<QN, PF_WAVES>(a, s);
 }
 
 }  // namespace

@@ -173,3 +173,20 @@ def test_prefill_config5_coarse_grid_exact_sets(device, kappa):
     rows = np.r_[rng.integers(skip, S, 1000), [skip] * 4, [S - 1] * 4]
     heads = np.r_[rng.integers(0, Hq, 1000), 0, 7, 16, Hq - 1, 0, 9, 22, Hq - 1]
     _check_rows(q, k, v, res, rows, heads, scale=scale, num_sink=sinks, kappa=kappa, exact_sets=True)
+
+
+@pytest.mark.parametrize("S", [511, 512, 513])
+@pytest.mark.parametrize("Hkv", [128, 171])
+def test_prefill_workgroup_sizes(device, S, Hkv):
+    """Grids on both sides of the line between workgroups of four waves and of
+    eight (512 workgroups of 256 rows), with a last row block of one row:
+    sampled rows of a few heads against the oracle."""
+    print(f"prefill workgroup sizes S={S} Hkv={Hkv}", flush=True)
+    q, k, v = _random_qkv(S, 2 * Hkv, Hkv, seed=S + Hkv, device=device)
+    scale = 128 ** -0.5
+    res = prefill_attention_topk(q, k, v, softmax_scale=scale, num_sink=4, kappa=8)
+    torch.cuda.synchronize()
+    pick = np.array([0, 1, 63, 127, 128, 255, 256, S - 2, S - 1])
+    heads = np.array([0, 5, 2 * Hkv - 1])
+    _check_rows(q, k, v, res, np.repeat(pick, heads.size), np.tile(heads, pick.size), scale=scale, num_sink=4, kappa=8,
+                exact_sets=False)

@@ -635,24 +635,35 @@ __global__ void weight_zero_kernel(float* __restrict__ weight, int64_t n, float*
 // one global atomic per touched community, and with 256 rows per workgroup
 // those (2.1 M at 32 heads x 32,751 rows, 512 communities) were most of the
 // launch.  Rows of 8 or 16 edges at 16-byte aligned addresses are read with
-// 16-byte loads.  82 us before at that size, 58 us now (67 MB of edges).
+// 16-byte loads.
+//
+// What bounds it are the LDS atomics: an f32 add takes some three cycles a
+// lane (9.4 M of them: 115,000 of a compute unit's 142,000 cycles), an f64 add
+// half of that.  So the weights gather in doubles up to TOPK_F64_COMMUNITIES,
+// in floats above, where only those fit a workgroup's 64 KB.  67 MB of edges,
+// 512 communities: 82 us at first, 58 us with the shares and loads above, 32 us
+// in doubles.  The whole state build at 512 / 2,000 / 3,900 / 7,500
+// communities: 157 / 169 / 187 / 217 us in floats, 123 / 134 / 151 / 187 in
+// doubles.  (Labels kept in LDS in 16 bits instead of read from L2: 63 us.)
 constexpr int TOPK_THREADS = 256;
 constexpr int TOPK_WORKGROUPS = 1024;
+constexpr int TOPK_F64_COMMUNITIES = 8192;  // 64 KB
 
-template <int VEC>  // 16-byte pieces of a row's edges; 0: any kappa, scalar loads
+template <int VEC, class W>  // VEC: 16-byte pieces of a row's edges (0: any kappa, scalar loads); W: the sums' type
 __global__ __launch_bounds__(TOPK_THREADS) void topk_weight_kernel(
     const int32_t* __restrict__ labels, int seq_len, int capacity, int lds_n, const int32_t* __restrict__ idx,
     const float* __restrict__ sc, int rows, int rows_per_wg, int kappa, int group, int row0, float lam,
     float* __restrict__ weight, float* __restrict__ total) {
   constexpr int K = VEC ? 4 * VEC : 16;
-  extern __shared__ float w_s[];  // communities [0, lds_n)
+  extern __shared__ double topk_lds[];
+  W* w_s = reinterpret_cast<W*>(topk_lds);  // communities [0, lds_n)
   const int h = blockIdx.y;
   const int g = h / group;
-  for (int c = threadIdx.x; c < lds_n; c += TOPK_THREADS) w_s[c] = 0.0f;
+  for (int c = threadIdx.x; c < lds_n; c += TOPK_THREADS) w_s[c] = W(0);
   __syncthreads();
   const int32_t* lab = labels + (int64_t)g * seq_len;
   auto add = [&](int c, float v) {
-    if (c >= 0 && c < lds_n) unsafeAtomicAdd(w_s + c, v);
+    if (c >= 0 && c < lds_n) unsafeAtomicAdd(w_s + c, (W)v);
     else if (c >= lds_n && c < capacity) unsafeAtomicAdd(weight + (int64_t)g * capacity + c, v);
   };
   const float half = 0.5f * lam, co = 1.0f - lam;
@@ -703,7 +714,7 @@ __global__ __launch_bounds__(TOPK_THREADS) void topk_weight_kernel(
   if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = mine;
   __syncthreads();
   for (int c = threadIdx.x; c < lds_n; c += TOPK_THREADS) {
-    const float v = w_s[c];
+    const float v = (float)w_s[c];
     if (v != 0.0f) unsafeAtomicAdd(weight + (int64_t)g * capacity + c, v);
   }
   if (threadIdx.x == 0) {
@@ -824,15 +835,17 @@ extern "C" int ckv_build_layer_state(const ckv_state_build_args* a, void* stream
       const int per_head = std::max(1, TOPK_WORKGROUPS / a->topk_heads);
       const int rows_per_wg = ((a->topk_rows + per_head - 1) / per_head + TOPK_THREADS - 1) / TOPK_THREADS * TOPK_THREADS;
       const dim3 tgrid((a->topk_rows + rows_per_wg - 1) / rows_per_wg, a->topk_heads);
+      const bool f64 = lds_n <= TOPK_F64_COMMUNITIES;
       auto topk = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, tgrid, dim3(TOPK_THREADS), (size_t)lds_n * sizeof(float), s, a->labels, a->seq_len,
+        hipLaunchKernelGGL(kernel, tgrid, dim3(TOPK_THREADS), (size_t)lds_n * (f64 ? 8 : 4), s, a->labels, a->seq_len,
                            a->community_capacity, lds_n, a->topk_indices, a->topk_scores, a->topk_rows, rows_per_wg,
                            a->topk_kappa, a->topk_group, a->topk_row0, a->lam, a->community_weight, a->total_weight);
       };
       const bool aligned = (((uintptr_t)a->topk_indices | (uintptr_t)a->topk_scores) & 15) == 0;
-      if (aligned && a->topk_kappa == 8) topk(topk_weight_kernel<2>);
-      else if (aligned && a->topk_kappa == 16) topk(topk_weight_kernel<4>);
-      else topk(topk_weight_kernel<0>);
+      if (aligned && a->topk_kappa == 8) f64 ? topk(topk_weight_kernel<2, double>) : topk(topk_weight_kernel<2, float>);
+      else if (aligned && a->topk_kappa == 16)
+        f64 ? topk(topk_weight_kernel<4, double>) : topk(topk_weight_kernel<4, float>);
+      else f64 ? topk(topk_weight_kernel<0, double>) : topk(topk_weight_kernel<0, float>);
     }
     if (a->edges > 0) {
       hipLaunchKernelGGL(edge_weight_kernel, dim3((unsigned)((a->edges + EDGES_PER_WG - 1) / EDGES_PER_WG)),

@@ -248,3 +248,35 @@ def test_state_build_weights_from_degrees(device, graphs, seq_len, n):
     with pytest.raises(ValueError, match="edge list"):
         build_layer_state(torch.from_numpy(ids).to(device), keys, retrieval_to_graph=tg, retrieval_to_kv=tg, num_sink=0,
                           max_decode_tokens=4, vertex_degree=torch.from_numpy(degree).to(device))
+
+
+@pytest.mark.parametrize("count,extra", [(8186, 6), (8186, 7)])
+def test_state_build_topk_many_communities(device, count, extra):
+    """Capacities on both sides of the line between sums in doubles and in
+    floats (8,192 communities), against the float64 closed form: some 10 float
+    terms a community, so 1e-5 relative."""
+    from community_kv_amd.graph.kernels.state_build import TopkEdges
+
+    rng = np.random.default_rng(count + extra)
+    seq_len, num_sink, kappa, lam = 9000, 2, 8, 0.5
+    row0 = num_sink + kappa - 1
+    rows = seq_len - row0
+    ids = rng.integers(0, count, (1, seq_len)).astype(np.int32)
+    ids[0, -1] = count - 1
+    idx = rng.integers(-1, seq_len + 1, size=(1, rows, kappa)).astype(np.int32)
+    sc = rng.random((1, rows, kappa)).astype(np.float32)
+    one = torch.zeros(1, dtype=torch.int32, device=device)
+    st = build_layer_state(torch.from_numpy(ids).to(device),
+                           torch.zeros(1, seq_len, 128, dtype=torch.bfloat16, device=device), retrieval_to_graph=one,
+                           retrieval_to_kv=one, num_sink=num_sink, max_decode_tokens=extra,
+                           topk_edges=TopkEdges(indices=torch.from_numpy(idx).to(device),
+                                                scores=torch.from_numpy(sc).to(device), row0=row0, group=1, lam=lam))
+    weight = np.zeros(st.community_weight.shape[1])
+    print(f"state build many communities capacity={weight.size}", flush=True)
+    ok = (idx[0] >= 0) & (idx[0] < seq_len)
+    p = np.where(ok, sc[0], 0.0).astype(np.float64)
+    s, s2 = p.sum(1), (p * p).sum(1)
+    np.add.at(weight, ids[0][np.where(ok, idx[0], 0)], lam / 2 * p + (1 - lam) * p * (s[:, None] + p))
+    np.add.at(weight, ids[0][row0:], lam / 2 * s)
+    np.testing.assert_allclose(st.community_weight.cpu().numpy()[0], weight, rtol=1e-5, atol=1e-5)
+    np.testing.assert_allclose(st.total_weight.cpu().numpy()[0], (lam * s + (1 - lam) * (s * s + s2)).sum(), rtol=1e-5)

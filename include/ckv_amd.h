@@ -3,10 +3,10 @@
  * (libckv_amd.so, built from community_kv_amd/csrc/).
  *
  * Every entry point takes plain device pointers and sizes, never allocates,
- * never synchronises the host, runs on the HIP stream it is given, and returns
- * 0 on success or a nonzero CKV_E* code with a message readable through
- * ckv_last_error().  Tensors are dense row-major; the only strides are those
- * of the KV cache.
+ * never synchronises the host (ckv_batch_prepare and ckv_leiden_run do, and say
+ * so), runs on the HIP stream it is given, and returns 0 on success or a
+ * nonzero CKV_E* code with a message readable through ckv_last_error().
+ * Tensors are dense row-major; the only strides are those of the KV cache.
  *
  * Reference interfaces replaced (paths relative to the reference repository):
  *   ckv_score_select        score_and_select()                attention/kernels/centroid_selection.py:537-556
@@ -34,6 +34,8 @@
  *   ckv_batched_leiden      batched_leiden() of the Leiden extension (graph/leiden/_csrc/bindings.cpp:40-103,
  *                           launch_batched_leiden in leiden.cu:43-205), called by run_leiden()
  *                           (graph/leiden/algorithm.py:51-161)
+ *   ckv_leiden_run          run_leiden() (graph/leiden/algorithm.py:51-161), every level in one call
+ *   ckv_dense_communities   the dense relabelling after it (graph/partition.py:252-286)
  *   ckv_aggregate_coo       aggregate_coo() of the same extension (bindings.cpp:118-170,
  *                           aggregate_upper_coo in aggregate.cu:88-184)
  *   ckv_densify_count,      _densify_per_graph() (graph/leiden/algorithm.py:30-48), as two calls

@@ -66,9 +66,9 @@ constexpr int ETHREADS = 256;
 // Control words of a level.  A sweep in which a vertex moves marks its slot of
 // its phase's ring; the next sweeps read the ring themselves, so no kernel runs
 // between sweeps to advance a state.  A slot is a word per XCD, each in a line
-// of its own: with a mark per moved vertex on one word a first sweep of 57,000
-// vertices took 64 us, 31 now.  Every RING sweeps fold_kernel moves the ring's
-// outcome to the base words.
+// of its own: with a mark per moved vertex on one word the first local-moving
+// sweeps of 32 8k graphs' levels averaged 64 us, 31 now.  Every RING sweeps
+// fold_kernel moves the ring's outcome to the base words.
 constexpr int RING = 16;
 constexpr int MARK_STRIDE = 32;              // words from one XCD's mark to the next
 constexpr int SLOT_WORDS = 8 * MARK_STRIDE;  // a sweep's slot
@@ -86,13 +86,8 @@ __device__ __host__ inline uint32_t pcg_hash(uint32_t x) {
   const uint32_t word = ((state >> ((state >> 28u) + 4u)) ^ state) * 277803737u;
   return (word >> 22u) ^ word;
 }
-__device__ inline uint32_t mix4(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
-  uint32_t h = pcg_hash(a);
-  h = pcg_hash(h ^ b);
-  h = pcg_hash(h ^ c);
-  return pcg_hash(h ^ d);
-}
-// mix4 of a salt = pcg_hash(pcg_hash(graph) ^ vertex) kept per vertex.
+// The reference's hash of (graph, vertex, c, d), each folded in by pcg_hash(h ^ x);
+// the first two are the vertex's salt.
 __device__ inline uint32_t salt_of(uint32_t g, uint32_t v) { return pcg_hash(pcg_hash(g) ^ v); }
 __device__ inline uint32_t mix_salt(uint32_t salt, uint32_t c, uint32_t d) { return pcg_hash(pcg_hash(salt ^ c) ^ d); }
 __device__ inline float unit_float(uint32_t h) { return (float)(h >> 8) * (1.0f / 16777216.0f); }
@@ -361,7 +356,8 @@ constexpr int GIANT_MIN = TABLE_CAP;  // rows longer than this take a workgroup 
 constexpr int GIANT_SLOTS = 4096;
 constexpr int GIANT_THREADS = 1024;
 constexpr int GIANT_BLOCKS = 512;  // two 65 KB workgroups per CU
-static_assert(SMALL_ROW == 32 * ROW_PER && MID_ROW == 64 * ROW_PER && GIANT_MIN == HUB_THREADS * ROW_PER, "rows fit their threads' registers");
+static_assert(SMALL_ROW == 32 * ROW_PER && MID_ROW == 64 * ROW_PER && GIANT_MIN == HUB_THREADS * ROW_PER,
+              "rows fit their threads' registers");
 
 // The rows longer than SMALL_ROW: mids (a wave each) from the front of `rows`,
 // hubs (a workgroup each) from its back, giants in a list of their own.
@@ -747,7 +743,8 @@ __device__ __forceinline__ bool move_vertex(const P& p, const Graph& gr, const M
 // Below two chunks a workgroup the long rows take LONG_BLOCKS workgroups of
 // their own in the same launch (all sweeps of eight 2k graphs, 2,000 chunks:
 // 577 us against 669 with every workgroup taking both); above, all workgroups
-// share both (57,000 vertices, 7,100 chunks: 1,885 us against 1,964).
+// share both (32 8k graphs, whose levels have 32,800 down to 7,100 chunks: all
+// sweeps 1,885 us with the line here, 1,964 with it at 16,384 chunks).
 struct Share {
   int32_t at, end, step;
 };
@@ -2461,8 +2458,8 @@ namespace {
 
 struct RunLayout {
   size_t row_ptr, col0, wt0, col[2], wt[2], beg[2], end[2], k[2], two_m, two_m0, totals[4], lab, moves[2], pairs[2], prop,
-      mover, salt, scale, ctl, hubs, giants, counts, flags, scan, dense, hist, first, members, dense_list, lists, words, temp,
-      temp_bytes, sort, total;
+      mover, salt, scale, ctl, hubs, giants, counts, flags, scan, dense, hist, first, members, dense_list,
+      lists, words, temp, temp_bytes, sort, total;
 };
 
 // Sorting scratch and the rows of the contracted levels share their place (the
@@ -2668,7 +2665,8 @@ extern "C" int ckv_leiden_run(const int32_t* edge_src, const int32_t* edge_dst, 
   const unsigned egrid = blocks(V0, ETHREADS);
   sigma_zero_kernel<<<egrid, ETHREADS, 0, st>>>(f64(L.totals[0]), V0);
   sigma_scatter_kernel<<<egrid, ETHREADS, 0, st>>>(labels, degree, V0, f64(L.totals[0]));
-  inside_kernel<<<blocks(V0, LWAVES), LTHREADS, 0, st>>>(gr0, labels, f64(L.totals[0]), f64(L.totals[1]), f64(L.totals[2]));
+  inside_kernel<<<blocks(V0, LWAVES), LTHREADS, 0, st>>>(gr0, labels, f64(L.totals[0]), f64(L.totals[1]),
+                                                         f64(L.totals[2]));
   double* sums = f64(L.k[0]);  // per graph: inside, square; then the result
   double* squares = f64(L.k[1]);
   graph_sum_kernel<<<graphs, SUM_THREADS, 0, st>>>(f64(L.totals[1]), seq_len, sums);

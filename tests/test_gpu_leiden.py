@@ -402,3 +402,19 @@ def test_sweep_row_classes(device, seed, rows, S, loops, sweeps, ordered):
     general = general[vertex.cpu().numpy()]
     pairs = np.unique(np.stack([general, part.cpu().numpy()]), axis=1).shape[1]
     assert pairs == np.unique(general).size == np.unique(part.cpu().numpy()).size
+
+
+def test_run_leiden_ranks_on_both_paths(device):
+    """Labels are ranked by a bitmap in LDS up to 262,144 vertices a graph and by
+    a scan above: one vertex without edges more gives the same communities."""
+    rng = np.random.default_rng(9)
+    S = 1 << 18
+    v = rng.choice(S, 3000, replace=False).astype(np.int64)
+    a, b = v[rng.integers(0, v.size, 12000)], v[rng.integers(0, v.size, 12000)]
+    key = np.unique(np.minimum(a, b)[a != b] * (S + 1) + np.maximum(a, b)[a != b])
+    w = (rng.integers(1, 64, key.size) / 64.0).astype(np.float32)
+    s, d, x = _dev(device, (key // (S + 1)).astype(np.int32), (key % (S + 1)).astype(np.int32), w)
+    print(f"leiden ranks edges={key.size}", flush=True)
+    got = [algorithm.run_leiden(s, d, x, G=1, seq_len=n, max_level=3, max_inner_iter=3, seed=2) for n in (S, S + 1)]
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    assert got[0][2] == pytest.approx(got[1][2], abs=1e-12)

@@ -512,7 +512,7 @@ __global__ __launch_bounds__(EDGE_THREADS) void edge_weight_kernel(
 // their communities, so a community weighs the sum of its members' degrees.
 // 262,144 degrees in place of 9.8 M edges with two label reads and LDS adds
 // each: 488 us (8 graphs of 32,768, 13,000 communities) and 1,434 us (32 of
-// 8,192) in edge_weight_kernel, 150 us with the totals here.
+// 8,192) in edge_weight_kernel, 110 us with the totals here.
 constexpr int DEGREE_THREADS = 256;
 
 __global__ __launch_bounds__(DEGREE_THREADS) void degree_weight_kernel(
@@ -534,18 +534,58 @@ __global__ __launch_bounds__(DEGREE_THREADS) void degree_weight_kernel(
 // totals of 10^5 depend on that order by up to 3e-5 (a single edge is smaller
 // than half their last bit), so it is kept, with the single edges added in a
 // register: one wave per graph, before and after the blocks (within 7e-6 of
-// the atomics on 4,000 to 32,768 positions, 2 to 32 graphs; 140 us in all at
-// 9.8 M edges).
+// the atomics on 4,000 to 32,768 positions, 2 to 32 graphs; 100 us in all at
+// 9.8 M edges: the look 14, a wave's 4,096 additions 25 twice, the blocks 36).
+//
+// That needs a list grouped by ascending graph with every source in a graph.
+// edge_order_kernel looks; of any other list the totals add up edge by edge,
+// sources outside the graphs left out.  Each of its workgroups leaves its
+// finding in a word of the weights, which are cleared afterwards: no word
+// needs clearing before it and the entry needs no workspace.
 constexpr int REST_EARLY_PER_GRAPH = 192, REST_EARLY_MOST = 4096;
+constexpr int ORDER_MOST = 1024;  // words a workgroup reads to know what was found
+
+__global__ __launch_bounds__(EDGE_THREADS) void edge_order_kernel(const int32_t* __restrict__ src, int64_t edges,
+                                                                  int seq_len, int64_t vertices, int* __restrict__ found) {
+  constexpr int U = 8;
+  const int64_t step = (int64_t)gridDim.x * EDGE_THREADS;
+  bool loose = false;
+  for (int64_t e0 = (int64_t)blockIdx.x * EDGE_THREADS + threadIdx.x; e0 < edges; e0 += U * step) {
+    int a[U], b[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t e = min(e0 + u * step, edges - 1);
+      b[u] = gload_i32(src + e);
+      a[u] = gload_i32(src + (e > 0 ? e - 1 : 0));
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      loose = loose || b[u] < 0 || b[u] >= vertices || (a[u] > b[u] && a[u] / seq_len > b[u] / seq_len);
+  }
+  const int any = __syncthreads_or(loose ? 1 : 0);
+  if (threadIdx.x == 0) found[blockIdx.x] = any ? 1 : 0;
+}
+
+// Whether any of the n words holds a finding (every thread of the workgroup calls).
+__device__ inline bool any_found(const int* __restrict__ found, int n) {
+  int mine = 0;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < n; i += blockDim.x) mine |= found[i];
+  return __syncthreads_or(mine) != 0;
+}
 
 __global__ __launch_bounds__(EDGE_THREADS) void edge_total_kernel(const int32_t* __restrict__ src,
                                                                   const float* __restrict__ w, int64_t edges,
-                                                                  int seq_len, float* __restrict__ total) {
+                                                                  int seq_len, int graphs,
+                                                                  const int* __restrict__ found, int founds,
+                                                                  float* __restrict__ total) {
   constexpr int U = 8;
   const int64_t e0 = (int64_t)blockIdx.x * EDGES_PER_WG;
   const int64_t e1 = min(edges, e0 + EDGES_PER_WG);
+  const bool loose = any_found(found, founds);
   const int g0 = src[e0] / seq_len;
-  const bool whole = src[e1 - 1] / seq_len == g0;  // (the list is grouped by graph)
+  const bool whole = !loose && src[e1 - 1] / seq_len == g0;
+  const bool g0_ok = !loose || (src[e0] >= 0 && g0 < graphs);
   float mine = 0.0f;
   for (int64_t b = e0 + threadIdx.x; b < e1; b += U * EDGE_THREADS) {
     float x[U];
@@ -553,7 +593,13 @@ __global__ __launch_bounds__(EDGE_THREADS) void edge_total_kernel(const int32_t*
     for (int u = 0; u < U; ++u) {
       const int64_t e = min(b + u * EDGE_THREADS, e1 - 1);
       x[u] = gload_f32(w + e);
-      if (!whole && src[e] / seq_len != g0) x[u] = 0.0f;
+      if (!whole) {
+        const int s = src[e];
+        const int g = s / seq_len;
+        if (loose && s >= 0 && g < graphs && (g != g0 || !g0_ok) && b + u * EDGE_THREADS < e1)
+          unsafeAtomicAdd(total + g, 2.0f * x[u]);
+        if (s < 0 || g != g0) x[u] = 0.0f;
+      }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -564,39 +610,65 @@ __global__ __launch_bounds__(EDGE_THREADS) void edge_total_kernel(const int32_t*
   mine = wave_sum_tree(mine);
   if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = mine;
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (threadIdx.x == 0 && g0_ok) {
     float t = 0.0f;
     for (int i = 0; i < EDGE_THREADS / 64; ++i) t = t + s_part[i];
     unsafeAtomicAdd(total + g0, t);
   }
 }
 
-// t plus the edges [e0, last) of graph g in order, up to the graph's end.
+// t plus the edges [e0, last) of graph g in order, up to the graph's end.  The
+// next 64 edges are on their way while these are added, from LDS four a read:
+// the additions wait for each other alone.
 __device__ inline float add_edges(const int32_t* __restrict__ src, const float* __restrict__ w, int64_t e0,
                                   int64_t last, int g, int seq_len, float t) {
+  __shared__ __align__(16) float x_s[64];
   const int lane = lane_id();
+  if (e0 >= last) return t;
+  float x = gload_f32(w + min(e0 + lane, last - 1));
+  int s = gload_i32(src + min(e0 + lane, last - 1));
   for (; e0 < last; e0 += 64) {
-    const int64_t e = min(e0 + lane, last - 1);
-    const float x = 2.0f * w[e];
-    const int n = __popcll(__ballot(e0 + lane < last && src[e] / seq_len == g));
+    const int64_t next = min(e0 + 64 + lane, last - 1);
+    const float xn = gload_f32(w + next);
+    const int sn = gload_i32(src + next);
+    const int n = __popcll(__ballot(e0 + lane < last && s / seq_len == g));
+    wave_sync();  // (the reads before are done)
+    x_s[lane] = 2.0f * x;
+    wave_sync();
     if (n == 64) {
+      float4 y[16];
 #pragma unroll
-      for (int i = 0; i < 64; ++i) t = t + ckv_u2f((uint32_t)__builtin_amdgcn_readlane((int)ckv_f2u(x), i));
+      for (int i = 0; i < 16; ++i) y[i] = reinterpret_cast<const float4*>(x_s)[i];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        t = t + y[i].x;
+        t = t + y[i].y;
+        t = t + y[i].z;
+        t = t + y[i].w;
+      }
     } else {
-      for (int i = 0; i < n; ++i) t = t + ckv_u2f((uint32_t)__builtin_amdgcn_readlane((int)ckv_f2u(x), i));
+      for (int i = 0; i < n; ++i) t = t + x_s[i];
       break;
     }
+    x = xn;
+    s = sn;
   }
   return t;
 }
 
 // One wave per graph: its edges that lie in an earlier graph's block, the
-// first `early` of them into a cleared total (late == 0) or the others.
+// first `early` of them into a cleared total (late == 0) or the others; of a
+// list in another order the cleared total alone.
 __global__ __launch_bounds__(64) void edge_rest_kernel(const int32_t* __restrict__ src, const float* __restrict__ w,
                                                        int64_t edges, int seq_len, int early, int late,
+                                                       const int* __restrict__ found, int founds,
                                                        float* __restrict__ total) {
   const int g = blockIdx.x;
   const int lane = threadIdx.x;
+  if (any_found(found, founds)) {
+    if (!late && lane == 0) total[g] = 0.0f;
+    return;
+  }
   const int64_t v0 = (int64_t)g * seq_len;
   // the first edge of this graph or a later one, 64 probes a round
   int64_t lo = 0, hi = edges;
@@ -618,7 +690,7 @@ __global__ __launch_bounds__(64) void edge_rest_kernel(const int32_t* __restrict
 __global__ void weight_zero_kernel(float* __restrict__ weight, int64_t n, float* __restrict__ total, int graphs) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) weight[i] = 0.0f;
-  if (i < graphs) total[i] = 0.0f;
+  if (total != nullptr && i < graphs) total[i] = 0.0f;
 }
 
 // Modularity weights straight from the prefill top-k edges: one thread per
@@ -866,19 +938,26 @@ extern "C" int ckv_degree_weights(const int32_t* labels, const double* degree, c
     return ckv_internal::set_error(CKV_E_INVALID, "graphs, seq_len and community_capacity must be positive");
   const hipStream_t s = (hipStream_t)stream;
   const int64_t n = (int64_t)graphs * community_capacity, v = (int64_t)graphs * seq_len;
-  hipLaunchKernelGGL(weight_zero_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, community_weight, n,
-                     total_weight, graphs);
+  if (edges > 0) {
+    const int early = std::min(REST_EARLY_MOST, REST_EARLY_PER_GRAPH * graphs);
+    const int64_t passes = (edges + 8 * EDGE_THREADS - 1) / (8 * EDGE_THREADS);
+    const int founds = (int)std::min<int64_t>(std::min<int64_t>(passes, ORDER_MOST), n);
+    int* found = reinterpret_cast<int*>(community_weight);
+    hipLaunchKernelGGL(edge_order_kernel, dim3(founds), dim3(EDGE_THREADS), 0, s, edge_src, edges, seq_len, v,
+                       found);
+    hipLaunchKernelGGL(edge_rest_kernel, dim3(graphs), dim3(64), 0, s, edge_src, edge_weight, edges, seq_len, early, 0,
+                       (const int*)found, founds, total_weight);
+    hipLaunchKernelGGL(edge_total_kernel, dim3((unsigned)((edges + EDGES_PER_WG - 1) / EDGES_PER_WG)),
+                       dim3(EDGE_THREADS), 0, s, edge_src, edge_weight, edges, seq_len, graphs, (const int*)found,
+                       founds, total_weight);
+    hipLaunchKernelGGL(edge_rest_kernel, dim3(graphs), dim3(64), 0, s, edge_src, edge_weight, edges, seq_len, early, 1,
+                       (const int*)found, founds, total_weight);
+  }
+  const int64_t clear = edges > 0 ? n : std::max<int64_t>(n, graphs);
+  hipLaunchKernelGGL(weight_zero_kernel, dim3((unsigned)((clear + 255) / 256)), dim3(256), 0, s, community_weight, n,
+                     edges > 0 ? nullptr : total_weight, graphs);
   hipLaunchKernelGGL(degree_weight_kernel, dim3((unsigned)((v + DEGREE_THREADS - 1) / DEGREE_THREADS)),
                      dim3(DEGREE_THREADS), 0, s, labels, degree, seq_len, graphs, community_capacity,
                      community_weight);
-  if (edges > 0) {
-    const int early = std::min(REST_EARLY_MOST, REST_EARLY_PER_GRAPH * graphs);
-    hipLaunchKernelGGL(edge_rest_kernel, dim3(graphs), dim3(64), 0, s, edge_src, edge_weight, edges, seq_len, early, 0,
-                       total_weight);
-    hipLaunchKernelGGL(edge_total_kernel, dim3((unsigned)((edges + EDGES_PER_WG - 1) / EDGES_PER_WG)),
-                       dim3(EDGE_THREADS), 0, s, edge_src, edge_weight, edges, seq_len, total_weight);
-    hipLaunchKernelGGL(edge_rest_kernel, dim3(graphs), dim3(64), 0, s, edge_src, edge_weight, edges, seq_len, early, 1,
-                       total_weight);
-  }
   return launch_check();
 }

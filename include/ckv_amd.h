@@ -308,7 +308,10 @@ int ckv_build_layer_state(const ckv_state_build_args* args, void* stream);
  * [graphs][seq_len], as ckv_leiden_run leaves them): community_weight[g][c] =
  * degrees of the positions labelled c (labels outside
  * [0, community_capacity) are dropped), total_weight[g] = twice the weight of
- * the graph's edges (the coalesced list that the degrees belong to). */
+ * the graph's edges (the coalesced list that the degrees belong to, in any
+ * order; edges whose source lies outside the graphs are left out.  A list
+ * grouped by ascending graph, as ckv_build_adjacency leaves it, is added up by
+ * blocks, any other edge by edge). */
 int ckv_degree_weights(const int32_t* labels, const double* degree, const int32_t* edge_src, const float* edge_weight,
                        int64_t edges, int32_t graphs, int32_t seq_len, int32_t community_capacity,
                        float* community_weight, float* total_weight, void* stream);

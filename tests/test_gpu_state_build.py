@@ -250,6 +250,41 @@ def test_state_build_weights_from_degrees(device, graphs, seq_len, n):
                           max_decode_tokens=4, vertex_degree=torch.from_numpy(degree).to(device))
 
 
+@pytest.mark.parametrize("order", ["shuffled", "descending", "rotated", "outside"])
+@pytest.mark.parametrize("graphs,seq_len,n", [(3, 1000, 5000), (2, 4000, 40000), (1, 300, 8193)])
+def test_state_build_degree_weights_any_edge_order(device, graphs, seq_len, n, order):
+    """Totals beside given degrees do not depend on the order of the edge list
+    (shuffled, graphs descending, graphs in blocks of their own but rotated),
+    and edges whose source lies outside the graphs are left out of them (dyadic
+    weights, sums below 2^12: exact)."""
+    rng = np.random.default_rng(n + graphs)
+    ids = rng.integers(0, 50, (graphs, seq_len)).astype(np.int32)
+    src, dst, _ = _edges(rng, graphs, seq_len, 0, n)
+    w = (rng.integers(1, 64, n) / 4096.0).astype(np.float32)
+    V = graphs * seq_len
+    if order == "outside":
+        src[:: 7] = rng.choice([-1, -seq_len, -2**31, V, V + seq_len, 2**31 - 1], src[::7].size)
+        src[0] = V
+    else:
+        at = {"shuffled": rng.permutation(n), "descending": np.arange(n)[::-1],
+              "rotated": np.roll(np.arange(n), n // 2)}[order]
+        src, dst, w = src[at].copy(), dst[at].copy(), w[at].copy()
+    ok = (src >= 0) & (src < V)
+    degree = (np.bincount(src[ok], weights=w[ok], minlength=V) + np.bincount(dst[ok], weights=w[ok], minlength=V))
+    tg = torch.arange(graphs, dtype=torch.int32, device=device)
+    print(f"state build degrees {order} graphs={graphs} S={seq_len} edges={n}", flush=True)
+    st = build_layer_state(torch.from_numpy(ids).to(device),
+                           torch.zeros(graphs, seq_len, 128, dtype=torch.bfloat16, device=device),
+                           retrieval_to_graph=tg, retrieval_to_kv=tg, num_sink=0, max_decode_tokens=4,
+                           edges=tuple(torch.from_numpy(e).to(device) for e in (src, dst, w)),
+                           vertex_degree=torch.from_numpy(degree).to(device))
+    np.testing.assert_array_equal(st.total_weight.cpu().numpy(),
+                                  np.bincount(src[ok] // seq_len, weights=2.0 * w[ok], minlength=graphs))
+    by_label = np.stack([np.bincount(ids[g], weights=degree.reshape(graphs, seq_len)[g],
+                                     minlength=st.community_weight.shape[1]) for g in range(graphs)])
+    np.testing.assert_array_equal(st.community_weight.cpu().numpy(), by_label)
+
+
 @pytest.mark.parametrize("count,extra", [(8186, 6), (8186, 7)])
 def test_state_build_topk_many_communities(device, count, extra):
     """Capacities on both sides of the line between sums in doubles and in

@@ -41,14 +41,21 @@ constexpr int D = CKV_HEAD_DIM;
 // Waves per workgroup, 32 packed (position, head) rows each.  A workgroup has a
 // compute unit to itself (LDS), so a short prompt lasts as long as its last row
 // block's chain of tiles: with PF_SHORT_WAVES the chain's tiles take less and
-// twice as many workgroups share the work.  Up to PF_SHORT_GRID workgroups of
-// PF_WAVES (two a compute unit; 32 query heads over 8 KV heads: 4,096 positions)
-// that is faster, above it the tiles staged for half the rows cost more:
-// 500 / 1,000 / 2,000 / 4,000 positions 53 / 93 / 200 / 339 us with eight waves
-// and 48 / 89 / 169 / 319 with four, 6,000 positions 509 and 616.
+// twice as many workgroups share the work.  That holds while nearly all of
+// those find a compute unit at once: up to PF_SHORT_GRID workgroups of PF_WAVES
+// (two thirds of the compute units; the shorter row blocks of the rest follow
+// the first ones that end), and while the chain is short, up to PF_SHORT_SEQ
+// positions.  Measured with eight and with four waves, kappa 8, us: 32 query
+// heads over 8 KV heads, 320 / 768 / 1,024 / 1,280 / 1,408 / 1,600 / 2,048 /
+// 4,096 positions (40 to 512 workgroups) 30 / 46 / 59 / 64 / 72 / 71 / 94 / 185
+// and 27 / 44 / 58 / 60 / 71 / 82 / 108 / 320; 64 over 8, 704 / 800 / 1,024
+// (176, 200, 256) 48 / 55 / 62 and 45 / 54 / 66; 16 over 8, 2,816 / 3,200 (176,
+// 200) 107 / 114 and 104 / 119; 8 over 2, 2,048 / 3,200 / 4,608 (64, 100, 144)
+// 84 / 114 / 145 and 83 / 118 / 149.  (Odd lengths and kappa 16: the same lines.)
 constexpr int PF_WAVES = 8;
 constexpr int PF_SHORT_WAVES = 4;
-constexpr int PF_SHORT_GRID = 512;
+constexpr int PF_SHORT_GRID = 176;
+constexpr int PF_SHORT_SEQ = 3072;
 constexpr int PF_KEYS = 64;             // keys per LDS tile
 constexpr int K_STRIDE = D + 8;         // 272-byte (17-chunk) K rows: 16-lane b128 reads hit distinct banks
 constexpr int V_STRIDE = D + 32;        // 320-byte (20-chunk) V rows: transposed b64 reads hit distinct banks
@@ -254,8 +261,11 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void prefill_mfma_kernel(ckv
   uint32_t row_thr = 0u;  // a lower bound of the row's QN-th best key (both halves)
   // Candidate filter: prefilter(max(own worst kept key, the other half's,
   // row_thr)).  It changes only when the queues do, so it is recomputed there
-  // instead of on every tile.
-  float tf = -FLT_MAX;
+  // instead of on every tile.  Rows past the prompt (the last block of an odd
+  // length) take no candidates: their scores are all zero, so every column
+  // would tie with the filter and be appended, in the block with the most
+  // tiles (8 heads over 2, 4,059 positions: 317 us so, 134 without).
+  float tf = row_ok ? -FLT_MAX : -NEG_INF;
   float m = NEG_INF;  // reference max of the raw score (scale > 0)
   float l = 0.0f;     // this half's share of the softmax denominator
 
@@ -293,7 +303,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void prefill_mfma_kernel(ckv
 #pragma unroll
     for (int i = 0; i < QN; ++i) rt = min(rt, max(qk[i], swap32_u32(qk[QN - 1 - i])));
     row_thr = rt;
-    tf = prefilter(max(max(q_min, swap32_u32(q_min)), row_thr));
+    tf = row_ok ? prefilter(max(max(q_min, swap32_u32(q_min)), row_thr)) : -NEG_INF;
   };
 
   // S^T (keys x rows) of the tile staged in `stage`: accumulator b holds keys
@@ -544,7 +554,8 @@ template <int QN>
 int launch_prefill(const ckv_prefill_args& a, hipStream_t s) {
   const int64_t packed = (int64_t)a.seq_len * (a.query_heads / a.kv_heads);
   const int64_t workgroups = (packed + 32 * PF_WAVES - 1) / (32 * PF_WAVES) * a.kv_heads;
-  return workgroups <= PF_SHORT_GRID ? launch_rows<QN, PF_SHORT_WAVES>(a, s) : launch_rows<QN, PF_WAVES>(a, s);
+  return workgroups <= PF_SHORT_GRID && a.seq_len <= PF_SHORT_SEQ ? launch_rows<QN, PF_SHORT_WAVES>(a, s)
+                                                                  : launch_rows<QN, PF_WAVES>(a, s);
 }
 
 }  // namespace

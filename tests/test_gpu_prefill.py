@@ -175,12 +175,13 @@ def test_prefill_config5_coarse_grid_exact_sets(device, kappa):
     _check_rows(q, k, v, res, rows, heads, scale=scale, num_sink=sinks, kappa=kappa, exact_sets=True)
 
 
-@pytest.mark.parametrize("S", [511, 512, 513])
-@pytest.mark.parametrize("Hkv", [128, 171])
+@pytest.mark.parametrize("S,Hkv", [(S, Hkv) for S in (511, 512, 513) for Hkv in (44, 45, 128, 171)]
+                         + [(3071, 3), (3072, 3), (3073, 3)])
 def test_prefill_workgroup_sizes(device, S, Hkv):
-    """Grids on both sides of the line between workgroups of four waves and of
-    eight (512 workgroups of 256 rows), with a last row block of one row:
-    sampled rows of a few heads against the oracle."""
+    """Both sides of the lines between workgroups of four waves and of eight
+    (176 workgroups of 256 rows: 44 KV heads of 512 positions; 3,072
+    positions), with last row blocks of one row and of all but one: sampled
+    rows of a few heads against the oracle."""
     print(f"prefill workgroup sizes S={S} Hkv={Hkv}", flush=True)
     q, k, v = _random_qkv(S, 2 * Hkv, Hkv, seed=S + Hkv, device=device)
     scale = 128 ** -0.5
@@ -190,3 +191,35 @@ def test_prefill_workgroup_sizes(device, S, Hkv):
     heads = np.array([0, 5, 2 * Hkv - 1])
     _check_rows(q, k, v, res, np.repeat(pick, heads.size), np.tile(heads, pick.size), scale=scale, num_sink=4, kappa=8,
                 exact_sets=False)
+
+
+def _best_us(f, runs=20):
+    """The fastest of `runs` calls on the GPU's clock."""
+    for _ in range(3):
+        f()
+    best = float("inf")
+    for _ in range(runs):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        f()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3)
+    return best
+
+
+def test_prefill_odd_lengths_keep_pace(device):
+    """Rows past the prompt cost no selection (their scores all tie: appending
+    every column made 4,059 positions 2.2 times as slow as 4,096), and twice
+    the positions on a grid that fills the chip take about twice the time
+    (three times where eight waves' work went to four)."""
+    def us(S, Hq, Hkv):
+        q, k, v = _random_qkv(S, Hq, Hkv, seed=S, device=device)
+        return _best_us(lambda: prefill_attention_topk(q, k, v, softmax_scale=128 ** -0.5, num_sink=10, kappa=8))
+
+    odd, even = us(4059, 8, 2), us(4096, 8, 2)
+    print(f"prefill 4,059 / 4,096 positions {odd:.0f} / {even:.0f} us", flush=True)
+    assert odd < 1.5 * even
+    once, twice = us(2048, 32, 8), us(4096, 32, 8)
+    print(f"prefill 2,048 / 4,096 positions {once:.0f} / {twice:.0f} us", flush=True)
+    assert twice < 2.5 * once

@@ -7,6 +7,8 @@ gains within an ulp)."""
 
 from __future__ import annotations
 
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -418,3 +420,54 @@ def test_run_leiden_ranks_on_both_paths(device):
     got = [algorithm.run_leiden(s, d, x, G=1, seq_len=n, max_level=3, max_inner_iter=3, seed=2) for n in (S, S + 1)]
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
     assert got[0][2] == pytest.approx(got[1][2], abs=1e-12)
+
+
+@pytest.mark.parametrize("at", ["front", "middle", "back", "spread"])
+def test_run_leiden_sparse_edge_lists(device, at):
+    """Vertices without edges before, between and behind those with edges, in
+    gaps on both sides of the length that one thread fills, in one graph of
+    three: labels equal the oracle's (dyadic weights: every sum exact)."""
+    rng = np.random.default_rng(len(at))
+    G, S, n = 3, 5000, 240
+    if at == "spread":
+        live = np.cumsum(np.concatenate([[0], np.tile([1, 2, 15, 16, 17, 18, 33, 64], 30)]))[:n]
+    else:
+        live = np.arange(n) + {"front": 0, "middle": 2300, "back": S - n}[at]
+    graph = {"front": 0, "middle": 1, "back": 2, "spread": 1}[at]
+    a, b = live[rng.integers(0, n, 900)], live[rng.integers(0, n, 900)]
+    key = np.unique((np.minimum(a, b) * S + np.maximum(a, b)))
+    src, dst = (key // S + graph * S).astype(np.int32), (key % S + graph * S).astype(np.int32)
+    w = (rng.integers(1, 64, key.size) / 64.0).astype(np.float32)
+    s, d, x = _dev(device, src, dst, w)
+    print(f"leiden sparse {at} edges={key.size}", flush=True)
+    vertex, part, q = algorithm.run_leiden(s, d, x, G=G, seq_len=S, max_inner_iter=4, seed=1)
+    rv, rp, rq = L.run_leiden(src, dst, w, graphs=G, seq_len=S, max_inner_iter=4, seed=1)
+    np.testing.assert_array_equal(vertex.cpu().numpy(), rv)
+    np.testing.assert_array_equal(part.cpu().numpy(), rp)
+    assert q == pytest.approx(rq, abs=1e-9)
+
+
+def test_run_leiden_graphs_without_edges_cost_little(device):
+    """Edges in the last of 32 graphs of 32,768 vertices: the run takes at most
+    a few times as long as on that graph alone (what a vertex without edges
+    costs; one thread that fills the others' row starts made it 60 times)."""
+    rng = np.random.default_rng(2)
+    G, S = 32, 32768
+    a = rng.integers(0, S - 200, 100000)
+    key = np.unique(a * S + a + rng.integers(1, 200, a.size))
+    w = torch.from_numpy((rng.integers(1, 64, key.size) / 64.0).astype(np.float32)).to(device)
+
+    def best_us(graphs):
+        off = (graphs - 1) * S
+        s, d = _dev(device, (key // S + off).astype(np.int32), (key % S + off).astype(np.int32))
+        best = float("inf")
+        for _ in range(6):
+            t0 = time.perf_counter()
+            algorithm.run_leiden(s, d, w, G=graphs, seq_len=S, max_inner_iter=4)
+            torch.cuda.synchronize()
+            best = min(best, (time.perf_counter() - t0) * 1e6)
+        return best
+
+    alone, among = best_us(1), best_us(G)
+    print(f"leiden one graph {alone:.0f} us, among {G} {among:.0f} us", flush=True)
+    assert among < 8.0 * alone

@@ -20,9 +20,21 @@
 //                     windows of consecutive ids summed in a dense LDS array
 //   scan + emit_kernel   edges to their places in the output
 //
-// The sums are f64 sums of the f32 entry weights, rounded once.
+// Rows of few entries (those without co-occurrence edges, lam = 1, and of one
+// column) are written out and sorted by pair all the same: there a posting,
+// which looks at all columns of its row, stands for one entry or two.
 //
-// Measured at that size (9.8 M edges out): 2.9 ms for the expansion, the
+//   expand_kernel     the entries, 64-bit keys (min, max)
+//   radix sort, reduce_by_key, unpack_kernel
+//
+// 32 x 32,751 rows without co-occurrence edges, 8 and 16 columns: 1,080 and
+// 3,850 us by postings, 730 and 1,280 so; 32 x 4,023 rows of 64: 2,030 and 630;
+// 32 x 32,758 of one column with them 500 and 345; of two: 500 by postings, 530
+// sorted.  By postings they also took scratch for kappa + 1 edges a posting.
+//
+// The sums are f64 sums of the f32 entry weights, rounded once, on both ways.
+//
+// Measured on 32 x 32,751 rows of 8 (9.8 M edges out): 2.9 ms for the expansion, the
 // 64-bit radix sort of its 46.9 M entries and their reduction before,
 // 1.2 ms so.  What bounds it now: the random reads of the rows (32 bytes
 // of columns and of scores per posting, from L2 and the Infinity Cache) and
@@ -65,7 +77,6 @@ struct TopkGraph {
   int32_t G, R, K, S;
   int shift;             // bits of a posting below its row
   float half_lam, co_lam;
-  int co;                // co-occurrence edges (lam < 1)
 };
 
 // Postings [first, last) of one vertex.
@@ -152,10 +163,10 @@ __device__ __forceinline__ Candidate candidate(const TopkGraph& t, uint32_t post
     r.u = (uint32_t)(base + (int32_t)l.p);
     r.ok = direct && base + l.p > v;
     r.w = w;
-    r.has_self = t.co || (direct && !r.ok);
-    if (t.co) r.self += (double)((l.s * l.s) * t.co_lam);
+    r.has_self = true;
+    r.self += (double)((l.s * l.s) * t.co_lam);
     if (direct && !r.ok) r.self += (double)w;
-  } else if (t.co && l.c >= 0 && l.c < t.S && base + l.c >= v) {
+  } else if (l.c >= 0 && l.c < t.S && base + l.c >= v) {
     const float w = (l.si * l.s) * t.co_lam;
     r.u = (uint32_t)(base + l.c);
     r.ok = base + l.c > v;
@@ -169,18 +180,18 @@ __device__ __forceinline__ Candidate candidate(const TopkGraph& t, uint32_t post
 // Walks the candidates q = first, first + step, ... of the run that starts at
 // posting a, FLIGHT at a time; add(candidate) for each, pause() after each FLIGHT
 // (a true return ends the walk).
-template <int KT, class Add, class Pause>
-__device__ __forceinline__ void walk(const TopkGraph& t, const uint32_t* __restrict__ postings, uint32_t a, uint64_t n,
+template <int KT, class N, class Add, class Pause>
+__device__ __forceinline__ void walk(const TopkGraph& t, const uint32_t* __restrict__ postings, uint32_t a, N n,
                                      uint32_t first, uint32_t step, int32_t v, int32_t base, Add add, Pause pause) {
   const uint32_t K = KT ? KT : (uint32_t)t.K;
-  for (uint64_t q0 = 0; q0 < n; q0 += (uint64_t)FLIGHT * step) {
+  for (N q0 = 0; q0 < n; q0 += (N)FLIGHT * step) {
     uint32_t post[FLIGHT], j[FLIGHT];
     Loaded l[FLIGHT];
 #pragma unroll
     for (int f = 0; f < FLIGHT; ++f) {
-      const uint64_t q = q0 + (uint64_t)f * step + first;
-      const uint64_t qc = q < n ? q : n - 1;  // (past the end: the last one again, not added)
-      const uint64_t p = KT ? qc / KT : qc / K;
+      const N q = q0 + (N)f * step + first;
+      const N qc = q < n ? q : n - 1;  // (past the end: the last one again, not added)
+      const N p = KT ? qc / (N)KT : qc / K;
       j[f] = (uint32_t)(qc - p * K);
       post[f] = postings[a + p];
     }
@@ -188,7 +199,7 @@ __device__ __forceinline__ void walk(const TopkGraph& t, const uint32_t* __restr
     for (int f = 0; f < FLIGHT; ++f) l[f] = load_candidate<KT>(t, post[f], (int)j[f]);
 #pragma unroll
     for (int f = 0; f < FLIGHT; ++f) {
-      if (q0 + (uint64_t)f * step + first < n) add(candidate<KT>(t, post[f], (int)j[f], l[f], v, base));
+      if (q0 + (N)f * step + first < n) add(candidate<KT>(t, post[f], (int)j[f], l[f], v, base));
     }
     if (pause()) break;
   }
@@ -228,8 +239,9 @@ __device__ __forceinline__ void gather_run(const TopkGraph& t, const uint32_t* _
   float w[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
+    if (64u * i >= size) break;  // (a multiple of 64; most runs have a table of 64 or 128)
     const uint32_t j = ln + 64 * i;
-    k[i] = j < size ? tk[j] : EMPTY;
+    k[i] = tk[j];
     w[i] = k[i] != EMPTY ? (float)ts[j] : 0.0f;
   }
   wave_lds_sync();
@@ -237,6 +249,7 @@ __device__ __forceinline__ void gather_run(const TopkGraph& t, const uint32_t* _
   int m = 0;
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
+    if (64u * i >= size) break;
     const uint64_t used = __ballot(k[i] != EMPTY);
     if (k[i] != EMPTY) {
       const int at = m + __popcll(used & ((((uint64_t)1) << ln) - 1));
@@ -612,6 +625,94 @@ __global__ __launch_bounds__(64 * WAVES) void emit_kernel(const uint32_t* __rest
   if (blockIdx.x == 0 && threadIdx.x == 0) *out_count = (int64_t)place[n - 1] + count[n - 1];
 }
 
+// ----------------------------------------------------------------- entries sorted by pair
+// Entry i of a row: the direct edges, then the co-occurrence pairs of the upper
+// triangle, row-major.  Entries with a column or position outside the sequence
+// carry the sentinel key, which sorts last.
+__global__ __launch_bounds__(THREADS) void expand_kernel(TopkGraph t, int per_row, int bits,
+                                                         uint64_t* __restrict__ keys, float* __restrict__ vals) {
+  const int64_t i = (int64_t)blockIdx.x * THREADS + threadIdx.x;
+  if (i >= (int64_t)t.G * t.R * per_row) return;
+  const int64_t row = i / per_row, at = row * t.K, base = row / t.R * t.S;
+  int e = (int)(i - row * per_row);
+  int64_t a, b;  // the ends' positions
+  float w;
+  if (e < t.K) {
+    a = t.pos[row];
+    b = t.idx[at + e];
+    w = t.sc[at + e] * t.half_lam;
+  } else {
+    int r = 0;
+    for (e -= t.K; e >= t.K - r; ++r) e -= t.K - r;
+    a = t.idx[at + r];
+    b = t.idx[at + r + e];
+    w = (t.sc[at + r] * t.sc[at + r + e]) * t.co_lam;
+  }
+  const bool ok = a >= 0 && a < t.S && b >= 0 && b < t.S;
+  const uint64_t lo = (uint64_t)(base + (a < b ? a : b)), hi = (uint64_t)(base + (a < b ? b : a));
+  keys[i] = ok ? (lo << bits) | hi : (uint64_t)((int64_t)t.G * t.S) << bits;
+  vals[i] = ok ? w : 0.0f;
+}
+
+// Ends of the pairs; a sentinel among them is the last and no edge.
+__global__ __launch_bounds__(THREADS) void unpack_kernel(const uint64_t* __restrict__ pairs,
+                                                         const int64_t* __restrict__ count, int bits, uint64_t V,
+                                                         int32_t* __restrict__ out_src, int32_t* __restrict__ out_dst,
+                                                         int64_t* __restrict__ out_count) {
+  const int64_t n = *count, i = (int64_t)blockIdx.x * THREADS + threadIdx.x;
+  if (i == 0) *out_count = (pairs[n - 1] >> bits) >= V ? n - 1 : n;
+  if (i >= n) return;
+  const uint64_t k = pairs[i];
+  out_src[i] = (int32_t)(k >> bits);
+  out_dst[i] = (int32_t)(k & (((uint64_t)1 << bits) - 1));
+}
+
+struct AsDouble {
+  __host__ __device__ double operator()(float x) const { return (double)x; }
+};
+using DoubleOf = rocprim::transform_iterator<const float*, AsDouble, double>;
+
+hipError_t sort_entries(void* temp, size_t& bytes, const uint64_t* keys_in, uint64_t* keys, const float* vals_in,
+                        float* vals, size_t n, int end_bit, hipStream_t st) {
+  return rocprim::radix_sort_pairs(temp, bytes, keys_in, keys, vals_in, vals, n, 0, (unsigned)end_bit, st);
+}
+hipError_t sum_entries(void* temp, size_t& bytes, const uint64_t* keys, const float* vals, size_t n, uint64_t* pairs,
+                       float* sums, int64_t* count, hipStream_t st) {
+  return rocprim::reduce_by_key(temp, bytes, keys, DoubleOf(vals, AsDouble()), n, pairs, sums, count,
+                                rocprim::plus<double>(), rocprim::equal_to<uint64_t>(), st);
+}
+
+// pairs takes the place of keys_in (free once they are sorted).
+struct SortLayout {
+  size_t keys_in, keys, vals_in, vals, count, temp, temp_bytes, total;
+};
+
+SortLayout sort_layout(int64_t n) {
+  SortLayout L{};
+  size_t off = 0;
+  auto take = [&](size_t bytes) {
+    const size_t at = off;
+    off += align256(bytes);
+    return at;
+  };
+  size_t sort = 0, sum = 0;
+  (void)sort_entries(nullptr, sort, nullptr, nullptr, nullptr, nullptr, (size_t)n, 64, (hipStream_t)0);
+  (void)sum_entries(nullptr, sum, nullptr, nullptr, (size_t)n, nullptr, nullptr, nullptr, (hipStream_t)0);
+  L.keys_in = take((size_t)n * 8);
+  L.keys = take((size_t)n * 8);
+  L.vals_in = take((size_t)n * 4);
+  L.vals = take((size_t)n * 4);
+  L.count = take(8);
+  L.temp_bytes = sort > sum ? sort : sum;
+  L.temp = take(L.temp_bytes);
+  L.total = off;
+  return L;
+}
+
+// Rows of at most two entries, or without co-occurrence edges.
+inline bool by_entries(int32_t kappa, float lam) { return !(lam < 1.0f) || kappa == 1; }
+
+// ----------------------------------------------------------------- host side
 struct AdjLayout {
   size_t keys_in, vals_in, keys, vals, temp, temp_bytes, count, place, short_runs, long_runs, dense, lists, tmp_id,
       tmp_w, total;
@@ -668,7 +769,7 @@ using namespace ckv;
 
 extern "C" size_t ckv_adjacency_workspace_bytes(int32_t graphs, int32_t rows, int32_t kappa, float lam) {
   if (graphs <= 0 || rows <= 0 || kappa <= 0) return 0;
-  (void)lam;
+  if (by_entries(kappa, lam)) return sort_layout(adjacency_entries(graphs, rows, kappa, lam)).total;
   return adj_layout(adjacency_postings(graphs, rows, kappa), kappa).total;
 }
 
@@ -694,8 +795,32 @@ extern "C" int ckv_build_adjacency(const int32_t* topk_indices, const float* top
   const int64_t n = adjacency_postings(graphs, rows, kappa);
   if (adjacency_entries(graphs, rows, kappa, lam) >= ((int64_t)1 << 31) - 1 || V >= (int64_t)1 << 30)
     return ckv_internal::set_error(CKV_E_LIMIT, "adjacency too large");
-  const AdjLayout L = adj_layout(n, kappa);
+  const TopkGraph t{topk_indices, topk_scores, query_positions, graphs, rows, kappa, seq_len,
+                    bits_for((uint64_t)kappa), lam / 2.0f, 1.0f - lam};
   char* ws = (char*)workspace;
+  if (by_entries(kappa, lam)) {
+    const int64_t entries = adjacency_entries(graphs, rows, kappa, lam);
+    const SortLayout L = sort_layout(entries);
+    uint64_t* keys_in = (uint64_t*)(ws + L.keys_in);
+    uint64_t* sorted = (uint64_t*)(ws + L.keys);
+    float* vals_in = (float*)(ws + L.vals_in);
+    float* vals = (float*)(ws + L.vals);
+    int64_t* pairs = (int64_t*)(ws + L.count);
+    const int bits = bits_for((uint64_t)V - 1);
+    expand_kernel<<<blocks_for(entries, THREADS), THREADS, 0, st>>>(t, (int)(entries / ((int64_t)graphs * rows)), bits,
+                                                                   keys_in, vals_in);
+    size_t temp = L.temp_bytes;
+    if (sort_entries(ws + L.temp, temp, keys_in, sorted, vals_in, vals, (size_t)entries, bits + bits_for((uint64_t)V),
+                     st) != hipSuccess)
+      return ckv_internal::set_error(CKV_E_LAUNCH, "entry sort failed");
+    temp = L.temp_bytes;
+    if (sum_entries(ws + L.temp, temp, sorted, vals, (size_t)entries, keys_in, out_weight, pairs, st) != hipSuccess)
+      return ckv_internal::set_error(CKV_E_LAUNCH, "entry sum failed");
+    unpack_kernel<<<blocks_for(entries, THREADS), THREADS, 0, st>>>(keys_in, pairs, bits, (uint64_t)V, out_src, out_dst,
+                                                                   out_count);
+    return launch_check();
+  }
+  const AdjLayout L = adj_layout(n, kappa);
   uint32_t* keys_in = (uint32_t*)(ws + L.keys_in);
   uint32_t* vals_in = (uint32_t*)(ws + L.vals_in);
   uint32_t* keys = (uint32_t*)(ws + L.keys);
@@ -708,8 +833,6 @@ extern "C" int ckv_build_adjacency(const int32_t* topk_indices, const float* top
   int32_t* lists = (int32_t*)(ws + L.lists);
   uint32_t* tmp_id = (uint32_t*)(ws + L.tmp_id);
   float* tmp_w = (float*)(ws + L.tmp_w);
-  const TopkGraph t{topk_indices, topk_scores, query_positions, graphs, rows, kappa, seq_len,
-                    bits_for((uint64_t)kappa), lam / 2.0f, 1.0f - lam, lam < 1.0f ? 1 : 0};
   auto gather = [&](auto width) -> int {
     constexpr int KT = decltype(width)::value;
     posting_kernel<KT><<<blocks_for((int64_t)graphs * rows, THREADS), THREADS, 0, st>>>(t, keys_in, vals_in, lists);

@@ -16,8 +16,9 @@
 //                     above the vertex gather in an LDS hash table (f64 sums) and leave
 //                     ordered by id
 //   gather_big_kernel the same by one workgroup per long run
-//   gather_dense_kernel  vertices with more neighbours than that table holds:
-//                     windows of consecutive ids summed in a dense LDS array
+//                     (the longest in parts, each added to a sum per id in memory)
+//   gather_dense_kernel  the sums of the longest in a row; vertices with more
+//                     neighbours than that table holds, summed in LDS by rank
 //   scan + emit_kernel   edges to their places in the output
 //
 // Rows of few entries (those without co-occurrence edges, lam = 1, and of one
@@ -64,11 +65,16 @@ constexpr int BIG_THREADS = 256;
 constexpr int BIG_SLOTS = 2048;        // 24 KB
 constexpr int BIG_MOST = 960;          // neighbours after which a vertex leaves for the dense list
 static_assert(BIG_MOST + FLIGHT * BIG_THREADS < BIG_SLOTS, "every insert between two checks finds a place");
-constexpr int BIG_BLOCKS = 1280;       // five workgroups a compute unit (24 KB + the id bitmap of 32k vertices)
+constexpr int BIG_BLOCKS = 1280;       // (four a compute unit at once: 24 KB + the id bitmap of 32k vertices)
 constexpr int MAP_WORDS = 4096;        // id bitmap of a graph: up to 131,072 vertices
 constexpr int DENSE_THREADS = 1024;
-constexpr int DENSE_WINDOW = 16384;    // ids per window: 128 KB of f64 sums
+constexpr int DENSE_IDS = 32 * MAP_WORDS;  // ids per bitmap
+constexpr int DENSE_SUMS = 14336;      // f64 sums per pass: 112 KB beside the bitmap's 32 KB
 constexpr int DENSE_BLOCKS = 256;
+constexpr int SPLIT_MIN = 4096;        // postings from which a run is taken by several workgroups
+constexpr int PART = 1024;             // postings of a part, at most PARTS_MOST of a run
+constexpr int PARTS_MOST = 1024;
+static_assert(SPLIT_MIN >= 4 * PART, "parts are full but for the last");
 
 struct TopkGraph {
   const int32_t* idx;    // [G * R][K]
@@ -84,7 +90,13 @@ struct Run {
   uint32_t first, last;
 };
 
-enum { LIST_SHORT = 0, LIST_LONG = 1, LIST_DENSE = 2, LIST_TICKET = 3, LIST_WORDS = 4 };
+// Postings [first, last) of the run that starts at posting `run`.
+struct Part {
+  uint32_t run, first, last;
+};
+
+enum { LIST_SHORT = 0, LIST_LONG = 1, LIST_SPLIT = 2, LIST_PARTS = 3, LIST_DENSE = 4, LIST_TICKET = 5,
+       LIST_DENSE_TICKET = 6, LIST_WORDS = 8 };
 
 // A posting names (row << shift) | i: column i of the row, or (i == K) its
 // position.  A position is a posting only if one of the row's columns lies
@@ -131,7 +143,7 @@ struct Loaded {
   int64_t p;     // the row's position (lane j == i only)
 };
 
-template <int KT>
+template <int KT, bool SCORES = true>
 __device__ __forceinline__ Loaded load_candidate(const TopkGraph& t, uint32_t posting, int j) {
   const int K = KT ? KT : t.K;
   const uint32_t row = posting >> t.shift;
@@ -139,8 +151,8 @@ __device__ __forceinline__ Loaded load_candidate(const TopkGraph& t, uint32_t po
   const int64_t at = (int64_t)row * K;
   Loaded l;
   l.c = t.idx[at + j];
-  l.s = t.sc[at + j];
-  l.si = t.sc[at + (i < K ? i : j)];
+  l.s = SCORES ? t.sc[at + j] : 0.0f;
+  l.si = SCORES ? t.sc[at + (i < K ? i : j)] : 0.0f;
   l.p = (j == i) ? t.pos[row] : -1;
   return l;
 }
@@ -179,8 +191,8 @@ __device__ __forceinline__ Candidate candidate(const TopkGraph& t, uint32_t post
 
 // Walks the candidates q = first, first + step, ... of the run that starts at
 // posting a, FLIGHT at a time; add(candidate) for each, pause() after each FLIGHT
-// (a true return ends the walk).
-template <int KT, class N, class Add, class Pause>
+// (a true return ends the walk).  Without SCORES the weights are not read.
+template <int KT, bool SCORES = true, class N, class Add, class Pause>
 __device__ __forceinline__ void walk(const TopkGraph& t, const uint32_t* __restrict__ postings, uint32_t a, N n,
                                      uint32_t first, uint32_t step, int32_t v, int32_t base, Add add, Pause pause) {
   const uint32_t K = KT ? KT : (uint32_t)t.K;
@@ -196,7 +208,7 @@ __device__ __forceinline__ void walk(const TopkGraph& t, const uint32_t* __restr
       post[f] = postings[a + p];
     }
 #pragma unroll
-    for (int f = 0; f < FLIGHT; ++f) l[f] = load_candidate<KT>(t, post[f], (int)j[f]);
+    for (int f = 0; f < FLIGHT; ++f) l[f] = load_candidate<KT, SCORES>(t, post[f], (int)j[f]);
 #pragma unroll
     for (int f = 0; f < FLIGHT; ++f) {
       if (q0 + (N)f * step + first < n) add(candidate<KT>(t, post[f], (int)j[f], l[f], v, base));
@@ -302,17 +314,19 @@ constexpr int LIST_THREADS = 1024;
 constexpr int LIST_GROUPS = 4;
 
 __global__ __launch_bounds__(LIST_THREADS) void list_kernel(const uint32_t* __restrict__ keys, uint32_t n, uint32_t V,
-                                                            uint32_t short_most, int32_t* __restrict__ count,
-                                                            Run* __restrict__ short_runs, Run* __restrict__ long_runs,
-                                                            int32_t* __restrict__ lists) {
+                                                            uint32_t short_most, uint32_t split_min,
+                                                            int32_t* __restrict__ count, Run* __restrict__ short_runs,
+                                                            Run* __restrict__ long_runs, Run* __restrict__ split_runs,
+                                                            Part* __restrict__ parts, int32_t* __restrict__ lists) {
   __shared__ int s_n[2], s_at[2];
   const int ln = lane();
   const uint64_t below = (((uint64_t)1) << ln) - 1;
   if (threadIdx.x < 2) s_n[threadIdx.x] = 0;
   __syncthreads();
   uint32_t stop[LIST_GROUPS];
-  int place[LIST_GROUPS];  // in the workgroup's part of list `kind`; kind 2: no run starts here
+  int place[LIST_GROUPS];  // in the workgroup's part of list `kind`
   int kind[LIST_GROUPS];
+  constexpr int NONE = -1;
 #pragma unroll
   for (int g = 0; g < LIST_GROUPS; ++g) {
     const uint32_t here = (blockIdx.x * LIST_GROUPS + g) * LIST_THREADS + threadIdx.x;
@@ -331,7 +345,8 @@ __global__ __launch_bounds__(LIST_THREADS) void list_kernel(const uint32_t* __re
     }
     const uint64_t later = ln == 63 ? 0ull : starts >> (ln + 1);
     stop[g] = later ? here + 1 + (uint32_t)__builtin_ctzll(later) : end;
-    kind[g] = !mine ? 2 : stop[g] - here <= short_most ? LIST_SHORT : LIST_LONG;
+    const uint32_t length = stop[g] - here;
+    kind[g] = !mine ? NONE : length <= short_most ? LIST_SHORT : length < split_min ? LIST_LONG : LIST_SPLIT;
     const uint64_t ms = __ballot(kind[g] == LIST_SHORT), ml = __ballot(kind[g] == LIST_LONG);
     int bs = 0, bl = 0;
     if (ln == 0) {
@@ -350,22 +365,57 @@ __global__ __launch_bounds__(LIST_THREADS) void list_kernel(const uint32_t* __re
     const uint32_t here = (blockIdx.x * LIST_GROUPS + g) * LIST_THREADS + threadIdx.x;
     if (kind[g] == LIST_SHORT) short_runs[s_at[0] + place[g]] = Run{here, stop[g]};
     if (kind[g] == LIST_LONG) long_runs[s_at[1] + place[g]] = Run{here, stop[g]};
+    if (kind[g] == LIST_SPLIT) {  // (few: n / split_min at most)
+      const uint32_t length = stop[g] - here;
+      const uint32_t size = max((uint32_t)PART, (length + PARTS_MOST - 1) / PARTS_MOST);
+      const uint32_t many = (length + size - 1) / size;
+      split_runs[atomicAdd(lists + LIST_SPLIT, 1)] = Run{here, stop[g]};
+      Part* to = parts + atomicAdd(lists + LIST_PARTS, (int)many);
+      for (uint32_t i = 0; i < many; ++i) to[i] = Part{here, here + i * size, min(here + (i + 1) * size, stop[g])};
+    }
   }
 }
 
 // The edges of the run that starts at posting a wait in tmp at a * (K + 1): a
 // posting brings at most K neighbours, the run one pair with itself; count[a]
 // holds their number (0 at postings that start no run).
+//
+// A split run's edges first stand as a sum per id from its vertex on, in the
+// ids' part of that place (a split run is long enough for them: split_length).
+// A sum that nothing was added to is -0.0: what is added is no -0.0, so no sum
+// becomes it.
+__host__ __device__ inline uint32_t split_length(int32_t S, int32_t K) {
+  const uint32_t fits = (uint32_t)((2 * (int64_t)S + 2 + K) / (K + 1));
+  return fits > (uint32_t)SPLIT_MIN ? fits : (uint32_t)SPLIT_MIN;
+}
+template <int KT>
+__device__ __forceinline__ double* split_sums(const TopkGraph& t, uint32_t a, uint32_t* tmp_id) {
+  const int64_t out = (int64_t)a * ((KT ? KT : t.K) + 1);
+  return reinterpret_cast<double*>(tmp_id + ((out + 1) & ~(int64_t)1));
+}
+constexpr double NOTHING = -0.0;
+__device__ inline bool is_nothing(double x) { return __builtin_bit_cast(uint64_t, x) == 0x8000000000000000ull; }
+constexpr int CHUNK = 4096;  // ids of a split run that a workgroup clears or copies at a time
+
 template <int KT>
 __global__ __launch_bounds__(64 * WAVES) void gather_kernel(TopkGraph t, const uint32_t* __restrict__ keys,
                                                             const uint32_t* __restrict__ postings,
                                                             const Run* __restrict__ runs,
+                                                            const Run* __restrict__ split_runs,
                                                             const int32_t* __restrict__ lists,
                                                             int32_t* __restrict__ count, uint32_t* __restrict__ tmp_id,
                                                             float* __restrict__ tmp_w) {
   __shared__ __align__(16) uint32_t tab_k[WAVES][WAVE_SLOTS];
   __shared__ double tab_s[WAVES][WAVE_SLOTS];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int32_t chunks = (t.S + CHUNK - 1) / CHUNK;
+  const int64_t clear = (int64_t)lists[LIST_SPLIT] * chunks;
+  for (int64_t it = blockIdx.x; it < clear; it += gridDim.x) {
+    const uint32_t a = split_runs[it / chunks].first;
+    const int32_t v = (int32_t)keys[a], ids = t.S - v % t.S, at = (int32_t)(it % chunks) * CHUNK;
+    double* sums = split_sums<KT>(t, a, tmp_id);
+    for (int i = at + threadIdx.x; i < min(ids, at + CHUNK); i += 64 * WAVES) sums[i] = NOTHING;
+  }
   const int32_t listed = lists[LIST_SHORT];
   for (int32_t it = blockIdx.x * WAVES + wave; it < listed; it += gridDim.x * WAVES) {
     const Run r = runs[it];
@@ -374,17 +424,23 @@ __global__ __launch_bounds__(64 * WAVES) void gather_kernel(TopkGraph t, const u
   }
 }
 
-// One workgroup per long run (taken in turn by a ticket: their lengths differ
-// by a hundredfold).  Up to BIG_MOST neighbours in the LDS table; a vertex that has more goes to the dense list.  The neighbours are
-// ordered by a bitmap of the graph's vertices (words of it dynamic LDS, with a
-// running count per word): the set bits below an id are its rank.  Counting
-// smaller ids instead, as the waves do for their few, grows with the square
-// (and orders graphs of more vertices than the bitmap has).
+// One workgroup per part of a split run and per long run (taken in turn by a
+// ticket: their lengths differ by a hundredfold).  A part's neighbours gather
+// in the LDS table as far as BIG_MOST of them go (the ones that many rows name
+// come early) and are added to the run's sums at its end; the others are added
+// there at once.
+//
+// A long run's neighbours: up to BIG_MOST in the table; a vertex that has more
+// goes to the dense list.  They are ordered by a bitmap of the graph's vertices
+// (words of it dynamic LDS, with a running count per word): the set bits below
+// an id are its rank.  Counting smaller ids instead, as the waves do for their
+// few, grows with the square (and orders graphs of more vertices than the
+// bitmap has).
 template <int KT>
 __global__ __launch_bounds__(BIG_THREADS) void gather_big_kernel(
     TopkGraph t, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ postings,
-    const Run* __restrict__ runs, Run* __restrict__ dense, int32_t* lists, int32_t* __restrict__ count,
-    uint32_t* __restrict__ tmp_id, float* __restrict__ tmp_w) {
+    const Run* __restrict__ runs, const Part* __restrict__ parts, Run* __restrict__ dense, int32_t* lists,
+    int32_t* __restrict__ count, uint32_t* __restrict__ tmp_id, float* __restrict__ tmp_w) {
   __shared__ __align__(16) uint32_t tk[BIG_SLOTS];
   __shared__ double ts[BIG_SLOTS];
   extern __shared__ uint32_t map_s[];  // [words] bits, [words] set bits before the word
@@ -392,7 +448,7 @@ __global__ __launch_bounds__(BIG_THREADS) void gather_big_kernel(
   __shared__ int wave_n[BIG_THREADS / 64];
   __shared__ int s_added, s_self, s_ticket;
   const int tid = threadIdx.x, wv = tid >> 6, ln = lane();
-  const int32_t listed = lists[LIST_LONG];
+  const int32_t split = lists[LIST_PARTS], listed = split + lists[LIST_LONG];
   const int words = t.S <= 32 * MAP_WORDS ? (t.S + 31) >> 5 : 0;
   uint32_t* before_s = map_s + words;
   while (true) {
@@ -400,7 +456,38 @@ __global__ __launch_bounds__(BIG_THREADS) void gather_big_kernel(
     __syncthreads();
     const int32_t it = s_ticket;
     if (it >= listed) return;
-    const uint32_t a = runs[it].first, b = runs[it].last;
+    if (it < split) {
+      const Part part = parts[it];
+      const int32_t v = (int32_t)keys[part.run];
+      const int32_t base = v / t.S * t.S;
+      double* sums = split_sums<KT>(t, part.run, tmp_id);
+      for (uint32_t j = tid; j < BIG_SLOTS; j += BIG_THREADS) {
+        tk[j] = EMPTY;
+        ts[j] = 0.0;
+      }
+      if (tid == 0) s_added = 0;
+      __syncthreads();
+      double self = 0.0;
+      bool any_self = false;
+      walk<KT>(t, postings, part.first, (uint64_t)(part.last - part.first) * (uint32_t)t.K, (uint32_t)tid, BIG_THREADS,
+               v, base,
+               [&](const Candidate& c) {
+                 any_self = any_self || c.has_self;
+                 self += c.self;
+                 if (c.ok && !insert_few(tk, ts, BIG_SLOTS, c.u, c.w, &s_added, BIG_MOST))
+                   unsafeAtomicAdd(sums + (c.u - (uint32_t)v), (double)c.w + 0.0);  // (no -0.0)
+               },
+               [] { return false; });
+      self = wave_sum_f64(self);
+      if (__ballot(any_self) != 0 && ln == 0) unsafeAtomicAdd(sums, self + 0.0);
+      __syncthreads();
+      for (uint32_t j = tid; j < BIG_SLOTS; j += BIG_THREADS) {
+        if (tk[j] != EMPTY) unsafeAtomicAdd(sums + (tk[j] - (uint32_t)v), ts[j] + 0.0);
+      }
+      __syncthreads();
+      continue;
+    }
+    const uint32_t a = runs[it - split].first, b = runs[it - split].last;
     const int32_t v = (int32_t)keys[a];
     const int32_t base = v / t.S * t.S;
     const uint64_t n = (uint64_t)(b - a) * (uint32_t)t.K;
@@ -528,93 +615,196 @@ __global__ __launch_bounds__(BIG_THREADS) void gather_big_kernel(
   }
 }
 
-// Vertices with more than BIG_MOST neighbours: their rows are read once per
-// window of DENSE_WINDOW consecutive ids, whose sums and marks lie in LDS in
-// id order.
-constexpr size_t dense_lds_bytes() { return DENSE_WINDOW * 8 + DENSE_WINDOW / 8; }
+// The runs that one LDS table does not hold.
+//
+// Split runs: a workgroup puts the sums that something was added to in a row.
+// Ids take the place of the sums: those of a round are read before they are
+// overwritten, and an id is half as long as a sum, so no later one is.
+//
+// Vertices of one workgroup with more than BIG_MOST neighbours: their rows are
+// read once for a bitmap of the neighbours, whose set bits below an id are its
+// rank, and once for every DENSE_SUMS ranks, whose sums lie in LDS in order
+// (graphs of more than DENSE_IDS vertices: bitmap by bitmap).  A pass per
+// window of 16,384 consecutive ids instead read the rows of a vertex with a few
+// thousand neighbours eight times at 131,072 positions.
+//
+// The whole graph of 32 heads in 8 graphs at 131,072 positions, columns drawn by
+// a power law: 9.1 ms; planted columns and one that all rows name 5.5, with all
+// heads in one graph 7.9; at 32,768 positions 1.4 and 1.2.  (Every run on one
+// workgroup: 26.4 ms, 30.9, 207; 3.5, 16.1.  The sort of all entries that the
+// gathering replaced: 11.5, 11.4, 9.7; 2.7, 2.2.)
+constexpr size_t dense_lds_bytes() { return DENSE_SUMS * 8 + MAP_WORDS * 8; }
+
+// Block-wide exclusive scan of one int per thread; the total in *sum.
+__device__ __forceinline__ int dense_scan(int x, int* wave_n, int* sum) {
+  const int wv = threadIdx.x >> 6;
+  int incl = x;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(incl, o);
+    if (lane() >= o) incl += y;
+  }
+  if (lane() == 63) wave_n[wv] = incl;
+  __syncthreads();
+  int at = incl - x, all = 0;
+  for (int i = 0; i < DENSE_THREADS / 64; ++i) {
+    if (i < wv) at += wave_n[i];
+    all += wave_n[i];
+  }
+  __syncthreads();
+  *sum = all;
+  return at;
+}
 
 template <int KT>
 __global__ __launch_bounds__(DENSE_THREADS) void gather_dense_kernel(
     TopkGraph t, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ postings,
-    const Run* __restrict__ dense, const int32_t* __restrict__ lists, int32_t* __restrict__ count,
-    uint32_t* __restrict__ tmp_id, float* __restrict__ tmp_w) {
+    const Run* __restrict__ split_runs, const Run* __restrict__ dense, int32_t* lists, int32_t* __restrict__ count,
+    uint32_t* tmp_id, float* __restrict__ tmp_w) {
   extern __shared__ double dense_s[];
-  uint32_t* mark = reinterpret_cast<uint32_t*>(dense_s + DENSE_WINDOW);
-  __shared__ int wave_n[DENSE_THREADS / 64];
-  constexpr int PER = DENSE_WINDOW / DENSE_THREADS;  // consecutive ids of a thread (half a mark word)
-  static_assert(PER == 16, "a thread owns half a mark word");
-  const int tid = threadIdx.x, wv = tid >> 6, ln = lane();
-  const int32_t listed = lists[LIST_DENSE];
-  for (int32_t it = blockIdx.x; it < listed; it += gridDim.x) {
-    const uint32_t a = dense[it].first, b = dense[it].last;
+  uint32_t* map = reinterpret_cast<uint32_t*>(dense_s + DENSE_SUMS);
+  uint32_t* below = map + MAP_WORDS;  // neighbours in the words before
+  __shared__ double red[DENSE_THREADS / 64];
+  __shared__ int wave_n[DENSE_THREADS / 64], s_ticket;
+  constexpr int OWN = MAP_WORDS / DENSE_THREADS;  // consecutive words of a thread
+  const int tid = threadIdx.x, wv = tid >> 6;
+  const int32_t split = lists[LIST_SPLIT], listed = split + lists[LIST_DENSE];
+  while (true) {
+    if (tid == 0) s_ticket = atomicAdd(lists + LIST_DENSE_TICKET, 1);
+    __syncthreads();
+    const int32_t it = s_ticket;
+    __syncthreads();
+    if (it >= listed) return;
+    if (it < split) {
+      constexpr int U = 4;
+      const uint32_t a = split_runs[it].first;
+      const int32_t v = (int32_t)keys[a], ids = t.S - v % t.S;
+      const int64_t out = (int64_t)a * (t.K + 1);
+      const double* sums = split_sums<KT>(t, a, tmp_id);
+      int done = 0;
+      for (int i0 = 0; i0 < ids; i0 += U * DENSE_THREADS) {
+        double x[U];
+        int own = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int i = i0 + U * tid + u;
+          x[u] = i < ids ? sums[i] : NOTHING;
+          own += is_nothing(x[u]) ? 0 : 1;
+        }
+        int m;
+        int64_t at = out + done + dense_scan(own, wave_n, &m);  // (its barriers: all sums of the round are read)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (!is_nothing(x[u])) {
+            tmp_id[at] = (uint32_t)(v + i0 + U * tid + u);
+            tmp_w[at] = (float)x[u];
+            ++at;
+          }
+        }
+        done += m;
+        __syncthreads();
+      }
+      if (tid == 0) count[a] = done;
+      continue;
+    }
+    const uint32_t a = dense[it - split].first, b = dense[it - split].last;
     const int32_t v = (int32_t)keys[a];
     const int32_t base = v / t.S * t.S;
     const uint64_t n = (uint64_t)(b - a) * (uint32_t)t.K;
     const int64_t out = (int64_t)a * (t.K + 1);
     int done = 0;
-    for (int32_t lo = v; lo < base + t.S; lo += DENSE_WINDOW) {
-      for (int j = tid; j < DENSE_WINDOW; j += DENSE_THREADS) dense_s[j] = 0.0;
-      for (int j = tid; j < DENSE_WINDOW / 32; j += DENSE_THREADS) mark[j] = 0u;
+    for (int32_t lo = v; lo < base + t.S; lo += DENSE_IDS) {
+      for (int j = tid; j < MAP_WORDS; j += DENSE_THREADS) map[j] = 0u;
       __syncthreads();
-      walk<KT>(t, postings, a, n, (uint32_t)tid, DENSE_THREADS, v, base,
-               [&](const Candidate& c) {
-                 if (c.has_self && lo == v) {
-                   unsafeAtomicAdd(dense_s, c.self);
-                   atomicOr(mark, 1u);
-                 }
-                 const int32_t d = (int32_t)c.u - lo;
-                 if (c.ok && d >= 0 && d < DENSE_WINDOW) {
-                   unsafeAtomicAdd(dense_s + d, (double)c.w);
-                   atomicOr(mark + (d >> 5), 1u << (d & 31));
-                 }
-               },
-               [] { return false; });
-      __syncthreads();
-      const uint32_t bits = (mark[tid >> 1] >> (16 * (tid & 1))) & 0xffffu;
-      const int own = __popc(bits);
-      int incl = own;
-      for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(incl, o);
-        if (ln >= o) incl += y;
+      bool any_self = false;
+      walk<KT, false>(t, postings, a, n, (uint32_t)tid, DENSE_THREADS, v, base,
+                      [&](const Candidate& c) {
+                        any_self = any_self || c.has_self;
+                        const uint32_t d = c.u - (uint32_t)lo;  // (below lo: beyond the bitmap)
+                        if (c.ok && d < (uint32_t)DENSE_IDS) atomicOr(map + (d >> 5), 1u << (d & 31));
+                      },
+                      [] { return false; });
+      const int lead = __syncthreads_or(any_self ? 1 : 0) != 0 && lo == v ? 1 : 0;
+      int mine = 0, m;
+#pragma unroll
+      for (int i = 0; i < OWN; ++i) mine += __popc(map[OWN * tid + i]);
+      int at = dense_scan(mine, wave_n, &m);
+      done += lead;
+      for (int i = 0; i < OWN; ++i) {
+        uint32_t bits = map[OWN * tid + i];
+        below[OWN * tid + i] = (uint32_t)at;
+        for (; bits != 0; bits &= bits - 1, ++at)
+          tmp_id[out + done + at] = (uint32_t)lo + 32u * (uint32_t)(OWN * tid + i) + (uint32_t)__builtin_ctz(bits);
       }
-      if (ln == 63) wave_n[wv] = incl;
-      __syncthreads();
-      int at = done + incl - own, m = 0;
-      for (int i = 0; i < DENSE_THREADS / 64; ++i) {
-        if (i < wv) at += wave_n[i];
-        m += wave_n[i];
-      }
-      for (int i = 0; i < PER; ++i) {
-        if ((bits >> i) & 1u) {
-          const int d = tid * PER + i;
-          tmp_id[out + at] = (uint32_t)(lo + d);
-          tmp_w[out + at] = (float)dense_s[d];
-          ++at;
+      for (int r0 = 0; r0 == 0 || r0 < m; r0 += DENSE_SUMS) {
+        const int ranks = min(m - r0, DENSE_SUMS);
+        for (int j = tid; j < ranks; j += DENSE_THREADS) dense_s[j] = 0.0;
+        __syncthreads();
+        double self = 0.0;
+        walk<KT>(t, postings, a, n, (uint32_t)tid, DENSE_THREADS, v, base,
+                 [&](const Candidate& c) {
+                   self += c.self;
+                   const uint32_t d = c.u - (uint32_t)lo;
+                   if (c.ok && d < (uint32_t)DENSE_IDS) {
+                     const int r = (int)below[d >> 5] + __popc(map[d >> 5] & ((1u << (d & 31)) - 1u)) - r0;
+                     if (r >= 0 && r < ranks) unsafeAtomicAdd(dense_s + r, (double)c.w);
+                   }
+                 },
+                 [] { return false; });
+        if (lead != 0 && r0 == 0) {
+          self = wave_sum_f64(self);
+          if (lane() == 0) red[wv] = self;
         }
+        __syncthreads();
+        if (lead != 0 && r0 == 0 && tid == 0) {
+          double total = 0.0;
+          for (int i = 0; i < DENSE_THREADS / 64; ++i) total += red[i];
+          tmp_id[out] = (uint32_t)v;
+          tmp_w[out] = (float)total;
+        }
+        for (int j = tid; j < ranks; j += DENSE_THREADS) tmp_w[out + done + r0 + j] = (float)dense_s[j];
+        __syncthreads();
       }
       done += m;
-      __syncthreads();
     }
     if (tid == 0) count[a] = done;
   }
 }
 
-// Copies the runs' edges to their places; the last posting's place ends the output.
+// Copies the runs' edges to their places, a wave per run; a workgroup per dense
+// run and per CHUNK of a split one.  The last posting's place ends the output.
 __global__ __launch_bounds__(64 * WAVES) void emit_kernel(const uint32_t* __restrict__ keys,
                                                           const int32_t* __restrict__ count,
                                                           const int32_t* __restrict__ place,
                                                           const Run* __restrict__ short_runs,
                                                           const Run* __restrict__ long_runs,
+                                                          const Run* __restrict__ split_runs,
+                                                          const Run* __restrict__ dense_runs,
                                                           const int32_t* __restrict__ lists, uint32_t n, int32_t K,
-                                                          const uint32_t* __restrict__ tmp_id,
+                                                          int32_t S, const uint32_t* __restrict__ tmp_id,
                                                           const float* __restrict__ tmp_w, int32_t* __restrict__ out_src,
                                                           int32_t* __restrict__ out_dst, float* __restrict__ out_w,
                                                           int64_t* __restrict__ out_count) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int32_t chunks = (S + CHUNK - 1) / CHUNK;
+  const int64_t pieces = (int64_t)lists[LIST_SPLIT] * chunks, items = pieces + lists[LIST_DENSE];
+  for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
+    const bool piece = it < pieces;
+    const uint32_t a = (piece ? split_runs[it / chunks] : dense_runs[it - pieces]).first;
+    const int i0 = piece ? (int)(it % chunks) * CHUNK : 0;
+    const int m = piece ? min(count[a], i0 + CHUNK) : count[a], at = place[a], v = (int)keys[a];
+    const int64_t from = (int64_t)a * (K + 1);
+#pragma unroll 4
+    for (int i = i0 + (int)threadIdx.x; i < m; i += 64 * WAVES) {
+      out_src[at + i] = v;
+      out_dst[at + i] = (int32_t)tmp_id[from + i];
+      out_w[at + i] = tmp_w[from + i];
+    }
+  }
   const int32_t shorts = lists[LIST_SHORT], listed = shorts + lists[LIST_LONG];
   for (int32_t it = blockIdx.x * WAVES + wave; it < listed; it += gridDim.x * WAVES) {
     const uint32_t a = (it < shorts ? short_runs[it] : long_runs[it - shorts]).first;
     const int m = count[a], at = place[a], v = (int)keys[a];
+    if (m > BIG_MOST + 1) continue;  // a dense run: copied above
     const int64_t from = (int64_t)a * (K + 1);
     for (int i = lane(); i < m; i += 64) {
       out_src[at + i] = v;
@@ -714,8 +904,8 @@ inline bool by_entries(int32_t kappa, float lam) { return !(lam < 1.0f) || kappa
 
 // ----------------------------------------------------------------- host side
 struct AdjLayout {
-  size_t keys_in, vals_in, keys, vals, temp, temp_bytes, count, place, short_runs, long_runs, dense, lists, tmp_id,
-      tmp_w, total;
+  size_t keys_in, vals_in, keys, vals, temp, temp_bytes, count, place, short_runs, long_runs, split_runs, parts, dense,
+      lists, tmp_id, tmp_w, total;
 };
 
 // n: postings (rows x (kappa + 1)).  A long run has more than WAVE_CANDIDATES / kappa of them.
@@ -738,6 +928,8 @@ AdjLayout adj_layout(int64_t n, int32_t kappa) {
   L.short_runs = take((size_t)n * sizeof(Run));
   L.long_runs = take(runs * sizeof(Run));
   L.dense = take(runs * sizeof(Run));
+  L.split_runs = take(((size_t)n / SPLIT_MIN + 1) * sizeof(Run));
+  L.parts = take(((size_t)n / PART + (size_t)n / SPLIT_MIN + 1) * sizeof(Part));
   L.lists = take(LIST_WORDS * 4);
   L.temp_bytes = sort > scan ? sort : scan;
   L.temp = take(L.temp_bytes);
@@ -830,6 +1022,8 @@ extern "C" int ckv_build_adjacency(const int32_t* topk_indices, const float* top
   Run* short_runs = (Run*)(ws + L.short_runs);
   Run* long_runs = (Run*)(ws + L.long_runs);
   Run* dense = (Run*)(ws + L.dense);
+  Run* split_runs = (Run*)(ws + L.split_runs);
+  Part* parts = (Part*)(ws + L.parts);
   int32_t* lists = (int32_t*)(ws + L.lists);
   uint32_t* tmp_id = (uint32_t*)(ws + L.tmp_id);
   float* tmp_w = (float*)(ws + L.tmp_w);
@@ -840,12 +1034,15 @@ extern "C" int ckv_build_adjacency(const int32_t* topk_indices, const float* top
         hipSuccess)
       return ckv_internal::set_error(CKV_E_LAUNCH, "posting sort failed");
     list_kernel<<<blocks_for(n, LIST_GROUPS * LIST_THREADS), LIST_THREADS, 0, st>>>(
-        keys, (uint32_t)n, (uint32_t)V, (uint32_t)(WAVE_CANDIDATES / kappa), count, short_runs, long_runs, lists);
-    gather_kernel<KT><<<WAVE_BLOCKS, 64 * WAVES, 0, st>>>(t, keys, vals, short_runs, lists, count, tmp_id, tmp_w);
+        keys, (uint32_t)n, (uint32_t)V, (uint32_t)(WAVE_CANDIDATES / kappa), split_length(seq_len, kappa), count,
+        short_runs, long_runs, split_runs, parts, lists);
+    gather_kernel<KT><<<WAVE_BLOCKS, 64 * WAVES, 0, st>>>(t, keys, vals, short_runs, split_runs, lists, count, tmp_id,
+                                                         tmp_w);
     const size_t map_bytes = seq_len <= 32 * MAP_WORDS ? (size_t)((seq_len + 31) / 32) * 8 : 0;
-    gather_big_kernel<KT><<<BIG_BLOCKS, BIG_THREADS, map_bytes, st>>>(t, keys, vals, long_runs, dense, lists, count,
-                                                                      tmp_id, tmp_w);
-    if (seq_len > BIG_MOST) {  // (a vertex has fewer neighbours than its graph has vertices)
+    gather_big_kernel<KT><<<BIG_BLOCKS, BIG_THREADS, map_bytes, st>>>(t, keys, vals, long_runs, parts, dense, lists,
+                                                                      count, tmp_id, tmp_w);
+    // (a vertex has fewer neighbours than its graph has vertices, and postings than its rows have entries)
+    if (seq_len > BIG_MOST || (int64_t)rows * (kappa + 1) >= SPLIT_MIN) {
       const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gather_dense_kernel<KT>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)dense_lds_bytes());
       if (e != hipSuccess) {
@@ -853,7 +1050,7 @@ extern "C" int ckv_build_adjacency(const int32_t* topk_indices, const float* top
         return ckv_internal::set_error(CKV_E_LAUNCH, hipGetErrorString(e));
       }
       gather_dense_kernel<KT><<<DENSE_BLOCKS, DENSE_THREADS, dense_lds_bytes(), st>>>(
-          t, keys, vals, dense, lists, count, tmp_id, tmp_w);
+          t, keys, vals, split_runs, dense, lists, count, tmp_id, tmp_w);
     }
     return 0;
   };
@@ -864,7 +1061,8 @@ extern "C" int ckv_build_adjacency(const int32_t* topk_indices, const float* top
   if (rc != 0) return rc;
   if (exclusive_scan_i32(ws + L.temp, L.temp_bytes, count, place, (size_t)n, st) != hipSuccess)
     return ckv_internal::set_error(CKV_E_LAUNCH, "edge scan failed");
-  emit_kernel<<<2048, 64 * WAVES, 0, st>>>(keys, count, place, short_runs, long_runs, lists, (uint32_t)n, kappa, tmp_id,
-                                           tmp_w, out_src, out_dst, out_weight, out_count);
+  emit_kernel<<<2048, 64 * WAVES, 0, st>>>(keys, count, place, short_runs, long_runs, split_runs, dense, lists,
+                                           (uint32_t)n, kappa, seq_len, tmp_id, tmp_w, out_src, out_dst, out_weight,
+                                           out_count);
   return launch_check();
 }

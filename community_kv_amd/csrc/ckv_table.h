@@ -54,4 +54,26 @@ __device__ inline bool insert(uint32_t* tk, double* ts, uint32_t size, uint32_t 
   return false;
 }
 
+// The same while *added, the new ids so far, is below `most`: false for a new
+// id afterwards (threads that look at once may add one each past it).
+__device__ inline bool insert_few(uint32_t* tk, double* ts, uint32_t size, uint32_t u, float w, int* added, int most) {
+  uint32_t h = hash_id(u) & (size - 1);
+  for (uint32_t probe = 0; probe < size; ++probe) {
+    const uint32_t cur = __hip_atomic_load(tk + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    bool mine = cur == u;
+    if (cur == EMPTY) {
+      if (__hip_atomic_load(added, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >= most) return false;
+      const uint32_t prev = atomicCAS(tk + h, EMPTY, u);
+      mine = prev == EMPTY || prev == u;
+      if (prev == EMPTY) atomicAdd(added, 1);
+    }
+    if (mine) {
+      unsafeAtomicAdd(ts + h, (double)w);
+      return true;
+    }
+    h = (h + 1) & (size - 1);
+  }
+  return false;
+}
+
 }  // namespace ckv

@@ -216,6 +216,54 @@ def test_build_adjacency_matches_oracle(device, lam, dyadic):
         np.testing.assert_allclose(w.cpu().numpy(), rw, rtol=2e-6)
 
 
+@pytest.mark.parametrize("R,S", [(9000, 3000), (4000, 40000), (300, 900)])
+def test_build_adjacency_weights_that_cancel(device, R, S):
+    """Edges whose weights add up to zero, or are all zero of either sign, are
+    edges all the same (raw scores may be negative), however they are gathered."""
+    from community_kv_amd.graph.partition import build_adjacency
+    from oracle import ckv_oracle as co
+
+    rng = np.random.default_rng(R)
+    idx = rng.integers(0, S, (1, R, 8)).astype(np.int32)
+    idx[..., 0] = 5
+    sc = (rng.integers(-2, 3, idx.shape) / 8.0).astype(np.float32)
+    sc[rng.random(sc.shape) < 0.1] = -0.0
+    sc[:, :, 0] = np.where(rng.random((1, R)) < 0.5, 0.0, 0.25)
+    pos = rng.integers(0, S, (1, R)).astype(np.int64)
+    print(f"build_adjacency cancelling weights R={R} S={S}", flush=True)
+    got = build_adjacency(*_dev(device, idx, sc, pos), seq_len=S, lam=0.5)
+    ref = co.build_adjacency(idx, sc, pos, seq_len=S, lam=0.5)
+    for a, b in zip(got, ref):
+        np.testing.assert_array_equal(a.cpu().numpy(), b)
+
+
+def test_build_adjacency_heavy_column_keeps_pace(device):
+    """A column that every row names costs little beside the same rows without
+    it (one workgroup reading all rows for it: 7 times with one graph)."""
+    from community_kv_amd.graph.partition import build_adjacency
+
+    g = torch.Generator(device=device).manual_seed(3)
+    heads, R, S = 32, 30000, 30000
+    pos = torch.arange(R, device=device).repeat(heads).unsqueeze(0)
+    idx = (pos.unsqueeze(-1) - torch.randint(0, 300, (1, heads * R, 8), device=device, generator=g)).clamp_min(0).int()
+    sc = torch.rand(1, heads * R, 8, device=device, generator=g)
+    heavy = idx.clone()
+    heavy[..., 0] = 3
+
+    def best_ms(columns):
+        best = float("inf")
+        for _ in range(5):
+            t0 = time.perf_counter()
+            build_adjacency(columns, sc, pos, seq_len=S, lam=0.5)
+            torch.cuda.synchronize()
+            best = min(best, (time.perf_counter() - t0) * 1e3)
+        return best
+
+    plain, with_it = best_ms(idx), best_ms(heavy)
+    print(f"build_adjacency {plain:.2f} ms, with a heavy column {with_it:.2f} ms", flush=True)
+    assert with_it < 2.5 * plain
+
+
 def test_build_adjacency_direct_edges_scratch_and_pace(device):
     """Without co-occurrence edges (lam = 1) a graph has one edge per column: it
     needs no more scratch per edge at 64 columns a row than at 8, and building
@@ -279,8 +327,14 @@ ADJACENCY_TIERS = [
     (2, 1500, 8, 900, 0, 0.0),       # short and long runs, fewer vertices than the workgroup table
     (1, 400, 16, 3000, 2, 0.2),      # the width with its own code; runs of 80 rows: the id bitmap orders them
     (1, 300, 5, 2000, 1, 1.0),       # any other width
-    (2, 6000, 8, 5000, 2, 1.0),      # more neighbours than the table: one dense window
-    (1, 4000, 8, 40000, 1, 1.0),     # three dense windows
+    (2, 6000, 8, 5000, 2, 1.0),      # more neighbours than the table: one pass of ranked sums
+    (1, 4000, 8, 40000, 1, 1.0),     # two passes
+    (1, 2500, 8, 290000, 1, 1.0),    # three bitmaps of ids
+    (1, 9000, 8, 3000, 2, 1.0),      # runs in parts
+    (2, 9000, 8, 500, 1, 1.0),       # of a graph whose vertices all fit the table
+    (1, 30000, 8, 70000, 1, 0.6),    # runs just long enough for a sum per id,
+    (1, 30000, 8, 70000, 1, 0.45),   # and too short for that
+    (1, 20000, 3, 9000, 2, 1.0),     # parts of a width without its own code
     (1, 700, 8, 140000, 1, 0.15),    # more vertices than the bitmap holds: ordered by counting
     (1, 57, 8, 300, 1, 1.0),         # a run one posting past the short ones
     (1, 1, 1, 1, 0, 0.0),            # the smallest graph: one vertex, one self loop
@@ -291,8 +345,8 @@ ADJACENCY_TIERS = [
 
 @pytest.mark.parametrize("G,R,kappa,S,hubs,share", ADJACENCY_TIERS)
 def test_build_adjacency_run_lengths(device, G, R, kappa, S, hubs, share):
-    """Every way a vertex's edges are gathered (one wave, one workgroup, dense
-    windows) and ordered, with columns on both sides of the row's position,
+    """Every way a vertex's edges are gathered (one wave, one workgroup, several
+    workgroups, by rank) and ordered, with columns on both sides of the row's position,
     repeated within a row and outside the sequence; dyadic scores make the sums
     exact, so the edge list must equal the oracle's bit for bit."""
     from community_kv_amd.graph.partition import build_adjacency

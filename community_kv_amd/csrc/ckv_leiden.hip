@@ -4,16 +4,16 @@
 // 43-205, local_moving.cu 69-210, refinement.cu 71-300, csr.cu 20-271,
 // aggregate.cu 24-184, helpers.cu 9-122) for MI355X:
 //
-//   * one wave64 per vertex; the vertex's neighbour communities are gathered
-//     into a per-wave LDS table by a leader loop (a chunk of 64 row entries at
-//     a time, ballot per distinct community, fp64 butterfly sum), so sums are
-//     formed in one fixed order and a low-degree vertex touches only its row;
+//   * a vertex takes half a wave, a wave or a workgroup by the length of its
+//     row, which its threads hold in registers; its neighbour communities
+//     gather in an LDS table by compare-and-swap, in f64 sums of arbitrary
+//     order (exact for weights within 29 bits of each other's range);
 //   * the sweep loops run without host round trips: every sweep's kernels
-//     are queued up front and read a device control word (moved count,
-//     up/down direction, stall count, done flag) that a one-wave control
-//     kernel advances after each sweep, so converged sweeps exit at once;
-//   * the symmetric CSR is one stable radix sort of (src, dst) keys, rows
-//     ordered by neighbour id.
+//     are queued up front and read from a ring of marks, one per sweep in which
+//     a vertex moved, where their phase stands (up or down moves, stalled,
+//     ended); sweeps after the end hand on what they were given or return;
+//   * the symmetric CSR of a list in any order is one stable radix sort of
+//     (src, dst) keys, rows ordered by neighbour id.
 //
 // Move rules follow the reference: synchronous moves on a snapshot, gain
 //   dQ = (k_v,new - k_v,old)/m + gamma k_v (Sigma_old - k_v - Sigma_new)/(2 m^2),
@@ -691,7 +691,7 @@ template <class P, bool FIRST>
 __device__ __forceinline__ bool move_vertex(const P& p, const Graph& gr, const MoveSweep& s, const MoveState& st,
                                             const Vertex& x, int32_t old) {
   int32_t choice = old;
-  if (!st.done && x.a != x.b && x.tm > 0.0) {
+  if (x.a != x.b && x.tm > 0.0) {
     Row r;
     load_row(p, gr, x.v, x.a, x.b, r);
     const double sig_old_excl = load_now(s.sigma + old) - x.kv;
@@ -775,12 +775,28 @@ __device__ __forceinline__ Share share_of(int32_t V, int32_t first) {
   return Share{(int32_t)(chunks * x / 8) + (b >> 3), (int32_t)(chunks * (x + 1) / 8), ((int32_t)gridDim.x - first) >> 3};
 }
 
+// A sweep after local moving has ended (every vertex stays): what it was given,
+// handed on.  Refinement needs nothing handed on: nothing reads the pairs and
+// totals of its last sweeps, and the labels are in place.
+__device__ __forceinline__ void hand_on(const MoveSweep& s, int32_t V) {
+  const int32_t step = (int32_t)(gridDim.x * HUB_THREADS);
+  for (int32_t v = (int32_t)(blockIdx.x * HUB_THREADS + threadIdx.x); v < V; v += step) {
+    s.lout[v] = s.lin[v];
+    s.next[v] = s.sigma[v];
+    s.clear[v] = 0.0;
+  }
+}
+
 template <bool FIRST>
 __global__ __launch_bounds__(HUB_THREADS, 8) void local_moving_kernel(Graph gr, MoveSweep s,
                                                                       RowLists l) {
   __shared__ SweepShared sh;  // (FIRST leaves the table out of use; its occupancy is full all the same)
   bool moved = false;
   const MoveState st = move_state(s.ctl, s.sweep);
+  if (!FIRST && st.done) {
+    hand_on(s, gr.V);
+    return;
+  }
   if constexpr (!FIRST) clear_tables(sh);
   const int32_t hubs = l.counts[1];
   const Share share = mid_share(l);
@@ -962,9 +978,8 @@ __device__ __forceinline__ Commit load_commit(const Graph& gr, const RefineSweep
 
 // Returns whether the vertex moves.
 template <class P>
-__device__ __forceinline__ bool commit_vertex(const P& p, const Graph& gr, const RefineSweep& s, bool done,
-                                              const Commit& x) {
-  const bool wants = !done && x.wants >= 0;  // (after the end the proposals are an earlier sweep's)
+__device__ __forceinline__ bool commit_vertex(const P& p, const Graph& gr, const RefineSweep& s, const Commit& x) {
+  const bool wants = x.wants >= 0;
   bool lost = false;
   if (wants) {
     const int32_t g = s.lc.graph_of.of(x.v);
@@ -1008,22 +1023,22 @@ template <bool FIRST>
 __global__ __launch_bounds__(HUB_THREADS, 8) void refine_commit_kernel(Graph gr, RefineSweep s,
                                                                        RowLists l) {
   __shared__ SweepShared sh;  // (the table stays out of use)
-  const bool done = refine_done(s.ctl, s.sweep);
+  if (refine_done(s.ctl, s.sweep)) return;
   bool moved = false;
   const int32_t hubs = l.counts[1], long_rows = hubs + l.counts[2];
   const Share share = mid_share(l);
   for (int32_t i = l.start(blockIdx.x); i < long_rows; i += l.long_blocks)
-    moved |= commit_vertex(Workgroup(sh), gr, s, done,
+    moved |= commit_vertex(Workgroup(sh), gr, s,
                   load_commit<FIRST>(gr, s, i < hubs ? l.rows[gr.V - 1 - i] : l.giants[i - hubs]));
   for (int32_t i = share.at; i < share.end; i += share.step)
-    moved |= commit_vertex(Wave(sh), gr, s, done, load_commit<FIRST>(gr, s, l.rows[i]));
+    moved |= commit_vertex(Wave(sh), gr, s, load_commit<FIRST>(gr, s, l.rows[i]));
   const Share mine = share_of(gr.V, l.first);
   const HalfWave p(sh);
   for (int32_t c = mine.at; c < mine.end; c += mine.step) {
     const int32_t v = c * GROUPS + (int32_t)(threadIdx.x >> 5);
     if (v >= gr.V) break;
     const Commit x = load_commit<FIRST>(gr, s, v);
-    if (x.b - x.a <= SMALL_ROW) moved |= commit_vertex(p, gr, s, done, x);
+    if (x.b - x.a <= SMALL_ROW) moved |= commit_vertex(p, gr, s, x);
   }
   mark_moved(mark_slot(s.ctl, false, s.sweep), moved);
 }
@@ -1188,13 +1203,14 @@ __global__ __launch_bounds__(GIANT_THREADS) void local_moving_giant_kernel(Graph
   __shared__ GiantShared sh;
   const int32_t count = l.counts[2];
   const MoveState st = move_state(s.ctl, s.sweep);
+  if (st.done) return;  // (handed on with the other rows)
   for (int32_t i = blockIdx.x; i < count; i += gridDim.x) {
     const int32_t v = l.giants[i];
     const int32_t old = FIRST ? v : s.lin[v];
     const int32_t g = v / gr.S;
     const double tm = gr.two_m[g];
     const double kv = gr.k_v[v];
-    if (st.done || !(tm > 0.0)) {
+    if (!(tm > 0.0)) {
       if (threadIdx.x == 0) finish_move(s, v, old, kv);
       continue;
     }

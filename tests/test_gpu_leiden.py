@@ -558,3 +558,27 @@ def test_run_leiden_graphs_without_edges_cost_little(device):
     alone, among = best_us(1), best_us(G)
     print(f"leiden one graph {alone:.0f} us, among {G} {among:.0f} us", flush=True)
     assert among < 8.0 * alone
+
+
+def test_run_leiden_sweeps_after_the_end_cost_little(device):
+    """Sweeps queued behind a phase's end leave the vertices alone: 64 sweeps of
+    a graph that settles in a few (30,000 leaves around one vertex, one
+    community in the end) take little longer than 8 (every vertex adding its
+    degree to that community's total once more a sweep: 5 times)."""
+    S = 30001
+    rng = np.random.default_rng(4)
+    s, d, w = _dev(device, np.zeros(S - 1, np.int32), np.arange(1, S, dtype=np.int32),
+                   (rng.integers(1, 64, S - 1) / 64.0).astype(np.float32))
+
+    def best_us(sweeps):
+        best = float("inf")
+        for _ in range(5):
+            t0 = time.perf_counter()
+            algorithm.run_leiden(s, d, w, G=1, seq_len=S, max_inner_iter=sweeps)
+            torch.cuda.synchronize()
+            best = min(best, (time.perf_counter() - t0) * 1e6)
+        return best
+
+    few, many = best_us(8), best_us(64)
+    print(f"leiden 8 sweeps {few:.0f} us, 64 sweeps {many:.0f} us", flush=True)
+    assert many < 2.5 * few

@@ -582,3 +582,24 @@ def test_run_leiden_sweeps_after_the_end_cost_little(device):
     few, many = best_us(8), best_us(64)
     print(f"leiden 8 sweeps {few:.0f} us, 64 sweeps {many:.0f} us", flush=True)
     assert many < 2.5 * few
+
+
+@pytest.mark.parametrize("S", [64, 127, 5000])
+def test_run_leiden_members_of_one_community(device, S):
+    """Members of a community counted and placed a wave at a time: whole waves of
+    one community, a few of it among others, fewer than are worth it, and a last
+    wave that is not full.  Labels equal the oracle's (dyadic weights)."""
+    rng = np.random.default_rng(S)
+    hubs = np.array([0, S // 2, S // 2 + 1])
+    home = np.where(np.arange(S) < S // 2, hubs[0], hubs[1 + (np.arange(S) % 16 == 0)])
+    pairs = {(min(a, b), max(a, b)) for a, b in zip(home.tolist(), range(S)) if a != b}
+    order = sorted(pairs)
+    src, dst = (np.array([p[i] for p in order], np.int32) for i in (0, 1))
+    w = (rng.integers(1, 64, src.size) / 64.0).astype(np.float32)
+    print(f"leiden members S={S}", flush=True)
+    s, d, x = _dev(device, src, dst, w)
+    vertex, part, q = algorithm.run_leiden(s, d, x, G=1, seq_len=S, max_inner_iter=6, seed=3)
+    rv, rp, rq = L.run_leiden(src, dst, w, graphs=1, seq_len=S, max_inner_iter=6, seed=3)
+    np.testing.assert_array_equal(vertex.cpu().numpy(), rv)
+    np.testing.assert_array_equal(part.cpu().numpy(), rp)
+    assert q == pytest.approx(rq, abs=1e-9)

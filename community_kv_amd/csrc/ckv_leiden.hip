@@ -1299,9 +1299,12 @@ __global__ __launch_bounds__(GIANT_THREADS) void refine_propose_giant_kernel(Gra
     int32_t thr;
     double e_sum;
     auto community_of = [&](int32_t u) {
-      if constexpr (FIRST) return s.parent[u] == pv ? u : -1;
-      const int2 q = FIRST ? int2{} : s.lin[u];
-      return q.x == pv ? q.y : -1;
+      if constexpr (FIRST) {
+        return s.parent[u] == pv ? u : -1;
+      } else {
+        const int2 q = s.lin[u];
+        return q.x == pv ? q.y : -1;
+      }
     };
     if (!giant_table(gr, community_of, v, a, b, sh, &thr, &e_sum)) {  // cannot happen: stay, flagged
       propose(old);

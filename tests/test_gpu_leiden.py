@@ -603,3 +603,68 @@ def test_run_leiden_members_of_one_community(device, S):
     np.testing.assert_array_equal(vertex.cpu().numpy(), rv)
     np.testing.assert_array_equal(part.cpu().numpy(), rp)
     assert q == pytest.approx(rq, abs=1e-9)
+
+
+@pytest.mark.parametrize("ordered", [True, False])
+@pytest.mark.parametrize("S", [32760, 32761, 40000])
+def test_sweeps_on_both_sides_of_the_grid_split(device, S, ordered):
+    """Up to 4,095 chunks of eight vertices the long rows have workgroups of
+    their own, from 4,096 on every workgroup takes hubs, mids and chunks in turn
+    from one table: rows of each class among short ones, several chunks a
+    workgroup, on ascending and on shuffled lists; one level's labels equal the
+    oracle's (dyadic weights: every sum exact)."""
+    rng = np.random.default_rng(S)
+    a = rng.integers(0, S, 3 * S)
+    b = np.clip(a + rng.integers(1, 40, a.size), 0, S - 1)
+    long_rows = [(129, 40), (200, 40), (256, 20), (257, 20), (600, 30), (1023, 10), (1025, 4), (3000, 2)]
+    heads = rng.choice(S, sum(n for _, n in long_rows), replace=False)
+    at = 0
+    for length, many in long_rows:
+        for v in heads[at:at + many]:
+            a = np.concatenate([a, np.full(length, v)])
+            b = np.concatenate([b, rng.choice(S, length, replace=False)])
+        at += many
+    key = np.unique((np.minimum(a, b) * S + np.maximum(a, b))[a != b])
+    if not ordered:
+        key = rng.permutation(key)
+    src, dst = (key // S).astype(np.int32), (key % S).astype(np.int32)
+    w = (rng.integers(1, 64, key.size) / 64.0).astype(np.float32)
+    print(f"leiden grid split S={S} edges={key.size} ordered={ordered}", flush=True)
+    s, d, x = _dev(device, src, dst, w)
+    kw = dict(seq_len=S, max_level=1, max_inner_iter=3, seed=5)
+    vertex, part, _ = algorithm.run_leiden(s, d, x, G=1, **kw)
+    rv, rp, _ = L.run_leiden(src, dst, w, graphs=1, **kw)
+    np.testing.assert_array_equal(vertex.cpu().numpy(), rv)
+    np.testing.assert_array_equal(part.cpu().numpy(), rp)
+
+
+def test_native_run_applies_environment_overrides(device, monkeypatch):
+    """The reference's environment variables reach the native run (sweeps and
+    temperature of the noise, and the noise itself)."""
+    src, dst, w = lg.planted(7, 2, 600, 9)
+    s, d, x = _dev(device, src, dst, w)
+    kw = dict(G=2, seq_len=600, seed=3)
+    explicit = algorithm.run_leiden(s, d, x, max_inner_iter=2, theta=0.5, use_boltzmann=True, **kw)
+    plain = algorithm.run_leiden(s, d, x, **kw)
+    monkeypatch.setenv("COMMUNITY_KV_LEIDEN_MAX_INNER_ITER", "2")
+    monkeypatch.setenv("COMMUNITY_KV_LEIDEN_THETA", "0.5")
+    monkeypatch.setenv("COMMUNITY_KV_LEIDEN_BOLTZMANN", "1")
+    got = algorithm.run_leiden(s, d, x, **kw)
+    assert torch.equal(got[1], explicit[1]) and got[2] == explicit[2]
+    assert plain[1].shape != got[1].shape or not torch.equal(plain[1], got[1])
+
+
+@pytest.mark.parametrize("dyadic", [True, False])
+def test_partition_modularity_of_an_edge_list(device, dyadic):
+    """ckv_partition_modularity (any labels, any edge order) against the same
+    formula in float64 on the host: sums of some 10^4 f64 terms."""
+    src, dst, w = lg.planted(11, 2, 900, 14, self_loops=5, isolated=20, dyadic=dyadic)
+    rng = np.random.default_rng(1)
+    order = rng.permutation(src.size)
+    src, dst, w = src[order], dst[order], w[order]
+    lab = rng.integers(0, 30, 1800).astype(np.int32)
+    print(f"partition modularity edges={src.size}", flush=True)
+    s, d, x, l = _dev(device, src, dst, w, lab)
+    got = algorithm._compute_disjoint_modularity(s, d, x, l, 1.25)
+    ref = algorithm._compute_disjoint_modularity(*(torch.from_numpy(a) for a in (src, dst, w, lab)), 1.25)
+    assert got == pytest.approx(ref, abs=1e-12)

@@ -285,15 +285,16 @@ def test_state_build_degree_weights_any_edge_order(device, graphs, seq_len, n, o
     np.testing.assert_array_equal(st.community_weight.cpu().numpy(), by_label)
 
 
-@pytest.mark.parametrize("count,extra", [(8186, 6), (8186, 7)])
+@pytest.mark.parametrize("count,extra", [(8186, 6), (8186, 7), (8192, 3), (8193, 3), (16384, 3), (16385, 3), (19000, 3)])
 def test_state_build_topk_many_communities(device, count, extra):
-    """Capacities on both sides of the line between sums in doubles and in
-    floats (8,192 communities), against the float64 closed form: some 10 float
-    terms a community, so 1e-5 relative."""
+    """Community counts on both sides of the line between sums in doubles and in
+    floats (8,192 communities, 64 KB of LDS either way) and of the one above
+    which the rest is added in global memory (16,384), against the float64
+    closed form: some 10 float terms a community, so 1e-5 relative."""
     from community_kv_amd.graph.kernels.state_build import TopkEdges
 
     rng = np.random.default_rng(count + extra)
-    seq_len, num_sink, kappa, lam = 9000, 2, 8, 0.5
+    seq_len, num_sink, kappa, lam = 9000 if count < 9000 else 20000, 2, 8, 0.5
     row0 = num_sink + kappa - 1
     rows = seq_len - row0
     ids = rng.integers(0, count, (1, seq_len)).astype(np.int32)

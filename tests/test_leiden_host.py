@@ -157,3 +157,52 @@ def test_run_leiden_raises_on_flagged_table_overflow(monkeypatch):
     with pytest.raises(RuntimeError, match="overflowed"):
         algorithm.run_leiden(torch.tensor([0], dtype=torch.int32), torch.tensor([1], dtype=torch.int32),
                              torch.ones(1), G=1, seq_len=2, max_level=1)
+
+
+class _FakeRun:
+    """ckv_leiden_run's place: notes its arguments and fails as told."""
+
+    def __init__(self, rc=0, message=b""):
+        self.rc, self.message, self.calls = rc, message, []
+
+    def ckv_leiden_run_workspace_bytes(self, edges, graphs, seq_len):
+        return 64
+
+    def ckv_leiden_run(self, *args):
+        self.calls.append(args)
+        return self.rc
+
+    def ckv_last_error(self):
+        return self.message
+
+
+def _native_run_on(monkeypatch, fake, **kw):
+    monkeypatch.setattr(algorithm.nat, "lib", lambda: fake)
+    monkeypatch.setattr(algorithm.nat, "require_device", lambda *t: torch.device("cpu"))
+    monkeypatch.setattr(algorithm.nat, "stream_handle", lambda device: 0)
+    edges = (torch.tensor([0], dtype=torch.int32), torch.tensor([1], dtype=torch.int32), torch.ones(1))
+    return algorithm.native_run(*edges, G=1, seq_len=4, max_level=2, resolution=1.0, seed=0, **kw)
+
+
+def test_native_run_takes_the_options_after_overrides(monkeypatch):
+    """What the environment leaves of the options is what ckv_leiden_run is given."""
+    ka = GOLDEN["leiden_env_overrides"]
+    for k, v in ka["env"].items():
+        monkeypatch.setenv(k, v)
+    theta, sweeps, boltzmann = algorithm.leiden_options(0.01, 16, False)
+    assert (theta, sweeps, boltzmann) == (ka["theta"], ka["max_inner_iter"], True)
+    fake = _FakeRun()
+    _native_run_on(monkeypatch, fake, theta=theta, max_inner_iter=sweeps, use_boltzmann=boltzmann)
+    args = fake.calls[0]
+    assert args[3:7] == (1, 1, 4, 2) and args[8] == ka["theta"] and args[9] == ka["max_inner_iter"] and args[11] == 1
+
+
+@pytest.mark.parametrize("rc,message,error,match", [
+    (1, b"edges must join two vertices of the same graph", ValueError, "same graph"),
+    (2, b"a neighbour-community table overflowed; the labels are not valid", RuntimeError, "Leiden: .*overflowed"),
+    (2, b"Leiden graph too large (vertices < 2^30, 2 * edges < 2^31)", RuntimeError, "too large"),
+])
+def test_native_run_errors(monkeypatch, rc, message, error, match):
+    """Errors of the native run reach the caller as the level loop's did."""
+    with pytest.raises(error, match=match):
+        _native_run_on(monkeypatch, _FakeRun(rc, message), theta=0.01, max_inner_iter=4, use_boltzmann=False)

@@ -424,6 +424,16 @@ __global__ __launch_bounds__(64 * WAVES) void gather_kernel(TopkGraph t, const u
   }
 }
 
+// A workgroup's first item is its own number, the next ones are taken in turn
+// (all threads call).  With a ticket for the first one too, 1,280 workgroups
+// queued 15 us for one word, in calls with nothing to do for them as well.
+__device__ inline int32_t next_ticket(int32_t* word, int* s_ticket) {
+  __syncthreads();
+  if (threadIdx.x == 0) *s_ticket = (int32_t)gridDim.x + atomicAdd(word, 1);
+  __syncthreads();
+  return *s_ticket;
+}
+
 // One workgroup per part of a split run and per long run (taken in turn by a
 // ticket: their lengths differ by a hundredfold).  A part's neighbours gather
 // in the LDS table as far as BIG_MOST of them go (the ones that many rows name
@@ -451,11 +461,7 @@ __global__ __launch_bounds__(BIG_THREADS) void gather_big_kernel(
   const int32_t split = lists[LIST_PARTS], listed = split + lists[LIST_LONG];
   const int words = t.S <= 32 * MAP_WORDS ? (t.S + 31) >> 5 : 0;
   uint32_t* before_s = map_s + words;
-  while (true) {
-    if (tid == 0) s_ticket = atomicAdd(lists + LIST_TICKET, 1);
-    __syncthreads();
-    const int32_t it = s_ticket;
-    if (it >= listed) return;
+  for (int32_t it = (int32_t)blockIdx.x; it < listed; it = next_ticket(lists + LIST_TICKET, &s_ticket)) {
     if (it < split) {
       const Part part = parts[it];
       const int32_t v = (int32_t)keys[part.run];
@@ -668,12 +674,7 @@ __global__ __launch_bounds__(DENSE_THREADS) void gather_dense_kernel(
   constexpr int OWN = MAP_WORDS / DENSE_THREADS;  // consecutive words of a thread
   const int tid = threadIdx.x, wv = tid >> 6;
   const int32_t split = lists[LIST_SPLIT], listed = split + lists[LIST_DENSE];
-  while (true) {
-    if (tid == 0) s_ticket = atomicAdd(lists + LIST_DENSE_TICKET, 1);
-    __syncthreads();
-    const int32_t it = s_ticket;
-    __syncthreads();
-    if (it >= listed) return;
+  for (int32_t it = (int32_t)blockIdx.x; it < listed; it = next_ticket(lists + LIST_DENSE_TICKET, &s_ticket)) {
     if (it < split) {
       constexpr int U = 4;
       const uint32_t a = split_runs[it].first;
@@ -1027,6 +1028,11 @@ extern "C" int ckv_build_adjacency(const int32_t* topk_indices, const float* top
   int32_t* lists = (int32_t*)(ws + L.lists);
   uint32_t* tmp_id = (uint32_t*)(ws + L.tmp_id);
   float* tmp_w = (float*)(ws + L.tmp_w);
+  // A vertex has fewer neighbours than its graph has vertices; in a graph small
+  // enough for every table runs are split, and that launch paid for (5 us of
+  // some 200), where it has rows enough to make one workgroup long.
+  const bool heavy = seq_len > BIG_MOST || (int64_t)rows * (kappa + 1) >= 16 * SPLIT_MIN;
+  const uint32_t split_min = heavy ? split_length(seq_len, kappa) : UINT32_MAX;
   auto gather = [&](auto width) -> int {
     constexpr int KT = decltype(width)::value;
     posting_kernel<KT><<<blocks_for((int64_t)graphs * rows, THREADS), THREADS, 0, st>>>(t, keys_in, vals_in, lists);
@@ -1034,15 +1040,14 @@ extern "C" int ckv_build_adjacency(const int32_t* topk_indices, const float* top
         hipSuccess)
       return ckv_internal::set_error(CKV_E_LAUNCH, "posting sort failed");
     list_kernel<<<blocks_for(n, LIST_GROUPS * LIST_THREADS), LIST_THREADS, 0, st>>>(
-        keys, (uint32_t)n, (uint32_t)V, (uint32_t)(WAVE_CANDIDATES / kappa), split_length(seq_len, kappa), count,
+        keys, (uint32_t)n, (uint32_t)V, (uint32_t)(WAVE_CANDIDATES / kappa), split_min, count,
         short_runs, long_runs, split_runs, parts, lists);
     gather_kernel<KT><<<WAVE_BLOCKS, 64 * WAVES, 0, st>>>(t, keys, vals, short_runs, split_runs, lists, count, tmp_id,
                                                          tmp_w);
     const size_t map_bytes = seq_len <= 32 * MAP_WORDS ? (size_t)((seq_len + 31) / 32) * 8 : 0;
     gather_big_kernel<KT><<<BIG_BLOCKS, BIG_THREADS, map_bytes, st>>>(t, keys, vals, long_runs, parts, dense, lists,
                                                                       count, tmp_id, tmp_w);
-    // (a vertex has fewer neighbours than its graph has vertices, and postings than its rows have entries)
-    if (seq_len > BIG_MOST || (int64_t)rows * (kappa + 1) >= SPLIT_MIN) {
+    if (heavy) {
       const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gather_dense_kernel<KT>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)dense_lds_bytes());
       if (e != hipSuccess) {

@@ -2868,7 +2868,8 @@ extern "C" int ckv_dense_communities(const int32_t* labels, int32_t graphs, int3
   if (!labels || !community_ids || !community_counts || !workspace || graphs <= 0 || seq_len <= 0 || width < 0)
     return ckv_internal::set_error(CKV_E_INVALID, "bad community arguments");
   const int64_t n = (int64_t)graphs * ((int64_t)seq_len + width);
-  if (n >= (int64_t)1 << 30) return ckv_internal::set_error(CKV_E_LIMIT, "too many vertices and labels");
+  if ((int64_t)graphs * seq_len >= (int64_t)1 << 30 || (int64_t)graphs * width >= (int64_t)1 << 30)
+    return ckv_internal::set_error(CKV_E_LIMIT, "too many vertices or labels (each below 2^30, as a run's are)");
   hipStream_t st = (hipStream_t)stream;
   int32_t* words = (int32_t*)workspace;
   int32_t* scan = (int32_t*)((char*)workspace + align256((size_t)n * 4));

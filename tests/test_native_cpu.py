@@ -200,3 +200,13 @@ def test_config_validation():
         CommunityKVConfig(assignment="kmeans")
     cfg = CommunityKVConfig(aggregation="query_group", local_window=128)
     assert cfg.aggregation.value == "query_group"
+
+
+@pytest.mark.parametrize("graphs,seq_len,width", [(1 << 10, 1 << 20, 0), (1, 5, 1 << 30), (3, 1 << 29, 7)])
+def test_dense_communities_limits(lib, graphs, seq_len, width):
+    """The relabelling after a run takes every run's vertices (below 2^30) with
+    as many labels, and refuses more before anything is queued (the pointers are
+    never read)."""
+    rc = lib.ckv_dense_communities(256, graphs, seq_len, width, 256, 256, 256, 0)
+    assert rc != 0 and b"2^30" in lib.ckv_last_error()
+    assert lib.ckv_dense_communities_workspace_bytes(1, (1 << 30) - 1, (1 << 30) - 1) >= 2 * 4 * ((1 << 31) - 2)

@@ -463,9 +463,9 @@ def run_partition(args, device):
     """Prefill partition of one config-2 layer (the second 'next' row): the
     top-8 edges of all 32 query heads from the prefill kernel on planted
     config-5 style inputs (32,768 tokens, 256 clusters), grouped into 8
-    QUERY_GROUP graphs, then ``partition_graphs``: build_adjacency (device
-    torch ops), native multi-level Leiden (ckv_batched_leiden /
-    ckv_aggregate_coo / ckv_densify_*), isolated fill and dense remap.  The
+    QUERY_GROUP graphs, then ``partition_graphs``: the coalesced graph
+    (ckv_build_adjacency), native multi-level Leiden (ckv_leiden_run) and the
+    dense relabelling (ckv_dense_communities).  The
     timed region is the whole partition; the Leiden part is timed alone too."""
     from community_kv_amd.attention.flash_attention import prefill_attention_topk
     from community_kv_amd.graph import partition as P

@@ -635,8 +635,8 @@ __global__ __launch_bounds__(BIG_THREADS) void gather_big_kernel(
 // thousand neighbours eight times at 131,072 positions.
 //
 // The whole graph of 32 heads in 8 graphs at 131,072 positions, columns drawn by
-// a power law: 9.1 ms; planted columns and one that all rows name 5.5, with all
-// heads in one graph 7.9; at 32,768 positions 1.4 and 1.2.  (Every run on one
+// a power law: 9.2 ms; planted columns and one that all rows name 5.6, with all
+// heads in one graph 8.1; at 32,768 positions 1.4 and 1.3.  (Every run on one
 // workgroup: 26.4 ms, 30.9, 207; 3.5, 16.1.  The sort of all entries that the
 // gathering replaced: 11.5, 11.4, 9.7; 2.7, 2.2.)
 constexpr size_t dense_lds_bytes() { return DENSE_SUMS * 8 + MAP_WORDS * 8; }

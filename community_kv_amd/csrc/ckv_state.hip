@@ -546,7 +546,8 @@ constexpr int REST_EARLY_PER_GRAPH = 192, REST_EARLY_MOST = 4096;
 constexpr int ORDER_MOST = 1024;  // words a workgroup reads to know what was found
 
 __global__ __launch_bounds__(EDGE_THREADS) void edge_order_kernel(const int32_t* __restrict__ src, int64_t edges,
-                                                                  int seq_len, int64_t vertices, int* __restrict__ found) {
+                                                                  int seq_len, int64_t vertices,
+                                                                  int* __restrict__ found) {
   constexpr int U = 8;
   const int64_t step = (int64_t)gridDim.x * EDGE_THREADS;
   bool loose = false;

@@ -180,7 +180,8 @@ def build_layer_state(community_ids: torch.Tensor, keys: torch.Tensor, *, retrie
     does with ``.item()``.  ``count_sink_labels`` counts communities over all
     positions (sinks included) instead of the non-sink ones;
     ``vertex_degree`` (f64, one per graph and position, of the graph of
-    ``edges``) saves the pass over the edges' labels where it is known.  (The workspace and edge copies return to the
+    ``edges``, whose order is free) saves the pass over the edges' labels where
+    it is known.  (The workspace and edge copies return to the
     caching allocator on this stream, so later work on it cannot overwrite
     them before the launches run.)"""
     return StateBuild(community_ids, keys, retrieval_to_graph=retrieval_to_graph, retrieval_to_kv=retrieval_to_kv,

@@ -4,8 +4,9 @@
 Device edges run ``ckv_leiden_run``: every level's local moving, refinement,
 densified labels and contraction on the device, one small read back per level.
 The extension's entry points (``batched_leiden``, ``aggregate_coo``) stay
-available one by one (``_load_module``); over host tensors ``run_leiden`` is
-the reference's own level loop around them.
+available one by one (``_load_module``) and take device tensors; over host
+tensors ``run_leiden`` is the reference's own level loop around whatever
+``_load_module`` returns.
 """
 
 from __future__ import annotations

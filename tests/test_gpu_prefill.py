@@ -222,4 +222,4 @@ def test_prefill_odd_lengths_keep_pace(device):
     assert odd < 1.5 * even
     once, twice = us(2048, 32, 8), us(4096, 32, 8)
     print(f"prefill 2,048 / 4,096 positions {once:.0f} / {twice:.0f} us", flush=True)
-    assert twice < 2.5 * once
+    assert twice < 2.7 * once
